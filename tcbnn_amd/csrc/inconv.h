@@ -1,0 +1,25 @@
+// What the first layer's kernels share: the problem and the matrix-core kernel's entry points.
+#pragma once
+
+#include "common.h"
+
+namespace tcbnn {
+
+struct InConvParams {
+    const float* in;       // [B][3][H][W]
+    const uint4* masks;    // [taps][opad32] {m0, m1, m2, pattern}, then the patterns alone: uint32 [taps][opad32]
+    const float* bn;
+    uint32_t* out;         // [OH][OW][ow][B]
+    int32_t* res;          // residual tensor in format res_fmt, or null
+    int res_fmt;           // TCBNN_RES_*
+    int H, W, B, O, opad, ow;
+    int R, S, stride_h, stride_w, pad_h, pad_w;
+    int PH, PW, pool_h, pool_w, OH, OW;
+};
+
+// First layer on the matrix cores (inconv_mfma.hip): whether it serves a problem, its launch, its kernel's name.
+bool inconv_mfma_applicable(const InConvParams& p);
+int launch_inconv_mfma(const InConvParams& p, hipStream_t stream);
+void inconv_mfma_kernel_name(const InConvParams& p, char* buf, size_t len);
+
+}  // namespace tcbnn

@@ -23,7 +23,7 @@
 
 #include <type_traits>
 
-#include "common.h"
+#include "inconv.h"
 
 namespace tcbnn {
 namespace {
@@ -32,18 +32,6 @@ constexpr int kThreads = 256;
 constexpr int kXT = 4;        // output columns per workgroup (one per wave)
 constexpr int kLB = 65;       // LDS row pitch in floats for 64 images (+1 against conflicts)
 constexpr int kMaxCols = 32;  // (kXT-1)*stride + S must fit
-
-struct InConvParams {
-    const float* in;       // [B][3][H][W]
-    const uint4* masks;    // [taps][opad32] {m0, m1, m2, 0}
-    const float* bn;
-    uint32_t* out;         // [OH][OW][ow][B]
-    int32_t* res;          // residual tensor in format res_fmt, or null
-    int res_fmt;           // TCBNN_RES_*
-    int H, W, B, O, opad, ow;
-    int R, S, stride_h, stride_w, pad_h, pad_w;
-    int PH, PW, pool_h, pool_w, OH, OW;
-};
 
 __device__ __forceinline__ float flip(float f, uint32_t m) {
     return __uint_as_float(__float_as_uint(f) ^ m);
@@ -820,6 +808,12 @@ static int inconv128_run(const tcbnn_inconv128_desc* d, void* stream, char* name
         return TCBNN_OK;
     }
     TCBNN_REQUIRE(d->input_layout == TCBNN_INCONV_INPUT_NCHW, "inconv128: unknown input_layout");
+    // 3-, 7- and 11-row filters on 32- or 64-channel tiles: matrix cores (inconv_mfma.hip says what it serves and why)
+    if (!force_linear && inconv_mfma_applicable(p)) {
+        if (name_buf == nullptr) return launch_inconv_mfma(p, (hipStream_t)stream);
+        inconv_mfma_kernel_name(p, name_buf, name_len);
+        return TCBNN_OK;
+    }
     if (name_buf != nullptr) {  // report the kernel instead of launching it
         if (!tiled) {
             snprintf(name_buf, name_len, "inconv_generic_kernel");

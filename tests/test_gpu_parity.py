@@ -885,6 +885,55 @@ def test_inconv128_linear_staging(gpu):
     assert proc.returncode == 0 and "linear staging ok" in proc.stdout, proc.stdout
 
 
+@pytest.mark.parametrize("b,h,w,R,S,stride,cout,pool,save,fmt,kind", [
+    # batches around the images of a tile, one image, ragged strips and bands, several channel groups, every stride class
+    (1, 224, 224, 7, 7, 4, 64, 1, True, None, "normal"), (5, 20, 20, 7, 7, 4, 64, 1, True, None, "normal"),
+    (9, 50, 70, 7, 5, 2, 128, 1, True, None, "normal"), (32, 64, 64, 7, 7, 2, 64, 1, False, None, "normal"),
+    (33, 30, 31, 3, 3, 1, 64, 1, True, None, "normal"), (40, 9, 13, 3, 4, 1, 192, 1, True, None, "normal"),
+    (8, 26, 26, 3, 3, 2, 64, 1, False, None, "normal"), (3, 60, 224, 11, 11, 4, 64, 2, False, None, "normal"),
+    (70, 24, 24, 11, 11, 4, 96, 2, False, None, "normal"),
+    (16, 40, 40, 7, 7, 4, 64, 1, True, 0, "normal"), (16, 40, 40, 7, 7, 4, 64, 1, True, 1, "normal"),
+    (16, 40, 40, 3, 3, 1, 64, 1, True, 0, "normal"), (16, 40, 40, 3, 3, 1, 64, 1, True, 2, "normal"),
+    # values that are all recomputed (outside fp16, below its steps, windows with NaN and infinity), sums that are whole
+    # numbers, windows of zeros, sums as large as the sum of |x|
+    (16, 40, 40, 7, 7, 4, 64, 1, True, None, "huge"), (16, 40, 40, 7, 7, 4, 64, 1, True, None, "tiny"),
+    (16, 40, 40, 7, 7, 4, 64, 1, True, None, "special"), (34, 60, 60, 11, 11, 4, 64, 2, False, None, "special"),
+    (34, 40, 40, 7, 7, 4, 64, 1, True, None, "whole"), (34, 33, 31, 3, 3, 1, 64, 1, True, None, "whole"),
+    (16, 40, 40, 7, 7, 4, 64, 1, True, None, "zeros"), (16, 40, 40, 7, 7, 4, 64, 1, True, None, "positive"),
+    (16, 20, 20, 3, 3, 1, 64, 1, False, None, "positive"), (16, 60, 60, 11, 11, 4, 64, 2, False, None, "positive")])
+def test_inconv128_matrix_cores(gpu, b, h, w, R, S, stride, cout, pool, save, fmt, kind):
+    """The first layer's matrix-core kernel gives the bits and residuals of the reference's order of additions."""
+    r = rng(b + h + R + cout)
+    x = r.standard_normal((b, 3, h, w)).astype(np.float32)
+    f = rm.pm1(r, (R, S, 3, cout))
+    bn = r.normal(0, np.sqrt(3 * R * S), cout).astype(np.float32)
+    bn[:7] = [0.0, -0.0, 1e-30, -1e-30, np.nan, np.inf, -np.inf]
+    if kind == "huge":
+        x *= 3e4
+    elif kind == "tiny":
+        x *= 1e-7
+    elif kind == "special":
+        x[0, 0, h // 2, w // 2], x[-1, 2, 0, 0], x[b // 2, 1, h - 1, w - 1] = np.nan, np.inf, -1e30
+    elif kind == "whole":
+        x = np.rint(x * 80).clip(-255, 255).astype(np.float32)
+    elif kind == "zeros":
+        x[:, :, :h // 2] = 0
+    elif kind == "positive":
+        x = np.abs(x)
+        f[..., :cout // 2] = 1
+        bn[7:cout // 2] += 3 * R * S * 0.8
+    want, wres = orc.inconv128(x, f, bn, stride, True, pool, save)
+    layer = gpu.InConv128LayerParam("Conv1", h, w, R, S, 3, cout, b, stride, stride, True, pool, pool, save, residual_format=fmt)
+    layer.initialize(x, gpu.ArrayWeights([f, bn]))
+    assert "mfma" in layer.kernel_name(), layer.kernel_name()
+    layer.forward()
+    gpuops.sync()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    if save:
+        np.testing.assert_array_equal(layer.download_residual(), wres)
+    layer.release()
+
+
 def test_inconv128_special_thresholds(gpu):
     """NaN, +-inf and exactly met thresholds in the first layer (kernel.cuh:655: bit = !(acc < bn))."""
     r = rng(321)
