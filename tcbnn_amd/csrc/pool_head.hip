@@ -1,6 +1,8 @@
 // Layers of the textbook ResNet wiring that the reference's drivers do not have: overlapping
 // OR / max pooling of a packed activation tensor with its residual, and the global-average-pool +
 // fp32 fully connected head.  Both are bound by HBM (one pass over their input).
+#include <algorithm>
+
 #include "common.h"
 
 namespace tcbnn {
@@ -83,111 +85,236 @@ __global__ __launch_bounds__(kThreads) void pool128_kernel(const PoolParams p) {
     reinterpret_cast<int4*>(p.rout)[((size_t)opix * p.groups + g) * p.B + b] = m;
 }
 
+// ---- 3x3 window, stride 2 (the textbook wiring's only pooling layer) -------------------------------------------------
+// A 12-bit residual's maximum is taken on packed 16-bit halves that hold a value each in their upper 12 bits; whatever
+// lies in the lower four only decides between equal values.
+typedef short v2s __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t max2x16(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(v2s, a), __builtin_bit_cast(v2s, b)));
+}
+// words w0..w2 of eight 12-bit values -> four pairs, and back
+__device__ __forceinline__ void i12_to_pairs(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t* q) {
+    constexpr uint32_t kLow = 0x0000ffffu;
+    auto pair = [](uint32_t low_at_4, uint32_t high_at_20) { return (low_at_4 & kLow) | (high_at_20 & ~kLow); };
+    q[0] = pair(w0 << 4, w0 << 8);
+    q[1] = pair(__builtin_amdgcn_alignbit(w1, w0, 20), w1 << 16);
+    q[2] = pair(w1 >> 12, __builtin_amdgcn_alignbit(w2, w1, 8));
+    q[3] = pair(w2 >> 4, w2);
+}
+__device__ __forceinline__ void i12_from_pairs(const uint32_t* q, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
+    int v[8];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        v[2 * k] = (int)(q[k] >> 4);
+        v[2 * k + 1] = (int)(q[k] >> 20);
+    }
+    i12_pack8(v, w0, w1, w2);
+}
+
+// A thread takes one unit (word of bits, or residual group) of one image and walks down `rows` output pixels of a
+// column: of the three input rows of a window the last is the next window's first, so an output costs six loads and not
+// nine, all of them in flight together.  Bound by HBM: 417 MB at 112x112, 64 channels, 12 bits, batch 256, in 86 us
+// (104 us with nine loads and a 64-bit division per output).
+template <int FMT>
+__global__ __launch_bounds__(kThreads) void pool3x3s2_kernel(const PoolParams p, int rows) {
+    const int rem = (int)(blockIdx.x * kThreads + threadIdx.x);
+    if (rem >= (p.cw + p.groups) * p.B) return;
+    const int u = rem / p.B, b = rem - u * p.B;
+    const int ox = blockIdx.y, x0 = ox * 2 - p.pad;
+    const int oy0 = blockIdx.z * rows, oy1 = min(p.OH, oy0 + rows);
+    // columns outside the frame repeat one inside it (padding < window: there is one)
+    int xs[3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) xs[s] = min(max(x0 + s, max(x0, 0)), min(x0 + 2, p.W - 1));
+    auto row_of = [&](int y) { return (size_t)y * p.W; };
+    if (u < p.cw) {  // OR of the window's words
+        const uint32_t* __restrict__ const src = p.in + (size_t)u * p.B + b;
+        const size_t px = (size_t)p.cw * p.B;
+        auto row = [&](int y) {
+            uint32_t v = 0u;
+            if (y >= 0 && y < p.H)
+#pragma unroll
+                for (int s = 0; s < 3; ++s) v |= src[(row_of(y) + xs[s]) * px];
+            return v;
+        };
+        uint32_t last = row(oy0 * 2 - p.pad);
+        for (int oy = oy0; oy < oy1; ++oy) {
+            const int y = oy * 2 - p.pad;
+            const uint32_t mid = row(y + 1), next = row(y + 2);
+            p.out[(((size_t)oy * p.OW + ox) * p.cw + u) * p.B + b] = last | mid | next;
+            last = next;
+        }
+        return;
+    }
+    const int g = u - p.cw;
+    constexpr int kQ = FMT == TCBNN_RES_I12 ? 8 : 4;  // registers of a group: pairs, or the four words
+    struct Group {
+        uint32_t q[kQ];
+    };
+    auto most = [](const Group& a, const Group& c) {
+        Group m;
+#pragma unroll
+        for (int k = 0; k < kQ; ++k)
+            m.q[k] = FMT == TCBNN_RES_I32 ? (uint32_t)max((int)a.q[k], (int)c.q[k]) : max2x16(a.q[k], c.q[k]);
+        return m;
+    };
+    auto load = [&](size_t pix) {
+        Group r;
+        if constexpr (FMT == TCBNN_RES_I12) {
+            const uint32_t* const w = reinterpret_cast<const uint32_t*>(p.rin);
+            const uint4 a = *reinterpret_cast<const uint4*>(w + i12_word_index(pix, (size_t)p.groups, g, p.B, b, 0));
+            const uint2 c = *reinterpret_cast<const uint2*>(w + i12_word_index(pix, (size_t)p.groups, g, p.B, b, 4));
+            i12_to_pairs(a.x, a.y, a.z, r.q);
+            i12_to_pairs(a.w, c.x, c.y, r.q + 4);
+        } else {
+            const uint4 a = reinterpret_cast<const uint4*>(p.rin)[(pix * p.groups + g) * p.B + b];
+            r.q[0] = a.x, r.q[1] = a.y, r.q[2] = a.z, r.q[3] = a.w;
+        }
+        return r;
+    };
+    auto row = [&](int y) { return most(most(load(row_of(y) + xs[0]), load(row_of(y) + xs[1])), load(row_of(y) + xs[2])); };
+    // (rows outside the frame repeat the nearest row inside, which is in the window: padding < window)
+    auto clamped = [&](int y, int oy) { return min(max(y, max(0, oy * 2 - p.pad)), min(p.H - 1, oy * 2 - p.pad + 2)); };
+    Group last = row(clamped(oy0 * 2 - p.pad, oy0));
+    for (int oy = oy0; oy < oy1; ++oy) {
+        const int y = oy * 2 - p.pad;
+        const Group mid = row(clamped(y + 1, oy)), next = row(clamped(y + 2, oy));
+        const Group m = most(most(last, mid), next);
+        const size_t pix = (size_t)oy * p.OW + ox;
+        if constexpr (FMT == TCBNN_RES_I12) {
+            uint32_t* const w = reinterpret_cast<uint32_t*>(p.rout);
+            uint32_t d[6];
+            i12_from_pairs(m.q, d[0], d[1], d[2]);
+            i12_from_pairs(m.q + 4, d[3], d[4], d[5]);
+            *reinterpret_cast<uint4*>(w + i12_word_index(pix, (size_t)p.groups, g, p.B, b, 0)) = make_uint4(d[0], d[1], d[2], d[3]);
+            *reinterpret_cast<uint2*>(w + i12_word_index(pix, (size_t)p.groups, g, p.B, b, 4)) = make_uint2(d[4], d[5]);
+        } else {
+            reinterpret_cast<uint4*>(p.rout)[(pix * p.groups + g) * p.B + b] = make_uint4(m.q[0], m.q[1], m.q[2], m.q[3]);
+        }
+        last = next;
+    }
+}
+
 struct HeadParams {
     const int32_t* rin;
     const float* w;
     const float* bias;
     float* out;
-    int P, C, B, N, groups, per_group, fmt;  // P = pixels
+    int P, C, B, N, groups, fmt;  // P = pixels
 };
 
 constexpr int kHeadImages = 8;     // images per workgroup
-constexpr int kHeadOutputs = 256;  // outputs per workgroup (one per thread)
+constexpr int kHeadOutputs = 128;  // outputs per workgroup: a thread takes one of them for four of the images
 constexpr int kHeadMaxC = 512;
+constexpr int kHeadChunk = 64;     // channels whose weights are in flight at a time
 
-// Workgroup = 8 images x 256 outputs.  Phase 1: the means of the 8 images, all channels, into LDS.
-// Phase 2: thread = output; per channel one coalesced weight load and eight fused multiply-adds on
-// means that every lane reads from the same LDS address (broadcast); channels in ascending order.
-__global__ __launch_bounds__(kThreads) void avgpool_fc_kernel(const HeadParams p) {
+// Workgroup = 8 images x 128 outputs.  Phase 1: the means of the 8 images, all channels, into LDS.  Phase 2: a thread
+// takes one output of four images; per channel one coalesced weight load (the workgroup's other half finds it in L1) and
+// four fused multiply-adds on means that every lane reads from the same LDS address; channels in ascending order.
+// Everything here is latency: a dependent chain of C multiply-adds (8 k cycles for 512 channels and four images at one
+// wave per SIMD) behind two trips to memory and the fetch of the code itself, which runs once.  So the grid is as many
+// workgroups as CUs at batch 256, all pixels of a 7x7 map are requested together, weights run 64 channels ahead, LDS reads
+// eight; and addresses advance on the scalar unit (wave-uniform base + lane offset) to keep the unrolled code short.
+// (8 images per thread, 8 pixels and 16 channels ahead, 128 workgroups, sums in a dynamically indexed array: 67 us at batch
+// 256 and at batch 20 alike; now 22 and 21 us for 7x7x512 -> 1000.)
+// Workgroups of the same images are gridDim.x apart in launch order: for a multiple of 8 image groups they share an L2.
+template <int FMT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void avgpool_fc_kernel(const HeadParams p) {
+    constexpr int kPer = (int)residual_group_channels(FMT);
+    constexpr int kPixels = FMT == TCBNN_RES_I12 ? 25 : 49;  // requested together (integer sums: the order does not matter)
     __shared__ __align__(16) float mean[kHeadMaxC][kHeadImages];
     const int tid = threadIdx.x;
     const int b0 = blockIdx.x * kHeadImages;
+    const int n = blockIdx.y * kHeadOutputs + (tid & (kHeadOutputs - 1)), i0 = tid / kHeadOutputs * 4;
+    // Weights eight channels at a time: a wave-uniform base and eight lane offsets.
+    unsigned w_lane[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) w_lane[q] = ((unsigned)q * (unsigned)p.N + (unsigned)min(n, p.N - 1)) * 4u;
+    float w[kHeadChunk];
+    auto request = [&](int c, int slot) {  // channels c .. c + 7 (c uniform), of no use past the last chunk
+        const char* const row = reinterpret_cast<const char*>(p.w) + (size_t)min(c, max(0, p.C - 8)) * p.N * 4;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) w[slot + q] = *reinterpret_cast<const float*>(row + (p.C >= 8 ? w_lane[q] : w_lane[0]));
+    };
+#pragma unroll
+    for (int q = 0; q < kHeadChunk; q += 8) request(q, q);
+
     const float npix = (float)p.P;
-    const int4* __restrict__ src = reinterpret_cast<const int4*>(p.rin);
+    const size_t pixel_b = (size_t)p.groups * residual_group_bytes(FMT) * p.B;
     for (int u = tid; u < p.groups * kHeadImages; u += kThreads) {
         const int g = u / kHeadImages, i = u % kHeadImages;  // image fastest: 128-byte runs
-        const int bb = min(b0 + i, p.B - 1);
-        if (p.fmt == TCBNN_RES_I12) {  // groups of 16 channels
-            int s16[16], v16[16];
+        const unsigned bb = (unsigned)min(b0 + i, p.B - 1);
+        const unsigned lane = (unsigned)g * (unsigned)residual_group_bytes(FMT) * (unsigned)p.B + bb * 16u;
+        const unsigned lane8 = (unsigned)g * 24u * (unsigned)p.B + (unsigned)p.B * 16u + bb * 8u;
+        int sum[kPer];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) s16[e] = 0;
-            for (int pix = 0; pix < p.P; ++pix) {
-                residual_load_group16(p.rin, p.fmt, (size_t)pix, p.C, g, p.B, bb, v16);
+        for (int k = 0; k < kPer; ++k) sum[k] = 0;
+        for (int pix0 = 0; pix0 < p.P; pix0 += kPixels) {
+            uint4 v[kPixels];
+            uint2 v2[FMT == TCBNN_RES_I12 ? kPixels : 1];
+            const char* at = reinterpret_cast<const char*>(p.rin) + (size_t)pix0 * pixel_b;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) s16[e] += v16[e];
+            for (int q = 0; q < kPixels; ++q) {
+                v[q] = *reinterpret_cast<const uint4*>(at + lane);
+                if constexpr (FMT == TCBNN_RES_I12) v2[q] = *reinterpret_cast<const uint2*>(at + lane8);
+                if (pix0 + q + 1 < p.P) at += pixel_b;  // (past the last pixel: the last one again, not added)
             }
+            auto add = [&](int q) {
+                if constexpr (FMT == TCBNN_RES_I12) {
+                    int e[16];
+                    i12_unpack8(v[q].x, v[q].y, v[q].z, e);
+                    i12_unpack8(v[q].w, v2[q].x, v2[q].y, e + 8);
 #pragma unroll
-            for (int e = 0; e < 16; ++e)
-                if (16 * g + e < p.C) mean[16 * g + e][i] = (float)s16[e] / npix;
-            continue;
-        }
-        int sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        // eight pixels requested at a time (a load per loop pass waits for each one in turn); integer sums, so
-        // the order does not matter
-        for (int pix0 = 0; pix0 < p.P; pix0 += 8) {
-            int4 v[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) v[q] = src[((size_t)min(pix0 + q, p.P - 1) * p.groups + g) * p.B + bb];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                if (pix0 + q >= p.P) continue;
-                if (p.fmt == TCBNN_RES_I16) {
-                    const int wv[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        sum[2 * k] += (int)(short)(wv[k] & 0xffff);
-                        sum[2 * k + 1] += wv[k] >> 16;
-                    }
+                    for (int k = 0; k < kPer; ++k) sum[k] += e[k];
                 } else {
-                    sum[0] += v[q].x;
-                    sum[1] += v[q].y;
-                    sum[2] += v[q].z;
-                    sum[3] += v[q].w;
+                    const int wv[4] = {(int)v[q].x, (int)v[q].y, (int)v[q].z, (int)v[q].w};
+#pragma unroll
+                    for (int k = 0; k < kPer; ++k)
+                        sum[k] += FMT == TCBNN_RES_I32 ? wv[k % 4] : (k % 2 == 0 ? (int)(short)(wv[k / 2] & 0xffff) : wv[k / 2] >> 16);
                 }
-            }
+            };
+#pragma unroll
+            for (int q = 0; q < kPixels; ++q)
+                if (pix0 + q < p.P) add(q);  // uniform
         }
-        for (int k = 0; k < p.per_group; ++k) {
-            const int c = g * p.per_group + k;
-            if (c < p.C) mean[c][i] = (float)sum[k] / npix;
-        }
+#pragma unroll
+        for (int k = 0; k < kPer; ++k)
+            if (g * kPer + k < p.C) mean[g * kPer + k][i] = (float)sum[k] / npix;
     }
     __syncthreads();
-    const int n = blockIdx.y * kHeadOutputs + tid;
-    if (n >= p.N) return;
-    float acc[kHeadImages];
+    if (b0 + i0 >= p.B) return;  // (a wave's lanes share i0)
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto channel = [&](const float4& m, float weight) {
+        acc[0] = __fmaf_rn(m.x, weight, acc[0]);
+        acc[1] = __fmaf_rn(m.y, weight, acc[1]);
+        acc[2] = __fmaf_rn(m.z, weight, acc[2]);
+        acc[3] = __fmaf_rn(m.w, weight, acc[3]);
+    };
+    int c0 = 0;
+    for (; c0 + kHeadChunk <= p.C; c0 += kHeadChunk) {
+        float4 m[2][8];
+        auto means = [&](int q0) {
 #pragma unroll
-    for (int i = 0; i < kHeadImages; ++i) acc[i] = 0.0f;
-    // weights of the next 16 channels are requested while the current 16 are used; the additions stay in ascending
-    // channel order
-    float wn[16];
+            for (int q = 0; q < 8; ++q) m[q0 / 8 % 2][q] = *reinterpret_cast<const float4*>(&mean[c0 + q0 + q][i0]);
+        };
+        means(0);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) wn[q] = p.w[(size_t)min(q, p.C - 1) * p.N + n];
-    for (int c0 = 0; c0 < p.C; c0 += 16) {
-        float wv[16];
+        for (int q0 = 0; q0 < kHeadChunk; q0 += 8) {
+            if (q0 + 8 < kHeadChunk) means(q0 + 8);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int q = 0; q < 16; ++q) wv[q] = wn[q];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) wn[q] = p.w[(size_t)min(c0 + 16 + q, p.C - 1) * p.N + n];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int c = min(c0 + q, p.C - 1);
-            const bool on = c0 + q < p.C;  // a channel past C leaves the sums as they are
-            const float4 m0 = *reinterpret_cast<const float4*>(&mean[c][0]);
-            const float4 m1 = *reinterpret_cast<const float4*>(&mean[c][4]);
-            acc[0] = on ? __fmaf_rn(m0.x, wv[q], acc[0]) : acc[0];
-            acc[1] = on ? __fmaf_rn(m0.y, wv[q], acc[1]) : acc[1];
-            acc[2] = on ? __fmaf_rn(m0.z, wv[q], acc[2]) : acc[2];
-            acc[3] = on ? __fmaf_rn(m0.w, wv[q], acc[3]) : acc[3];
-            acc[4] = on ? __fmaf_rn(m1.x, wv[q], acc[4]) : acc[4];
-            acc[5] = on ? __fmaf_rn(m1.y, wv[q], acc[5]) : acc[5];
-            acc[6] = on ? __fmaf_rn(m1.z, wv[q], acc[6]) : acc[6];
-            acc[7] = on ? __fmaf_rn(m1.w, wv[q], acc[7]) : acc[7];
+            for (int q = 0; q < 8; ++q) channel(m[q0 / 8 % 2][q], w[q0 + q]);
+            __builtin_amdgcn_sched_barrier(0);
+            request(c0 + kHeadChunk + q0, q0);
         }
     }
+    for (; c0 < p.C; ++c0)  // (what is left of a channel count that 64 does not divide)
+        channel(*reinterpret_cast<const float4*>(&mean[c0][i0]), p.w[(size_t)c0 * p.N + min(n, p.N - 1)]);
+    if (n >= p.N) return;
     const float bias = p.bias[n];
 #pragma unroll
-    for (int i = 0; i < kHeadImages; ++i)
-        if (b0 + i < p.B) p.out[(size_t)(b0 + i) * p.N + n] = __fadd_rn(acc[i], bias);
+    for (int i = 0; i < 4; ++i)
+        if (b0 + i0 + i < p.B) p.out[(size_t)(b0 + i0 + i) * p.N + n] = __fadd_rn(acc[i], bias);
 }
 
 }  // namespace
@@ -234,6 +361,21 @@ extern "C" int tcbnn_pool128_forward(const tcbnn_pool128_desc* d, void* stream) 
     const long long total = (long long)(p.cw + p.groups) * p.B * p.OH * p.OW;
     const long long blocks = (total + kThreads - 1) / kThreads;
     TCBNN_REQUIRE(blocks <= 0x7fffffffLL, "pool128: grid too large");
+    if (p.window == 3 && p.stride == 2 && p.OW <= 65535 && p.OH <= 65535 && (long long)(p.cw + p.groups) * p.B < (1LL << 31) - kThreads) {
+        // output rows per thread: eight, fewer while that leaves the chip's 1024 SIMDs under eight waves each
+        const long long columns = (long long)(p.cw + p.groups) * p.B * p.OW;
+        const int rows = (int)std::min(8LL, std::max(1LL, columns * p.OH / (8192LL * 64)));
+        const dim3 grid((unsigned)(((long long)(p.cw + p.groups) * p.B + kThreads - 1) / kThreads), (unsigned)p.OW, (unsigned)((p.OH + rows - 1) / rows));
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, p, rows); };
+        if (p.fmt == TCBNN_RES_I12)
+            launch(pool3x3s2_kernel<TCBNN_RES_I12>);
+        else if (p.fmt == TCBNN_RES_I16)
+            launch(pool3x3s2_kernel<TCBNN_RES_I16>);
+        else
+            launch(pool3x3s2_kernel<TCBNN_RES_I32>);
+        TCBNN_LAUNCH_CHECK("pool3x3s2_kernel");
+        return TCBNN_OK;
+    }
     hipLaunchKernelGGL(pool128_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, (hipStream_t)stream, p);
     TCBNN_LAUNCH_CHECK("pool128_kernel");
     return TCBNN_OK;
@@ -261,10 +403,16 @@ extern "C" int tcbnn_avgpool_fc_forward(const tcbnn_avgpool_fc_desc* d, void* st
     p.B = d->batch;
     p.N = d->out_features;
     p.fmt = d->residual_format;
-    p.per_group = (int)residual_group_channels(p.fmt);
-    p.groups = (p.C + p.per_group - 1) / p.per_group;
+    const int per_group = (int)residual_group_channels(p.fmt);
+    p.groups = (p.C + per_group - 1) / per_group;
     const dim3 grid((unsigned)((p.B + kHeadImages - 1) / kHeadImages), (unsigned)((p.N + kHeadOutputs - 1) / kHeadOutputs));
-    hipLaunchKernelGGL(avgpool_fc_kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, p);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, p); };
+    if (p.fmt == TCBNN_RES_I12)
+        launch(avgpool_fc_kernel<TCBNN_RES_I12>);
+    else if (p.fmt == TCBNN_RES_I16)
+        launch(avgpool_fc_kernel<TCBNN_RES_I16>);
+    else
+        launch(avgpool_fc_kernel<TCBNN_RES_I32>);
     TCBNN_LAUNCH_CHECK("avgpool_fc_kernel");
     return TCBNN_OK;
 }

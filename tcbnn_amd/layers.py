@@ -897,6 +897,8 @@ class Pool128LayerParam:
         check(lib.tcbnn_pool128_forward(C.byref(d), _stream_handle(stream)))
 
     def kernel_name(self):
+        if self.window == 3 and self.stride == 2:
+            return "pool3x3s2_kernel<%d>" % (self.input_residual_gpu.format if self.pool_residual else 0)
         return "pool128_kernel"
 
     download_packed = _ConvGeometry.download_packed
@@ -949,7 +951,7 @@ class AvgPoolFcLayerParam:
         check(lib.tcbnn_avgpool_fc_forward(C.byref(d), _stream_handle(stream)))
 
     def kernel_name(self):
-        return "avgpool_fc_kernel"
+        return "avgpool_fc_kernel<%d>" % self.input_residual_gpu.format
 
     def download_output(self):
         return self.output_gpu.to_numpy(np.float32, (self.batch, self.out_features))

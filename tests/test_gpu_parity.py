@@ -1365,6 +1365,20 @@ def test_avgpool_fc(gpu, b, h, c, n, fmt):
     layer.release()
 
 
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("b,h,c,pad", [(2, 5, 16, 0), (6, 8, 33, 2), (66, 4, 64, 1), (4, 3, 130, 2)])
+def test_pool3x3_stride2(gpu, b, h, c, pad, fmt):
+    """The rolling 3x3 / stride 2 kernel at the frame's edges: every padding, odd and even frames, channel tails."""
+    test_pool128(gpu, b, h, c, 3, 2, pad, fmt)
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("b,h,c,n", [(2, 7, 4, 3), (9, 8, 64, 129), (12, 5, 200, 128), (5, 2, 512, 1)])
+def test_avgpool_fc_tails(gpu, b, h, c, n, fmt):
+    """Channel counts below and off the 64-channel chunks, more pixels than are requested at once, ragged outputs."""
+    test_avgpool_fc(gpu, b, h, c, n, fmt)
+
+
 def test_forward_captured_in_a_hip_graph(gpu):
     """The whole forward (no allocation, no memset) is captured into a HIP graph and replayed several
     times, with eager work and synchronisations between the replays and a new input before the last
