@@ -109,31 +109,32 @@ __device__ __forceinline__ float minus_half(float x, h2 pair) {
     return d;
 }
 
-// 16 channels of one image and pixel, streamed past the caches (read two launches later): 12 bits each, 16 bytes at `at`
-// and 8 at `at8`; 16 or 32 bits, 16-byte pieces `piece` bytes apart from `at` on.  Lanes without a value pass offsets
+// 16 channels of one image and pixel: 12 bits each, 16 bytes at `at` and 8 at `at8`; 16 or 32 bits, 16-byte pieces
+// `piece` bytes apart from `at` on.  Ordinary stores: a tile's eight images are whole 128-byte lines only if the batch is a
+// multiple of 8, and otherwise the cache has to join the halves (CIFAR ResNet at batch 170: 33.9 us with non-temporal
+// stores, 23.0 us with these; at batch 256 28.5 and 27.7 us).  Lanes without a value pass offsets
 // beyond the tensor and store nothing.  (No scalar offset register on these stores: a 128-bit buffer store with one,
 // directly followed by a VALU write of its data, can store the new value.)
 template <int RES>
 __device__ __forceinline__ void store_residual_group(__amdgpu_buffer_rsrc_t rsrc, int fmt, unsigned at, unsigned at8, unsigned piece,
                                                      const int* v) {
-    constexpr int kNonTemporal = 2;
     if constexpr (RES == RES_12) {
         uint32_t d[6];
         i12_pack8(v, d[0], d[1], d[2]);
         i12_pack8(v + 8, d[3], d[4], d[5]);
-        __builtin_amdgcn_raw_buffer_store_b128(v4u{d[0], d[1], d[2], d[3]}, rsrc, (int)at, 0, kNonTemporal);
-        __builtin_amdgcn_raw_buffer_store_b64(v2u{d[4], d[5]}, rsrc, (int)at8, 0, kNonTemporal);
+        __builtin_amdgcn_raw_buffer_store_b128(v4u{d[0], d[1], d[2], d[3]}, rsrc, (int)at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b64(v2u{d[4], d[5]}, rsrc, (int)at8, 0, 0);
     } else if (fmt == TCBNN_RES_I16) {
 #pragma unroll
         for (int e = 0; e < 16; e += 8)
             __builtin_amdgcn_raw_buffer_store_b128(v4u{(uint32_t)((v[e] & 0xffff) | (v[e + 1] << 16)), (uint32_t)((v[e + 2] & 0xffff) | (v[e + 3] << 16)),
                                                        (uint32_t)((v[e + 4] & 0xffff) | (v[e + 5] << 16)), (uint32_t)((v[e + 6] & 0xffff) | (v[e + 7] << 16))},
-                                                   rsrc, (int)(at + (unsigned)(e / 8) * piece), 0, kNonTemporal);
+                                                   rsrc, (int)(at + (unsigned)(e / 8) * piece), 0, 0);
     } else {
 #pragma unroll
         for (int e = 0; e < 16; e += 4)
             __builtin_amdgcn_raw_buffer_store_b128(v4u{(uint32_t)v[e], (uint32_t)v[e + 1], (uint32_t)v[e + 2], (uint32_t)v[e + 3]}, rsrc,
-                                                   (int)(at + (unsigned)(e / 4) * piece), 0, kNonTemporal);
+                                                   (int)(at + (unsigned)(e / 4) * piece), 0, 0);
     }
 }
 
