@@ -1,9 +1,8 @@
 // FP4 matrix-core kernel for LARGE bit-GEMMs: the stand-alone bit matrix product (BMMAS_new,
 // tensorcore_kernel.cu:336-356: C = K - 2 popc(A xor B)) and fully connected layers at large batch
 // (Fc128LayerFMT / Out128LayerFMT, kernel.cuh:174-280; e.g. the 1024 -> 1024 layers of the MLP at batch
-// 8192), where K is a whole number of 64-bit words per row.  The generic implicit-GEMM
-// kernel serves the same problems, but pays for its generality in every k-step (tap bookkeeping, frame and
-// range tests, weights expanded with masks behind two barriers per block).
+// 8192).  The generic implicit-GEMM kernel serves the same problems, but pays for its generality in every k-step (tap
+// bookkeeping, frame and range tests, weights expanded with masks behind two barriers per block).
 //
 //   workgroup = 4 waves = (4 x MT x 32 rows of the batch / of A) x 64 output columns;
 //   wave      = MT image tiles x 2 column tiles: 2 MT MFMAs (32 x 32 x 64, FP4) per k-step;
@@ -44,13 +43,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     const int ng = blockIdx.x % n_groups, rb = blockIdx.x / n_groups;
     const int n0 = ng * (32 * kNT);
     const int b0 = (rb * kWaves + wave) * (32 * MT);
-    // 64-bit k-steps (cw is even, host checked), run in whole groups of kAhead.  Nothing is masked: a pad bit is 0 in
-    // both operands (the layouts' convention), and so is every bit of a step past K (rows: outside the descriptor's
-    // range; weights: staged as 0).  A 0 bit expands to +1.0 on both sides, so each such position adds exactly +1
-    // to the dot product, and the known count is taken off in the epilogue.
-    const int true_steps = p.cw / 2;
-    const int steps = (true_steps + kAhead - 1) / kAhead * kAhead;
-    const int corr = 32 * p.cw - p.k_tap + 64 * (steps - true_steps);
+    // 64-bit k-steps, run in whole groups of kAhead.  Nothing is masked: a pad bit is 0 in both operands (the layouts'
+    // convention), and so is every bit of a word past K: the upper half of the last step of an odd cw, and the steps
+    // that fill up the group (rows: outside the descriptor's range; weights: staged as 0).  A 0 bit expands to +1.0 on
+    // both sides, so each such position adds exactly +1 to the dot product, and the known count is taken off in the
+    // epilogue.
+    const int steps = (p.cw + 2 * kAhead - 1) / (2 * kAhead) * kAhead;
+    const int corr = 64 * steps - p.k_tap;
 
     // ---- weights: this wave stages fragments f = wave + 4 i = (k-step ql = wave/2 + 2 i, column tile wave % 2)
     const int snt = wave & 1, sq = wave >> 1;
@@ -61,7 +60,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
         for (int i = 0; i < kFrags; ++i) {
             const int q = q0 + sq + 2 * i;
-            wx[i] = q < true_steps ? wrow[2 * q] : 0u;
+            if (2 * q + 1 < p.cw) wx[i] = wrow[2 * q];  // (uniform)
+            else wx[i] = 2 * q + h < p.cw ? wrow[2 * q] : 0u;
         }
     };
     int csum = 0;  // this lane's share of its column's constant C: the words it stages, pad steps included
@@ -299,7 +299,7 @@ bool gemm_mfma_applicable(const BgemmParams& p) {
     if (p.PH * p.PW != 1 || p.R * p.S != 1 || p.pool_h * p.pool_w != 1) return false;
     if (p.res_in != nullptr || p.res_out != nullptr) return false;
     if (p.mode != EPI_THRESH && p.mode != EPI_AFFINE && p.mode != EPI_RAW) return false;
-    if (p.cw % 2 != 0 || p.k_tap > 32 * p.cw) return false;               // whole 64-bit k-steps
+    if (p.k_tap > 32 * p.cw) return false;
     if ((long long)p.cw * p.B * 4 >= (1LL << 31)) return false;          // 32-bit buffer offsets
     // large enough to give every CU a workgroup with two image tiles per wave; smaller problems are bound by
     // launch and fill and stay with the kernels written for them
