@@ -1,0 +1,601 @@
+// FP4 matrix-core kernel of the bit convolutions and bit products whose batch is not a multiple of 32 images wide or
+// whose whole work is small: the columns of the product are (pixel, image) pairs numbered through,
+// column = pixel * batch + image, so a 32-column MFMA tile is full whatever the batch is.  (The kernels that give a
+// tile 32 images of ONE pixel multiply 32 / batch times too much at a batch below 32.)
+//
+//   tile      = MT x 32 columns by NT x 32 output channels, one wave; with 2x2 OR-pooling a column is a window, and its
+//               four pixels are either the MT = 4 column tiles (the window is reduced in the lane's own registers) or,
+//               where that leaves too few waves, four groups of 8 lanes of one tile;
+//   K         = the words of the filter row, (tap, input word) numbered through.  A group is 8 words: lane half h owns
+//               words 8g + 4h .. + 3, one 128-bit load per channel tile straight from the packed filter rows, and the
+//               matching four activation words; step i multiplies word 8g + 4h + i.  Cin = 32 or 96 costs no padding;
+//   borders   : a lane's invalid taps are bits of a mask; such an activation is not loaded (its offset lies outside the
+//               buffer) and enters as FP4 zero, the reference's "exclude" rule (kernel.cuh:752-768).  Where an
+//               activation word of the group lies relative to the column's first tap, and which tap it belongs to, is
+//               a table in LDS, filled once per workgroup;
+//   small work: K is split over the waves of a workgroup (up to 8) so that a launch of few tiles still spreads over
+//               the machine; the partial sums, exact integers, meet in LDS.
+//
+// What bounds it: the small launches by latency (one or two memory round trips, then the launch itself), the larger
+// ones by instruction issue: expanding the operands takes 7 VALU instructions per fragment, plus 5 per column tile and
+// step for address and border, against 32 cycles per MFMA.
+#include <algorithm>
+
+#include "common.h"
+#include "mfma_util.h"
+
+namespace tcbnn {
+namespace {
+
+using namespace mfma;
+
+// what happens to the sums
+constexpr int FM_BITS = 0;    // threshold, packed bits
+constexpr int FM_RES = 1;     // residual injected from a source of the same size and / or saved; threshold
+constexpr int FM_RESPOOL = 2; // residual injected as the 2x2 maximum of a source twice the size
+constexpr int FM_RAW = 3;     // int32 dot products
+// 2x2 OR-pooling: none; the window's four pixels in lanes 8 apart of one column tile; in the four column tiles of a wave
+constexpr int FW_NONE = 0, FW_LANES = 1, FW_TILES = 2;
+
+constexpr int kTapNone = 31;  // tap number of a word past K: its mask bit is always "invalid"
+constexpr int kMaxWords = 4096;
+
+// n / d for n < 2^31 by multiplication (Granlund and Montgomery's round-up method)
+struct FastDiv {
+    uint32_t mul, shift, d;
+};
+FastDiv fast_div(uint32_t d) {
+    uint32_t s = 0;
+    while ((1ull << s) < d) ++s;
+    return {(uint32_t)((((1ull << s) - d) << 32) / d + 1), s, d};
+}
+__device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv& f) { return (__umulhi(n, f.mul) + n) >> f.shift; }
+
+struct FlatArgs {
+    FastDiv by_batch, by_row, by_cw, by_s;  // columns per item, items per row, words per tap, taps per filter row
+    int cols, n_tiles_c, n_groups, kw_tot, groups, per_slice, slices;
+    int total;  // tiles (column groups x channel groups) of the launch
+    unsigned act_bytes, wgt_bytes;
+    int res_lim;
+};
+
+constexpr int raw_pitch(int nt) { return 32 * nt + 4; }  // words; an odd multiple of 4: conflict-free both ways
+constexpr int max_waves(int mt, int nt) { return mt * nt == 1 ? 8 : 4; }
+// groups of operand words in flight per wave (registers)
+constexpr int ring_depth(int mt, int nt, int fm) { return mt * nt >= 8 ? 1 : (mt * nt >= 4 || fm == FM_RESPOOL ? 2 : 4); }
+
+template <int MT, int NT, int FM, int RF, int WIN>
+__global__ __launch_bounds__(64 * max_waves(MT, NT)) __attribute__((amdgpu_waves_per_eu(MT * NT == 1 ? 4 : 2))) void
+bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, const uint32_t* __restrict__ wgt,
+                     const float* __restrict__ bnp, const int32_t* __restrict__ rin, const FlatArgs f) {
+    static_assert(WIN == FW_NONE || (FM == FM_BITS && MT == (WIN == FW_TILES ? 4 : 1)), "see FW_*");
+    static_assert(FM != FM_RESPOOL || MT == 1, "four source pixels per column");
+    constexpr bool kRes = FM == FM_RES || FM == FM_RESPOOL;
+    constexpr int D = ring_depth(MT, NT, FM);
+    extern __shared__ v4i lds_dyn[];
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int waves = blockDim.x >> 6;
+    // Tiles are dealt so that each XCD (workgroups go to the 8 of them in turn) gets a contiguous run: neighbouring
+    // pixels share activation rows, and the channel groups of a column tile all of them.
+    const int per_wg = f.slices > 1 ? 1 : waves;
+    const int wgs = (f.total + per_wg - 1) / per_wg;
+    const int per_xcd = (wgs + 7) / 8;
+    const int wg = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    const int slice = f.slices > 1 ? wave : 0;
+    const int tile = f.slices > 1 ? wg : wg * waves + wave;
+    const bool live = (int)(blockIdx.x >> 3) < per_xcd && wg < wgs && tile < f.total;  // (uniform per wave)
+    const int ct = live ? tile / f.n_groups : 0, ng = live ? tile % f.n_groups : 0;
+    const int n0 = ng * (32 * NT);
+
+    v4i* red = lds_dyn;                                                           // [slices - 1][MT * NT][4][64]
+    int* raw_area = reinterpret_cast<int*>(red + (size_t)(f.slices - 1) * MT * NT * 256);
+    constexpr int kRawWords = FM == FM_RAW ? 32 * raw_pitch(NT) + 64 : 0;         // per tile of the workgroup
+    int2* tab = reinterpret_cast<int2*>(raw_area + per_wg * kRawWords);           // [8 * groups]
+
+    const int g_begin = slice * f.per_slice, g_end = live ? min(f.groups, g_begin + f.per_slice) : 0;
+
+    // ---- weights: lane (j, h) reads words 8g + 4h .. + 3 of its channel's row (past the last row: zeros; past the end
+    // of a row: the next row's words, which meet activations that are zero)
+    const __amdgpu_buffer_rsrc_t r_wgt =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(wgt), 0, (int)f.wgt_bytes, 0x00020000);
+    unsigned wvoff[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+        wvoff[nt] = ((unsigned)(n0 + nt * 32 + row_to_channel(j)) * (unsigned)f.kw_tot + 4u * (unsigned)h) * 4u;
+    v4i aw[D][NT];
+    auto request_w = [&](int slot, int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+            aw[slot][nt] = __builtin_amdgcn_raw_buffer_load_b128(r_wgt, (int)wvoff[nt], g * 32, 0);
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (g_begin + d < g_end) request_w(d, g_begin + d);
+
+    // ---- columns
+    const unsigned row_b = (unsigned)p.B * 4u, pix_b = (unsigned)p.cw * row_b;
+    unsigned base[MT], inval[MT];  // byte offset of the column's first tap (may be "negative"); mask of its invalid taps
+    int cpix[WIN == FW_TILES ? 1 : MT], cb[WIN == FW_TILES ? 1 : MT], cy[MT], cx[MT];
+    bool cok[WIN == FW_TILES ? 1 : MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        constexpr bool tiles = WIN == FW_TILES;
+        const int sub = tiles ? mt : j >> 3;  // pixel of the window
+        if (!tiles || mt == 0) {
+            const unsigned col = WIN == FW_LANES ? (unsigned)ct * 8u + (unsigned)(j & 7)
+                                                 : (unsigned)(tiles ? ct : ct * MT + mt) * 32u + (unsigned)j;
+            const unsigned cc = min(col, (unsigned)f.cols - 1u);
+            const unsigned item = div_by(cc, f.by_batch);
+            cok[mt] = live && col < (unsigned)f.cols;
+            cpix[mt] = (int)item;
+            cb[mt] = (int)(cc - item * f.by_batch.d);
+        }
+        const int k = tiles ? 0 : mt;
+        const unsigned iy = div_by((unsigned)cpix[k], f.by_row), ix = (unsigned)cpix[k] - iy * f.by_row.d;
+        cy[mt] = WIN != FW_NONE ? 2 * (int)iy + (sub >> 1) : (int)iy;
+        cx[mt] = WIN != FW_NONE ? 2 * (int)ix + (sub & 1) : (int)ix;
+        const int ay0 = cy[mt] * p.stride_h - p.pad_h, ax0 = cx[mt] * p.stride_w - p.pad_w;
+        base[mt] = (unsigned)(ay0 * p.W + ax0) * pix_b + (unsigned)cb[k] * 4u;
+        // valid taps: rows lo_y .. hi_y, columns lo_x .. hi_x
+        const int lo_x = max(0, -ax0), hi_x = min(p.S, p.W - ax0);
+        const unsigned run = hi_x > lo_x ? ((1u << hi_x) - 1u) & ~((1u << lo_x) - 1u) : 0u;
+        unsigned ok = 0;
+        for (int r = 0; r < p.R; ++r)
+            if (ay0 + r >= 0 && ay0 + r < p.H) ok |= run << (r * p.S);
+        inval[mt] = cok[k] ? ~ok : 0xffffffffu;
+    }
+
+    // ---- operands of the epilogue, requested ahead of K
+    const bool fin = live && slice == 0;  // (uniform) this wave finishes the tile
+    float thr[NT][16];
+    constexpr int NRAW = RF == TCBNN_RES_I12 ? 6 : (RF == TCBNN_RES_I16 ? 8 : 16);
+    constexpr int NSRC = FM == FM_RESPOOL ? 4 : 1;
+    int rraw[kRes ? MT * NT : 1][NSRC][NRAW];
+    if (FM != FM_RAW && fin) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) thr[nt][v] = bnp[min(n0 + nt * 32 + 16 * h + v, p.N - 1)];
+    }
+    if constexpr (kRes) {
+        if (fin && f.res_lim > 0) {
+            const unsigned G = (unsigned)(p.res_in_ch + (int)residual_group_channels(RF) - 1) / (unsigned)residual_group_channels(RF);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const int b = cb[mt];
+#pragma unroll
+                for (int s = 0; s < NSRC; ++s) {
+                    const size_t spix = FM == FM_RESPOOL
+                                            ? (size_t)(2 * cy[mt] + (s >> 1)) * (size_t)(2 * p.PW) + (size_t)(2 * cx[mt] + (s & 1))
+                                            : (size_t)cy[mt] * p.PW + cx[mt];
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) {
+                        const int cbase = n0 + nt * 32 + 16 * h;
+                        int* dst = rraw[mt * NT + nt][s];
+                        if constexpr (RF == TCBNN_RES_I12) {
+                            if (cbase < p.res_in_ch) {
+                                const uint32_t* w = reinterpret_cast<const uint32_t*>(rin) + (spix * G + cbase / 16) * (size_t)p.B * 6;
+                                const v4i a = *reinterpret_cast<const v4i*>(w + (size_t)b * 4);
+                                const int2 c = *reinterpret_cast<const int2*>(w + (size_t)p.B * 4 + (size_t)b * 2);
+                                dst[0] = a[0], dst[1] = a[1], dst[2] = a[2], dst[3] = a[3], dst[4] = c.x, dst[5] = c.y;
+                            }
+                        } else {
+                            constexpr int kCh = (int)residual_group_channels(RF);
+#pragma unroll
+                            for (int g = 0; g < 16 / kCh; ++g)
+                                if (cbase + kCh * g < p.res_in_ch) {
+                                    const v4i a = reinterpret_cast<const v4i*>(rin)[(spix * G + cbase / kCh + g) * (size_t)p.B + b];
+                                    dst[4 * g] = a[0], dst[4 * g + 1] = a[1], dst[4 * g + 2] = a[2], dst[4 * g + 3] = a[3];
+                                }
+                        }
+                    }
+                }
+            }
+        }
+    }
+
+    // ---- the table of K: byte offset of word k's activation from the column's first tap, and its tap
+    for (int k = tid; k < 8 * f.groups; k += blockDim.x) {
+        const unsigned tap = div_by((unsigned)k, f.by_cw), w = (unsigned)k - tap * f.by_cw.d;
+        const unsigned r = div_by(tap, f.by_s), s = tap - r * f.by_s.d;
+        tab[k] = k < f.kw_tot ? make_int2((int)((r * (unsigned)p.W + s) * pix_b + w * row_b), (int)tap) : make_int2(0, kTapNone);
+    }
+    __syncthreads();
+
+    const __amdgpu_buffer_rsrc_t r_act =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(act), 0, (int)f.act_bytes, 0x00020000);
+    uint32_t bw[D][MT][4];
+    int tp[D][4];
+    auto request_b = [&](int slot, int g) __attribute__((always_inline)) {
+        const v4i* t = reinterpret_cast<const v4i*>(tab + 8 * g + 4 * h);
+        const v4i t0 = t[0], t1 = t[1];
+        const int off[4] = {t0[0], t0[2], t1[0], t1[2]};
+        tp[slot][0] = t0[1], tp[slot][1] = t0[3], tp[slot][2] = t1[1], tp[slot][3] = t1[3];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                // all ones where the tap is invalid: the offset then lies outside the buffer, the load returns 0
+                const unsigned m = (unsigned)__builtin_amdgcn_sbfe((int)inval[mt], (unsigned)tp[slot][i], 1u);
+                bw[slot][mt][i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r_act, (int)((base[mt] + (unsigned)off[i]) | m), 0, 0);
+            }
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (g_begin + d < g_end) request_b(d, g_begin + d);
+
+    v16f acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[mt][nt][v] = 0.0f;
+
+    // +-1 in FP4 as in expand_f4, zero where the tap is invalid (its word was returned as 0)
+    auto expand_col = [&](uint32_t x, unsigned c) __attribute__((always_inline)) {
+        v4i r;
+        auto bfi = [&](uint32_t shifted) __attribute__((always_inline)) {
+            int d;
+            asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(d) : "s"(0x88888888u), "v"(shifted), "v"(c));
+            return d;
+        };
+        r[0] = bfi(x << 3);
+        r[1] = bfi(x << 2);
+        r[2] = bfi(x << 1);
+        r[3] = bfi(x);
+        return r;
+    };
+    for (int g0 = g_begin; g0 < g_end; g0 += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const int g = g0 + d;
+            if (g < g_end) {  // (uniform)
+                const int left = f.kw_tot - 8 * g;  // steps past the row's last word in both halves are not multiplied
+                v4i a[NT];
+                uint32_t x[MT][4];
+                int tq[4];
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) a[nt] = aw[d][nt];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    tq[i] = tp[d][i];
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) x[mt][i] = bw[d][mt][i];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (i < left) {
+                        v4i bf[MT], af[NT];
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) {
+                            const unsigned m = (unsigned)__builtin_amdgcn_sbfe((int)inval[mt], (unsigned)tq[i], 1u);
+                            bf[mt] = expand_col(x[mt][i], ~m & 0x22222222u);
+                        }
+#pragma unroll
+                        for (int nt = 0; nt < NT; ++nt) af[nt] = expand_f4((uint32_t)a[nt][i]);
+#pragma unroll
+                        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                            for (int mt = 0; mt < MT; ++mt) acc[mt][nt] = Acc<FMT_F4>::mma(af[nt], bf[mt], acc[mt][nt]);
+                    }
+                if (g + D < g_end) {
+                    request_w(d, g + D);
+                    request_b(d, g + D);
+                }
+            }
+        }
+    }
+
+    // ---- the slices' sums meet in LDS; wave 0 of the workgroup finishes the tile
+    if (f.slices > 1) {
+        if (slice > 0) {
+#pragma unroll
+            for (int t = 0; t < MT * NT; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const v16f& s = acc[t / NT][t % NT];
+                    red[(((slice - 1) * MT * NT + t) * 4 + q) * 64 + lane] =
+                        v4i{(int)s[4 * q], (int)s[4 * q + 1], (int)s[4 * q + 2], (int)s[4 * q + 3]};
+                }
+        }
+        __syncthreads();
+        if (slice > 0) return;
+    }
+    if (!live) return;
+
+    const int padbits = 32 * p.cw - p.k_tap;  // a tap's pad bits are 0 in both operands: each adds +1
+    const int ow = (p.N + 31) / 32;
+    uint32_t orw[NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int k = WIN == FW_TILES ? 0 : mt;
+        const int b = cb[k];
+        const bool ok = cok[k];
+        const int corr = padbits * (p.R * p.S - __popc(inval[mt] & ((1u << (p.R * p.S)) - 1u)));
+        const size_t pix = (size_t)cy[mt] * p.PW + cx[mt];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const int cbase = n0 + nt * 32 + 16 * h;
+            int dot[16];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) dot[v] = (int)acc[mt][nt][v] - corr;
+            for (int s = 1; s < f.slices; ++s)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const v4i o = red[(((s - 1) * MT * NT + mt * NT + nt) * 4 + q) * 64 + lane];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) dot[4 * q + e] += o[e];
+                }
+            if constexpr (FM == FM_RAW) {
+                int* mine = raw_area + (f.slices > 1 ? 0 : wave) * kRawWords;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<v4i*>(mine + j * raw_pitch(NT) + nt * 32 + 16 * h + 4 * q) =
+                        v4i{dot[4 * q], dot[4 * q + 1], dot[4 * q + 2], dot[4 * q + 3]};
+                continue;
+            }
+            if constexpr (kRes) {
+                if (f.res_lim > 0) {
+                    int rv[16];
+#pragma unroll
+                    for (int s = 0; s < NSRC; ++s) {
+                        const int* w = rraw[mt * NT + nt][s];
+                        int t[16];
+                        if constexpr (RF == TCBNN_RES_I12) {
+                            i12_unpack8((uint32_t)w[0], (uint32_t)w[1], (uint32_t)w[2], t);
+                            i12_unpack8((uint32_t)w[3], (uint32_t)w[4], (uint32_t)w[5], t + 8);
+                        } else if constexpr (RF == TCBNN_RES_I16) {
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) t[2 * e] = (w[e] << 16) >> 16, t[2 * e + 1] = w[e] >> 16;
+                        } else {
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) t[v] = w[v];
+                        }
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) rv[v] = s == 0 ? t[v] : max(rv[v], t[v]);
+                    }
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) dot[v] += cbase + v < f.res_lim ? rv[v] : 0;
+                }
+            }
+            uint32_t hw = 0;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const uint32_t bit = cbase + v < p.N ? thresh_bit(dot[v], thr[nt][v], p.nan_bit) : 0u;
+                hw = hw + hw + bit;
+            }
+            if constexpr (kRes) {
+                if (p.res_out != nullptr) {
+                    if (ok && cbase < p.N) {
+                        int rs[16];
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) rs[v] = cbase + v < p.N ? dot[v] : 0;  // (0 past N inside a group)
+                        if (p.res_out_fmt == TCBNN_RES_I12) {
+                            residual_store_group16(p.res_out, TCBNN_RES_I12, pix, p.N, cbase / 16, p.B, b, rs);
+                        } else if (p.res_out_fmt == TCBNN_RES_I16) {
+                            v4i* dst = reinterpret_cast<v4i*>(p.res_out) + (pix * (size_t)((p.N + 7) / 8) + cbase / 8) * p.B + b;
+#pragma unroll
+                            for (int g = 0; g < 2; ++g)
+                                if (cbase + 8 * g < p.N)
+                                    dst[(size_t)g * p.B] = v4i{(rs[8 * g] & 0xffff) | (rs[8 * g + 1] << 16),
+                                                               (rs[8 * g + 2] & 0xffff) | (rs[8 * g + 3] << 16),
+                                                               (rs[8 * g + 4] & 0xffff) | (rs[8 * g + 5] << 16),
+                                                               (rs[8 * g + 6] & 0xffff) | (rs[8 * g + 7] << 16)};
+                        } else {
+                            v4i* dst = reinterpret_cast<v4i*>(p.res_out) + (pix * (size_t)((p.N + 3) / 4) + cbase / 4) * p.B + b;
+#pragma unroll
+                            for (int g = 0; g < 4; ++g)
+                                if (cbase + 4 * g < p.N)
+                                    dst[(size_t)g * p.B] = v4i{rs[4 * g], rs[4 * g + 1], rs[4 * g + 2], rs[4 * g + 3]};
+                        }
+                    }
+                }
+            }
+            // the half word of lane + 32 completes the word of lane j
+            const uint32_t other = __builtin_amdgcn_permlane32_swap(hw, hw, false, false)[1];
+            uint32_t word = (hw << 16) | other;
+            if constexpr (WIN == FW_TILES) {
+                orw[nt] = mt == 0 ? word : orw[nt] | word;
+                if (mt < MT - 1) continue;
+                word = orw[nt];
+            }
+            if constexpr (WIN == FW_LANES) {
+                word |= (uint32_t)__shfl_xor((int)word, 8);
+                word |= (uint32_t)__shfl_xor((int)word, 16);
+            }
+            if ((WIN == FW_LANES ? lane < 8 : h == 0) && ok) {
+                const size_t opix = WIN != FW_NONE ? (size_t)cpix[0] : pix;
+                uint32_t* dst = p.out_bits + opix * (size_t)p.bits_pix_stride + b;
+                const int w = ng * NT + nt;
+                if (w < p.bits_row_words) dst[(size_t)w * p.B] = word;
+                if (ng == f.n_groups - 1 && nt == NT - 1)  // the pixel's padding words
+                    for (int z = max(ow, f.n_groups * NT); z < p.bits_row_words; ++z) dst[(size_t)z * p.B] = 0;
+            }
+        }
+        if constexpr (FM == FM_RAW) {
+            // int32 output: a lane holds 16 channels of one column; through LDS (the same wave writes and reads) a
+            // store instruction covers whole channel runs of its columns instead of 64 pieces of 16 bytes
+            int* mine = raw_area + (f.slices > 1 ? 0 : wave) * kRawWords;
+            long long* start = reinterpret_cast<long long*>(mine + 32 * raw_pitch(NT));
+            const long long at = (long long)pix * p.raw_pix_stride + (long long)b * p.raw_b_stride + n0;
+            if (h == 0) start[j] = ok ? at : -1;
+            const int chans = min(32 * NT, p.N - n0);
+            const bool vec = chans == 32 * NT && p.raw_pix_stride % 4 == 0 && p.raw_b_stride % 4 == 0 &&
+                             (reinterpret_cast<uintptr_t>(p.out_i32) & 15) == 0;  // (uniform)
+            if (vec) {
+                constexpr int kCols = 8 * NT, kRows = 64 / kCols;
+                const int rl = lane / kCols, cl = lane % kCols;
+#pragma unroll
+                for (int r = 0; r < 32; r += kRows) {
+                    const v4i q = *reinterpret_cast<const v4i*>(mine + (r + rl) * raw_pitch(NT) + 4 * cl);
+                    const long long to = start[r + rl];
+                    if (to >= 0) *reinterpret_cast<v4i*>(p.out_i32 + to + 4 * cl) = q;
+                }
+            } else {
+                constexpr int kCols = 32, kRows = 2;
+                const int rl = lane / kCols, cl = lane % kCols;
+                for (int r = 0; r < 32; r += kRows) {
+                    const long long to = start[r + rl];
+                    for (int c = cl; c < chans; c += kCols)
+                        if (to >= 0) p.out_i32[to + c] = mine[(r + rl) * raw_pitch(NT) + c];
+                }
+            }
+        }
+    }
+}
+
+struct FlatPlan {
+    int mt, nt, slices, win;
+};
+
+int flat_mode(const BgemmParams& p) {
+    if (p.mode == EPI_RAW) return FM_RAW;
+    if (p.res_in == nullptr && p.res_out == nullptr) return FM_BITS;
+    return p.res_in != nullptr && p.res_pool ? FM_RESPOOL : FM_RES;
+}
+
+// column tiles (of MT x 32, or of 32 windows) times channel groups
+long long flat_tiles(const BgemmParams& p, int mt, int nt, int win) {
+    const long long items = win != FW_NONE ? (long long)(p.PH / 2) * (p.PW / 2) : (long long)p.PH * p.PW;
+    const long long per = win == FW_LANES ? 8 : (win == FW_TILES ? 32 : 32LL * mt);
+    return (items * p.B + per - 1) / per * ((p.N + 32 * nt - 1) / (32 * nt));
+}
+
+// The largest tile that still gives each of the 1024 SIMDs a wave (every expanded fragment then feeds more MFMAs); tiles
+// of one MFMA are split along K until the SIMDs are busy or a slice is one group.  Measured on the 8 x 8 .. 56 x 56
+// layers of the networks at batch 1 .. 64: eight slices 5.9 us against 8.3 us unsplit for 512 -> 512 channels at 7 x 7,
+// batch 8; more than eight gained nothing (the one wave that adds the sums up takes as long as it saves).
+FlatPlan flat_plan(const BgemmParams& p) {
+    const int groups = (p.R * p.S * p.cw + 7) / 8;
+    const int fm = flat_mode(p);
+    constexpr int kSimds = 1024;
+    FlatPlan f = {1, 1, 1, p.pool_h == 2 ? FW_LANES : FW_NONE};
+    if (f.win != FW_NONE) {
+        if (flat_tiles(p, 4, 2, FW_TILES) >= kSimds) f = {4, 2, 1, FW_TILES};
+        else if (flat_tiles(p, 4, 1, FW_TILES) >= kSimds) f = {4, 1, 1, FW_TILES};
+    } else if (fm != FM_RESPOOL) {  // (with a residual a 4 x 2 tile does not fit the registers)
+        if (fm != FM_RES && flat_tiles(p, 4, 2, FW_NONE) >= kSimds) f.mt = 4, f.nt = 2;
+        else if (flat_tiles(p, 2, 2, FW_NONE) >= kSimds) f.mt = 2, f.nt = 2;
+    }
+    if (f.mt * f.nt == 1) {
+        const long long tiles = flat_tiles(p, 1, 1, f.win);
+        while (f.slices < max_waves(1, 1) && tiles * f.slices < kSimds && 2 * f.slices <= groups) f.slices *= 2;
+    }
+    return f;
+}
+
+template <int MT, int NT, int FM, int RF, int WIN>
+int launch(const BgemmParams& p, const FlatPlan& pl, hipStream_t stream) {
+    FlatArgs f;
+    const int row = WIN != FW_NONE ? p.PW / 2 : p.PW;
+    const long long items = WIN != FW_NONE ? (long long)(p.PH / 2) * (p.PW / 2) : (long long)p.PH * p.PW;
+    f.by_batch = fast_div((uint32_t)p.B);
+    f.by_row = fast_div((uint32_t)row);
+    f.by_cw = fast_div((uint32_t)p.cw);
+    f.by_s = fast_div((uint32_t)p.S);
+    f.cols = (int)(items * p.B);
+    f.n_groups = (p.N + 32 * NT - 1) / (32 * NT);
+    f.kw_tot = p.R * p.S * p.cw;
+    f.groups = (f.kw_tot + 7) / 8;
+    f.per_slice = (f.groups + pl.slices - 1) / pl.slices;
+    f.slices = pl.slices;
+    const long long total = flat_tiles(p, MT, NT, WIN);
+    f.total = (int)total;
+    f.n_tiles_c = (int)(total / f.n_groups);
+    f.act_bytes = (unsigned)(4LL * p.H * p.W * p.cw * p.B);
+    f.wgt_bytes = (unsigned)(4LL * pad32(p.N) * f.kw_tot);
+    f.res_lim = p.res_in != nullptr ? std::min(std::min(p.res_limit, p.res_in_ch), p.N) : 0;
+    const int waves = pl.slices > 1 ? pl.slices : 4, per_wg = pl.slices > 1 ? 1 : waves;
+    const long long wgs = (total + per_wg - 1) / per_wg, blocks = (wgs + 7) / 8 * 8;
+    const size_t lds = (size_t)(pl.slices - 1) * MT * NT * 4096 +
+                       (FM == FM_RAW ? (size_t)per_wg * (32 * raw_pitch(NT) + 64) * 4 : 0) + (size_t)f.groups * 64;
+    if (blocks <= 0 || blocks > 0x7fffffffLL || lds > 64 * 1024) return fail(TCBNN_EINVAL, "bgemm_flat: launch too large");
+    hipLaunchKernelGGL((bgemm_flat_f4_kernel<MT, NT, FM, RF, WIN>), dim3((unsigned)blocks), dim3(64 * waves), lds, stream, p,
+                       p.act, p.wgt, p.bn, p.res_in, f);
+    TCBNN_LAUNCH_CHECK("bgemm_flat_f4_kernel");
+    return TCBNN_OK;
+}
+
+template <int MT, int NT>
+int launch_res(const BgemmParams& p, const FlatPlan& pl, hipStream_t stream) {
+    const int fmt = p.res_in != nullptr ? p.res_in_fmt : TCBNN_RES_I32;
+    if (fmt == TCBNN_RES_I12) return launch<MT, NT, FM_RES, TCBNN_RES_I12, FW_NONE>(p, pl, stream);
+    if (fmt == TCBNN_RES_I16) return launch<MT, NT, FM_RES, TCBNN_RES_I16, FW_NONE>(p, pl, stream);
+    return launch<MT, NT, FM_RES, TCBNN_RES_I32, FW_NONE>(p, pl, stream);
+}
+
+}  // namespace
+
+bool bgemm_flat_applicable(const BgemmParams& p) {
+    if (p.ksplit > 1 || (p.mode != EPI_THRESH && p.mode != EPI_RAW)) return false;
+    const int kw_tot = p.R * p.S * p.cw;
+    if (p.R * p.S >= kTapNone || kw_tot > kMaxWords - 8) return false;
+    const bool res = p.res_in != nullptr || p.res_out != nullptr;
+    const bool pool1 = p.pool_h == 1 && p.pool_w == 1;
+    const bool pool2 = p.pool_h == 2 && p.pool_w == 2 && p.PH % 2 == 0 && p.PW % 2 == 0 && !res && p.mode == EPI_THRESH;
+    if (!pool1 && !pool2) return false;
+    if (p.res_out_pool) return false;
+    const long long cols = (long long)p.PH * p.PW * p.B;
+    return cols < (1LL << 30) && 4LL * p.H * p.W * p.cw * p.B < (1LL << 31) && 4LL * (p.N + 64) * kw_tot < (1LL << 31);
+}
+
+// Both kernels serve the 3x3 layers of conv3x3_mfma.hip: which is faster?  An estimate of both launches in microseconds,
+// fitted to 623 measured pairs (all layers of five networks at batch 1 .. 200, and int32 convolutions with 64 .. 512
+// input channels, 64 .. 512 output channels, 8 x 8 .. 56 x 56 pixels, batch 2 .. 200): choosing by it costs 0.5 % over
+// choosing by measurement, always taking the persistent kernel 20 %.
+bool bgemm_flat_preferred(const BgemmParams& p) {
+    if (!conv3x3_mfma_applicable(p) || !bgemm_flat_applicable(p)) return false;
+    const double steps = 9.0 * p.cw / 2, pix = (double)p.PH * p.PW, n_tiles = (p.N + 31) / 32;
+    const bool raw = p.mode == EPI_RAW, res = p.res_in != nullptr || p.res_out != nullptr, pool = p.pool_h == 2;
+    // Outside what was measured, or where nothing is to be gained, the persistent kernel stays: partial channel tiles
+    // (its other instantiations), un-pooled layers of 32 images and more (full tiles there too), and pooled ones of
+    // fewer windows than fill two tiles.
+    const int res_lim = p.res_in != nullptr ? std::min(std::min(p.res_limit, p.res_in_ch), p.N) : 0;
+    if (!raw && (p.N % 64 != 0 || res_lim % 32 != 0 || (p.B >= 32 && !pool))) return false;
+    if (pool && (long long)p.OH * p.OW * p.B < 16) return false;
+    const int mt = conv3x3_mfma_image_tiles(p);
+    const double b_groups = (p.B + 32 * mt - 1) / (32 * mt);
+    const double mib = raw ? 4e-6 * pix * p.B * p.N : 0.0;  // output, MB
+    // persistent kernel: staging the weights, then the longer of one work item's MFMAs and the whole machine's
+    const double item = 0.0175 * steps * 2 * mt * (pool ? 4 : 1);
+    const double all = 23e-6 * pix * b_groups * mt * n_tiles * steps;
+    const double t_persistent = 4.0 + 0.02 * steps + std::max(item, all) + (res ? 1.2 : 0.0) + 0.24 * mib;
+    // this kernel: full tiles, but operands expanded for every tile and a prologue per tile (the share of short K)
+    const double mfmas = (double)(((long long)p.PH * p.PW * p.B + 31) / 32) * n_tiles * steps;
+    const double t_flat = 4.4 + 1e-6 * mfmas * (40.0 + 380.0 / steps) + 0.015 * steps + (res ? 0.5 : 0.0) + 0.16 * mib;
+    return t_flat < t_persistent;
+}
+
+void bgemm_flat_kernel_name(const BgemmParams& p, char* buf, size_t len) {
+    const FlatPlan f = flat_plan(p);
+    const int fm = flat_mode(p);
+    const int rf = (fm == FM_RES || fm == FM_RESPOOL) && p.res_in != nullptr ? p.res_in_fmt : TCBNN_RES_I32;
+    snprintf(buf, len, "bgemm_flat_f4_kernel<%d, %d, %d, %d, %d>", f.mt, f.nt, fm, rf, f.win);
+}
+
+int launch_bgemm_flat(const BgemmParams& p, hipStream_t stream) {
+    const FlatPlan pl = flat_plan(p);
+    const int fm = flat_mode(p);
+    if (pl.win == FW_LANES) return launch<1, 1, FM_BITS, TCBNN_RES_I32, FW_LANES>(p, pl, stream);
+    if (pl.win == FW_TILES)
+        return pl.nt == 2 ? launch<4, 2, FM_BITS, TCBNN_RES_I32, FW_TILES>(p, pl, stream)
+                          : launch<4, 1, FM_BITS, TCBNN_RES_I32, FW_TILES>(p, pl, stream);
+    if (fm == FM_RESPOOL) {
+        if (p.res_in_fmt == TCBNN_RES_I12) return launch<1, 1, FM_RESPOOL, TCBNN_RES_I12, FW_NONE>(p, pl, stream);
+        if (p.res_in_fmt == TCBNN_RES_I16) return launch<1, 1, FM_RESPOOL, TCBNN_RES_I16, FW_NONE>(p, pl, stream);
+        return launch<1, 1, FM_RESPOOL, TCBNN_RES_I32, FW_NONE>(p, pl, stream);
+    }
+    if (fm == FM_RES)
+        return pl.mt == 1 ? launch_res<1, 1>(p, pl, stream) : launch_res<2, 2>(p, pl, stream);
+    if (fm == FM_RAW)
+        return pl.mt == 1 ? launch<1, 1, FM_RAW, TCBNN_RES_I32, FW_NONE>(p, pl, stream)
+                          : (pl.mt == 2 ? launch<2, 2, FM_RAW, TCBNN_RES_I32, FW_NONE>(p, pl, stream)
+                                        : launch<4, 2, FM_RAW, TCBNN_RES_I32, FW_NONE>(p, pl, stream));
+    return pl.mt == 1 ? launch<1, 1, FM_BITS, TCBNN_RES_I32, FW_NONE>(p, pl, stream)
+                      : (pl.mt == 2 ? launch<2, 2, FM_BITS, TCBNN_RES_I32, FW_NONE>(p, pl, stream)
+                                    : launch<4, 2, FM_BITS, TCBNN_RES_I32, FW_NONE>(p, pl, stream));
+}
+
+}  // namespace tcbnn

@@ -509,6 +509,10 @@ int mfma_ksplit(const BgemmParams& p, int variant) {
 }  // namespace
 
 void bgemm_mfma_kernel_name(const BgemmParams& p, int variant, char* buf, size_t len) {
+    if (variant == TCBNN_VARIANT_MFMA_F4 && bgemm_flat_preferred(p)) {
+        bgemm_flat_kernel_name(p, buf, len);
+        return;
+    }
     if (variant == TCBNN_VARIANT_MFMA_F4 && conv3x3_mfma_applicable(p)) {
         conv3x3_mfma_kernel_name(p, buf, len);
         return;
@@ -521,6 +525,10 @@ void bgemm_mfma_kernel_name(const BgemmParams& p, int variant, char* buf, size_t
         fc_mfma_kernel_name(p, buf, len);
         return;
     }
+    if (variant == TCBNN_VARIANT_MFMA_F4 && bgemm_flat_applicable(p)) {
+        bgemm_flat_kernel_name(p, buf, len);
+        return;
+    }
     BgemmParams q = p;
     q.ksplit = mfma_ksplit(p, variant);
     snprintf(buf, len, "bgemm_mfma_kernel<%d, %d, %d>", variant == TCBNN_VARIANT_MFMA_F4 ? FMT_F4 : FMT_I8,
@@ -529,10 +537,12 @@ void bgemm_mfma_kernel_name(const BgemmParams& p, int variant, char* buf, size_t
 
 int launch_bgemm_mfma(const BgemmParams& p_in, int variant, hipStream_t stream) {
     if (int rc = validate_bgemm(p_in)) return rc;
+    if (variant == TCBNN_VARIANT_MFMA_F4 && bgemm_flat_preferred(p_in)) return launch_bgemm_flat(p_in, stream);
     if (variant == TCBNN_VARIANT_MFMA_F4 && conv3x3_mfma_applicable(p_in))
         return launch_conv3x3_mfma(p_in, stream);
     if (variant == TCBNN_VARIANT_MFMA_F4 && gemm_mfma_applicable(p_in)) return launch_gemm_mfma(p_in, stream);
     if (variant == TCBNN_VARIANT_MFMA_F4 && fc_mfma_applicable(p_in)) return launch_fc_mfma(p_in, stream);
+    if (variant == TCBNN_VARIANT_MFMA_F4 && bgemm_flat_applicable(p_in)) return launch_bgemm_flat(p_in, stream);
     if ((long long)p_in.cw * p_in.B * 4 >= (1LL << 31))
         return fail(TCBNN_EUNSUPPORTED, "bgemm: one pixel's activation words must stay below 2 GiB");
     BgemmParams p = p_in;

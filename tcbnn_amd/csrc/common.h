@@ -222,10 +222,15 @@ __host__ __device__ inline size_t fc_weight_row_words(int npad, int kw) { return
 __host__ __device__ inline size_t fc_weight_lane_words(int npad, int kw) { return (size_t)npad * 8 * ((kw + 7) / 8); }
 // persistent FP4 matrix-core kernel for 3x3 convolutions with Cin = 64 / 128 / 192 / 256 / 384 / 512
 bool conv3x3_mfma_applicable(const BgemmParams& p);
+int conv3x3_mfma_image_tiles(const BgemmParams& p);  // 32-image tiles per wave
 int launch_conv3x3_mfma(const BgemmParams& p, hipStream_t stream);
 void conv3x3_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len);
 // FP4 matrix-core kernel for small fully connected layers (K split over the waves of a workgroup)
 // large unmasked bit-GEMMs (stand-alone product, FC layers at large batch)
+bool bgemm_flat_applicable(const BgemmParams& p);
+bool bgemm_flat_preferred(const BgemmParams& p);  // over conv3x3_mfma, where both apply
+int launch_bgemm_flat(const BgemmParams& p, hipStream_t stream);
+void bgemm_flat_kernel_name(const BgemmParams& p, char* buf, size_t len);
 bool gemm_mfma_applicable(const BgemmParams& p);
 int launch_gemm_mfma(const BgemmParams& p, hipStream_t stream);
 void gemm_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len);

@@ -1329,6 +1329,8 @@ bool conv3x3_mfma_applicable(const BgemmParams& p) {
            (long long)p.PH * p.PW < (1 << 24) && within_2gib(p);
 }
 
+int conv3x3_mfma_image_tiles(const BgemmParams& p) { return pick(p).mt; }
+
 void conv3x3_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len) {
     const Pick k = pick(p);
     const int res_lim = p.res_in != nullptr ? std::min(std::min(p.res_limit, p.res_in_ch), p.N) : 0;

@@ -1365,6 +1365,47 @@ def test_avgpool_fc(gpu, b, h, c, n, fmt):
     layer.release()
 
 
+@pytest.mark.parametrize("b,h,cin,cout,R,pool,res", [
+    # the flat kernel's tiles and their edges: one MFMA, K in eight slices and in one; 2 x 2; 4 x 2 (column and channel remainders)
+    (1, 1, 32, 1, 1, 1, None), (3, 5, 512, 64, 3, 1, None), (7, 50, 96, 310, 3, 1, None), (9, 64, 32, 250, 1, 1, None),
+    # windows in lanes, in four column tiles of one and of two channel tiles; FC-ready padding words
+    (1, 2, 64, 40, 5, 2, None), (3, 6, 512, 128, 3, 2, None), (5, 64, 96, 250, 3, 2, None), (9, 64, 32, 230, 1, 2, None),
+    # residuals in both tile sizes and all formats
+    (2, 6, 512, 64, 3, 1, 2), (6, 64, 96, 230, 1, 1, 2), (5, 64, 32, 250, 1, 1, 1), (5, 64, 32, 250, 1, 1, 0)])
+def test_conv128_flat_columns(gpu, b, h, cin, cout, R, pool, res):
+    r = rng(7 * b + h + cin + cout)
+    x = rm.pm1(r, (b, h, h, cin))
+    f = rm.pm1(r, (R, R, cin, cout))
+    bn = r.normal(0, np.sqrt(R * R * cin), cout).astype(np.float32)
+    inp, filt = orc.pack_conv_input_nhwc(x), orc.pack_conv_filter(f)
+    kw, okw = {}, {}
+    if res is not None:
+        src = r.integers(-900, 900, size=(h, h, b, cout)).astype(np.int32)
+        okw = dict(save_residual=True, inject_residual=True, residual_channels=cout // 2 if cout % 64 == 0 else cout - 1,
+                   res_in=src)
+        kw = dict(okw, in_fmt=res, out_fmt=res)
+    want, wres = orc.conv128(inp, filt, bn, cin, cout, R, R, 1, True, pool, pool == 2, **okw)
+    layer = _run_conv_layer(gpu, "mfma_f4", x, f, bn, 1, pool, pool == 2, **kw)
+    assert layer.kernel_name().startswith("bgemm_flat_f4_kernel<"), layer.kernel_name()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    if res is not None:
+        np.testing.assert_array_equal(layer.download_residual(), wres)
+    layer.release()
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 32, 32), (33, 64, 8192), (700, 2048, 160), (1025, 3072, 96),
+                                   # the large kernel with an odd number of words per row
+                                   (4100, 992, 32), (4100, 1056, 544), (8200, 1024, 7200)])
+def test_bmm_flat_and_odd_words(gpu, m, n, k):
+    test_bmm(gpu, "mfma_f4", m, n, k)
+
+
+@pytest.mark.parametrize("b,h,cin,cout,R,stride", [(1, 1, 32, 8, 5, 1), (7, 50, 96, 320, 3, 1), (9, 64, 32, 256, 1, 1),
+                                                   (3, 7, 512, 100, 3, 2), (2, 33, 128, 255, 3, 1)])
+def test_bconv_flat_columns(gpu, b, h, cin, cout, R, stride):
+    test_bconv_odd_shapes(gpu, "mfma_f4", b, h, cin, cout, R, stride)
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2])
 @pytest.mark.parametrize("b,h,c,pad", [(2, 5, 16, 0), (6, 8, 33, 2), (66, 4, 64, 1), (4, 3, 130, 2)])
 def test_pool3x3_stride2(gpu, b, h, c, pad, fmt):
