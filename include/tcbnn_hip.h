@@ -128,6 +128,18 @@ int tcbnn_inconv_residual_bound_of_input(const float* input_host, int batch, int
 /* max |x| over a HOST array (on a few host threads; +infinity if any value is NaN or infinite): the cheap first test of
  * a new first-layer batch against the recorded bound, before the window scan above. */
 float tcbnn_host_abs_max(const float* values_host, size_t count);
+/* Uploads of new input batches.  An uploader holds pinned memory (at most 64 MiB; arrays of up to `bytes` bytes, longer
+ * ones go through it in turns) and shares a few worker threads with the process's other uploaders; they end with the
+ * last one.  tcbnn_upload copies `bytes` of HOST memory to the device, in the order of the null stream, and is complete
+ * when it returns.  tcbnn_upload_stage (an uploader created with staged = 1) copies an array of floats out of
+ * HOST memory, takes max |x| on the way (as tcbnn_host_abs_max) and leaves the destination alone;
+ * tcbnn_upload_commit then writes the staged array to `dst`.  Calls on one uploader exclude each other. */
+typedef struct tcbnn_uploader tcbnn_uploader;
+int tcbnn_uploader_create(size_t bytes, int staged, tcbnn_uploader** out);
+void tcbnn_uploader_destroy(tcbnn_uploader* uploader);
+int tcbnn_upload(tcbnn_uploader* uploader, void* dst, const void* src_host, size_t bytes);
+int tcbnn_upload_stage(tcbnn_uploader* uploader, const float* src_host, size_t count, float* abs_max);
+int tcbnn_upload_commit(tcbnn_uploader* uploader, void* dst);
 int tcbnn_conv_residual_bound(int input_channels, int filter_height, int filter_width, int injected_bound);
 int tcbnn_residual_format_for_bound(int bound);
 int tcbnn_residual_format_narrowest(int bound, int batch);

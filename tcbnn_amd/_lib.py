@@ -101,6 +101,11 @@ ABI = {
     "tcbnn_residual_bytes": (c_size_t, [c_int] * 5),
     "tcbnn_inconv_residual_bound": (c_int, [c_int, c_int, C.c_float]),
     "tcbnn_host_abs_max": (C.c_float, [c_void_p, c_size_t]),
+    "tcbnn_uploader_create": (c_int, [c_size_t, c_int, C.POINTER(c_void_p)]),
+    "tcbnn_uploader_destroy": (None, [c_void_p]),
+    "tcbnn_upload": (c_int, [c_void_p, c_void_p, c_void_p, c_size_t]),
+    "tcbnn_upload_stage": (c_int, [c_void_p, c_void_p, c_size_t, C.POINTER(C.c_float)]),
+    "tcbnn_upload_commit": (c_int, [c_void_p, c_void_p]),
     "tcbnn_conv_residual_bound": (c_int, [c_int] * 4),
     "tcbnn_residual_format_for_bound": (c_int, [c_int]),
     "tcbnn_residual_format_narrowest": (c_int, [c_int, c_int]),
@@ -163,6 +168,8 @@ _hip.hipGetErrorString.restype = C.c_char_p
 _hip.hipGetErrorString.argtypes = [c_int]
 _hip.hipMalloc.argtypes = [C.POINTER(c_void_p), c_size_t]
 _hip.hipFree.argtypes = [c_void_p]
+_hip.hipHostMalloc.argtypes = [C.POINTER(c_void_p), c_size_t, C.c_uint]
+_hip.hipHostFree.argtypes = [c_void_p]
 _hip.hipMemcpy.argtypes = [c_void_p, c_void_p, c_size_t, c_int]
 _hip.hipMemset.argtypes = [c_void_p, c_int, c_size_t]
 _hip.hipMemsetAsync.argtypes = [c_void_p, c_int, c_size_t, c_void_p]

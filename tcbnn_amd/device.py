@@ -58,6 +58,71 @@ class DeviceBuffer:
             pass
 
 
+class PinnedBuffer:
+    """Owning handle on pinned host memory, for results that are downloaded over and over."""
+
+    def __init__(self, nbytes):
+        self.nbytes = int(nbytes)
+        p = C.c_void_p(0)
+        hip_check(hip.hipHostMalloc(C.byref(p), max(self.nbytes, 4), 0), "hipHostMalloc(%d)" % self.nbytes)
+        self.ptr = p.value
+        self.bytes = np.ctypeslib.as_array((C.c_uint8 * self.nbytes).from_address(self.ptr))
+
+    def download(self, src, dtype, shape):
+        """A new array of the device buffer's first bytes (a copy to pageable memory takes 25 us where this takes 10)."""
+        out = np.empty(shape, dtype=dtype)
+        assert out.nbytes <= min(self.nbytes, src.nbytes), (out.nbytes, self.nbytes, src.nbytes)
+        if out.nbytes:
+            hip_check(hip.hipMemcpy(self.ptr, src.ptr, out.nbytes, _lib.D2H), "hipMemcpy D2H")
+            out.reshape(-1).view(np.uint8)[:] = self.bytes[:out.nbytes]
+        return out
+
+    def free(self):
+        if getattr(self, "ptr", None):
+            self.bytes = None
+            hip.hipHostFree(self.ptr)
+            self.ptr = None
+
+    def __del__(self):
+        try:
+            self.free()
+        except Exception:
+            pass
+
+
+class Uploader:
+    """Uploads of new input batches through pinned memory (tcbnn_upload)."""
+
+    def __init__(self, nbytes, staged=False):
+        p = C.c_void_p(0)
+        _lib.check(_lib.lib.tcbnn_uploader_create(int(nbytes), int(staged), C.byref(p)))
+        self.handle = p.value
+
+    def upload(self, dst, arr):
+        assert arr.nbytes <= dst.nbytes
+        _lib.check(_lib.lib.tcbnn_upload(self.handle, dst.ptr, arr.ctypes.data, arr.nbytes))
+
+    def stage(self, arr):
+        """max |x| of the array, which commit() writes to its destination."""
+        most = C.c_float(0)
+        _lib.check(_lib.lib.tcbnn_upload_stage(self.handle, arr.ctypes.data, arr.size, C.byref(most)))
+        return most.value
+
+    def commit(self, dst):
+        _lib.check(_lib.lib.tcbnn_upload_commit(self.handle, dst.ptr))
+
+    def free(self):
+        if getattr(self, "handle", None):
+            _lib.lib.tcbnn_uploader_destroy(self.handle)
+            self.handle = None
+
+    def __del__(self):
+        try:
+            self.free()
+        except Exception:
+            pass
+
+
 class Stream:
     """A HIP stream at the default priority."""
 

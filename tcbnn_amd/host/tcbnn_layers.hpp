@@ -635,11 +635,13 @@ class InConv128LayerParam {  // param.h:701-870
     void set_input(float* input) {
         CHECK_NULL_POINTER(input);
         CHECK_NULL_POINTER(input_gpu);
+        if (uploader == NULL) TCBNN_SAFE_CALL(tcbnn_uploader_create(input_bytes(), save_residual ? 1 : 0, &uploader));
         if (save_residual) {
+            float abs_max = 0.0f;
+            TCBNN_SAFE_CALL(tcbnn_upload_stage(uploader, input, (size_t)input_size(), &abs_max));
             const tcbnn_host::ResidualInfo* u = tcbnn_host::find_residual(output_residual_gpu);
             const int recorded = u != NULL ? u->bound : residual_info.bound;
-            const int coarse = tcbnn_inconv_residual_bound(filter_height, filter_width,
-                                                           tcbnn_host_abs_max(input, (size_t)input_size()));
+            const int coarse = tcbnn_inconv_residual_bound(filter_height, filter_width, abs_max);
             if (coarse > recorded) {
                 const int limit = tcbnn_host::residual_bound_limit(output_residual_gpu);
                 const int bound = coarse <= limit ? coarse : residual_bound_of(input);
@@ -651,9 +653,11 @@ class InConv128LayerParam {  // param.h:701-870
                 }
                 tcbnn_host::raise_residual_bound(output_residual_gpu, bound);
             }
+            TCBNN_SAFE_CALL(tcbnn_upload_commit(uploader, input_gpu));
+        } else {
+            TCBNN_SAFE_CALL(tcbnn_upload(uploader, input_gpu, input, input_bytes()));
         }
         this->input = input;
-        HIP_SAFE_CALL(hipMemcpy(input_gpu, input, input_bytes(), hipMemcpyHostToDevice));
         pack_input();
     }
     uin32* get_output_gpu() { return this->output_gpu; }
@@ -713,6 +717,8 @@ class InConv128LayerParam {  // param.h:701-870
         SAFE_FREE_HOST(output);
         SAFE_FREE_GPU(input_gpu);
         SAFE_FREE_GPU(input_packed_gpu);
+        tcbnn_uploader_destroy(uploader);
+        uploader = NULL;
         SAFE_FREE_GPU(output_gpu);
         SAFE_FREE_GPU(filter_gpu);
         SAFE_FREE_GPU(bn_gpu);
@@ -757,6 +763,7 @@ class InConv128LayerParam {  // param.h:701-870
     uin32* output_fmt_gpu = NULL;        // reference-layout copies of the output and the saved residual
     int* output_residual_ref_gpu = NULL;
     bool packed_input = false;           // use_packed_input()
+    tcbnn_uploader* uploader = NULL;     // set_input's pinned memory, made by the first call
     float* input_packed_gpu = NULL;      // [Hp][Wp][batch][3] copy of input_gpu (un-pooled layers, on request)
 };
 

@@ -20,7 +20,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import lib, check
-from .device import DeviceBuffer
+from .device import DeviceBuffer, PinnedBuffer, Uploader
 
 
 def STEP8(x):
@@ -256,7 +256,7 @@ class In128LayerParam(_ReferenceLayoutIO):
         self.name = name
         self.input_height = self.output_height = input_height
         self.input_width = self.output_width = input_width
-        self.input_gpu = self.output_gpu = None
+        self.input_gpu = self.output_gpu = self._uploader = None
 
     def output_bit_size(self):
         return PAD8(self.output_height) * STEP128(self.output_width)
@@ -273,7 +273,10 @@ class In128LayerParam(_ReferenceLayoutIO):
         return self
 
     def set_input(self, input):
-        self.input_gpu.upload(np.ascontiguousarray(input, dtype=np.float32))
+        x = np.ascontiguousarray(input, dtype=np.float32)
+        if self._uploader is None:
+            self._uploader = Uploader(self.input_gpu.nbytes)
+        self._uploader.upload(self.input_gpu, x)
 
     def get_output_gpu(self):
         return self.output_gpu
@@ -294,10 +297,10 @@ class In128LayerParam(_ReferenceLayoutIO):
 
     def release(self):
         self._release_ref_bufs()
-        for b in (self.input_gpu, self.output_gpu):
+        for b in (self.input_gpu, self.output_gpu, self._uploader):
             if b is not None:
                 b.free()
-        self.input_gpu = self.output_gpu = None
+        self.input_gpu = self.output_gpu = self._uploader = None
 
 
 def _fc_download_fmt(buf, batch, features):
@@ -404,7 +407,7 @@ class Out128LayerParam(_ReferenceLayoutIO):
         self.output_height, self.output_width = input_height, weight_width
         self.variant = variant
         self.weight = self.bn_scale = self.bn_bias = None
-        self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = self.input_gpu = None
+        self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = self.input_gpu = self._host = None
 
     def weight_size(self):
         return self.weight_height * self.weight_width
@@ -451,14 +454,16 @@ class Out128LayerParam(_ReferenceLayoutIO):
         return buf.value.decode()
 
     def download_output(self):
-        return self.output_gpu.to_numpy(np.float32, (self.output_height, self.output_width))
+        if self._host is None:
+            self._host = PinnedBuffer(self.output_gpu.nbytes)
+        return self._host.download(self.output_gpu, np.float32, (self.output_height, self.output_width))
 
     def release(self):
         self._release_ref_bufs()
-        for b in (self.weight_gpu, self.bn_scale_gpu, self.bn_bias_gpu, self.output_gpu):
+        for b in (self.weight_gpu, self.bn_scale_gpu, self.bn_bias_gpu, self.output_gpu, self._host):
             if b is not None:
                 b.free()
-        self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = None
+        self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = self._host = None
 
 
 class _ConvGeometry(_ReferenceLayoutIO):
@@ -598,7 +603,7 @@ class InConv128LayerParam(_ConvGeometry):
         self.save_residual = save_residual
         self.filter = self.bn = None
         self.input_gpu = self.filter_gpu = self.bn_gpu = self.output_gpu = self.output_residual_gpu = None
-        self.input_packed_gpu = None
+        self.input_packed_gpu = self._uploader = None
         self._derive()
 
     def input_size(self):
@@ -663,10 +668,11 @@ class InConv128LayerParam(_ConvGeometry):
         skipped when R*S*3*max|x| already fits."""
         x = np.ascontiguousarray(input, dtype=np.float32)
         assert x.size == self.input_size(), (x.size, self.input_size())
+        if self._uploader is None:
+            self._uploader = Uploader(self.input_gpu.nbytes, staged=self.save_residual)
         if self.save_residual:
             buf = self.output_residual_gpu
-            coarse = lib.tcbnn_inconv_residual_bound(self.filter_height, self.filter_width,
-                                                     lib.tcbnn_host_abs_max(x.ctypes.data, x.size))
+            coarse = lib.tcbnn_inconv_residual_bound(self.filter_height, self.filter_width, self._uploader.stage(x))
             limit = _residual_bound_limit(buf)
             if coarse > buf.bound:
                 bound = coarse if coarse <= limit else self._residual_bound(x)
@@ -674,7 +680,9 @@ class InConv128LayerParam(_ConvGeometry):
                     raise _lib.TcbnnError("input magnitude (window sums of |x| up to %d) exceeds what the residual "
                                           "formats chosen at initialize() hold (up to %d)" % (bound, limit))
                 _raise_residual_bound(buf, bound)
-        self.input_gpu.upload(x)
+            self._uploader.commit(self.input_gpu)
+        else:
+            self._uploader.upload(self.input_gpu, x)
         self._pack_input()
 
     def _desc(self):
@@ -701,11 +709,11 @@ class InConv128LayerParam(_ConvGeometry):
     def release(self):
         self._release_ref_bufs()
         for b in (self.input_gpu, self.input_packed_gpu, self.filter_gpu, self.bn_gpu, self.output_gpu,
-                  self.output_residual_gpu):
+                  self.output_residual_gpu, self._uploader):
             if b is not None:
                 b.free()
         self.input_gpu = self.filter_gpu = self.bn_gpu = self.output_gpu = self.output_residual_gpu = None
-        self.input_packed_gpu = None
+        self.input_packed_gpu = self._uploader = None
 
 
 class Conv128LayerParam(_ConvGeometry):
@@ -924,7 +932,7 @@ class AvgPoolFcLayerParam:
         self.name = name
         self.input_height, self.input_width = input_height, input_width
         self.channels, self.batch, self.out_features = channels, batch, out_features
-        self.input_residual_gpu = self.weight_gpu = self.bias_gpu = self.output_gpu = None
+        self.input_residual_gpu = self.weight_gpu = self.bias_gpu = self.output_gpu = self._host = None
 
     def initialize(self, config_file, input_residual_gpu):
         if input_residual_gpu is None:
@@ -954,10 +962,12 @@ class AvgPoolFcLayerParam:
         return "avgpool_fc_kernel<%d>" % self.input_residual_gpu.format
 
     def download_output(self):
-        return self.output_gpu.to_numpy(np.float32, (self.batch, self.out_features))
+        if self._host is None:
+            self._host = PinnedBuffer(self.output_gpu.nbytes)
+        return self._host.download(self.output_gpu, np.float32, (self.batch, self.out_features))
 
     def release(self):
-        for b in (self.weight_gpu, self.bias_gpu, self.output_gpu):
+        for b in (self.weight_gpu, self.bias_gpu, self.output_gpu, self._host):
             if b is not None:
                 b.free()
-        self.weight_gpu = self.bias_gpu = self.output_gpu = None
+        self.weight_gpu = self.bias_gpu = self.output_gpu = self._host = None

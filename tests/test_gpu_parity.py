@@ -1406,6 +1406,28 @@ def test_bconv_flat_columns(gpu, b, h, cin, cout, R, stride):
     test_bconv_odd_shapes(gpu, "mfma_f4", b, h, cin, cout, R, stride)
 
 
+@pytest.mark.parametrize("n", [1, 32767, 32769, 131073, (1 << 20) - 1, (1 << 20) + 5, (4 << 20) + 3, (17 << 20) + 1])
+def test_uploads_through_pinned_memory(gpu, n):
+    """Edges of an uploader: one value, pieces of 128 KiB, worker threads, overlapped chunks, streaming stores, arrays
+    longer than the pinned memory; the maximum sees every value and the destination nothing before the commit."""
+    from tcbnn_amd.device import DeviceBuffer, Uploader
+    x = rng(n).standard_normal(n).astype(np.float32)
+    x[-1] = -9.5
+    dst = DeviceBuffer.zeros(x.nbytes)
+    staged, plain = Uploader(x.nbytes, staged=True), Uploader(x.nbytes)
+    assert staged.stage(x) == 9.5
+    assert not dst.to_numpy(np.float32, (n,)).any()
+    staged.commit(dst)
+    np.testing.assert_array_equal(dst.to_numpy(np.float32, (n,)), x)
+    y = -x
+    y[n // 2] = np.nan
+    assert staged.stage(y) == np.inf
+    plain.upload(dst, y[:n])
+    np.testing.assert_array_equal(dst.to_numpy(np.float32, (n,)), y)
+    for b in (staged, plain, dst):
+        b.free()
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2])
 @pytest.mark.parametrize("b,h,c,pad", [(2, 5, 16, 0), (6, 8, 33, 2), (66, 4, 64, 1), (4, 3, 130, 2)])
 def test_pool3x3_stride2(gpu, b, h, c, pad, fmt):
