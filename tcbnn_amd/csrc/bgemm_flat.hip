@@ -20,6 +20,7 @@
 // ones by instruction issue: expanding the operands takes 7 VALU instructions per fragment, plus 5 per column tile and
 // step for address and border, against 32 cycles per MFMA.
 #include <algorithm>
+#include <initializer_list>
 
 #include "common.h"
 #include "mfma_util.h"
@@ -51,12 +52,23 @@ FastDiv fast_div(uint32_t d) {
 }
 __device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv& f) { return (__umulhi(n, f.mul) + n) >> f.shift; }
 
+// Everything the kernel reads, and nothing else: it is fetched in one go at the start (see fetch_now).
 struct FlatArgs {
-    FastDiv by_batch, by_row, by_cw, by_s;  // columns per item, items per row, words per tap, taps per filter row
-    int cols, n_tiles_c, n_groups, kw_tot, groups, per_slice, slices;
-    int total;  // tiles (column groups x channel groups) of the launch
+    const uint32_t* act;
+    const uint32_t* wgt;
+    const float* bn;
+    const int32_t* res_in;
+    uint32_t* out_bits;
+    int32_t* out_i32;
+    int32_t* res_out;
+    long long bits_pix_stride, raw_pix_stride, raw_b_stride;
+    FastDiv by_batch, by_row, by_cw, by_s, by_groups;  // columns per item, items per row, words per tap, taps per filter row
+    int B, cw, H, W, R, S, stride_h, stride_w, pad_h, pad_w, PW, N, k_tap, nan_bit, bits_row_words;
+    int res_in_ch, res_out_fmt, res_lim;
+    int cols, n_groups, kw_tot, groups, per_slice, slices;
+    int total;         // tiles (column groups x channel groups) of the launch
+    int wgs, per_xcd;  // workgroups with work, and how many of them an XCD gets
     unsigned act_bytes, wgt_bytes;
-    int res_lim;
 };
 
 constexpr int raw_pitch(int nt) { return 32 * nt + 4; }  // words; an odd multiple of 4: conflict-free both ways
@@ -64,45 +76,56 @@ constexpr int max_waves(int mt, int nt) { return mt * nt == 1 ? 8 : 4; }
 // groups of operand words in flight per wave (registers)
 constexpr int ring_depth(int mt, int nt, int fm) { return mt * nt >= 8 ? 1 : (mt * nt >= 4 || fm == FM_RESPOOL ? 2 : 4); }
 
+template <typename T>
+__device__ __forceinline__ void fetch_one(T v) {
+    asm volatile("" ::"s"(v));
+}
+
 template <int MT, int NT, int FM, int RF, int WIN>
 __global__ __launch_bounds__(64 * max_waves(MT, NT)) __attribute__((amdgpu_waves_per_eu(MT * NT == 1 ? 4 : 2))) void
-bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, const uint32_t* __restrict__ wgt,
-                     const float* __restrict__ bnp, const int32_t* __restrict__ rin, const FlatArgs f) {
+bgemm_flat_f4_kernel(const FlatArgs p) {
     static_assert(WIN == FW_NONE || (FM == FM_BITS && MT == (WIN == FW_TILES ? 4 : 1)), "see FW_*");
     static_assert(FM != FM_RESPOOL || MT == 1, "four source pixels per column");
     constexpr bool kRes = FM == FM_RES || FM == FM_RESPOOL;
     constexpr int D = ring_depth(MT, NT, FM);
+    // Left to the compiler, an argument is a scalar load right before its first use: four round trips one after the
+    // other before the first activation is asked for.
+    auto fetch_now = [](auto... v) __attribute__((always_inline)) { (void)std::initializer_list<int>{(fetch_one(v), 0)...}; };
+    fetch_now(p.act, p.wgt, p.by_batch.mul, p.by_row.mul, p.by_cw.mul, p.by_s.mul, p.by_groups.mul, p.B, p.cw, p.H, p.W, p.R,
+              p.S, p.stride_h, p.stride_w, p.pad_h, p.pad_w, p.PW, p.N, p.k_tap, p.cols, p.kw_tot, p.groups, p.slices, p.wgs,
+              p.act_bytes, p.wgt_bytes);
+    if constexpr (FM == FM_RAW) fetch_now(p.out_i32, p.raw_pix_stride, p.raw_b_stride);
+    else fetch_now(p.bn, p.out_bits, p.bits_pix_stride, p.nan_bit, p.bits_row_words);
+    if constexpr (kRes) fetch_now(p.res_in, p.res_out, p.res_in_ch, p.res_out_fmt, p.res_lim);
     extern __shared__ v4i lds_dyn[];
     const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int waves = blockDim.x >> 6;
     // Tiles are dealt so that each XCD (workgroups go to the 8 of them in turn) gets a contiguous run: neighbouring
     // pixels share activation rows, and the channel groups of a column tile all of them.
-    const int per_wg = f.slices > 1 ? 1 : waves;
-    const int wgs = (f.total + per_wg - 1) / per_wg;
-    const int per_xcd = (wgs + 7) / 8;
-    const int wg = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    const int slice = f.slices > 1 ? wave : 0;
-    const int tile = f.slices > 1 ? wg : wg * waves + wave;
-    const bool live = (int)(blockIdx.x >> 3) < per_xcd && wg < wgs && tile < f.total;  // (uniform per wave)
-    const int ct = live ? tile / f.n_groups : 0, ng = live ? tile % f.n_groups : 0;
+    const int per_wg = p.slices > 1 ? 1 : waves;
+    const int wg = (int)(blockIdx.x & 7) * p.per_xcd + (int)(blockIdx.x >> 3);
+    const int slice = p.slices > 1 ? wave : 0;
+    const int tile = p.slices > 1 ? wg : wg * waves + wave;
+    const bool live = wg < p.wgs && tile < p.total;  // (uniform per wave)
+    const int ct = live ? (int)div_by((unsigned)tile, p.by_groups) : 0, ng = live ? tile - ct * p.n_groups : 0;
     const int n0 = ng * (32 * NT);
 
     v4i* red = lds_dyn;                                                           // [slices - 1][MT * NT][4][64]
-    int* raw_area = reinterpret_cast<int*>(red + (size_t)(f.slices - 1) * MT * NT * 256);
+    int* raw_area = reinterpret_cast<int*>(red + (size_t)(p.slices - 1) * MT * NT * 256);
     constexpr int kRawWords = FM == FM_RAW ? 32 * raw_pitch(NT) + 64 : 0;         // per tile of the workgroup
     int2* tab = reinterpret_cast<int2*>(raw_area + per_wg * kRawWords);           // [8 * groups]
 
-    const int g_begin = slice * f.per_slice, g_end = live ? min(f.groups, g_begin + f.per_slice) : 0;
+    const int g_begin = slice * p.per_slice, g_end = live ? min(p.groups, g_begin + p.per_slice) : 0;
 
     // ---- weights: lane (j, h) reads words 8g + 4h .. + 3 of its channel's row (past the last row: zeros; past the end
     // of a row: the next row's words, which meet activations that are zero)
     const __amdgpu_buffer_rsrc_t r_wgt =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(wgt), 0, (int)f.wgt_bytes, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.wgt), 0, (int)p.wgt_bytes, 0x00020000);
     unsigned wvoff[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
-        wvoff[nt] = ((unsigned)(n0 + nt * 32 + row_to_channel(j)) * (unsigned)f.kw_tot + 4u * (unsigned)h) * 4u;
+        wvoff[nt] = ((unsigned)(n0 + nt * 32 + row_to_channel(j)) * (unsigned)p.kw_tot + 4u * (unsigned)h) * 4u;
     v4i aw[D][NT];
     auto request_w = [&](int slot, int g) __attribute__((always_inline)) {
 #pragma unroll
@@ -125,14 +148,14 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
         if (!tiles || mt == 0) {
             const unsigned col = WIN == FW_LANES ? (unsigned)ct * 8u + (unsigned)(j & 7)
                                                  : (unsigned)(tiles ? ct : ct * MT + mt) * 32u + (unsigned)j;
-            const unsigned cc = min(col, (unsigned)f.cols - 1u);
-            const unsigned item = div_by(cc, f.by_batch);
-            cok[mt] = live && col < (unsigned)f.cols;
+            const unsigned cc = min(col, (unsigned)p.cols - 1u);
+            const unsigned item = div_by(cc, p.by_batch);
+            cok[mt] = live && col < (unsigned)p.cols;
             cpix[mt] = (int)item;
-            cb[mt] = (int)(cc - item * f.by_batch.d);
+            cb[mt] = (int)(cc - item * p.by_batch.d);
         }
         const int k = tiles ? 0 : mt;
-        const unsigned iy = div_by((unsigned)cpix[k], f.by_row), ix = (unsigned)cpix[k] - iy * f.by_row.d;
+        const unsigned iy = div_by((unsigned)cpix[k], p.by_row), ix = (unsigned)cpix[k] - iy * p.by_row.d;
         cy[mt] = WIN != FW_NONE ? 2 * (int)iy + (sub >> 1) : (int)iy;
         cx[mt] = WIN != FW_NONE ? 2 * (int)ix + (sub & 1) : (int)ix;
         const int ay0 = cy[mt] * p.stride_h - p.pad_h, ax0 = cx[mt] * p.stride_w - p.pad_w;
@@ -156,10 +179,10 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) thr[nt][v] = bnp[min(n0 + nt * 32 + 16 * h + v, p.N - 1)];
+            for (int v = 0; v < 16; ++v) thr[nt][v] = p.bn[min(n0 + nt * 32 + 16 * h + v, p.N - 1)];
     }
     if constexpr (kRes) {
-        if (fin && f.res_lim > 0) {
+        if (fin && p.res_lim > 0) {
             const unsigned G = (unsigned)(p.res_in_ch + (int)residual_group_channels(RF) - 1) / (unsigned)residual_group_channels(RF);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
@@ -175,7 +198,7 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
                         int* dst = rraw[mt * NT + nt][s];
                         if constexpr (RF == TCBNN_RES_I12) {
                             if (cbase < p.res_in_ch) {
-                                const uint32_t* w = reinterpret_cast<const uint32_t*>(rin) + (spix * G + cbase / 16) * (size_t)p.B * 6;
+                                const uint32_t* w = reinterpret_cast<const uint32_t*>(p.res_in) + (spix * G + cbase / 16) * (size_t)p.B * 6;
                                 const v4i a = *reinterpret_cast<const v4i*>(w + (size_t)b * 4);
                                 const int2 c = *reinterpret_cast<const int2*>(w + (size_t)p.B * 4 + (size_t)b * 2);
                                 dst[0] = a[0], dst[1] = a[1], dst[2] = a[2], dst[3] = a[3], dst[4] = c.x, dst[5] = c.y;
@@ -185,7 +208,7 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
 #pragma unroll
                             for (int g = 0; g < 16 / kCh; ++g)
                                 if (cbase + kCh * g < p.res_in_ch) {
-                                    const v4i a = reinterpret_cast<const v4i*>(rin)[(spix * G + cbase / kCh + g) * (size_t)p.B + b];
+                                    const v4i a = reinterpret_cast<const v4i*>(p.res_in)[(spix * G + cbase / kCh + g) * (size_t)p.B + b];
                                     dst[4 * g] = a[0], dst[4 * g + 1] = a[1], dst[4 * g + 2] = a[2], dst[4 * g + 3] = a[3];
                                 }
                         }
@@ -196,15 +219,15 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
     }
 
     // ---- the table of K: byte offset of word k's activation from the column's first tap, and its tap
-    for (int k = tid; k < 8 * f.groups; k += blockDim.x) {
-        const unsigned tap = div_by((unsigned)k, f.by_cw), w = (unsigned)k - tap * f.by_cw.d;
-        const unsigned r = div_by(tap, f.by_s), s = tap - r * f.by_s.d;
-        tab[k] = k < f.kw_tot ? make_int2((int)((r * (unsigned)p.W + s) * pix_b + w * row_b), (int)tap) : make_int2(0, kTapNone);
+    for (int k = tid; k < 8 * p.groups; k += blockDim.x) {
+        const unsigned tap = div_by((unsigned)k, p.by_cw), w = (unsigned)k - tap * p.by_cw.d;
+        const unsigned r = div_by(tap, p.by_s), s = tap - r * p.by_s.d;
+        tab[k] = k < p.kw_tot ? make_int2((int)((r * (unsigned)p.W + s) * pix_b + w * row_b), (int)tap) : make_int2(0, kTapNone);
     }
     __syncthreads();
 
     const __amdgpu_buffer_rsrc_t r_act =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(act), 0, (int)f.act_bytes, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.act), 0, (int)p.act_bytes, 0x00020000);
     uint32_t bw[D][MT][4];
     int tp[D][4];
     auto request_b = [&](int slot, int g) __attribute__((always_inline)) {
@@ -252,7 +275,7 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
         for (int d = 0; d < D; ++d) {
             const int g = g0 + d;
             if (g < g_end) {  // (uniform)
-                const int left = f.kw_tot - 8 * g;  // steps past the row's last word in both halves are not multiplied
+                const int left = p.kw_tot - 8 * g;  // steps past the row's last word in both halves are not multiplied
                 v4i a[NT];
                 uint32_t x[MT][4];
                 int tq[4];
@@ -289,7 +312,7 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
     }
 
     // ---- the slices' sums meet in LDS; wave 0 of the workgroup finishes the tile
-    if (f.slices > 1) {
+    if (p.slices > 1) {
         if (slice > 0) {
 #pragma unroll
             for (int t = 0; t < MT * NT; ++t)
@@ -321,7 +344,7 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
             int dot[16];
 #pragma unroll
             for (int v = 0; v < 16; ++v) dot[v] = (int)acc[mt][nt][v] - corr;
-            for (int s = 1; s < f.slices; ++s)
+            for (int s = 1; s < p.slices; ++s)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const v4i o = red[(((s - 1) * MT * NT + mt * NT + nt) * 4 + q) * 64 + lane];
@@ -329,7 +352,7 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
                     for (int e = 0; e < 4; ++e) dot[4 * q + e] += o[e];
                 }
             if constexpr (FM == FM_RAW) {
-                int* mine = raw_area + (f.slices > 1 ? 0 : wave) * kRawWords;
+                int* mine = raw_area + (p.slices > 1 ? 0 : wave) * kRawWords;
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     *reinterpret_cast<v4i*>(mine + j * raw_pitch(NT) + nt * 32 + 16 * h + 4 * q) =
@@ -337,7 +360,7 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
                 continue;
             }
             if constexpr (kRes) {
-                if (f.res_lim > 0) {
+                if (p.res_lim > 0) {
                     int rv[16];
 #pragma unroll
                     for (int s = 0; s < NSRC; ++s) {
@@ -357,7 +380,7 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
                         for (int v = 0; v < 16; ++v) rv[v] = s == 0 ? t[v] : max(rv[v], t[v]);
                     }
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) dot[v] += cbase + v < f.res_lim ? rv[v] : 0;
+                    for (int v = 0; v < 16; ++v) dot[v] += cbase + v < p.res_lim ? rv[v] : 0;
                 }
             }
             uint32_t hw = 0;
@@ -410,14 +433,14 @@ bgemm_flat_f4_kernel(const BgemmParams p, const uint32_t* __restrict__ act, cons
                 uint32_t* dst = p.out_bits + opix * (size_t)p.bits_pix_stride + b;
                 const int w = ng * NT + nt;
                 if (w < p.bits_row_words) dst[(size_t)w * p.B] = word;
-                if (ng == f.n_groups - 1 && nt == NT - 1)  // the pixel's padding words
-                    for (int z = max(ow, f.n_groups * NT); z < p.bits_row_words; ++z) dst[(size_t)z * p.B] = 0;
+                if (ng == p.n_groups - 1 && nt == NT - 1)  // the pixel's padding words
+                    for (int z = max(ow, p.n_groups * NT); z < p.bits_row_words; ++z) dst[(size_t)z * p.B] = 0;
             }
         }
         if constexpr (FM == FM_RAW) {
             // int32 output: a lane holds 16 channels of one column; through LDS (the same wave writes and reads) a
             // store instruction covers whole channel runs of its columns instead of 64 pieces of 16 bytes
-            int* mine = raw_area + (f.slices > 1 ? 0 : wave) * kRawWords;
+            int* mine = raw_area + (p.slices > 1 ? 0 : wave) * kRawWords;
             long long* start = reinterpret_cast<long long*>(mine + 32 * raw_pitch(NT));
             const long long at = (long long)pix * p.raw_pix_stride + (long long)b * p.raw_b_stride + n0;
             if (h == 0) start[j] = ok ? at : -1;
@@ -488,32 +511,40 @@ FlatPlan flat_plan(const BgemmParams& p) {
 
 template <int MT, int NT, int FM, int RF, int WIN>
 int launch(const BgemmParams& p, const FlatPlan& pl, hipStream_t stream) {
-    FlatArgs f;
+    FlatArgs f{};
     const int row = WIN != FW_NONE ? p.PW / 2 : p.PW;
     const long long items = WIN != FW_NONE ? (long long)(p.PH / 2) * (p.PW / 2) : (long long)p.PH * p.PW;
+    f.act = p.act, f.wgt = p.wgt, f.bn = p.bn, f.res_in = p.res_in;
+    f.out_bits = p.out_bits, f.out_i32 = p.out_i32, f.res_out = p.res_out;
+    f.bits_pix_stride = p.bits_pix_stride, f.raw_pix_stride = p.raw_pix_stride, f.raw_b_stride = p.raw_b_stride;
+    f.n_groups = (p.N + 32 * NT - 1) / (32 * NT);
     f.by_batch = fast_div((uint32_t)p.B);
     f.by_row = fast_div((uint32_t)row);
     f.by_cw = fast_div((uint32_t)p.cw);
     f.by_s = fast_div((uint32_t)p.S);
+    f.by_groups = fast_div((uint32_t)f.n_groups);
+    f.B = p.B, f.cw = p.cw, f.H = p.H, f.W = p.W, f.R = p.R, f.S = p.S;
+    f.stride_h = p.stride_h, f.stride_w = p.stride_w, f.pad_h = p.pad_h, f.pad_w = p.pad_w;
+    f.PW = p.PW, f.N = p.N, f.k_tap = p.k_tap, f.nan_bit = p.nan_bit, f.bits_row_words = p.bits_row_words;
+    f.res_in_ch = p.res_in_ch, f.res_out_fmt = p.res_out_fmt;
+    f.res_lim = p.res_in != nullptr ? std::min(std::min(p.res_limit, p.res_in_ch), p.N) : 0;
     f.cols = (int)(items * p.B);
-    f.n_groups = (p.N + 32 * NT - 1) / (32 * NT);
     f.kw_tot = p.R * p.S * p.cw;
     f.groups = (f.kw_tot + 7) / 8;
     f.per_slice = (f.groups + pl.slices - 1) / pl.slices;
     f.slices = pl.slices;
     const long long total = flat_tiles(p, MT, NT, WIN);
     f.total = (int)total;
-    f.n_tiles_c = (int)(total / f.n_groups);
     f.act_bytes = (unsigned)(4LL * p.H * p.W * p.cw * p.B);
     f.wgt_bytes = (unsigned)(4LL * pad32(p.N) * f.kw_tot);
-    f.res_lim = p.res_in != nullptr ? std::min(std::min(p.res_limit, p.res_in_ch), p.N) : 0;
     const int waves = pl.slices > 1 ? pl.slices : 4, per_wg = pl.slices > 1 ? 1 : waves;
     const long long wgs = (total + per_wg - 1) / per_wg, blocks = (wgs + 7) / 8 * 8;
+    f.wgs = (int)wgs;
+    f.per_xcd = (int)(blocks / 8);
     const size_t lds = (size_t)(pl.slices - 1) * MT * NT * 4096 +
                        (FM == FM_RAW ? (size_t)per_wg * (32 * raw_pitch(NT) + 64) * 4 : 0) + (size_t)f.groups * 64;
     if (blocks <= 0 || blocks > 0x7fffffffLL || lds > 64 * 1024) return fail(TCBNN_EINVAL, "bgemm_flat: launch too large");
-    hipLaunchKernelGGL((bgemm_flat_f4_kernel<MT, NT, FM, RF, WIN>), dim3((unsigned)blocks), dim3(64 * waves), lds, stream, p,
-                       p.act, p.wgt, p.bn, p.res_in, f);
+    hipLaunchKernelGGL((bgemm_flat_f4_kernel<MT, NT, FM, RF, WIN>), dim3((unsigned)blocks), dim3(64 * waves), lds, stream, f);
     TCBNN_LAUNCH_CHECK("bgemm_flat_f4_kernel");
     return TCBNN_OK;
 }
