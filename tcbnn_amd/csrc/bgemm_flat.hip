@@ -509,6 +509,17 @@ FlatPlan flat_plan(const BgemmParams& p) {
     return f;
 }
 
+// LDS of a workgroup: the sums of the slices, the staging area of int32 output, the table of K.  A workgroup gets 64 KiB
+// of it; a long K of int32 output can need more (above 4000 words where it is split over eight waves, above 3712 where
+// four waves stage a 2 x 2 tile each), and such a problem is left to the generic kernel.
+constexpr size_t kLdsMost = 64 * 1024;
+int flat_waves(const FlatPlan& pl) { return pl.slices > 1 ? pl.slices : 4; }
+int flat_tiles_per_wg(const FlatPlan& pl) { return pl.slices > 1 ? 1 : 4; }
+size_t flat_lds_bytes(const BgemmParams& p, const FlatPlan& pl) {
+    const size_t raw = p.mode == EPI_RAW ? (size_t)flat_tiles_per_wg(pl) * (32 * raw_pitch(pl.nt) + 64) * 4 : 0;
+    return (size_t)(pl.slices - 1) * pl.mt * pl.nt * 4096 + raw + (size_t)((p.R * p.S * p.cw + 7) / 8) * 64;
+}
+
 template <int MT, int NT, int FM, int RF, int WIN>
 int launch(const BgemmParams& p, const FlatPlan& pl, hipStream_t stream) {
     FlatArgs f{};
@@ -537,13 +548,12 @@ int launch(const BgemmParams& p, const FlatPlan& pl, hipStream_t stream) {
     f.total = (int)total;
     f.act_bytes = (unsigned)(4LL * p.H * p.W * p.cw * p.B);
     f.wgt_bytes = (unsigned)(4LL * pad32(p.N) * f.kw_tot);
-    const int waves = pl.slices > 1 ? pl.slices : 4, per_wg = pl.slices > 1 ? 1 : waves;
+    const int waves = flat_waves(pl), per_wg = flat_tiles_per_wg(pl);
     const long long wgs = (total + per_wg - 1) / per_wg, blocks = (wgs + 7) / 8 * 8;
     f.wgs = (int)wgs;
     f.per_xcd = (int)(blocks / 8);
-    const size_t lds = (size_t)(pl.slices - 1) * MT * NT * 4096 +
-                       (FM == FM_RAW ? (size_t)per_wg * (32 * raw_pitch(NT) + 64) * 4 : 0) + (size_t)f.groups * 64;
-    if (blocks <= 0 || blocks > 0x7fffffffLL || lds > 64 * 1024) return fail(TCBNN_EINVAL, "bgemm_flat: launch too large");
+    const size_t lds = flat_lds_bytes(p, pl);
+    if (blocks <= 0 || blocks > 0x7fffffffLL || lds > kLdsMost) return fail(TCBNN_EINVAL, "bgemm_flat: launch too large");
     hipLaunchKernelGGL((bgemm_flat_f4_kernel<MT, NT, FM, RF, WIN>), dim3((unsigned)blocks), dim3(64 * waves), lds, stream, f);
     TCBNN_LAUNCH_CHECK("bgemm_flat_f4_kernel");
     return TCBNN_OK;
@@ -569,7 +579,8 @@ bool bgemm_flat_applicable(const BgemmParams& p) {
     if (!pool1 && !pool2) return false;
     if (p.res_out_pool) return false;
     const long long cols = (long long)p.PH * p.PW * p.B;
-    return cols < (1LL << 30) && 4LL * p.H * p.W * p.cw * p.B < (1LL << 31) && 4LL * (p.N + 64) * kw_tot < (1LL << 31);
+    return cols < (1LL << 30) && 4LL * p.H * p.W * p.cw * p.B < (1LL << 31) && 4LL * (p.N + 64) * kw_tot < (1LL << 31) &&
+           flat_lds_bytes(p, flat_plan(p)) <= kLdsMost;
 }
 
 // Both kernels serve the 3x3 layers of conv3x3_mfma.hip: which is faster?  An estimate of both launches in microseconds,

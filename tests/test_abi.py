@@ -75,6 +75,21 @@ def test_errors_are_codes_not_exits():
         _lib.check(-1)
 
 
+def test_no_long_k_is_refused_for_its_lds():
+    """Int32 products and convolutions whose K is too long for the LDS of one kernel go to another one: on both sides of
+    every such limit a call fails for want of a device and of nothing else (where there is one, nothing is called: the
+    pointers are made up)."""
+    from tcbnn_amd import _lib
+    L = _lib.lib
+    if _lib.device_count() > 0:
+        pytest.skip("made-up pointers")
+    for m, n, k in ((32, 32, 128000), (32, 32, 128032), (1, 4096, 130816), (1, 4096, 130848)):
+        assert L.tcbnn_bmm(16, 16, 16, m, n, k, _lib.VARIANT_MFMA_F4, None) == -3, (m, n, k, L.tcbnn_last_error())
+    for b, hw, cin, cout in ((64, 28, 4736, 256), (64, 28, 4768, 256), (64, 28, 5120, 256), (64, 56, 4800, 512)):
+        assert L.tcbnn_bconv(16, 16, 16, b, hw, hw, cin, cout, 5, 5, 1, 1, 2, 2, hw, hw, _lib.VARIANT_MFMA_F4, None) == -3, \
+            (b, hw, cin, cout, L.tcbnn_last_error())
+
+
 def test_network_specs_match_reference_wiring():
     from tcbnn_amd import nets
     spec = nets.imagenet_resnet_spec(batch=256)

@@ -29,7 +29,9 @@ def _variant(gpu, name):
                                    # K of 3, 8 and 24 k-steps (groups of 8, weight blocks of 16)
                                    (4100, 992, 192), (4100, 992, 512), (9000, 2048, 1536), (8192, 1024, 1024),
                                    # a last column group of 32 (its rows leave element-wise, the others through LDS)
-                                   (4100, 1056, 192)])
+                                   (4100, 1056, 192),
+                                   # K on both sides of what the LDS of the kernel for small products holds
+                                   (32, 32, 128000), (32, 32, 128032), (1, 4096, 130816)])
 def test_bmm(gpu, variant, m, n, k):
     r = rng(m + n + k)
     a = r.integers(0, 2 ** 32, size=(m, k // 32), dtype=np.uint64).astype(np.uint32)
