@@ -86,7 +86,7 @@ float magnitude(uint32_t pattern) {
 
 // One pass over an array, in pieces that any thread may take; chunks are runs of pieces.
 struct Job {
-    char* dst = nullptr;  // null: maximum only
+    char* dst = nullptr;
     const char* src = nullptr;
     size_t bytes = 0;
     std::atomic<size_t> next{0};
@@ -99,9 +99,9 @@ struct Job {
         const size_t p = next.fetch_add(1, std::memory_order_relaxed);
         if (p >= pieces()) return false;
         const size_t at = p * kPiece, n = std::min(kPiece, bytes - at);
-        const uint32_t m = copy_max(dst != nullptr ? reinterpret_cast<uint32_t*>(dst + at) : nullptr,
-                                    reinterpret_cast<const uint32_t*>(src + at), n / 4, bytes >= kStreamFrom);
-        if (n % 4 != 0 && dst != nullptr) memcpy(dst + at + n / 4 * 4, src + at + n / 4 * 4, n % 4);
+        const uint32_t m = copy_max(reinterpret_cast<uint32_t*>(dst + at), reinterpret_cast<const uint32_t*>(src + at), n / 4,
+                                    bytes >= kStreamFrom);
+        if (n % 4 != 0) memcpy(dst + at + n / 4 * 4, src + at + n / 4 * 4, n % 4);
         uint32_t seen = most.load(std::memory_order_relaxed);
         while (m > seen && !most.compare_exchange_weak(seen, m, std::memory_order_relaxed)) {
         }
@@ -111,6 +111,19 @@ struct Job {
         return true;
     }
 };
+
+// Up to n threads that run `work`: as many as can be had, none at worst (a limit on threads or memory is no reason to give
+// up what the caller can do alone, and a half-filled vector of running threads must not be destroyed).
+template <class F>
+std::vector<std::thread> start_threads(int n, F work) {
+    std::vector<std::thread> t;
+    try {
+        t.reserve((size_t)std::max(0, n));
+        while ((int)t.size() < n) t.emplace_back(work);
+    } catch (const std::exception&) {
+    }
+    return t;
+}
 
 // Worker threads, shared by all uploaders of the process and gone with the last of them.  One job at a time; a caller that
 // finds them busy does its job alone.
@@ -124,10 +137,7 @@ class Workers {
         if (!w) one = w = std::make_shared<Workers>();
         return w;
     }
-    Workers() {
-        const int n = std::min(kMostWorkers, (int)std::thread::hardware_concurrency() - 1);
-        for (int i = 0; i < n; ++i) threads_.emplace_back([this] { loop(); });
-    }
+    Workers() : threads_(start_threads(std::min(kMostWorkers, (int)std::thread::hardware_concurrency() - 1), [this] { loop(); })) {}
     ~Workers() {
         {
             std::lock_guard<std::mutex> l(m_);
@@ -174,11 +184,11 @@ class Workers {
     }
     std::mutex owner_, m_;
     std::condition_variable wake_, idle_;
-    std::vector<std::thread> threads_;
     Job* job_ = nullptr;
     uint64_t round_ = 0;
     int inside_ = 0;
     bool stop_ = false;
+    std::vector<std::thread> threads_;  // (last: started when all that they use is there)
 };
 
 }  // namespace
@@ -240,12 +250,15 @@ int pass(tcbnn_uploader* u, void* to, const void* src, size_t bytes, uint32_t* m
 
 extern "C" {
 
+// (no exception leaves an entry point: allocations of the host side that fail are an error code)
+static int out_of_memory(const char* what) { return fail(TCBNN_EINVAL, "%s: out of host memory", what); }
+
 int tcbnn_uploader_create(size_t bytes, int staged, tcbnn_uploader** out) {
     if (out == nullptr) return fail(TCBNN_ENULL, "NULL pointer: out");
     *out = nullptr;
     if (bytes == 0) return fail(TCBNN_EINVAL, "uploader: nothing to upload");
     std::unique_ptr<tcbnn_uploader> u(new (std::nothrow) tcbnn_uploader);
-    if (!u) return fail(TCBNN_EINVAL, "uploader: out of memory");
+    if (!u) return out_of_memory("uploader");
     u->bytes = bytes;
     u->pinned_bytes = std::min(kPinnedMost, (bytes + kPiece - 1) / kPiece * kPiece);
     if (int rc = check_hip(hipHostMalloc(&u->pinned, u->pinned_bytes, hipHostMallocDefault), "hipHostMalloc")) return rc;
@@ -257,7 +270,7 @@ int tcbnn_uploader_create(size_t bytes, int staged, tcbnn_uploader** out) {
     if (bytes > 4 * kPiece) {
         try {
             u->workers = Workers::get();
-        } catch (const std::exception&) {  // (no threads to be had: the caller's own does the work)
+        } catch (const std::exception&) {  // (no memory for them: the caller's own thread does the work)
         }
     }
     *out = u.release();
@@ -276,7 +289,11 @@ int tcbnn_upload(tcbnn_uploader* u, void* dst, const void* src_host, size_t byte
     if (bytes > u->bytes) return fail(TCBNN_EINVAL, "upload: longer than the uploader was made for");
     std::lock_guard<std::mutex> l(u->m);
     u->staged = 0;
-    return pass(u, dst, src_host, bytes, nullptr);
+    try {
+        return pass(u, dst, src_host, bytes, nullptr);
+    } catch (const std::bad_alloc&) {
+        return out_of_memory("upload");
+    }
 }
 
 int tcbnn_upload_stage(tcbnn_uploader* u, const float* src_host, size_t count, float* abs_max) {
@@ -287,7 +304,11 @@ int tcbnn_upload_stage(tcbnn_uploader* u, const float* src_host, size_t count, f
     std::lock_guard<std::mutex> l(u->m);
     u->on_device = u->device != nullptr;
     uint32_t most = 0;
-    if (int rc = pass(u, u->device, src_host, bytes, &most)) return rc;
+    try {
+        if (int rc = pass(u, u->device, src_host, bytes, &most)) return rc;
+    } catch (const std::bad_alloc&) {
+        return out_of_memory("upload_stage");
+    }
     u->staged = bytes;
     *abs_max = magnitude(most);
     return TCBNN_OK;
@@ -309,23 +330,25 @@ int tcbnn_upload_commit(tcbnn_uploader* u, void* dst) {
 // max |x| over a host array, on a few host threads (NaN or infinity anywhere: +infinity)
 float tcbnn_host_abs_max(const float* values_host, size_t count) {
     if (values_host == nullptr || count == 0) return 0.0f;
-    Job job;
-    job.src = reinterpret_cast<const char*>(values_host);
-    job.bytes = 4 * count;
-    job.chunk_end.push_back(job.pieces());
-    job.left.reset(new std::atomic<size_t>[1]);
-    job.left[0] = job.pieces();
-    std::vector<std::thread> helpers;
+    std::atomic<size_t> next{0};
+    std::atomic<uint32_t> most{0};
+    constexpr size_t kFloats = kPiece / 4;
+    auto work = [&] {
+        uint32_t m = 0;
+        for (;;) {
+            const size_t at = next.fetch_add(kFloats, std::memory_order_relaxed);
+            if (at >= count) break;
+            m = std::max(m, copy_max(nullptr, reinterpret_cast<const uint32_t*>(values_host) + at, std::min(kFloats, count - at), false));
+        }
+        uint32_t seen = most.load(std::memory_order_relaxed);
+        while (m > seen && !most.compare_exchange_weak(seen, m, std::memory_order_relaxed)) {
+        }
+    };
     const size_t n = std::min<size_t>(std::min<size_t>(count >> 20, 8), std::thread::hardware_concurrency());
-    for (size_t t = 1; t < n; ++t)
-        helpers.emplace_back([&job] {
-            while (job.work()) {
-            }
-        });
-    while (job.work()) {
-    }
+    std::vector<std::thread> helpers = start_threads((int)n - 1, work);
+    work();
     for (std::thread& t : helpers) t.join();
-    return magnitude(job.most.load());
+    return magnitude(most.load());
 }
 
 }  // extern "C"

@@ -9,6 +9,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -194,8 +196,8 @@ int tcbnn_residual_format_narrowest(int bound, int batch) {
 // magnitude is at most the window's sum of |x| (all three channels); fp32 rounding of the 3*R*S additions adds at
 // most 3*R*S*2^-24 of that relative, far inside the 0.1 % + 1 of slack taken here.  Per image: prefix sums of
 // |x| down the columns give every window's column sums with one subtraction, a prefix sum along the row gives the
-// window (double precision: the cancellation error is below 1e-10 of the sums).  Images are dealt to a few host
-// threads.
+// window (double precision: the cancellation error is below 1e-10 of the sums).  A few host threads, as many as can be
+// had, take images one after the other; without memory for the prefix sums the bound is unknown (INT32_MAX).
 int tcbnn_inconv_residual_bound_of_input(const float* input_host, int batch, int height, int width,
                                          int filter_height, int filter_width, int stride_height,
                                          int stride_width, int padding) {
@@ -208,44 +210,53 @@ int tcbnn_inconv_residual_bound_of_input(const float* input_host, int batch, int
     const int ow = tcbnn_conv_out(width, filter_width, stride_width, padding, 1);
     if (oh <= 0 || ow <= 0) return INT32_MAX;
     const size_t plane = (size_t)height * width;
-    const int n_threads = std::max(1, std::min(std::min(batch, 16), (int)std::thread::hardware_concurrency()));
-    std::vector<double> worst(n_threads, 0.0);
-    std::vector<char> bad(n_threads, 0);
-    auto scan = [&](int t) {
-        std::vector<double> down((size_t)(height + 1) * width), along(width + 1);
-        for (int b = t; b < batch && !bad[t]; b += n_threads) {
-            const float* img = input_host + (size_t)b * 3 * plane;
-            for (int x = 0; x < width; ++x) down[x] = 0.0;
-            for (int y = 0; y < height; ++y)
-                for (int x = 0; x < width; ++x) {
-                    const size_t i = (size_t)y * width + x;
-                    const double a = std::fabs((double)img[i]) + std::fabs((double)img[plane + i]) + std::fabs((double)img[2 * plane + i]);
-                    if (!(a <= 1e30)) bad[t] = 1;  // NaN or infinity
-                    down[(size_t)(y + 1) * width + x] = down[i] + a;
-                }
-            for (int y = 0; y < oh; ++y) {
-                const int y0 = std::max(0, y * stride_height - pad_h), y1 = std::min(height, y * stride_height - pad_h + filter_height);
-                if (y1 <= y0) continue;
-                along[0] = 0.0;
-                for (int x = 0; x < width; ++x)
-                    along[x + 1] = along[x] + (down[(size_t)y1 * width + x] - down[(size_t)y0 * width + x]);
-                for (int x = 0; x < ow; ++x) {
-                    const int x0 = std::max(0, x * stride_width - pad_w), x1 = std::min(width, x * stride_width - pad_w + filter_width);
-                    if (x1 > x0) worst[t] = std::max(worst[t], along[x1] - along[x0]);
+    std::atomic<int> next{0};
+    std::atomic<bool> bad{false};
+    std::mutex guard;
+    double worst = 0.0;
+    auto scan = [&] {
+        double w = 0.0;
+        try {
+            std::vector<double> down((size_t)(height + 1) * width), along(width + 1);
+            for (int b; !bad.load(std::memory_order_relaxed) && (b = next.fetch_add(1, std::memory_order_relaxed)) < batch;) {
+                const float* img = input_host + (size_t)b * 3 * plane;
+                for (int x = 0; x < width; ++x) down[x] = 0.0;
+                for (int y = 0; y < height; ++y)
+                    for (int x = 0; x < width; ++x) {
+                        const size_t i = (size_t)y * width + x;
+                        const double a = std::fabs((double)img[i]) + std::fabs((double)img[plane + i]) + std::fabs((double)img[2 * plane + i]);
+                        if (!(a <= 1e30)) bad = true;  // NaN or infinity
+                        down[(size_t)(y + 1) * width + x] = down[i] + a;
+                    }
+                for (int y = 0; y < oh; ++y) {
+                    const int y0 = std::max(0, y * stride_height - pad_h), y1 = std::min(height, y * stride_height - pad_h + filter_height);
+                    if (y1 <= y0) continue;
+                    along[0] = 0.0;
+                    for (int x = 0; x < width; ++x)
+                        along[x + 1] = along[x] + (down[(size_t)y1 * width + x] - down[(size_t)y0 * width + x]);
+                    for (int x = 0; x < ow; ++x) {
+                        const int x0 = std::max(0, x * stride_width - pad_w), x1 = std::min(width, x * stride_width - pad_w + filter_width);
+                        if (x1 > x0) w = std::max(w, along[x1] - along[x0]);
+                    }
                 }
             }
+        } catch (const std::bad_alloc&) {
+            bad = true;
         }
+        std::lock_guard<std::mutex> l(guard);
+        worst = std::max(worst, w);
     };
     std::vector<std::thread> pool;
-    for (int t = 1; t < n_threads; ++t) pool.emplace_back(scan, t);
-    scan(0);
-    for (std::thread& th : pool) th.join();
-    double w = 0.0;
-    for (int t = 0; t < n_threads; ++t) {
-        if (bad[t]) return INT32_MAX;
-        w = std::max(w, worst[t]);
+    try {
+        const int n = std::min(std::min(batch, 16), (int)std::thread::hardware_concurrency());
+        pool.reserve(16);
+        while ((int)pool.size() + 1 < n) pool.emplace_back(scan);
+    } catch (const std::exception&) {  // (those that run take the images of those that do not)
     }
-    const double bound = w * 1.001 + 1.0;
+    scan();
+    for (std::thread& th : pool) th.join();
+    if (bad) return INT32_MAX;
+    const double bound = worst * 1.001 + 1.0;
     return bound < (double)(INT32_MAX / 2) ? (int)std::ceil(bound) : INT32_MAX;
 }
 

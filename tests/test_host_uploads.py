@@ -1,0 +1,65 @@
+"""The host side of uploads without a GPU: what happens when threads or memory cannot be had, and what several callers of one
+uploader see.  Each test runs in a process of its own with tests/native/host_stub.c preloaded, so that HIP's memory calls work
+on ordinary memory and can be told to fail."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes as C, threading
+import numpy as np
+import tcbnn_amd
+from tcbnn_amd import _lib, device, layers
+L = _lib.lib
+stub = C.CDLL(STUB)
+def knob(name, value):
+    C.c_int.in_dll(stub, "stub_" + name).value = value
+def allocations():
+    return C.c_int.in_dll(stub, "stub_allocations").value
+device.hip = stub
+r = np.random.default_rng(1)
+def floats(n):
+    return r.standard_normal(n).astype(np.float32)
+def uploader(nbytes, staged=0):
+    p = C.c_void_p(0)
+    assert L.tcbnn_uploader_create(nbytes, staged, C.byref(p)) == 0, L.tcbnn_last_error()
+    return p
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("native") / "host_stub.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(ROOT, "tests/native/host_stub.c"), "-ldl"], check=True)
+
+    def go(body):
+        preload = ":".join([so] + [v for v in [os.environ.get("LD_PRELOAD")] if v])
+        env = dict(os.environ, LD_PRELOAD=preload, PYTHONPATH=ROOT, OMP_NUM_THREADS="1", OPENBLAS_NUM_THREADS="1")
+        code = "STUB = %r\n" % so + PRELUDE + textwrap.dedent(body) + "\nprint('done')\n"
+        p = subprocess.run([sys.executable, "-c", code], env=env, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=240)
+        assert p.returncode == 0 and p.stdout.strip().endswith("done"), "exit %d: %s" % (p.returncode, p.stdout[-2000:])
+    return go
+
+
+@pytest.mark.parametrize("left", [0, 1, 3])
+def test_fewer_threads_than_asked_for_are_enough(run, left):
+    """A thread that cannot be created, the first or a later one, costs speed and nothing else."""
+    run("""
+    knob("threads_left", %d)
+    x = floats((3 << 20) + 5)
+    u = uploader(x.nbytes, 1)
+    y, most = np.empty_like(x), C.c_float(0)
+    assert L.tcbnn_upload_stage(u, x.ctypes.data, x.size, C.byref(most)) == 0 and L.tcbnn_upload_commit(u, y.ctypes.data) == 0
+    assert np.array_equal(x, y) and most.value == np.abs(x).max()
+    L.tcbnn_uploader_destroy(u)
+    assert L.tcbnn_host_abs_max(x.ctypes.data, x.size) == np.abs(x).max()
+    im = floats((12, 3, 9, 9))
+    bound = L.tcbnn_inconv_residual_bound_of_input(im.ctypes.data, 12, 9, 9, 9, 9, 9, 9, 0)
+    most = np.abs(im.astype(np.float64)).sum((1, 2, 3)).max()
+    assert most <= bound <= most * 1.001 + 2
+    """ % left)
