@@ -133,7 +133,9 @@ float tcbnn_host_abs_max(const float* values_host, size_t count);
  * last one.  tcbnn_upload copies `bytes` of HOST memory to the device, in the order of the null stream, and is complete
  * when it returns.  tcbnn_upload_stage (an uploader created with staged = 1) copies an array of floats out of
  * HOST memory, takes max |x| on the way (as tcbnn_host_abs_max) and leaves the destination alone;
- * tcbnn_upload_commit then writes the staged array to `dst`.  Calls on one uploader exclude each other. */
+ * tcbnn_upload_commit then writes the staged array to `dst`.  Each call on one uploader excludes the others.  A stage and
+ * its commit are two calls about the ONE array that an uploader keeps staged: the next stage replaces it from its first
+ * byte on, and threads that share an uploader hold a lock of their own across the two. */
 typedef struct tcbnn_uploader tcbnn_uploader;
 int tcbnn_uploader_create(size_t bytes, int staged, tcbnn_uploader** out);
 void tcbnn_uploader_destroy(tcbnn_uploader* uploader);

@@ -302,6 +302,7 @@ int tcbnn_upload_stage(tcbnn_uploader* u, const float* src_host, size_t count, f
     if (bytes > u->bytes || (u->device == nullptr && bytes > u->pinned_bytes))
         return fail(TCBNN_EINVAL, "upload_stage: longer than the uploader was made for");
     std::lock_guard<std::mutex> l(u->m);
+    u->staged = 0;  // (what was staged before is overwritten from here on, whether this call succeeds or not)
     u->on_device = u->device != nullptr;
     uint32_t most = 0;
     try {

@@ -1,5 +1,6 @@
 """Device memory, streams and events for the Python host mirror (thin HIP runtime plumbing)."""
 import ctypes as C
+import threading
 
 import numpy as np
 
@@ -59,10 +60,12 @@ class DeviceBuffer:
 
 
 class PinnedBuffer:
-    """Owning handle on pinned host memory, for results that are downloaded over and over."""
+    """Owning handle on pinned host memory, for results that are downloaded over and over (by one thread at a time:
+    download() takes turns)."""
 
     def __init__(self, nbytes):
         self.nbytes = int(nbytes)
+        self.lock = threading.Lock()
         p = C.c_void_p(0)
         hip_check(hip.hipHostMalloc(C.byref(p), max(self.nbytes, 4), 0), "hipHostMalloc(%d)" % self.nbytes)
         self.ptr = p.value
@@ -73,8 +76,9 @@ class PinnedBuffer:
         out = np.empty(shape, dtype=dtype)
         assert out.nbytes <= min(self.nbytes, src.nbytes), (out.nbytes, self.nbytes, src.nbytes)
         if out.nbytes:
-            hip_check(hip.hipMemcpy(self.ptr, src.ptr, out.nbytes, _lib.D2H), "hipMemcpy D2H")
-            out.reshape(-1).view(np.uint8)[:] = self.bytes[:out.nbytes]
+            with self.lock:
+                hip_check(hip.hipMemcpy(self.ptr, src.ptr, out.nbytes, _lib.D2H), "hipMemcpy D2H")
+                out.reshape(-1).view(np.uint8)[:] = self.bytes[:out.nbytes]
         return out
 
     def free(self):
@@ -121,6 +125,34 @@ class Uploader:
             self.free()
         except Exception:
             pass
+
+
+class InputUploads:
+    """New batches for a layer's input buffer.  put() is one call per batch, whichever threads they come from: the
+    uploader keeps ONE staged batch, so what stages it, judges it and commits it must not be interleaved."""
+
+    def __init__(self, staged=False):
+        self.staged = staged
+        self.uploader = None
+        self.lock = threading.Lock()
+
+    def put(self, dst, x, accept=None):
+        """Replaces the contents of `dst` by `x`.  accept(max |x|) (staged uploads) raises to refuse the batch; the
+        buffer then keeps what it holds."""
+        with self.lock:
+            if self.uploader is None:
+                self.uploader = Uploader(dst.nbytes, self.staged)
+            if accept is None:
+                self.uploader.upload(dst, x)
+            else:
+                accept(self.uploader.stage(x))
+                self.uploader.commit(dst)
+
+    def free(self):
+        with self.lock:
+            if self.uploader is not None:
+                self.uploader.free()
+                self.uploader = None
 
 
 class Stream:

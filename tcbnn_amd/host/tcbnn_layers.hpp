@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <map>
+#include <mutex>
 #include <vector>
 
 #include "../../include/tcbnn_hip.h"
@@ -635,6 +636,8 @@ class InConv128LayerParam {  // param.h:701-870
     void set_input(float* input) {
         CHECK_NULL_POINTER(input);
         CHECK_NULL_POINTER(input_gpu);
+        // (one batch at a time: an uploader keeps one staged array, which is staged, judged and committed here)
+        std::lock_guard<std::mutex> one_batch(upload_guard);
         if (uploader == NULL) TCBNN_SAFE_CALL(tcbnn_uploader_create(input_bytes(), save_residual ? 1 : 0, &uploader));
         if (save_residual) {
             float abs_max = 0.0f;
@@ -763,6 +766,7 @@ class InConv128LayerParam {  // param.h:701-870
     uin32* output_fmt_gpu = NULL;        // reference-layout copies of the output and the saved residual
     int* output_residual_ref_gpu = NULL;
     bool packed_input = false;           // use_packed_input()
+    std::mutex upload_guard;
     tcbnn_uploader* uploader = NULL;     // set_input's pinned memory, made by the first call
     float* input_packed_gpu = NULL;      // [Hp][Wp][batch][3] copy of input_gpu (un-pooled layers, on request)
 };

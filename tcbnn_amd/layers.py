@@ -20,7 +20,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import lib, check
-from .device import DeviceBuffer, PinnedBuffer, Uploader
+from .device import DeviceBuffer, InputUploads, PinnedBuffer
 
 
 def STEP8(x):
@@ -256,7 +256,7 @@ class In128LayerParam(_ReferenceLayoutIO):
         self.name = name
         self.input_height = self.output_height = input_height
         self.input_width = self.output_width = input_width
-        self.input_gpu = self.output_gpu = self._uploader = None
+        self.input_gpu = self.output_gpu = self._uploads = None
 
     def output_bit_size(self):
         return PAD8(self.output_height) * STEP128(self.output_width)
@@ -269,14 +269,12 @@ class In128LayerParam(_ReferenceLayoutIO):
             raise _lib.TcbnnError("Error: NULL pointer (input)")
         x = np.ascontiguousarray(input, dtype=np.float32).reshape(self.input_height, self.input_width)
         self.input_gpu = DeviceBuffer.from_numpy(x)
+        self._uploads = InputUploads()
         self.output_gpu = DeviceBuffer(4 * lib.tcbnn_fc_act_words(self.output_height, self.output_width))
         return self
 
     def set_input(self, input):
-        x = np.ascontiguousarray(input, dtype=np.float32)
-        if self._uploader is None:
-            self._uploader = Uploader(self.input_gpu.nbytes)
-        self._uploader.upload(self.input_gpu, x)
+        self._uploads.put(self.input_gpu, np.ascontiguousarray(input, dtype=np.float32))
 
     def get_output_gpu(self):
         return self.output_gpu
@@ -297,10 +295,10 @@ class In128LayerParam(_ReferenceLayoutIO):
 
     def release(self):
         self._release_ref_bufs()
-        for b in (self.input_gpu, self.output_gpu, self._uploader):
+        for b in (self.input_gpu, self.output_gpu, self._uploads):
             if b is not None:
                 b.free()
-        self.input_gpu = self.output_gpu = self._uploader = None
+        self.input_gpu = self.output_gpu = self._uploads = None
 
 
 def _fc_download_fmt(buf, batch, features):
@@ -603,7 +601,7 @@ class InConv128LayerParam(_ConvGeometry):
         self.save_residual = save_residual
         self.filter = self.bn = None
         self.input_gpu = self.filter_gpu = self.bn_gpu = self.output_gpu = self.output_residual_gpu = None
-        self.input_packed_gpu = self._uploader = None
+        self.input_packed_gpu = self._uploads = None
         self._derive()
 
     def input_size(self):
@@ -633,6 +631,7 @@ class InConv128LayerParam(_ConvGeometry):
         x = np.ascontiguousarray(input, dtype=np.float32)
         assert x.size == self.input_size(), (x.size, self.input_size())
         self.input_gpu = DeviceBuffer.from_numpy(x)
+        self._uploads = InputUploads(staged=self.save_residual)
         if self._packed_floats():
             self.input_packed_gpu = DeviceBuffer(4 * self._packed_floats())
             self._pack_input()
@@ -668,11 +667,10 @@ class InConv128LayerParam(_ConvGeometry):
         skipped when R*S*3*max|x| already fits."""
         x = np.ascontiguousarray(input, dtype=np.float32)
         assert x.size == self.input_size(), (x.size, self.input_size())
-        if self._uploader is None:
-            self._uploader = Uploader(self.input_gpu.nbytes, staged=self.save_residual)
-        if self.save_residual:
+
+        def accept(abs_max):
             buf = self.output_residual_gpu
-            coarse = lib.tcbnn_inconv_residual_bound(self.filter_height, self.filter_width, self._uploader.stage(x))
+            coarse = lib.tcbnn_inconv_residual_bound(self.filter_height, self.filter_width, abs_max)
             limit = _residual_bound_limit(buf)
             if coarse > buf.bound:
                 bound = coarse if coarse <= limit else self._residual_bound(x)
@@ -680,9 +678,8 @@ class InConv128LayerParam(_ConvGeometry):
                     raise _lib.TcbnnError("input magnitude (window sums of |x| up to %d) exceeds what the residual "
                                           "formats chosen at initialize() hold (up to %d)" % (bound, limit))
                 _raise_residual_bound(buf, bound)
-            self._uploader.commit(self.input_gpu)
-        else:
-            self._uploader.upload(self.input_gpu, x)
+
+        self._uploads.put(self.input_gpu, x, accept if self.save_residual else None)
         self._pack_input()
 
     def _desc(self):
@@ -709,11 +706,11 @@ class InConv128LayerParam(_ConvGeometry):
     def release(self):
         self._release_ref_bufs()
         for b in (self.input_gpu, self.input_packed_gpu, self.filter_gpu, self.bn_gpu, self.output_gpu,
-                  self.output_residual_gpu, self._uploader):
+                  self.output_residual_gpu, self._uploads):
             if b is not None:
                 b.free()
         self.input_gpu = self.filter_gpu = self.bn_gpu = self.output_gpu = self.output_residual_gpu = None
-        self.input_packed_gpu = self._uploader = None
+        self.input_packed_gpu = self._uploads = None
 
 
 class Conv128LayerParam(_ConvGeometry):

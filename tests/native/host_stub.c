@@ -45,6 +45,7 @@ int hipMemcpy(void* d, const void* s, size_t n, int kind) {
     memcpy(d, s, n);
     return 0;
 }
+int hipMemset(void* d, int v, size_t n) { memset(d, v, n); return 0; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* stream) { (void)stream; return hipMemcpy(d, s, n, kind); }
 int hipStreamSynchronize(void* stream) { (void)stream; return 0; }
 int hipDeviceSynchronize(void) { return 0; }

@@ -21,6 +21,8 @@ def knob(name, value):
     C.c_int.in_dll(stub, "stub_" + name).value = value
 def allocations():
     return C.c_int.in_dll(stub, "stub_allocations").value
+for name in ("hipMalloc", "hipHostMalloc", "hipFree", "hipHostFree", "hipMemcpy", "hipMemset"):
+    getattr(stub, name).argtypes = getattr(_lib.hip, name).argtypes
 device.hip = stub
 r = np.random.default_rng(1)
 def floats(n):
@@ -63,3 +65,81 @@ def test_fewer_threads_than_asked_for_are_enough(run, left):
     most = np.abs(im.astype(np.float64)).sum((1, 2, 3)).max()
     assert most <= bound <= most * 1.001 + 2
     """ % left)
+
+
+def test_a_failed_or_refused_stage_leaves_nothing_to_commit(run):
+    """Staging overwrites what was staged before: after a stage that failed on the way there is nothing to commit."""
+    run("""
+    x, z = floats(3 << 20), floats(3 << 20)     # 12 MiB: goes on to the device copy chunk by chunk
+    u = uploader(x.nbytes, 1)
+    y, most = np.zeros_like(x), C.c_float(0)
+    assert L.tcbnn_upload_stage(u, x.ctypes.data, x.size, C.byref(most)) == 0
+    knob("copies_left", 1)
+    assert L.tcbnn_upload_stage(u, z.ctypes.data, z.size, C.byref(most)) == -3
+    knob("copies_left", -1)
+    assert L.tcbnn_upload_commit(u, y.ctypes.data) == -1 and not y.any()
+    assert L.tcbnn_upload_stage(u, z.ctypes.data, z.size, C.byref(most)) == 0 and L.tcbnn_upload_commit(u, y.ctypes.data) == 0
+    assert np.array_equal(y, z)
+    L.tcbnn_uploader_destroy(u)
+    assert allocations() == 0
+    """)
+
+
+def test_two_threads_with_new_batches_for_one_layer(run):
+    """set_input from two threads: each batch is staged, judged and committed as a whole, one after the other."""
+    run("""
+    n = 3 * 20 * 20 * 8
+    layer = layers.InConv128LayerParam("Conv1", 20, 20, 3, 3, 3, 64, 8, save_residual=True)
+    layer.input_gpu = device.DeviceBuffer.zeros(4 * n)
+    layer._uploads = device.InputUploads(staged=True)
+    class Residual:
+        bound, format, channels, readers = 2000, _lib.RES_I12, 64, []
+    layer.output_residual_gpu = Residual()
+    layers._residual_bound_limit = lambda buf: 2047
+    first = [floats(n), floats(n)]
+    for x in first:
+        layer.set_input(x)                       # the uploader exists now
+    staged = threading.Barrier(2, timeout=2)
+    stage = device.Uploader.stage
+    def stage_and_wait(self, arr):
+        most = stage(self, arr)
+        try:
+            staged.wait()                        # lets the other thread stage too, where it can
+        except threading.BrokenBarrierError:
+            pass
+        return most
+    device.Uploader.stage = stage_and_wait
+    failed = []
+    def call(x):
+        try:
+            layer.set_input(x)
+        except Exception as e:
+            failed.append(e)
+    threads = [threading.Thread(target=call, args=(x,)) for x in first]
+    [t.start() for t in threads]; [t.join() for t in threads]
+    assert not failed, failed
+    got = layer.input_gpu.to_numpy(np.float32, (n,))
+    assert any(np.array_equal(got, x) for x in first)
+    """)
+
+
+def test_two_threads_downloading_through_one_pinned_buffer(run):
+    run("""
+    import time
+    a, b = device.DeviceBuffer.from_numpy(floats(1000)), device.DeviceBuffer.from_numpy(floats(1000))
+    host = device.PinnedBuffer(4000)
+    class Slow:
+        def __getattr__(self, name):
+            return getattr(stub, name)
+        def hipMemcpy(self, *args):
+            rc = stub.hipMemcpy(*args)
+            time.sleep(0.05)
+            return rc
+    device.hip = Slow()
+    got = {}
+    def call(i, src):
+        got[i] = host.download(src, np.float32, (1000,))
+    threads = [threading.Thread(target=call, args=(i, s)) for i, s in enumerate((a, b))]
+    [t.start() for t in threads]; [t.join() for t in threads]
+    assert np.array_equal(got[0], a.to_numpy(np.float32, (1000,))) and np.array_equal(got[1], b.to_numpy(np.float32, (1000,)))
+    """)
