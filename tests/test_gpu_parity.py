@@ -936,6 +936,45 @@ def test_inconv128_matrix_cores(gpu, b, h, w, R, S, stride, cout, pool, save, fm
     layer.release()
 
 
+@pytest.mark.parametrize("b,h,R,stride,pool,kind", [(16, 40, 7, 4, 1, "normal"), (16, 40, 7, 4, 1, "mixed"), (16, 30, 7, 2, 1, "spikes"),
+                                                    (16, 20, 3, 1, 1, "normal"), (16, 20, 3, 1, 1, "mixed"), (16, 20, 3, 1, 1, "spikes"),
+                                                    (16, 60, 11, 4, 2, "normal"), (16, 60, 11, 4, 2, "mixed"), (16, 60, 11, 4, 2, "spikes")])
+def test_inconv128_thresholds_at_the_ordered_sums(gpu, b, h, R, stride, pool, kind):
+    """Every channel's threshold is the reference's own ordered sum of some pixel, or the next float above or below it: one
+    rounding in another order shows in a bit.  Magnitudes from 1e-3 to 1e4 in one window, and few large values among many
+    that the matrix cores' sums lose bits of."""
+    r = rng(1000 + b + h + R + len(kind))
+    cout = 64
+    x = r.standard_normal((b, 3, h, h)).astype(np.float32)
+    if kind == "mixed":
+        x *= (10.0 ** r.uniform(-3, 4, x.shape)).astype(np.float32)
+    elif kind == "spikes":
+        x = np.where(r.random(x.shape) < 0.3, x * np.float32(4096), x * np.float32(2e-4)).astype(np.float32)
+    f = rm.pm1(r, (R, R, 3, cout))
+    pad, _, out = rm.conv_pad_out(h, R, stride, True, 1)
+    bn = np.empty(cout, np.float32)
+    for o in range(cout):
+        i, y0, x0 = int(r.integers(b)), int(r.integers(2, out - 2)) * stride - pad, int(r.integers(2, out - 2)) * stride - pad
+        acc = np.float32(0)
+        for t in range(R):
+            for s in range(R):
+                if 0 <= y0 + t < h and 0 <= x0 + s < h:
+                    v = x[i, :, y0 + t, x0 + s] * f[t, s, :, o]
+                    acc = acc + ((v[0] + v[1]) + v[2])
+        bn[o] = [acc, np.nextafter(acc, np.float32(np.inf)), np.nextafter(acc, np.float32(-np.inf))][o % 3]
+    save = pool == 1
+    want, wres = orc.inconv128(x, f, bn, stride, True, pool, save)
+    layer = gpu.InConv128LayerParam("Conv1", h, h, R, R, 3, cout, b, stride, stride, True, pool, pool, save)
+    layer.initialize(x, gpu.ArrayWeights([f, bn]))
+    assert "mfma" in layer.kernel_name(), layer.kernel_name()
+    layer.forward()
+    gpuops.sync()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    if save:
+        np.testing.assert_array_equal(layer.download_residual(), wres)
+    layer.release()
+
+
 def test_inconv128_special_thresholds(gpu):
     """NaN, +-inf and exactly met thresholds in the first layer (kernel.cuh:655: bit = !(acc < bn))."""
     r = rng(321)
