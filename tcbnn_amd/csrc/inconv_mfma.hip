@@ -8,8 +8,10 @@
 //   2. a bound E of |S - acc| is known per pixel (below), so wherever S is further than E from the threshold, and from
 //      every integer where a residual is saved, the bit and the residual of S are those of acc;
 //   3. the few values within E (0.1 % with a residual, a few in 10^5 without) are put on a list and recomputed in the
-//      reference's order by the same wave, which then repairs the stored bit and residual.
-// The results are therefore the reference's, bit for bit, for every input; only the time depends on the data.
+//      reference's order by the same wave, which then repairs the stored bit and residual;
+//   4. where that is not few (flat areas, large magnitudes), a wave leaves the list for passes that cost a bounded factor.
+// The results are therefore the reference's, bit for bit, for every input; only the time depends on the data, and by a
+// small factor (below).
 //
 // The bound.  u = 2^-24, A = sum of |x| under the window, T = R*S taps.  A rounding of a running sum is at most u times
 // that sum, which is at most what has been added so far and at most |S| plus what is still to come: (A + |S|) / 2.  The
@@ -26,9 +28,26 @@
 // last tap, unused otherwise), so the accumulators hold S - E: a bit is certainly 1 where S - E >= bn, certainly 0 below
 // bn - 2E.
 // Inputs outside the fp16 range, infinities and NaN make E infinite: all values of such a window are recomputed.
-// Whole-number inputs (images of 0..255, inputs binarised to +-1) put every sum ON an integer; their sums are exact in
-// both orders, so once a wave meets more than half a tile of doubtful values, rows are checked while they are staged, and windows of
-// whole numbers below 512 run with E = 0.
+//
+// Many values in doubt.  A saved residual puts every sum ON an integer in doubt, and images have areas of such sums: bars of
+// +-1 after scaling to [-1, 1], saturated white, bytes, a flat grey of 0.2 (every fifth channel); and E grows with the
+// magnitudes: bytes less a mean leave 7 % of the sums in doubt, values in the thousands all of them.  One by one (four at a
+// time, a trip to memory and 49 dependent additions) a tile full of them takes 512 rounds, a hundred multiplications' time.
+//   grid    : while every row a wave has staged is multiples of 1/256 (bytes, bytes / 128 - 1, +-1), sums of windows with
+//             a sum of |x| below 2^16 are exact: every partial sum is a multiple of 1/256 below 2^24 / 256, in both orders.
+//             E is 0.  Rows are checked as long as that holds; other inputs pay for the first window.
+//   COMMON  : a wave's first pass; it ends at an item with many values in doubt (kManyInLane, kManyLanesCommon; where no
+//             residual is saved: at a full list).  The test and the exit cost it 1.5 %; what the later passes do cost 3-9 %
+//             inside its loop, by its registers.
+//   MARKED  : the window is staged again, and rows from then on, with a mark at every column that is off that grid (the
+//             fourth channel of the lo plane).  An item looks at its windows' marks first; E is 0 where there is none.
+//   ORDERED : where that still leaves many, sums in the reference's order, 32 columns x 64 channels at a time, as fp32
+//             products on the matrix cores (ordered_sums): no values in doubt but those that are no numbers.
+// A single wave that leaves the common pass takes 80 us longer (code that no other wave has fetched), and the launch with
+// it: the lines lie where none of 25000 items of bytes / 255 (0.6 % in doubt) reaches them.
+// ResNet-18's first layer at batch 256, us, in brackets with the list alone: normal data 107 (111), bytes / 128 - 1 92 (245),
+// images in [-1, 1] with bars and patches of +-1 over a third 117 (7690), bytes / 255 147 (163), a third of 0.2 grey 271
+// (1490), bytes less a mean 326 (1404), normal x 1000 336 (14150); the additions on the VALU (inconv.hip) take 138 for any.
 //
 // Work split.  A team owns NI images x a strip of xo output columns x a band of output rows, and walks down the rows:
 // the input rows of the window stay in LDS (a ring; stride_h new rows per output row, every input row is read and split
@@ -63,6 +82,10 @@ constexpr int rounds_of(int r) { return r == 3 ? 3 : 5; }  // staging units (col
 constexpr bool bound_for_half(int r) { return r > 3; }
 constexpr bool ring_shared(int r) { return r > 7; }          // four waves to a ring, else one
 constexpr int kListCap = 64;   // doubtful values a wave keeps
+// A wave's passes (top of this file), and what counts as many values in doubt: one lane with this many (of its column's 32;
+// a flat area), or this many lanes (of 64) with any.
+enum Mode : int { COMMON, MARKED, ORDERED };
+constexpr int kManyInLane = 8, kManyLanesCommon = 28, kManyLanesMarked = 32;
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -104,7 +127,23 @@ struct Geometry {
     float half_scale;
     float bound_add;
     float small_squares;     // sum of hi^2 below which the sum of |x| is below 1/2
+    float exact_squares;     // ... below which sums of multiples of 1/256 are exact
 };
+
+// The kernel's argument.  Code that seldom runs reads it anew from the argument segment (seldom_args): fields that
+// only such code needs are then not kept in scalar registers, and spilled, all the way through the common one.  (The
+// segment's address is a register of the kernel itself: taken in a function that is not inlined it would be 0.)
+struct KernelArgs {
+    InConvParams p;
+    Geometry q;
+    const uint32_t* pats;
+    unsigned out_bytes, res_bytes;
+};
+typedef const KernelArgs __attribute__((address_space(4))) * SeldomArgs;
+__device__ __forceinline__ SeldomArgs seldom_args(SeldomArgs a) {
+    asm volatile("" : "+s"(a));
+    return a;
+}
 
 // x - (float)pair[I], exact: one multiply-add with a half-precision operand
 template <int I>
@@ -160,9 +199,12 @@ __device__ __forceinline__ float add_row_taps(float acc, float m, int left) {
 
 template <int R, int NQ, int MT, int RES, int POOL, int PAIRS>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgroups_per_cu(R)))) void inconv_mfma_kernel(
-    const InConvParams p, const Geometry q, const float* __restrict__ in, const uint32_t* __restrict__ pats,
-    const float* __restrict__ bn, unsigned out_bytes, unsigned res_bytes) {
+    const KernelArgs args) {
+    const SeldomArgs args_at = (SeldomArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    const InConvParams& p = args.p;
+    const Geometry& q = args.q;
     static_assert(MT * POOL <= 2 && !(RES != RES_NONE && POOL > 1), "doubtful values of an item are 32 bits of a register");
+    static_assert(!(ring_shared(R) && RES != RES_NONE), "a wave of a shared ring cannot leave its pass at an item");
     constexpr int NK = R * NQ;  // MFMA steps: four taps (of one filter row) x four channels each
     constexpr int kRounds = rounds_of(R);
     constexpr unsigned kOutOfRange = 0x80000000u;
@@ -197,15 +239,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
     const int plane = q.ring * row_bytes;
     float* const thr = reinterpret_cast<float*>(lds);
     uint32_t* const list = reinterpret_cast<uint32_t*>(lds) + p.O + wave * 2 * kListCap;
-    int* const not_whole = reinterpret_cast<int*>(lds) + p.O + 4 * 2 * kListCap;
+    int* const flags = reinterpret_cast<int*>(lds) + p.O + 4 * 2 * kListCap;  // kShared: rows off the grid; many doubts
     char* const rows = lds + (p.O + 4 * 2 * kListCap + 4) * 4 + (kShared ? 0 : wave * 2 * plane);
 
     // ---- thresholds (NaN: -infinity, the bit is 1 either way)
     for (int i = tid; i < p.O; i += kThreads) {
-        const float t = bn[i];
+        const float t = p.bn[i];
         thr[i] = t != t ? -INFINITY : t;
     }
-    if (tid == 0) *not_whole = 0;
+    if (tid < 2) flags[tid] = 0;
     __syncthreads();
     if (idle) return;
 
@@ -221,7 +263,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const int s = 4 * (k % NQ) + 2 * h + t;
-                const uint32_t pt = pats[(size_t)((k / NQ) * p.S + min(s, p.S - 1)) * p.opad + o];
+                const uint32_t pt = args.pats[(size_t)((k / NQ) * p.S + min(s, p.S - 1)) * p.opad + o];
                 uint32_t d0 = 0x3c003c00u | ((pt & 4u) << 13) | (pt << 30 & 0x80000000u), d1 = 0x3c00u | ((pt & 1u) << 15);
                 if (s >= p.S) d0 = d1 = 0u;
                 if (k == NK - 1 && t == 0) d1 |= h == 0 ? 0x3c000000u : 0u;  // the slot that -E enters through
@@ -235,7 +277,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
     const unsigned plane_b = (unsigned)(p.H * p.W) * 4u;
     const int ax_first = x0 * p.stride_w - p.pad_w;
     const bool edge = ax_first < 0 || ax_first + 2 * q.np > p.W;  // uniform
-    __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(in + (size_t)b0 * 3 * p.H * p.W), 0,
+    __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.in + (size_t)b0 * 3 * p.H * p.W), 0,
                                                                     (int)((unsigned)min(NI, p.B - b0) * 3u * plane_b), 0x00020000);
     unsigned voff[kRounds];  // byte offset of the left column (out of range: no such image)
     unsigned cell[kRounds];  // cell in a row | left column in the frame << 16 | right one << 17 | row << 20
@@ -250,7 +292,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
     }
     const int rounds = q.rounds;
     v2f x[kRounds][3];
-    auto fetch = [&](int ay_first, int n_rows) {
+    auto fetch = [&](int ay_first, int n_rows) __attribute__((always_inline)) {
         const int row_b = ay_first * p.W * 4;
         const bool inner = !edge && ay_first >= 0 && ay_first + q.adv <= p.H;  // uniform (units past n_rows read what nobody uses)
 #pragma unroll
@@ -275,9 +317,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
             }
         }
     };
-    bool whole = true;  // every row staged so far is whole numbers below 512 (rows are checked as long as that holds)
-    auto split_and_store = [&](int n_rows, int slot0) {
-        bool all_whole = true;
+    bool grid = true;  // every row staged so far is multiples of 1/256 (rows are checked as long as that holds)
+    // marks: the fourth channel of the lo plane says which columns are not multiples of 1/256
+    auto split_and_store = [&](auto marks, int n_rows, int slot0) __attribute__((always_inline)) {
+        bool on_grid = true;
 #pragma unroll
         for (int k = 0; k < kRounds; ++k) {
             if (k >= rounds) break;  // uniform
@@ -294,6 +337,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
                 lo[2 * t] = __builtin_bit_cast(uint32_t, al);
                 lo[2 * t + 1] = __builtin_bit_cast(uint32_t, cl);
             }
+            if constexpr (decltype(marks)::value) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    float off = 0.0f;
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) off = __builtin_fmaxf(off, __builtin_amdgcn_fractf(f[3 * t + c] * 256.0f));
+                    lo[2 * t + 1] |= off > 0.0f ? 0x10000u : 0u;
+                }
+            }
             asm volatile("" : "+v"(cell[k]));
             const unsigned row = cell[k] >> 20;
             if (row < (unsigned)n_rows) {
@@ -302,26 +354,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
                 *reinterpret_cast<v4u*>(dst) = hi;
                 *reinterpret_cast<v4u*>(dst + plane) = lo;
             }
-            if (whole) {  // uniform
+            if (grid) {  // uniform
 #pragma unroll
-                for (int t = 0; t < 6; ++t) all_whole = all_whole & (((__builtin_rintf(f[t]) == f[t]) & (__builtin_fabsf(f[t]) < 512.0f)) | (row >= (unsigned)n_rows));
+                for (int t = 0; t < 6; ++t) on_grid = on_grid & ((__builtin_amdgcn_fractf(f[t] * 256.0f) == 0.0f) | (row >= (unsigned)n_rows));
             }
         }
-        if (whole) {
-            const bool mine = __ballot(!all_whole) == 0;
+        if (grid) {
+            const bool mine = __ballot(!on_grid) == 0;
             if constexpr (kShared) {
-                if (!mine && lane == 0) *not_whole = 1;
+                if (!mine && lane == 0) flags[0] = 1;
             } else {
-                whole = mine;
+                grid = mine;
             }
         }
     };
 
     // ---- doubtful values: recomputed in the reference's order, 16 lanes per value (lane t of a row: tap 16 c + t), the
-    // list's last four at a time
+    // list's last four at a time.  One trip to memory: inputs, signs and the residual's words are asked for together (the
+    // words after the sums, and the threshold from memory: two more trips, 111 us for 107, bytes / 255 163 for 147)
     int count = 0;  // entries on this wave's list (uniform)
     constexpr int NC = (R * 4 * NQ + 15) / 16;
-    auto recompute = [&]() {
+    auto recompute = [&]() __attribute__((always_inline)) {
+        const SeldomArgs a = seldom_args(args_at);
+        const auto& p = a->p;
+        const auto& q = a->q;
+        const uint32_t* const pats = a->pats;
         float f[NC][3];
         uint32_t pt[NC];
         const int pending = min(count, 4);
@@ -334,6 +391,33 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
         const int ay0 = (int)(ex >> 16) * p.stride_h - p.pad_h, ax0 = (int)(ex & 0xffffu) * p.stride_w - p.pad_w;
         const int o = (int)(ey & 0xffffu);
         const unsigned im = (ey >> 16) * 3u * plane_b;
+        const bool active = (lane >> 4) < pending;
+        const int bb = b0 + (int)(ey >> 16);
+        const unsigned pix = (ex >> 16) / POOL * (unsigned)p.OW + (ex & 0xffffu) / POOL;  // (host: tensors below 2 GiB)
+        // What the residual's words hold is asked for now, with the inputs.  Bits [fix_shift, ...) of the 32-bit word fix_at,
+        // under fix_mask, are the value's from bit fix_drop on; only this lane changes them, neighbours in the same word are
+        // left alone (exclusive or with what differs).
+        uint32_t* const residual = reinterpret_cast<uint32_t*>(p.res);
+        size_t fix_at = 0;
+        int fix_shift = 0, fix_drop = 0;
+        uint32_t fix_mask = 0u, old = 0u;
+        if constexpr (RES == RES_12) {
+            const int bit = 12 * (o & 15), here = min(12, 32 - (bit & 31));
+            const bool second = t16 == 1;
+            fix_shift = second ? 0 : bit & 31;
+            fix_drop = second ? here : 0;
+            fix_mask = t16 < 2 ? (1u << (second ? 12 - here : here)) - 1u : 0u;
+            fix_at = i12_word_index(pix, (size_t)((p.O + 15) / 16), o >> 4, p.B, bb, (bit >> 5) + (second ? 1 : 0));
+        } else if constexpr (RES == RES_WIDE) {
+            fix_at = residual_index(p.res_fmt, pix, p.O, o, p.B, bb);
+            if (p.res_fmt == TCBNN_RES_I16) {
+                fix_shift = (int)(fix_at & 1) * 16;
+                fix_mask = t16 == 0 ? 0xffffu : 0u;
+                fix_at >>= 1;
+            }
+        }
+        const bool fix = active && fix_mask != 0u;
+        if (RES != RES_NONE && fix) old = __hip_atomic_load(residual + fix_at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             const int tap = 16 * c + t16, r = (int)((unsigned)tap * q.s_magic >> 16), s = tap - r * p.S;
@@ -358,51 +442,33 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
                 else
                     acc = add_row_taps<0, 16, false>(acc, m, taps - 16 * c);
             }
-            if (t16 == 0 && (lane >> 4) < pending) {
-                const int y = (int)(ex >> 16), xx = (int)(ex & 0xffffu), o = (int)(ey & 0xffffu);
-                const int bb = b0 + (int)(ey >> 16);
-                const unsigned pix = (unsigned)(y / POOL * p.OW + xx / POOL);  // (host: tensors below 2 GiB)
-                if (!(acc < bn[o]))
-                    __hip_atomic_fetch_or(p.out + ((pix * (unsigned)p.ow + (unsigned)(o >> 5)) * (unsigned)p.B + (unsigned)bb), 0x80000000u >> (o & 31), __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT);
-                if constexpr (RES != RES_NONE) {
-                    const uint32_t v = (uint32_t)(int)acc;
-                    uint32_t* const w = reinterpret_cast<uint32_t*>(p.res);
-                    // bits [bit, bit + width) of the 32-bit words from word `at` on hold the value; only this lane changes
-                    // them, neighbours in the same word are left alone (exclusive or with what differs)
-                    auto repair = [&](size_t at, int bit, uint32_t mask, uint32_t val) {
-                        const uint32_t old = __hip_atomic_load(w + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> bit;
-                        const uint32_t d = ((old ^ val) & mask) << bit;
-                        if (d != 0u) __hip_atomic_fetch_xor(w + at, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    };
-                    if constexpr (RES == RES_12) {
-                        const size_t G = (size_t)((p.O + 15) / 16);
-                        const int bit = 12 * (o & 15), k = bit >> 5, sh = bit & 31, here = min(12, 32 - sh);
-                        repair(i12_word_index(pix, G, o >> 4, p.B, bb, k), sh, (1u << here) - 1u, v);
-                        if (here < 12)
-                            repair(i12_word_index(pix, G, o >> 4, p.B, bb, k + 1), 0, (1u << (12 - here)) - 1u, v >> here);
-                    } else if (p.res_fmt == TCBNN_RES_I16) {
-                        const size_t i = residual_index(TCBNN_RES_I16, pix, p.O, o, p.B, bb);
-                        repair(i >> 1, (int)(i & 1) * 16, 0xffffu, v);
-                    } else {
-                        w[residual_index(TCBNN_RES_I32, pix, p.O, o, p.B, bb)] = v;
-                    }
-                }
+            // (the row's 16 lanes all hold the sum: lane 2 sets the bit, lanes 0 and 1 repair the one or two words)
+            if (active && t16 == 2 && !(acc < thr[o]))
+                __hip_atomic_fetch_or(p.out + ((pix * (unsigned)p.ow + (unsigned)(o >> 5)) * (unsigned)p.B + (unsigned)bb), 0x80000000u >> (o & 31), __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+            if constexpr (RES != RES_NONE) {
+                const uint32_t v = (uint32_t)(int)acc;
+                const uint32_t d = ((old >> fix_shift ^ v >> fix_drop) & fix_mask) << fix_shift;
+                if (fix && d != 0u) __hip_atomic_fetch_xor(residual + fix_at, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (RES == RES_WIDE && active && t16 == 0 && p.res_fmt == TCBNN_RES_I32) residual[fix_at] = v;
             }
         }
     };
 
-    // ---- first window of the band
+    // ---- the window
     int ay0 = oy_begin * POOL * p.stride_h - p.pad_h;  // first input row of the step's window
     int s0 = 0;                                        // its ring slot
-    for (int done = 0; done < q.ring; done += q.adv) {
-        const int n = min(q.adv, q.ring - done);
-        fetch(ay0 + done, n);
-        split_and_store(n, done);
-    }
+    auto stage_window = [&](auto marks) __attribute__((always_inline)) {
+        for (int done = 0; done < q.ring; done += q.adv) {
+            const int n = min(q.adv, q.ring - done), slot = s0 + done;
+            fetch(ay0 + done, n);
+            split_and_store(marks, n, slot >= q.ring ? slot - q.ring : slot);
+        }
+    };
+    stage_window(std::false_type{});
 
-    const __amdgpu_buffer_rsrc_t out_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)out_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t res_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.res, 0, (int)res_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t out_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)args.out_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t res_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.res, 0, (int)args.res_bytes, 0x00020000);
     // Where this lane stores, relative to the item (uniform): its output word, its 16 residuals (12-bit: the 8-byte part
     // apart); beyond the tensors for an image past the batch.
     const unsigned uB = (unsigned)p.B, group_b = (RES == RES_12 ? 24u : (p.res_fmt == TCBNN_RES_I16 ? 32u : 64u)) * uB;
@@ -419,183 +485,359 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
         }
     }
 
-    for (int oy = oy_begin; oy < oy_end; ++oy) {
-        const bool more = oy + 1 < oy_end;  // uniform
-        if constexpr (kShared) {
-            __syncthreads();
-            if (whole) whole = __builtin_amdgcn_readfirstlane(*not_whole) == 0;
-        }
-        if (more) fetch(ay0 + q.ring, q.adv);
-        for (int g = wg0; g < n_groups; g += wg_step) {
-            uint32_t word[MT];
-            uint32_t doubt = 0u;
-            // A lane's place (column of the tile: image and pixel; half of the channels) is worked out anew from a lane
-            // index the compiler cannot carry over: kept across the multiplication, the addresses made from it spill.
-            int ln = lane;
-            asm volatile("" : "+v"(ln));
+    // ---- a whole item in the reference's order: words, residuals; in doubt stay sums that are no numbers.
+    // A tap's eight possible values are four and their negatives, so adding one of them to 32 x 32 sums is a product with a
+    // matrix of one +-1 and three 0 per row: two v_mfma_f32_32x32x2_f32, each one fp32 addition per sum (adding the zeros
+    // changes nothing; tests/test_gpu_matrix_core.py).
+    auto ordered_sums = [&](int oy, int g, uint32_t* word, uint32_t& doubt) __attribute__((always_inline)) {
+        const SeldomArgs a = seldom_args(args_at);
+        const auto& p = a->p;
+        const uint32_t* const pats = a->pats;
+        int ln = lane;
+        asm volatile("" : "+v"(ln));  // (nothing derived from it is kept outside)
+        const int h = ln >> 5, img = ln & (NI - 1), xc = x0 + g * NX + ((ln & 31) >> a->q.ni_log2);
+        const bool valid = b0 + img < p.B && xc < xcols;
+        const int ax0 = xc * p.stride_w - p.pad_w, o0 = tile0 * 32 + mfma::row_to_channel(ln & 31);
+        const unsigned im = (unsigned)img * 3u * plane_b, flip = (unsigned)h << 31;
+        doubt = 0u;
 #pragma unroll
-            for (int m = 0; m < MT; ++m) word[m] = 0u;
+        for (int m = 0; m < MT; ++m) word[m] = 0u;
 #pragma unroll 1
-            for (int py = 0; py < POOL; ++py) {
-                v16f acc[MT];
+        for (int py = 0; py < POOL; ++py) {
+            const int ay0 = (oy * POOL + py) * p.stride_h - p.pad_h, r_end = min(R, p.H - ay0);
+            v16f acc[MT];
 #pragma unroll
-                for (int m = 0; m < MT; ++m)
+            for (int m = 0; m < MT; ++m)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
-                const int first_col = (g * NX + ((ln & 31) >> q.ni_log2)) * p.stride_w;
-                const int lane_at = (ln & (NI - 1)) * q.pp * 16 + (PAIRS == PAIRS_SPLIT ? (first_col >> 2) * 16 + (ln >> 5) * q.odd_pairs * 16
-                                                                                       : first_col * 8 + (ln >> 5) * 16);
-                auto fragment = [&](int r, int j, int plane_off) -> v4i {
-                    int slot = s0 + py * p.stride_h + r;
-                    slot = slot >= q.ring ? slot - q.ring : slot;
-                    const char* const at = rows + (slot * row_bytes + plane_off) + lane_at + j * (PAIRS == PAIRS_SPLIT ? 16 : 32);
-                    if constexpr (PAIRS != PAIRS_ANY)
-                        return __builtin_bit_cast(v4i, *reinterpret_cast<const h8*>(at));
-                    else
-                        return __builtin_bit_cast(v4i, static_cast<h8>(*reinterpret_cast<const h8u*>(at)));
-                };
-                // lo steps, then hi steps; a step's fragment is requested kAhead steps ahead
-                constexpr int kAhead = 4;
-                v4i ahead[kAhead];
+                for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
+            // a filter row at a time, requested one row ahead; out of the frame: zeros, which add nothing
+            constexpr int kTaps = 4 * NQ;
+            float next[kTaps][3];
+            uint32_t next_pt[kTaps][MT];
+            auto request = [&](int r) __attribute__((always_inline)) {
+                const unsigned at0 = im + (unsigned)((ay0 + r) * p.W + ax0) * 4u;
 #pragma unroll
-                for (int k = 0; k < kAhead; ++k) ahead[k] = fragment(k % NK / NQ, k % NK % NQ, k < NK ? plane : 0);
-                float sq = 0.0f, two_e = 0.0f, half_a = 0.0f, wide_shift = 0.0f, wide_two_e = 0.0f;
-                bool bad = false, small = false;  // small: |S| and |acc| are below 1/2, the residual is 0
+                for (int j = 0; j < NQ; ++j) {
+                    const int ax = ax0 + 4 * j;
+                    const unsigned at = at0 + 16u * j;
+                    if (__ballot(valid & ((ax < 0) | (ax + 4 > p.W))) == 0) {  // uniform
 #pragma unroll
-                for (int k = 0; k < 2 * NK; ++k) {
-                    v4i v = ahead[k % kAhead];
-                    if (k + kAhead < 2 * NK)
-                        ahead[k % kAhead] = fragment((k + kAhead) % NK / NQ, (k + kAhead) % NK % NQ, k + kAhead < NK ? plane : 0);
-                    if (k >= NK) {
+                        for (int ch = 0; ch < 3; ++ch) {
+                            const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(valid ? at : kOutOfRange), (int)(ch * plane_b), 0));
 #pragma unroll
-                        for (int d = 0; d < 4; ++d) {
-                            const int two = v[d];
-                            sq = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, two), __builtin_bit_cast(h2, two), sq, false);
+                            for (int t = 0; t < 4; ++t) next[4 * j + t][ch] = v[t];
+                        }
+                    } else {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            const bool inside = valid & (ax + t >= 0) & (ax + t < p.W);
+#pragma unroll
+                            for (int ch = 0; ch < 3; ++ch)
+                                next[4 * j + t][ch] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(inside ? at + 4u * t : kOutOfRange), (int)(ch * plane_b), 0));
                         }
                     }
-                    if (k == 2 * NK - 1) {
-                        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(sq), __float_as_uint(sq), false, false);
-                        const float all = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-                        const float root = __builtin_amdgcn_sqrtf(all), full = root * q.bound_scale_full + q.bound_add;
-                        small = all < q.small_squares;
-                        bad = !(all < 4.0e9f) || !(full < 3.0e4f);
-                        _Float16 eh = (_Float16)(root * q.bound_scale + q.bound_add);
-                        half_a = root * q.half_scale;
-                        wide_two_e = 2.002f * full;
-                        if (whole && !bad) {
-                            eh = (_Float16)0.0f;
-                            half_a = INFINITY;
-                        }
-                        two_e = 2.002f * (float)eh;
-                        wide_shift = (float)eh - full;
-                        if (lane < 32) v[1] |= (int)((uint32_t)(__builtin_bit_cast(uint16_t, eh) | 0x8000u) << 16);
-                    }
-#pragma unroll
-                    for (int m = 0; m < MT; ++m)
-                        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, wf[k % NK][m]), __builtin_bit_cast(h8, v), acc[m], 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
                 }
-                // ---- bits (MSB first; the sign of S - E - bn, inverted), residual, doubtful values
-                asm volatile("" : "+v"(ln));
-                const int h = ln >> 5;
-                const bool valid = b0 + (ln & (NI - 1)) < p.B && x0 + g * NX + ((ln & 31) >> q.ni_log2) < xcols;
+                const uint32_t* const row = pats + (unsigned)(r * p.S * p.opad);  // (uniform)
 #pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    const v4f* const tp = reinterpret_cast<const v4f*>(thr + (tile0 + m) * 32 + 16 * h);
-                    // Signs are collected MSB first (bit 15 - i: channel i).  w: S - E < bn, dm: values in doubt.  Integers
-                    // within E are common (in every other tile) and collected like the bits; thresholds within E and sums
-                    // above A/2 (E is less than a bound for those) are rare: the tile's nearest distance below a threshold
-                    // and its largest |S| tell whether to look for them.
-                    uint32_t w = 0u, dm = 0u;
-                    int nearest = INT32_MAX;
-                    float most = 0.0f;
-                    {
-                        const v4f th[4] = {tp[0], tp[1], tp[2], tp[3]};
+                for (int t = 0; t < kTaps; ++t)
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            const float d = acc[m][i] - th[i >> 2][i & 3];
-                            w = __builtin_amdgcn_alignbit(w, __float_as_uint(d), 31);
-                            nearest = min(nearest, __float_as_int(d));
-                            if constexpr (kHalf) most = __builtin_fmaxf(most, __builtin_fabsf(acc[m][i]));
-                            if constexpr (RES != RES_NONE)
-                                dm = __builtin_amdgcn_alignbit(dm, __float_as_uint(__builtin_amdgcn_fractf(-acc[m][i]) - two_e), 31);
-                        }
-                    }
-                    if constexpr (RES != RES_NONE) dm = small ? 0u : dm;
-                    // (NaN: `bad` is set)
-                    if (__ballot(bad | (kHalf & !(most <= half_a)) | (nearest <= (int)(0x80000000u | __float_as_uint(two_e)))) != 0) {
-                        const bool wide = kHalf & !(most <= half_a);  // this lane's sums with the full bound
-                        const float shift = wide ? wide_shift : 0.0f, two = wide ? wide_two_e : two_e;
-                        uint32_t w2 = 0u, r = 0u;
-                        w = 0u;
+                    for (int m = 0; m < MT; ++m) next_pt[t][m] = row[(unsigned)(min(t, p.S - 1) * p.opad + o0 + 32 * m)];
+            };
+            const int r_begin = max(0, -ay0);
+            if (r_begin < r_end) request(r_begin);
+#pragma unroll 1
+            for (int r = r_begin; r < r_end; ++r) {
+                float f[kTaps][3];
+                uint32_t pt[kTaps][MT];
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            float a = acc[m][i];
-                            asm volatile("" : "+v"(a));  // (evaluated again here: not kept from above)
-                            a += shift;
-                            const float d = a - tp[i >> 2][i & 3];
-                            w = __builtin_amdgcn_alignbit(w, __float_as_uint(d), 31);
-                            w2 = __builtin_amdgcn_alignbit(w2, __float_as_uint(d + two), 31);
-                            if constexpr (RES != RES_NONE) r = __builtin_amdgcn_alignbit(r, __float_as_uint(__builtin_amdgcn_fractf(-a) - two), 31);
-                        }
-                        w = bad ? 0xffffu : w;
-                        dm = bad ? 0xffffu : (w & ~w2) | (wide || !small ? r : 0u);
-                    }
-                    doubt |= (valid ? dm & 0xffffu : 0u) << (16 * (POOL > 1 ? py : m));
-                    word[m] |= ~w & 0xffffu;  // (a bit in doubt is 0 here: the recomputation only ever sets it)
-                    if constexpr (RES != RES_NONE) {
-                        int v[16];
+                for (int t = 0; t < kTaps; ++t) {
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) v[i] = (int)acc[m][i];
-                        const unsigned item = (unsigned)(oy * p.PW + x0 + g * NX) * pixel_b + (unsigned)((tile0 + m) * 2) * group_b;
-                        store_residual_group<RES>(res_rsrc, p.res_fmt, valid ? place_res + item : kOutOfRange,
-                                                  RES == RES_12 ? (valid ? place_res8 + item : kOutOfRange) : 0u, uB * 16u, v);
-                        __builtin_amdgcn_sched_barrier(0);  // (one tile at a time: registers)
+                    for (int ch = 0; ch < 3; ++ch) f[t][ch] = next[t][ch];
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) pt[t][m] = next_pt[t][m];
+                }
+                if (r + 1 < r_end) request(r + 1);
+#pragma unroll
+                for (int t = 0; t < kTaps; ++t) {
+                    if (t >= p.S) break;  // uniform
+                    const float f2 = __uint_as_float(__float_as_uint(f[t][2]) ^ flip);
+                    const float same = (f[t][0] + f[t][1]) + f2, other = (f[t][0] - f[t][1]) + f2;
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) {
+                        // pattern 4 neg0 + 2 neg1 + neg2; a pattern from 4 on is the negative of the inverted one
+                        const uint32_t neg = (uint32_t)((int)(pt[t][m] << 29) >> 31), c = (pt[t][m] ^ neg) & 3u;
+                        const uint32_t one = 0x3f800000u | (neg & 0x80000000u);
+                        acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(c == (uint32_t)h ? one : 0u), same, acc[m], 0, 0, 0);
+                        acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(c == (uint32_t)h + 2u ? one : 0u), other, acc[m], 0, 0, 0);
                     }
                 }
             }
-            // ---- output words: two tiles: lane half h stores the word of tile h; one tile: half 0 stores
-            asm volatile("" : "+v"(ln));
-            const int h = ln >> 5, img = ln & (NI - 1), xc = x0 + g * NX + ((ln & 31) >> q.ni_log2);
-            const auto sw = __builtin_amdgcn_permlane32_swap(word[0], word[MT - 1], false, false);
-            uint32_t full = (sw[0] << 16) | sw[1];
-            if constexpr (POOL > 1) full |= (uint32_t)__shfl_xor((int)full, NI);  // the window's other column
-            const unsigned item_word = ((unsigned)(oy * p.OW + (x0 + g * NX) / POOL) * (unsigned)p.ow + (unsigned)tile0) * uB * 4u;
-            __builtin_amdgcn_raw_buffer_store_b32(full, out_rsrc, (int)(xc < xcols ? place_word + item_word : kOutOfRange), 0, 0);
-            // ---- doubtful values of this item go on the list, one per lane at a time.  Recomputed are those of earlier
-            // items (their stores are older than this item's, so nothing of this item is waited for), four at a time, and
-            // all that are there where the list is full and after the wave's last item.
-            const bool last = !more && g + wg_step >= n_groups;
-            if (count >= 4) {
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RES != RES_NONE ? 2 * MT + 1 : 1) : "memory");
-                recompute();
-            }
-            for (;;) {
-                unsigned long long who;
-                int c;
-                while ((c = __builtin_amdgcn_readfirstlane(__popcll(who = __ballot(doubt != 0u)))) != 0 && count + c <= kListCap) {
-                    if (doubt != 0u) {
-                        const int bit = __ffs(doubt) - 1;
-                        doubt &= doubt - 1u;
-                        const int at = count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0u));
-                        const int py = POOL > 1 ? bit >> 4 : 0, m = POOL > 1 ? 0 : bit >> 4;
-                        list[2 * at] = (uint32_t)(oy * POOL + py) << 16 | (uint32_t)xc;
-                        list[2 * at + 1] = (uint32_t)((tile0 + m) * 32 + 16 * h + 15 - (bit & 15)) | (uint32_t)img << 16;
-                    }
-                    count += c;
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const v4f* const tp = reinterpret_cast<const v4f*>(thr + (tile0 + m) * 32 + 16 * h);
+                uint32_t w = 0u;
+                float zero = 0.0f;  // an infinity or NaN among a tap's values makes NaN of it, times 0, in every sum
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    w = __builtin_amdgcn_alignbit(w, __float_as_uint(acc[m][i] - tp[i >> 2][i & 3]), 31);
+                    zero = __builtin_fmaf(acc[m][i], 0.0f, zero);
                 }
-                if (c == 0 && (!last || count == 0)) break;
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                do recompute();
-                while (count > kListCap / 2);
+                const bool bad = !(zero == 0.0f);
+                word[m] |= bad ? 0u : ~w & 0xffffu;
+                doubt |= (bad && valid ? 0xffffu : 0u) << (16 * (POOL > 1 ? py : m));
+                if constexpr (RES != RES_NONE) {
+                    int v[16];
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v[i] = (int)acc[m][i];
+                    const unsigned item = (unsigned)(oy * p.PW + x0 + g * NX) * pixel_b + (unsigned)((tile0 + m) * 2) * group_b;
+                    store_residual_group<RES>(res_rsrc, p.res_fmt, valid ? place_res + item : kOutOfRange,
+                                              RES == RES_12 ? (valid ? place_res8 + item : kOutOfRange) : 0u, uB * 16u, v);
+                    __builtin_amdgcn_sched_barrier(0);  // (one tile at a time: registers)
+                }
             }
         }
-        if constexpr (kShared) __syncthreads();
-        if (more) split_and_store(q.adv, s0);
-        ay0 += q.adv;
-        s0 += q.adv;
-        s0 = s0 >= q.ring ? s0 - q.ring : s0;
+    };
+
+    // ---- the band's items, in up to three passes.  The common one ends at an item with many values in doubt.  That item and
+    // the rest of the band are then done with marks (common sums, exact where a window has none), and from an item on where
+    // that still leaves many, in the reference's order.  (A shared ring is left by all its waves together, before the next
+    // row, and for ordered sums.)
+    int oy = oy_begin, g = wg0;
+    bool many = false;
+    auto pass = [&](auto mode) __attribute__((always_inline)) {
+        constexpr bool kMarked = decltype(mode)::value == MARKED, kOrdered = decltype(mode)::value == ORDERED;
+        constexpr int kManyLanes = kMarked ? kManyLanesMarked : kManyLanesCommon;
+        // Few sums are ever in doubt where no residual is saved: that there are many is seen by the list, and the pass ends
+        // with the row, which costs its loop less.
+        constexpr bool kRowExit = RES == RES_NONE && !kShared;
+        int first_g = n_groups;
+        many = false;
+        for (; oy < oy_end; ++oy) {
+            const bool more = oy + 1 < oy_end;  // uniform
+            if constexpr (kShared && !kOrdered) {
+                __syncthreads();
+                if (grid) grid = __builtin_amdgcn_readfirstlane(flags[0]) == 0;
+                if (__builtin_amdgcn_readfirstlane(flags[1]) != 0) return;  // (written between the two barriers only)
+            }
+            if (!kOrdered && more) fetch(ay0 + q.ring, q.adv);
+            while (g < n_groups) {
+                uint32_t word[MT];
+                uint32_t doubt = 0u;
+                // A lane's place (column of the tile: image and pixel; half of the channels) is worked out anew from a lane
+                // index the compiler cannot carry over: kept across the multiplication, the addresses made from it spill.
+                int ln = lane;
+                asm volatile("" : "+v"(ln));
+#pragma unroll
+                for (int m = 0; m < MT; ++m) word[m] = 0u;
+                if constexpr (!kOrdered) {
+#pragma unroll 1
+                    for (int py = 0; py < POOL; ++py) {
+                        v16f acc[MT];
+#pragma unroll
+                        for (int m = 0; m < MT; ++m)
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
+                        const int first_col = (g * NX + ((ln & 31) >> q.ni_log2)) * p.stride_w;
+                        const int lane_at = (ln & (NI - 1)) * q.pp * 16 + (PAIRS == PAIRS_SPLIT ? (first_col >> 2) * 16 + (ln >> 5) * q.odd_pairs * 16
+                                                                                               : first_col * 8 + (ln >> 5) * 16);
+                        auto fragment = [&](int r, int j, int plane_off) -> v4i {
+                            int slot = s0 + py * p.stride_h + r;
+                            slot = slot >= q.ring ? slot - q.ring : slot;
+                            const char* const at = rows + (slot * row_bytes + plane_off) + lane_at + j * (PAIRS == PAIRS_SPLIT ? 16 : 32);
+                            if constexpr (PAIRS != PAIRS_ANY)
+                                return __builtin_bit_cast(v4i, *reinterpret_cast<const h8*>(at));
+                            else
+                                return __builtin_bit_cast(v4i, static_cast<h8>(*reinterpret_cast<const h8u*>(at)));
+                        };
+                        bool exact = false;  // this lane's window has no mark
+                        if constexpr (kMarked) {
+                            uint32_t marks = 0u;
+#pragma unroll 2
+                            for (int k = 0; k < NK; ++k) {
+                                const v4i v = fragment(k / NQ, k % NQ, plane);
+                                const int s = 4 * (k % NQ) + 2 * (ln >> 5);
+                                marks |= (s < p.S ? (uint32_t)v[1] : 0u) | (s + 1 < p.S ? (uint32_t)v[3] : 0u);
+                            }
+                            const auto sw = __builtin_amdgcn_permlane32_swap(marks, marks, false, false);
+                            exact = (sw[0] | sw[1]) < 0x10000u;
+                        }
+                        // lo steps, then hi steps; a step's fragment is requested kAhead steps ahead
+                        constexpr int kAhead = 4;
+                        v4i ahead[kAhead];
+#pragma unroll
+                        for (int k = 0; k < kAhead; ++k) ahead[k] = fragment(k % NK / NQ, k % NK % NQ, k < NK ? plane : 0);
+                        float sq = 0.0f, two_e = 0.0f, half_a = 0.0f, wide_shift = 0.0f, wide_two_e = 0.0f;
+                        bool bad = false, small = false;  // small: |S| and |acc| are below 1/2, the residual is 0
+#pragma unroll
+                        for (int k = 0; k < 2 * NK; ++k) {
+                            v4i v = ahead[k % kAhead];
+                            if (k + kAhead < 2 * NK)
+                                ahead[k % kAhead] = fragment((k + kAhead) % NK / NQ, (k + kAhead) % NK % NQ, k + kAhead < NK ? plane : 0);
+                            if (k >= NK) {
+#pragma unroll
+                                for (int d = 0; d < 4; ++d) {
+                                    const int two = v[d];
+                                    sq = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, two), __builtin_bit_cast(h2, two), sq, false);
+                                }
+                            }
+                            if (kMarked && k == NK - 1 && lane < 32) v[1] &= 0xffff;  // (a mark where -E will enter)
+                            if (k == 2 * NK - 1) {
+                                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(sq), __float_as_uint(sq), false, false);
+                                const float all = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+                                const float root = __builtin_amdgcn_sqrtf(all), full = root * q.bound_scale_full + q.bound_add;
+                                small = all < q.small_squares;
+                                bad = !(all < 4.0e9f) || !(full < 3.0e4f);
+                                _Float16 eh = (_Float16)(root * q.bound_scale + q.bound_add);
+                                half_a = root * q.half_scale;
+                                wide_two_e = 2.002f * full;
+                                if ((grid | exact) & (all < q.exact_squares)) {
+                                    eh = (_Float16)0.0f;
+                                    half_a = INFINITY;
+                                }
+                                two_e = 2.002f * (float)eh;
+                                wide_shift = (float)eh - full;
+                                if (lane < 32) v[1] |= (int)((uint32_t)(__builtin_bit_cast(uint16_t, eh) | 0x8000u) << 16);
+                            }
+#pragma unroll
+                            for (int m = 0; m < MT; ++m)
+                                acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, wf[k % NK][m]), __builtin_bit_cast(h8, v), acc[m], 0, 0, 0);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                        // ---- bits (MSB first; the sign of S - E - bn, inverted), residual, doubtful values
+                        asm volatile("" : "+v"(ln));
+                        const int h = ln >> 5;
+                        const bool valid = b0 + (ln & (NI - 1)) < p.B && x0 + g * NX + ((ln & 31) >> q.ni_log2) < xcols;
+#pragma unroll
+                        for (int m = 0; m < MT; ++m) {
+                            const v4f* const tp = reinterpret_cast<const v4f*>(thr + (tile0 + m) * 32 + 16 * h);
+                            // Signs are collected MSB first (bit 15 - i: channel i).  w: S - E < bn, dm: values in doubt.  Integers
+                            // within E are common (in every other tile) and collected like the bits; thresholds within E and sums
+                            // above A/2 (E is less than a bound for those) are rare: the tile's nearest distance below a threshold
+                            // and its largest |S| tell whether to look for them.
+                            uint32_t w = 0u, dm = 0u;
+                            int nearest = INT32_MAX;
+                            float most = 0.0f;
+                            {
+                                const v4f th[4] = {tp[0], tp[1], tp[2], tp[3]};
+#pragma unroll
+                                for (int i = 0; i < 16; ++i) {
+                                    const float d = acc[m][i] - th[i >> 2][i & 3];
+                                    w = __builtin_amdgcn_alignbit(w, __float_as_uint(d), 31);
+                                    nearest = min(nearest, __float_as_int(d));
+                                    if constexpr (kHalf) most = __builtin_fmaxf(most, __builtin_fabsf(acc[m][i]));
+                                    if constexpr (RES != RES_NONE)
+                                        dm = __builtin_amdgcn_alignbit(dm, __float_as_uint(__builtin_amdgcn_fractf(-acc[m][i]) - two_e), 31);
+                                }
+                            }
+                            if constexpr (RES != RES_NONE) dm = small ? 0u : dm;
+                            // (NaN: `bad` is set)
+                            if (__ballot(bad | (kHalf & !(most <= half_a)) | (nearest <= (int)(0x80000000u | __float_as_uint(two_e)))) != 0) {
+                                const bool wide = kHalf & !(most <= half_a);  // this lane's sums with the full bound
+                                const float shift = wide ? wide_shift : 0.0f, two = wide ? wide_two_e : two_e;
+                                uint32_t w2 = 0u, r = 0u;
+                                w = 0u;
+#pragma unroll
+                                for (int i = 0; i < 16; ++i) {
+                                    float a = acc[m][i];
+                                    asm volatile("" : "+v"(a));  // (evaluated again here: not kept from above)
+                                    a += shift;
+                                    const float d = a - tp[i >> 2][i & 3];
+                                    w = __builtin_amdgcn_alignbit(w, __float_as_uint(d), 31);
+                                    w2 = __builtin_amdgcn_alignbit(w2, __float_as_uint(d + two), 31);
+                                    if constexpr (RES != RES_NONE) r = __builtin_amdgcn_alignbit(r, __float_as_uint(__builtin_amdgcn_fractf(-a) - two), 31);
+                                }
+                                w = bad ? 0xffffu : w;
+                                dm = bad ? 0xffffu : (w & ~w2) | (wide || !small ? r : 0u);
+                            }
+                            doubt |= (valid ? dm & 0xffffu : 0u) << (16 * (POOL > 1 ? py : m));
+                            word[m] |= ~w & 0xffffu;  // (a bit in doubt is 0 here: the recomputation only ever sets it)
+                            if constexpr (RES != RES_NONE) {
+                                int v[16];
+#pragma unroll
+                                for (int i = 0; i < 16; ++i) v[i] = (int)acc[m][i];
+                                const unsigned item = (unsigned)(oy * p.PW + x0 + g * NX) * pixel_b + (unsigned)((tile0 + m) * 2) * group_b;
+                                store_residual_group<RES>(res_rsrc, p.res_fmt, valid ? place_res + item : kOutOfRange,
+                                                          RES == RES_12 ? (valid ? place_res8 + item : kOutOfRange) : 0u, uB * 16u, v);
+                                __builtin_amdgcn_sched_barrier(0);  // (one tile at a time: registers)
+                            }
+                        }
+                    }
+                }
+                if constexpr (kOrdered) ordered_sums(oy, g, word, doubt);
+                // ---- output words: two tiles: lane half h stores the word of tile h; one tile: half 0 stores
+                asm volatile("" : "+v"(ln));
+                const int h = ln >> 5, img = ln & (NI - 1), xc = x0 + g * NX + ((ln & 31) >> q.ni_log2);
+                const auto sw = __builtin_amdgcn_permlane32_swap(word[0], word[MT - 1], false, false);
+                uint32_t full = (sw[0] << 16) | sw[1];
+                if constexpr (POOL > 1) full |= (uint32_t)__shfl_xor((int)full, NI);  // the window's other column
+                const unsigned item_word = ((unsigned)(oy * p.OW + (x0 + g * NX) / POOL) * (unsigned)p.ow + (unsigned)tile0) * uB * 4u;
+                __builtin_amdgcn_raw_buffer_store_b32(full, out_rsrc, (int)(xc < xcols ? place_word + item_word : kOutOfRange), 0, 0);
+                // ---- doubtful values of this item go on the list, one per lane at a time.  Recomputed are those of earlier
+                // items (their stores are older than this item's, so nothing of this item is waited for), four at a time, and
+                // all that are there where the list is full and after the wave's last item.
+                const bool last = !more && g + wg_step >= n_groups;
+                if (count >= 4) {
+                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RES != RES_NONE ? 2 * MT + 1 : 1) : "memory");
+                    recompute();
+                }
+                unsigned long long who = __ballot(doubt != 0u);
+                const int earlier = count;
+                if (!kOrdered && RES != RES_NONE && who != 0) {  // uniform
+                    many = __builtin_popcountll(who) >= kManyLanes || __ballot(__builtin_popcount(doubt) >= kManyInLane) != 0;
+                    if (many) who = 0;  // (what is stored of this item is stored again)
+                }
+                if (!kOrdered && kRowExit && many) who = 0;
+                for (;;) {
+                    int c;
+                    while ((c = __builtin_amdgcn_readfirstlane(__popcll(who))) != 0 && count + c <= kListCap) {
+                        if (doubt != 0u) {
+                            const int bit = __ffs(doubt) - 1;
+                            doubt &= doubt - 1u;
+                            const int at = count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0u));
+                            const int py = POOL > 1 ? bit >> 4 : 0, m = POOL > 1 ? 0 : bit >> 4;
+                            list[2 * at] = (uint32_t)(oy * POOL + py) << 16 | (uint32_t)xc;
+                            list[2 * at + 1] = (uint32_t)((tile0 + m) * 32 + 16 * h + 15 - (bit & 15)) | (uint32_t)img << 16;
+                        }
+                        count += c;
+                        who = __ballot(doubt != 0u);
+                    }
+                    if (c == 0 && (!last || count == 0 || (!kShared && many))) break;
+                    if (!kOrdered && RES == RES_NONE && c != 0) {  // the list is full
+                        many = true;
+                        if constexpr (kRowExit) {
+                            first_g = g;
+                            count = earlier;
+                            break;
+                        }
+                    }
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    do recompute();
+                    while (count > kListCap / 2);
+                }
+                if (RES != RES_NONE && many) return;
+                g += wg_step;
+            }
+            if (kRowExit && many) {
+                g = first_g;
+                return;
+            }
+            g = wg0;
+            if constexpr (kShared && !kOrdered) {
+                __syncthreads();
+                if (many && lane == 0) flags[1] = 1;
+            }
+            if (!kOrdered && more) split_and_store(std::bool_constant<kMarked>{}, q.adv, s0);
+            ay0 += q.adv;
+            s0 += q.adv;
+            s0 = s0 >= q.ring ? s0 - q.ring : s0;
+        }
+    };
+    pass(std::integral_constant<Mode, COMMON>{});
+    if (!kShared && oy < oy_end) {
+        stage_window(std::true_type{});
+        pass(std::integral_constant<Mode, MARKED>{});
     }
+    if (oy < oy_end) pass(std::integral_constant<Mode, ORDERED>{});
 }
 
 // ---------------------------------------------------------------- host side
@@ -721,6 +963,7 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     q.half_scale = (float)(0.49 * a_scale);
     q.bound_add = (float)(3.0 * T * std::ldexp(1.0, -24) + std::ldexp(1.0, -22));
     q.small_squares = (float)(0.2 / (3.0 * T));
+    q.exact_squares = (float)(60000.0 * 60000.0 / (3.0 * T));  // (sum of |x| below 2^16 = 2^24 / 256)
     *out = c;
     return true;
 }
@@ -753,7 +996,7 @@ int launch(const InConvParams& p, const Choice& c, int dev, hipStream_t stream) 
     }
     const uint32_t* pats = reinterpret_cast<const uint32_t*>(p.masks) + (size_t)p.R * p.S * p.opad * 4;
     hipLaunchKernelGGL((inconv_mfma_kernel<R, NQ, MT, RES, POOL, PAIRS>), dim3((unsigned)c.grid), dim3(kThreads),
-                       c.lds_bytes, stream, p, c.q, p.in, pats, p.bn, (unsigned)c.out_bytes, (unsigned)c.res_bytes);
+                       c.lds_bytes, stream, KernelArgs{p, c.q, pats, (unsigned)c.out_bytes, (unsigned)c.res_bytes});
     TCBNN_LAUNCH_CHECK("inconv_mfma_kernel");
     return TCBNN_OK;
 }

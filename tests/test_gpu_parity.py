@@ -936,6 +936,86 @@ def test_inconv128_matrix_cores(gpu, b, h, w, R, S, stride, cout, pool, save, fm
     layer.release()
 
 
+def _flat_images(r, b, h, w, kind):
+    """Images whose first-layer sums meet integers (or thresholds of 0) in whole areas, or everywhere."""
+    x = (r.random((b, 3, h, w)) * 2 - 1).astype(np.float32)
+    level = np.float32(1)
+    if kind == "quantised":           # sums that are multiples of 1/128
+        return (np.rint(r.random((b, 3, h, w)) * 255) / 128 - 1).astype(np.float32)
+    if kind == "mean_subtracted":     # bytes less a mean: large sums, of which one in fifteen is within E of an integer
+        return (np.rint(r.random((b, 3, h, w)) * 255) - np.array([103.939, 116.779, 123.68])[None, :, None, None]).astype(np.float32)
+    if kind == "grey":                # no multiples of 1/256: every fifth sum is a whole number but for its roundings
+        level = np.float32(0.2)
+    elif kind == "grid_and_dust":     # flat areas that are NOT what their fp16 halves say
+        level = np.float32(0.25)
+    x[:, :, :h // 4] = -level         # bar
+    for i in range(b):                # patches at every parity of place and width
+        y0, x0 = int(r.integers(0, h - h // 3)), int(r.integers(0, w - w // 3))
+        x[i, :, y0:y0 + h // 3 + i % 3, x0:x0 + w // 3 + i % 4] = level
+    if kind == "grid_and_dust":
+        dust = r.random(x.shape) < 0.02
+        x[dust & (np.abs(x) == 0.25)] *= np.float32(1 + 2.0 ** -23)
+        x[r.random(x.shape) < 0.01] = np.float32(1e-42)
+    elif kind == "special":
+        x[0, 0, h // 5, w // 2], x[-1, 2, 1, 1], x[b // 2, 1, h // 2, w - 1], x[0, 1, 0, 0] = np.nan, np.inf, -1e30, 3e38
+    return x
+
+
+@pytest.mark.parametrize("kind", ["flat", "quantised", "grey", "mean_subtracted", "grid_and_dust", "special"])
+@pytest.mark.parametrize("b,h,w,R,S,stride,cout,pool,save", [(16, 60, 60, 7, 7, 4, 64, 1, True), (9, 50, 70, 7, 5, 2, 128, 1, True),
+                                                             (33, 30, 31, 3, 3, 1, 64, 1, True), (10, 26, 26, 3, 3, 2, 128, 1, False),
+                                                             (3, 150, 170, 7, 7, 2, 64, 1, False), (34, 70, 90, 11, 11, 4, 64, 2, False)])
+def test_inconv128_areas_in_doubt(gpu, b, h, w, R, S, stride, cout, pool, save, kind):
+    """The first layer's passes for many doubtful values: exact sums of windows on the grid of 1/256, ordered sums, and what
+    is left for the list; thresholds of 0, of whole numbers and of whole numbers' neighbours."""
+    r = rng(7000 + b + h + R)
+    x = _flat_images(r, b, h, w, kind)
+    f = rm.pm1(r, (R, S, 3, cout))
+    bn = np.rint(r.normal(0, np.sqrt(R * S), cout)).astype(np.float32)
+    bn[:8] = 0
+    bn[8:16] = np.nextafter(bn[8:16], np.float32(100))
+    with np.errstate(all="ignore"):
+        want, wres = orc.inconv128(x, f, bn, stride, True, pool, save)
+    for fmt in ([None, gpu._lib.RES_I32] if save else [None]):
+        layer = gpu.InConv128LayerParam("Conv1", h, w, R, S, 3, cout, b, stride, stride, True, pool, pool, save, residual_format=fmt)
+        layer.initialize(x, gpu.ArrayWeights([f, bn]))
+        assert "mfma" in layer.kernel_name(), layer.kernel_name()
+        layer.forward()
+        gpuops.sync()
+        np.testing.assert_array_equal(layer.download_packed(), want)
+        if save:
+            np.testing.assert_array_equal(layer.download_residual(), wres)
+        layer.release()
+
+
+def test_inconv128_time_does_not_hang_on_the_images(gpu):
+    """Bars and patches of +-1 over a third of the images cost next to nothing over random ones, and images of which every
+    sum is in doubt a small factor (one by one, sums in doubt took 70 and 130 times as long)."""
+    from tcbnn_amd.device import Event
+    r = rng(5)
+    b, h = 128, 224
+    f, bn = rm.pm1(r, (7, 7, 3, 64)), r.normal(0, 12, 64).astype(np.float32)
+    us = {}
+    for kind in ("random", "flat", "mean_subtracted", "thousands"):
+        x = r.standard_normal((b, 3, h, h)).astype(np.float32) * (1000 if kind == "thousands" else 1)
+        if kind in ("flat", "mean_subtracted"):
+            x = _flat_images(r, b, h, h, kind)
+        layer = gpu.InConv128LayerParam("Conv1", h, h, 7, 7, 3, 64, b, 4, 4, True, 1, 1, True)
+        layer.initialize(np.ascontiguousarray(x, dtype=np.float32), gpu.ArrayWeights([f, bn]))
+        layer.forward()
+        us[kind] = 1e9
+        for _ in range(4):
+            e0, e1 = Event(), Event()
+            e0.record()
+            for _ in range(4):
+                layer.forward()
+            e1.record()
+            e1.synchronize()
+            us[kind] = min(us[kind], e0.elapsed_ms(e1) * 250)
+        layer.release()
+    assert us["flat"] < 1.5 * us["random"] and max(us.values()) < 6 * us["random"], us
+
+
 @pytest.mark.parametrize("b,h,R,stride,pool,kind", [(16, 40, 7, 4, 1, "normal"), (16, 40, 7, 4, 1, "mixed"), (16, 30, 7, 2, 1, "spikes"),
                                                     (16, 20, 3, 1, 1, "normal"), (16, 20, 3, 1, 1, "mixed"), (16, 20, 3, 1, 1, "spikes"),
                                                     (16, 60, 11, 4, 2, "normal"), (16, 60, 11, 4, 2, "mixed"), (16, 60, 11, 4, 2, "spikes")])
