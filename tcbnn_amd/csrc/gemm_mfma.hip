@@ -29,7 +29,10 @@ constexpr int kFrags = kBlk * kNT / kWaves;  // fragments a wave stages per bloc
 
 // Row words are expanded without shifts (expand_rows_f4 in mfma_util.h): the accumulator ends as the dot product
 // plus a per-column constant, which the staging lanes count as they go and the epilogue takes off.
-template <int MT, int EPI>
+// ODD: an odd number of words per row (the stand-alone product alone can have one; a fully connected layer's rows are whole
+// 128-bit units): the last k-step's upper words do not exist.  As a test in every staging it cost the MLP, whose hidden
+// layers' whole K is one staging block, 1.2 % (43.2 us for 42.7 at batch 8192).
+template <int MT, int EPI, bool ODD>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_mfma_f4_kernel(
     const BgemmParams p, const uint32_t* __restrict__ act, const uint32_t* __restrict__ wgt,
     const float* __restrict__ bnp, const float* __restrict__ bias, int n_groups) {
@@ -60,8 +63,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
         for (int i = 0; i < kFrags; ++i) {
             const int q = q0 + sq + 2 * i;
-            if (2 * q + 1 < p.cw) wx[i] = wrow[2 * q];  // (uniform)
-            else wx[i] = 2 * q + h < p.cw ? wrow[2 * q] : 0u;
+            wx[i] = 0u;
+            if (ODD ? 2 * q + h < p.cw : 2 * q < p.cw) wx[i] = wrow[2 * q];  // (not ODD: uniform)
         }
     };
     int csum = 0;  // this lane's share of its column's constant C: the words it stages, pad steps included
@@ -299,7 +302,7 @@ bool gemm_mfma_applicable(const BgemmParams& p) {
     if (p.PH * p.PW != 1 || p.R * p.S != 1 || p.pool_h * p.pool_w != 1) return false;
     if (p.res_in != nullptr || p.res_out != nullptr) return false;
     if (p.mode != EPI_THRESH && p.mode != EPI_AFFINE && p.mode != EPI_RAW) return false;
-    if (p.k_tap > 32 * p.cw) return false;
+    if (p.k_tap > 32 * p.cw || (p.cw % 2 != 0 && p.mode != EPI_RAW)) return false;
     if ((long long)p.cw * p.B * 4 >= (1LL << 31)) return false;          // 32-bit buffer offsets
     // large enough to give every CU a workgroup with two image tiles per wave; smaller problems are bound by
     // launch and fill and stay with the kernels written for them
@@ -308,7 +311,7 @@ bool gemm_mfma_applicable(const BgemmParams& p) {
 }
 
 void gemm_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len) {
-    snprintf(buf, len, "gemm_mfma_f4_kernel<%d, %d>", gemm_mt(p), p.mode);
+    snprintf(buf, len, "gemm_mfma_f4_kernel<%d, %d, %s>", gemm_mt(p), p.mode, p.cw % 2 != 0 ? "true" : "false");
 }
 
 template <int MT>
@@ -318,18 +321,24 @@ static int launch_gemm_mt(const BgemmParams& p, hipStream_t stream) {
     const long long blocks = row_blocks * n_groups;
     if (blocks <= 0 || blocks > 0x7fffffffLL) return fail(TCBNN_EINVAL, "gemm grid too large");
     const dim3 grid((unsigned)blocks), block(kThreads);
+    const bool odd = p.cw % 2 != 0;
+    TCBNN_REQUIRE(!odd || p.mode == EPI_RAW, "gemm: an odd number of words per row");
     switch (p.mode) {
         case EPI_THRESH:
-            hipLaunchKernelGGL((gemm_mfma_f4_kernel<MT, EPI_THRESH>), grid, block, 0, stream, p, p.act, p.wgt, p.bn,
+            hipLaunchKernelGGL((gemm_mfma_f4_kernel<MT, EPI_THRESH, false>), grid, block, 0, stream, p, p.act, p.wgt, p.bn,
                                p.bn, n_groups);
             break;
         case EPI_AFFINE:
-            hipLaunchKernelGGL((gemm_mfma_f4_kernel<MT, EPI_AFFINE>), grid, block, 0, stream, p, p.act, p.wgt,
+            hipLaunchKernelGGL((gemm_mfma_f4_kernel<MT, EPI_AFFINE, false>), grid, block, 0, stream, p, p.act, p.wgt,
                                p.bn_scale, p.bn_bias, n_groups);
             break;
         default:
-            hipLaunchKernelGGL((gemm_mfma_f4_kernel<MT, EPI_RAW>), grid, block, 0, stream, p, p.act, p.wgt, p.bn,
-                               p.bn, n_groups);
+            if (odd)
+                hipLaunchKernelGGL((gemm_mfma_f4_kernel<MT, EPI_RAW, true>), grid, block, 0, stream, p, p.act, p.wgt, p.bn,
+                                   p.bn, n_groups);
+            else
+                hipLaunchKernelGGL((gemm_mfma_f4_kernel<MT, EPI_RAW, false>), grid, block, 0, stream, p, p.act, p.wgt, p.bn,
+                                   p.bn, n_groups);
     }
     TCBNN_LAUNCH_CHECK("gemm_mfma_f4_kernel");
     return TCBNN_OK;

@@ -90,6 +90,16 @@ def test_no_long_k_is_refused_for_its_lds():
             (b, hw, cin, cout, L.tcbnn_last_error())
 
 
+def test_large_products_test_for_odd_words_only_where_there_can_be_any():
+    """Fully connected layers, whose rows are whole 128-bit units, run an instantiation without that test."""
+    import ctypes as C
+    from tcbnn_amd import _lib
+    name = C.create_string_buffer(128)
+    d = _lib.Fc128Desc(1, 1, 1, 1, 8192, 784, 1024, _lib.VARIANT_MFMA_F4, None, 0)
+    _lib.check(_lib.lib.tcbnn_fc128_kernel_name(C.byref(d), name, 128))
+    assert name.value == b"gemm_mfma_f4_kernel<2, 0, false>"
+
+
 def test_network_specs_match_reference_wiring():
     from tcbnn_amd import nets
     spec = nets.imagenet_resnet_spec(batch=256)
