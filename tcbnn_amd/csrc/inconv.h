@@ -17,9 +17,9 @@ struct InConvParams {
     int PH, PW, pool_h, pool_w, OH, OW;
 };
 
-// First layer on the matrix cores (inconv_mfma.hip): whether it serves a problem, its launch, its kernel's name.
-bool inconv_mfma_applicable(const InConvParams& p);
-int launch_inconv_mfma(const InConvParams& p, hipStream_t stream);
-void inconv_mfma_kernel_name(const InConvParams& p, char* buf, size_t len);
+// First layer on the matrix cores (inconv_mfma.hip): its kernel's name (false: it does not serve the problem), its launch
+// (`served`: whether it does; if not, nothing has been launched).
+bool inconv_mfma_kernel_name(const InConvParams& p, char* buf, size_t len);
+int launch_inconv_mfma(const InConvParams& p, hipStream_t stream, bool* served);
 
 }  // namespace tcbnn

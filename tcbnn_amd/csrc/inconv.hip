@@ -809,10 +809,11 @@ static int inconv128_run(const tcbnn_inconv128_desc* d, void* stream, char* name
     }
     TCBNN_REQUIRE(d->input_layout == TCBNN_INCONV_INPUT_NCHW, "inconv128: unknown input_layout");
     // 3-, 7- and 11-row filters on 32- or 64-channel tiles: matrix cores (inconv_mfma.hip says what it serves and why)
-    if (!force_linear && inconv_mfma_applicable(p)) {
-        if (name_buf == nullptr) return launch_inconv_mfma(p, (hipStream_t)stream);
-        inconv_mfma_kernel_name(p, name_buf, name_len);
-        return TCBNN_OK;
+    if (!force_linear && name_buf != nullptr && inconv_mfma_kernel_name(p, name_buf, name_len)) return TCBNN_OK;
+    if (!force_linear && name_buf == nullptr) {
+        bool served = false;
+        const int rc = launch_inconv_mfma(p, (hipStream_t)stream, &served);
+        if (served || rc != TCBNN_OK) return rc;
     }
     if (name_buf != nullptr) {  // report the kernel instead of launching it
         if (!tiled) {

@@ -856,9 +856,11 @@ struct Choice {
 
 size_t lds_extra(int channels) { return (size_t)(channels + 4 * 2 * kListCap + 4) * 4; }
 
-// Shapes with an instantiation, and how a launch is split.  `cus`: compute units.
-bool choose(const InConvParams& p, int cus, Choice* out) {
-    Choice c{};
+// The instantiation for a problem's form, if there is one: what the networks' first layers need.  (For other forms, 5x5
+// filters, pooled 3x3, 32-channel or odd-stride 7x7 layers, there is none and nothing has been measured: the kernels of
+// inconv.hip serve them.)
+bool instantiated(const InConvParams& p, Choice* out) {
+    Choice& c = *out;
     c.r = p.R;
     c.nq = (p.S + 3) / 4;
     c.res = p.res == nullptr ? RES_NONE : (p.res_fmt == TCBNN_RES_I12 ? RES_12 : RES_WIDE);
@@ -873,6 +875,13 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     } else {
         return false;
     }
+    return true;
+}
+
+// How a launch is split; false for sizes that the kernel does not take.  `cus`: compute units.
+bool choose(const InConvParams& p, int cus, Choice* out) {
+    Choice c{};
+    if (!instantiated(p, &c)) return false;
     c.wg_per_cu = workgroups_per_cu(c.r);
     Geometry& q = c.q;
     q.adv = c.pool * p.stride_h;
@@ -1003,22 +1012,21 @@ int launch(const InConvParams& p, const Choice& c, int dev, hipStream_t stream) 
 
 }  // namespace
 
-bool inconv_mfma_applicable(const InConvParams& p) {
+bool inconv_mfma_kernel_name(const InConvParams& p, char* buf, size_t len) {
     Choice c;
-    return choose(p, 256, &c);
-}
-
-void inconv_mfma_kernel_name(const InConvParams& p, char* buf, size_t len) {
-    Choice c;
-    choose(p, 256, &c);
+    if (!choose(p, 256, &c)) return false;
     snprintf(buf, len, "inconv_mfma_kernel<%d, %d, %d, %d, %d, %d>", c.r, c.nq, c.mt, c.res, c.pool, c.pairs);
+    return true;
 }
 
-int launch_inconv_mfma(const InConvParams& p, hipStream_t stream) {
+int launch_inconv_mfma(const InConvParams& p, hipStream_t stream, bool* served) {
+    Choice c{};
+    *served = instantiated(p, &c);
+    if (!*served) return TCBNN_OK;
     int dev = 0, cus = 0;
     if (int rc = device_info(&dev, &cus)) return rc;
-    Choice c;
-    TCBNN_REQUIRE(choose(p, cus, &c), "inconv128: no matrix-core kernel for this shape");
+    *served = choose(p, cus, &c);
+    if (!*served) return TCBNN_OK;
     auto with_residual = [&](auto go) { return c.res == RES_12 ? go(std::integral_constant<int, RES_12>{}) : (c.res == RES_WIDE ? go(std::integral_constant<int, RES_WIDE>{}) : go(std::integral_constant<int, RES_NONE>{})); };
     if (c.r == 3)
         return with_residual([&](auto res) {
