@@ -128,10 +128,12 @@ int tcbnn_inconv_residual_bound_of_input(const float* input_host, int batch, int
 /* max |x| over a HOST array (on a few host threads; +infinity if any value is NaN or infinite): the cheap first test of
  * a new first-layer batch against the recorded bound, before the window scan above. */
 float tcbnn_host_abs_max(const float* values_host, size_t count);
-/* Uploads of new input batches.  An uploader holds pinned memory (at most 64 MiB; arrays of up to `bytes` bytes, longer
- * ones go through it in turns) and shares a few worker threads with the process's other uploaders; they end with the
- * last one.  tcbnn_upload copies `bytes` of HOST memory to the device, in the order of the null stream, and is complete
- * when it returns.  tcbnn_upload_stage (an uploader created with staged = 1) copies an array of floats out of
+/* Uploads of new input batches.  An uploader serves arrays of up to `bytes` bytes.  It holds pinned memory (at most
+ * 64 MiB), with staged = 1 and from 4 MiB on device memory for one array, and shares a few worker threads with the
+ * process's other uploaders; they end with the last one.  Where one of these cannot be had tcbnn_uploader_create returns
+ * TCBNN_EHIP (a thread that cannot be started is done without), and a plain copy does the same work.  tcbnn_upload copies
+ * `bytes` of HOST memory to the device, in the order of the null stream, and is complete when it returns.
+ * tcbnn_upload_stage (an uploader created with staged = 1) copies an array of floats out of
  * HOST memory, takes max |x| on the way (as tcbnn_host_abs_max) and leaves the destination alone;
  * tcbnn_upload_commit then writes the staged array to `dst`.  Each call on one uploader excludes the others.  A stage and
  * its commit are two calls about the ONE array that an uploader keeps staged: the next stage replaces it from its first

@@ -5,6 +5,9 @@
 // array (632 us there, 244 us for 2.4 MB).  Here one pass copies a piece into pinned memory and takes its maximum, the
 // pieces are shared with a few worker threads, and chunks go to the device as they fill up; the transfer is then all that
 // is left (set_input of 38.5 MB 1961 -> 800 us, of 2.4 MB 346 -> 92, of 0.6 MB 96 -> 45).
+// An uploader has to be made first, and the pages of its pinned memory are slow when they are first written (38.5 MB: 0.9 ms
+// and 3.5 ms), so the layers make one for their second batch, not for the first.  (16 MiB of pinned memory, used as a ring or
+// in two halves, cost 2 ms less there, and 90 to 260 us on every batch of 38.5 MB after it.)
 #include <hip/hip_runtime_api.h>
 #include <string.h>
 
@@ -204,6 +207,10 @@ struct tcbnn_uploader {
     bool on_device = false;  // the staged array is there (else in pinned memory)
     size_t staged = 0;
     std::shared_ptr<Workers> workers;
+    ~tcbnn_uploader() {
+        if (device != nullptr) (void)hipFree(device);
+        if (pinned != nullptr) (void)hipHostFree(pinned);
+    }
 };
 
 namespace {
@@ -261,12 +268,12 @@ int tcbnn_uploader_create(size_t bytes, int staged, tcbnn_uploader** out) {
     if (!u) return out_of_memory("uploader");
     u->bytes = bytes;
     u->pinned_bytes = std::min(kPinnedMost, (bytes + kPiece - 1) / kPiece * kPiece);
-    if (int rc = check_hip(hipHostMalloc(&u->pinned, u->pinned_bytes, hipHostMallocDefault), "hipHostMalloc")) return rc;
-    if (staged && bytes >= kOverlapFrom)
-        if (int rc = check_hip(hipMalloc(&u->device, bytes), "hipMalloc")) {
-            (void)hipHostFree(u->pinned);
-            return rc;
-        }
+    int rc = check_hip(hipHostMalloc(&u->pinned, u->pinned_bytes, hipHostMallocDefault), "hipHostMalloc");
+    if (rc == TCBNN_OK && staged && bytes >= kOverlapFrom) rc = check_hip(hipMalloc(&u->device, bytes), "hipMalloc");
+    if (rc != TCBNN_OK) {
+        (void)hipGetLastError();  // (a caller without an uploader copies as it is: the next launch is not to report this)
+        return rc;
+    }
     if (bytes > 4 * kPiece) {
         try {
             u->workers = Workers::get();
@@ -278,9 +285,6 @@ int tcbnn_uploader_create(size_t bytes, int staged, tcbnn_uploader** out) {
 }
 
 void tcbnn_uploader_destroy(tcbnn_uploader* u) {
-    if (u == nullptr) return;
-    if (u->device != nullptr) (void)hipFree(u->device);
-    if (u->pinned != nullptr) (void)hipHostFree(u->pinned);
     delete u;
 }
 

@@ -638,10 +638,15 @@ class InConv128LayerParam {  // param.h:701-870
         CHECK_NULL_POINTER(input_gpu);
         // (one batch at a time: an uploader keeps one staged array, which is staged, judged and committed here)
         std::lock_guard<std::mutex> one_batch(upload_guard);
-        if (uploader == NULL) TCBNN_SAFE_CALL(tcbnn_uploader_create(input_bytes(), save_residual ? 1 : 0, &uploader));
+        // The first batch is scanned and copied as it is: an uploader costs more to make than it saves on one batch.
+        // Where none can be made every batch goes that way.
+        if (++batches == 2 && tcbnn_uploader_create(input_bytes(), save_residual ? 1 : 0, &uploader) != TCBNN_OK) uploader = NULL;
         if (save_residual) {
             float abs_max = 0.0f;
-            TCBNN_SAFE_CALL(tcbnn_upload_stage(uploader, input, (size_t)input_size(), &abs_max));
+            if (uploader != NULL)
+                TCBNN_SAFE_CALL(tcbnn_upload_stage(uploader, input, (size_t)input_size(), &abs_max));
+            else
+                abs_max = tcbnn_host_abs_max(input, (size_t)input_size());
             const tcbnn_host::ResidualInfo* u = tcbnn_host::find_residual(output_residual_gpu);
             const int recorded = u != NULL ? u->bound : residual_info.bound;
             const int coarse = tcbnn_inconv_residual_bound(filter_height, filter_width, abs_max);
@@ -656,10 +661,13 @@ class InConv128LayerParam {  // param.h:701-870
                 }
                 tcbnn_host::raise_residual_bound(output_residual_gpu, bound);
             }
-            TCBNN_SAFE_CALL(tcbnn_upload_commit(uploader, input_gpu));
-        } else {
-            TCBNN_SAFE_CALL(tcbnn_upload(uploader, input_gpu, input, input_bytes()));
         }
+        if (uploader == NULL)
+            HIP_SAFE_CALL(hipMemcpy(input_gpu, input, input_bytes(), hipMemcpyHostToDevice));
+        else if (save_residual)
+            TCBNN_SAFE_CALL(tcbnn_upload_commit(uploader, input_gpu));
+        else
+            TCBNN_SAFE_CALL(tcbnn_upload(uploader, input_gpu, input, input_bytes()));
         this->input = input;
         pack_input();
     }
@@ -722,6 +730,7 @@ class InConv128LayerParam {  // param.h:701-870
         SAFE_FREE_GPU(input_packed_gpu);
         tcbnn_uploader_destroy(uploader);
         uploader = NULL;
+        batches = 0;
         SAFE_FREE_GPU(output_gpu);
         SAFE_FREE_GPU(filter_gpu);
         SAFE_FREE_GPU(bn_gpu);
@@ -767,7 +776,8 @@ class InConv128LayerParam {  // param.h:701-870
     int* output_residual_ref_gpu = NULL;
     bool packed_input = false;           // use_packed_input()
     std::mutex upload_guard;
-    tcbnn_uploader* uploader = NULL;     // set_input's pinned memory, made by the first call
+    tcbnn_uploader* uploader = NULL;     // set_input's pinned memory, made by the second call
+    unsigned batches = 0;                // calls of set_input
     float* input_packed_gpu = NULL;      // [Hp][Wp][batch][3] copy of input_gpu (un-pooled layers, on request)
 };
 

@@ -20,7 +20,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import lib, check
-from .device import DeviceBuffer, InputUploads, PinnedBuffer
+from .device import DeviceBuffer, Downloads, InputUploads
 
 
 def STEP8(x):
@@ -405,7 +405,8 @@ class Out128LayerParam(_ReferenceLayoutIO):
         self.output_height, self.output_width = input_height, weight_width
         self.variant = variant
         self.weight = self.bn_scale = self.bn_bias = None
-        self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = self.input_gpu = self._host = None
+        self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = self.input_gpu = None
+        self._downloads = Downloads()
 
     def weight_size(self):
         return self.weight_height * self.weight_width
@@ -452,16 +453,14 @@ class Out128LayerParam(_ReferenceLayoutIO):
         return buf.value.decode()
 
     def download_output(self):
-        if self._host is None:
-            self._host = PinnedBuffer(self.output_gpu.nbytes)
-        return self._host.download(self.output_gpu, np.float32, (self.output_height, self.output_width))
+        return self._downloads.get(self.output_gpu, np.float32, (self.output_height, self.output_width))
 
     def release(self):
         self._release_ref_bufs()
-        for b in (self.weight_gpu, self.bn_scale_gpu, self.bn_bias_gpu, self.output_gpu, self._host):
+        for b in (self.weight_gpu, self.bn_scale_gpu, self.bn_bias_gpu, self.output_gpu, self._downloads):
             if b is not None:
                 b.free()
-        self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = self._host = None
+        self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = None
 
 
 class _ConvGeometry(_ReferenceLayoutIO):
@@ -929,7 +928,8 @@ class AvgPoolFcLayerParam:
         self.name = name
         self.input_height, self.input_width = input_height, input_width
         self.channels, self.batch, self.out_features = channels, batch, out_features
-        self.input_residual_gpu = self.weight_gpu = self.bias_gpu = self.output_gpu = self._host = None
+        self.input_residual_gpu = self.weight_gpu = self.bias_gpu = self.output_gpu = None
+        self._downloads = Downloads()
 
     def initialize(self, config_file, input_residual_gpu):
         if input_residual_gpu is None:
@@ -959,12 +959,10 @@ class AvgPoolFcLayerParam:
         return "avgpool_fc_kernel<%d>" % self.input_residual_gpu.format
 
     def download_output(self):
-        if self._host is None:
-            self._host = PinnedBuffer(self.output_gpu.nbytes)
-        return self._host.download(self.output_gpu, np.float32, (self.batch, self.out_features))
+        return self._downloads.get(self.output_gpu, np.float32, (self.batch, self.out_features))
 
     def release(self):
-        for b in (self.weight_gpu, self.bias_gpu, self.output_gpu, self._host):
+        for b in (self.weight_gpu, self.bias_gpu, self.output_gpu, self._downloads):
             if b is not None:
                 b.free()
-        self.weight_gpu = self.bias_gpu = self.output_gpu = self._host = None
+        self.weight_gpu = self.bias_gpu = self.output_gpu = None
