@@ -78,6 +78,7 @@ def layer_work(L, spec=(), res_bytes=None, pooled=()):
     res_bytes = res_bytes or {}
     from tcbnn_amd import nets
     bops, flops = nets.binary_ops([L])
+    mfma_flops = 0.0
     B = L["batch"]
     if L["kind"] == "in":
         byts = B * L["features"] * 4 + B * L["features"] / 8
@@ -96,6 +97,8 @@ def layer_work(L, spec=(), res_bytes=None, pooled=()):
         out_bits = B * poh * pow_ * L["cout"] / 8
         if L["kind"] == "inconv":
             byts = B * 3 * L["h"] * L["w"] * 4 + out_bits + L["r"] * L["s"] * 3 * L["cout"] * 4
+            # fp16 products of the matrix-core kernel: four taps of four channels to a step, high and low parts
+            mfma_flops = 2.0 * B * oh * ow * L["cout"] * 2 * 16 * L["r"] * -(-L["s"] // 4)
             if L["save_residual"]:
                 byts += B * oh * ow * L["cout"] * res_bytes.get(L["name"], 4)
         else:
@@ -108,7 +111,7 @@ def layer_work(L, spec=(), res_bytes=None, pooled=()):
                 ch = min([L["residual_channels"], L["cout"]] + src_ch)
                 src_pixels = 4 if L["residual_pool"] and L.get("res_src") not in pooled else 1
                 byts += B * oh * ow * src_pixels * ch * res_bytes.get(L.get("res_src"), 4)
-    return dict(bops=bops, flops=flops, bytes=float(byts))
+    return dict(bops=bops, flops=flops, bytes=float(byts), mfma_flops=mfma_flops)
 
 
 def roofline_of(name, g, variant):
@@ -136,16 +139,21 @@ def roofline_of(name, g, variant):
         "ops_per_byte": round(intensity, 1) if g["bytes"] else None,
         "binary_tops": round(tops, 2), "hbm_gbs": round(gbs, 1),
     }
-    if g.get("flops"):
-        # The fp32 first layer is far from the HBM roof because its additions bind it: one dependent fp32 add per
-        # (tap, output channel, pixel, image) is the least the reference's summation order allows (its 2 flops per
+    if g.get("flops") and "mfma" in name:
+        # The first layer on the matrix cores: what it executes there, fp16 products of the inputs' high and low parts.
+        # `bound` stays the roof its algorithmic bytes put it under; the counters show neither pipe full.
+        done = g["mfma_flops"] / secs / 1e12
+        rec["matrix_fp16"] = {"flops_per_launch": round(g["mfma_flops"] / g["launches"]), "achieved": round(done, 1),
+                              "peak": 2500.0, "unit": "TFLOP/s", "frac": round(done / 2500.0, 4)}
+        rec["binding"] = "waves waiting for memory and for issue slots, under two per SIMD; see matrix_fp16"
+    elif g.get("flops"):
+        # The fp32 first layer on the VALU is far from the HBM roof because its additions bind it: one dependent fp32 add
+        # per (tap, output channel, pixel, image) is the least the reference's summation order allows (its 2 flops per
         # input value and tap are 6 per such add).  Peak: the published 157.3 TFLOP/s counts packed FMAs; plain adds
         # issue at a quarter of that (64 lanes per CU and clock).
         adds = g["flops"] / 6.0
         rec["valu_fp32"] = {"adds_per_launch": round(adds / g["launches"]), "achieved": round(adds / secs / 1e12, 2),
                             "peak": round(157.3 / 4, 1), "unit": "Tadd/s", "frac": round(adds / secs / 1e12 / (157.3 / 4), 4)}
-        # `bound` stays the roof the kernel's algorithmic bytes and operations put it under; what the hardware
-        # counters show it waiting for is the issue rate of its dependent fp32 additions
         rec["binding"] = "valu (dependent fp32 adds in the reference's summation order); see valu_fp32"
     return rec
 
@@ -438,9 +446,10 @@ def main():
         name = layer.kernel_name() if hasattr(layer, "kernel_name") else \
             {"in": "in128_kernel"}[L["kind"]]
         w = layer_work(L, spec, res_bytes, pooled)
-        g = groups.setdefault(name, dict(bops=0.0, flops=0.0, bytes=0.0, ms=0.0, launches=0))
+        g = groups.setdefault(name, dict(bops=0.0, flops=0.0, mfma_flops=0.0, bytes=0.0, ms=0.0, launches=0))
         g["bops"] += w["bops"]
         g["flops"] += w["flops"]
+        g["mfma_flops"] += w["mfma_flops"]
         g["bytes"] += w["bytes"]
         g["ms"] += layer_ms[L["name"]]
         g["launches"] += 1

@@ -36,6 +36,11 @@ def test_one_json_line_with_the_contract_keys(gpu):
     for key in ("bound", "achieved", "peak", "unit", "frac", "traffic"):
         assert key in r, key
     assert r["bound"] in ("hbm", "mfma") and abs(r["frac"] - r["achieved"] / r["peak"]) < 1e-3
+    # the first layer's record says what its kernel executes: products on the matrix cores, not additions on the VALU
+    assert "inconv_mfma" in r["kernel"] and "valu_fp32" not in r and "valu" not in r["binding"]
+    m = r["matrix_fp16"]
+    assert m["flops_per_launch"] == 256 * 56 * 56 * 64 * 2 * 2 * 16 * 14 and 0 < m["frac"] < 1
+    assert abs(m["achieved"] - m["flops_per_launch"] / r["avg_launch_ms"] / 1e9) <= 0.02 * m["achieved"]
     c = d["cpu_baseline"]
     for key in ("value", "unit", "cores", "kind", "sample"):
         assert key in c, key
