@@ -7,8 +7,10 @@
 // are no multiplies (the sign is applied by flipping the fp32 sign bit with a
 // precomputed mask), hence no FMA contraction either.
 //
-// Two kernels:
-//   inconv_tiled_kernel (pool 1x1): workgroup = one output row y, 4 consecutive output
+// The layers of the networks go to the matrix cores (inconv_mfma.hip, same bits and residuals); the kernels here serve what
+// that file has no instantiation for (other filter heights and poolings, channels that are no multiple of 64 or, at 11x11,
+// of 32, strides outside its forms, tensors of 2 GiB) and packed input:
+//   inconv_tiled_kernel (pool 1x1, or a pool_w of at most 2 without a residual): workgroup = one output row y, 4 consecutive output
 //     columns, 64 images (lane = image); a wave owns two of the columns and 32 of the 64 output
 //     channels of a pass.  For each filter row the needed
 //     input row segment of the 64 images is read with lanes running along the image row
@@ -244,7 +246,7 @@ __device__ __forceinline__ void inconv_store_residual(const float* acc, int32_t*
 // three channels of a tap are constant offsets apart and the 64 images of a wave's tap read fall into 64 different
 // banks (3 kSegStride is odd).  The host selects it when a segment fits the stride.
 constexpr int inconv_seg_stride(int nst) { return nst == 4 ? 5 : (nst == 8 ? 9 : (nst == 16 ? 21 : 31)); }
-// Where it is used: 16 passes (segments of 11 to 21 columns: 7-wide filters at strides 2 to 4, three waves' worth of
+// Where it is used: 16 passes (segments of 11 to 21 columns: 5- and 7-wide filters at strides 2 to 4, three waves' worth of
 // segments per pass), where it measured 2-4 % faster than staging through registers.  With 8 passes (3x3 filters at
 // stride 1: three taps per row) it measured 3-5 % slower and with 24 (11-wide filters, three waves per SIMD) 20 %.
 constexpr bool inconv_straight_to_lds(int nst, int ncols) { return nst == 16 && ncols <= inconv_seg_stride(nst); }

@@ -2,7 +2,7 @@
 // matrix cores, with the bits and residuals of the reference's own fp32 order of additions
 //     acc = 0; for r, for s (in-frame taps): acc += ((+-f0) + (+-f1)) + (+-f2);  bit = !(acc < bn);  residual = (int)acc.
 // On the VALU that order costs one dependent fp32 add per (tap, channel, pixel): 73 us at the very least for ResNet-18's
-// first layer at batch 256, 123-142 us in practice.  Here it is computed as a filtered predicate:
+// first layer at batch 256, 121-138 us in practice.  Here it is computed as a filtered predicate:
 //   1. every input is split into two fp16 numbers, x = hi + lo (22-23 bits), and S = sum of +-hi + sum of +-lo runs on
 //      v_mfma_f32_32x32x16_f16: products are exact, sums are fp32;
 //   2. a bound E of |S - acc| is known per pixel (below), so wherever S is further than E from the threshold, and from
@@ -23,10 +23,9 @@
 // The lo steps run first, on sums below 2^-10 A.  For A stands sqrt(3 T sum of hi^2), whose squares are one v_dot2 per
 // loaded dword and which such small values hardly enter: by Cauchy and Schwarz the losses of all halves add the most to
 // the rest of the bound where m = 0, and then 2 R NQ / (3 T) < 0.25 u A; 2.25 roundings are taken per step, not 2.  From
-// 7 rows on E is taken for |S| <= A/2 (partial sums
-// below 3/4 A); a lane with a larger sum looks again with the full bound.  -E itself enters the sum as one more product (the fourth channel of the
-// last tap, unused otherwise), so the accumulators hold S - E: a bit is certainly 1 where S - E >= bn, certainly 0 below
-// bn - 2E.
+// 7 rows on E is taken for |S| <= A/2 (partial sums below 3/4 A); a lane with a larger sum looks again with the full
+// bound.  -E itself enters the sum as one more product (the fourth channel of the last tap, unused otherwise), so the
+// accumulators hold S - E: a bit is certainly 1 where S - E >= bn, certainly 0 below bn - 2E.
 // Inputs outside the fp16 range, infinities and NaN make E infinite: all values of such a window are recomputed.
 //
 // Many values in doubt.  A saved residual puts every sum ON an integer in doubt, and images have areas of such sums: bars of
@@ -60,11 +59,15 @@
 // values).  11-row filters, whose rings are larger, share one among the four waves of a workgroup.  The four waves of a
 // workgroup are neighbouring strips; work of one image tile goes to one XCD.
 //
-// What binds it: instruction issue, 960 VALU instructions per 32 columns x 64 channels (7x7, 12-bit residual; 224 for 3x3
-// without one) next to 56 (12) MFMAs, two (four) waves per SIMD; HBM would allow 40 us for ResNet-18's layer at batch 256.
-// Measured, events around 20 launches, before (VALU adds, inconv.hip) -> here: ResNet-18 7x7/4 batch 256 123 -> 117 us,
-// batch 8 54 -> 16; 7x7/2 batch 256 458 -> 317, batch 20 154 -> 43; VGG-16 3x3 batch 256 402 -> 222, batch 5 130 -> 14;
-// AlexNet 11x11/4 batch 200 425 -> 129, batch 3 139 -> 17.
+// What binds it: nothing by itself.  At ResNet-18's layer (batch 256, 12-bit residual; 950 VALU instructions and 56 MFMAs per
+// 32 columns x 64 channels) the VALU is busy 38 % of the time and the matrix cores 18 %; a wave waits 31 % of its time for
+// counters (memory, LDS) and 28 % for its turn to issue: 1792 waves, under two per SIMD, do not hide one another's waits.
+// In a network's pass, where the images come from HBM and not from the memory-side cache, the first of these grows.  (HBM
+// would allow 40 us.)
+// Measured, us, VALU adds (inconv.hip) -> here.  A launch within the network's pass, kernel trace, batch 256: ResNet-18 7x7/4
+// 127 -> 121 (launch after launch on one batch 121 -> 98), 7x7/2 423 -> 315, VGG-16 3x3 399 -> 207, AlexNet 11x11/4 310 -> 137,
+// CIFAR ResNet 3x3 27 -> 27, CIFAR VGG (no residual) 23 -> 18.  Events around 20 launches: ResNet-18 batch 8 52 -> 14; 7x7/2
+// batch 20 151 -> 38; VGG-16 batch 5 129 -> 14; CIFAR ResNet batch 77 26 -> 18; AlexNet batch 200 403 -> 134, batch 3 137 -> 16.
 #include <algorithm>
 #include <atomic>
 #include <cmath>

@@ -1,6 +1,6 @@
 // Layers of the textbook ResNet wiring that the reference's drivers do not have: overlapping
 // OR / max pooling of a packed activation tensor with its residual, and the global-average-pool +
-// fp32 fully connected head.  Both are bound by HBM (one pass over their input).
+// fp32 fully connected head.  The pooling is one pass over its input; the head is latency (below).
 #include <algorithm>
 
 #include "common.h"
@@ -113,8 +113,9 @@ __device__ __forceinline__ void i12_from_pairs(const uint32_t* q, uint32_t& w0, 
 
 // A thread takes one unit (word of bits, or residual group) of one image and walks down `rows` output pixels of a
 // column: of the three input rows of a window the last is the next window's first, so an output costs six loads and not
-// nine, all of them in flight together.  Bound by HBM: 417 MB at 112x112, 64 channels, 12 bits, batch 256, in 86 us
-// (104 us with nine loads and a 64-bit division per output).
+// nine, all of them in flight together.  417 MB at 112x112, 64 channels, 12 bits, batch 256, in 86 us (104 us with nine
+// loads and a 64-bit division per output): three quarters of the copy rate; a wave waits for memory (44 % of its time) and
+// for the other waves' unpacking, maxima and packing (47 %).
 template <int FMT>
 __global__ __launch_bounds__(kThreads) void pool3x3s2_kernel(const PoolParams p, int rows) {
     const int rem = (int)(blockIdx.x * kThreads + threadIdx.x);
