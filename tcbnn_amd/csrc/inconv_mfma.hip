@@ -62,8 +62,9 @@
 // What binds it: nothing by itself.  At ResNet-18's layer (batch 256, 12-bit residual; 950 VALU instructions and 56 MFMAs per
 // 32 columns x 64 channels) the VALU is busy 38 % of the time and the matrix cores 18 %; a wave waits 31 % of its time for
 // counters (memory, LDS) and 28 % for its turn to issue: 1792 waves, under two per SIMD, do not hide one another's waits.
-// In a network's pass, where the images come from HBM and not from the memory-side cache, the first of these grows.  (HBM
-// would allow 40 us.)
+// In a network's pass, where the images come from HBM and not from the memory-side cache, the first of these grows.  HBM
+// would allow 40 us; the launch fetches 336 MB, 2.2 times the images: a strip's rows are 80 bytes, and lines that neighbouring
+// strips share come more than once.
 // Measured, us, VALU adds (inconv.hip) -> here.  A launch within the network's pass, kernel trace, batch 256: ResNet-18 7x7/4
 // 127 -> 121 (launch after launch on one batch 121 -> 98), 7x7/2 423 -> 315, VGG-16 3x3 399 -> 207, AlexNet 11x11/4 310 -> 137,
 // CIFAR ResNet 3x3 27 -> 27, CIFAR VGG (no residual) 23 -> 18.  Events around 20 launches: ResNet-18 batch 8 52 -> 14; 7x7/2
