@@ -19,7 +19,7 @@
 // What bounds it, with counters: the small launches latency, one or two memory round trips and the launch itself (3x3 layers
 // at batch 8, 5.6-6.3 us: waves wait for memory 52-64 % of their time, VALU busy 20-33 %, matrix cores 4 %).  The larger ones
 // instruction issue: expanding the operands takes 7 VALU instructions per fragment, plus 5 per column tile and step for
-// address and border, against 32 cycles per MFMA (AlexNet's 5x5 layer at batch 200, 50 us: VALU 63 %, matrix cores 27 %, of
+// address and border, against 32 cycles per MFMA (AlexNet's 5x5 layer at batch 256, 50 us: VALU 63 %, matrix cores 27 %, of
 // the same issue slots).  1x1 layers with a residual at batch 256 (19.5 us) their traffic: 40 % waiting, 54 % VALU, 3 %
 // matrix cores.
 #include <algorithm>
