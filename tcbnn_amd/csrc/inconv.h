@@ -1,4 +1,4 @@
-// What the first layer's kernels share: the problem and the matrix-core kernel's entry points.
+// What the first layer's kernels share: the problem and the matrix-core kernels' entry points.
 #pragma once
 
 #include "common.h"
@@ -21,5 +21,9 @@ struct InConvParams {
 // (`served`: whether it does; if not, nothing has been launched).
 bool inconv_mfma_kernel_name(const InConvParams& p, char* buf, size_t len);
 int launch_inconv_mfma(const InConvParams& p, hipStream_t stream, bool* served);
+// The kernel that it leaves few rows of 11x11 filters to (inconv_mfma_ring.hip); `dev` below kInConvDevices
+constexpr int kInConvDevices = 64;
+bool inconv_mfma_ring_serves(const InConvParams& p);
+int launch_inconv_mfma_ring(const InConvParams& p, int dev, int cus, hipStream_t stream, bool* served);
 
 }  // namespace tcbnn

@@ -7,7 +7,7 @@
 // are no multiplies (the sign is applied by flipping the fp32 sign bit with a
 // precomputed mask), hence no FMA contraction either.
 //
-// The layers of the networks go to the matrix cores (inconv_mfma.hip, same bits and residuals); the kernels here serve what
+// The layers of the networks go to the matrix cores (inconv_mfma.hip, inconv_mfma_ring.hip, same bits and residuals); the kernels here serve what
 // that file has no instantiation for (other filter heights and poolings, channels that are no multiple of 64 or, at 11x11,
 // of 32, strides outside its forms, tensors of 2 GiB) and packed input:
 //   inconv_tiled_kernel (pool 1x1, or a pool_w of at most 2 without a residual): workgroup = one output row y, 4 consecutive output
@@ -810,7 +810,8 @@ static int inconv128_run(const tcbnn_inconv128_desc* d, void* stream, char* name
         return TCBNN_OK;
     }
     TCBNN_REQUIRE(d->input_layout == TCBNN_INCONV_INPUT_NCHW, "inconv128: unknown input_layout");
-    // 3-, 7- and 11-row filters on 32- or 64-channel tiles: matrix cores (inconv_mfma.hip says what it serves and why)
+    // 3-, 7- and 11-row filters on 32- or 64-channel tiles: matrix cores (inconv_mfma.hip and
+    // inconv_mfma_ring.hip say what they serve and why)
     if (!force_linear && name_buf != nullptr && inconv_mfma_kernel_name(p, name_buf, name_len)) return TCBNN_OK;
     if (!force_linear && name_buf == nullptr) {
         bool served = false;

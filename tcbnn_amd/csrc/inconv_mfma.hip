@@ -13,62 +13,55 @@
 // The results are therefore the reference's, bit for bit, for every input; only the time depends on the data, and by a
 // small factor (below).
 //
-// The bound.  u = 2^-24, A = sum of |x| under the window, T = R*S taps.  A rounding of a running sum is at most u times
-// that sum, which is at most what has been added so far and at most |S| plus what is still to come: (A + |S|) / 2.  The
-// ordered sum has T such roundings and 2 u A more inside its taps; the split drops at most 2 u |x| per input (and 2^-25
-// where fp16 runs out of exponents).  An MFMA adds its 16 products in two halves of eight (six, without the fourth channel).
-// A half rounds its result once, and what lies below u times its largest product M is lost, of each product and of the sum
-// that they are added to (tests/test_gpu_matrix_core.py holds the instruction to this).  An fp16 number has 11 bits, so
-// only products below 2^-13 M lose anything: m of them and the sum, (m + 1) u M at most, where the sum is below M.
-// The lo steps run first, on sums below 2^-10 A.  For A stands sqrt(3 T sum of hi^2), whose squares are one v_dot2 per
-// loaded dword and which such small values hardly enter: by Cauchy and Schwarz the losses of all halves add the most to
-// the rest of the bound where m = 0, and then 2 R NQ / (3 T) < 0.25 u A; 2.25 roundings are taken per step, not 2.  From
-// 7 rows on E is taken for |S| <= A/2 (partial sums below 3/4 A); a lane with a larger sum looks again with the full
-// bound.  -E itself enters the sum as one more product (the fourth channel of the last tap, unused otherwise), so the
-// accumulators hold S - E: a bit is certainly 1 where S - E >= bn, certainly 0 below bn - 2E.
-// Inputs outside the fp16 range, infinities and NaN make E infinite: all values of such a window are recomputed.
+// The bound.  u = 2^-24, A = sum of |x| under the window, A_k = what of it has been multiplied up to step k.  A rounding of a
+// running sum is at most u times that sum, and the sum is at most A_k: there is one rounding per tap in the reference's order,
+// and there are four per step here (an MFMA adds its 16 products in two halves of eight and rounds each once; lo, then hi;
+// tests/test_gpu_matrix_core.py holds the instruction to this).  Added to these: 2 u A inside the reference's taps; 2 u A that
+// the split drops (and 2^-25 per input where fp16 runs out of exponents); and what lies below u times a half's largest product
+// M, which is lost of each product and of the sum they are added to: an fp16 number has 11 bits, so only products below
+// 2^-13 M lose anything, with the sum at most 8 u M, and the M of all halves are at most A (those of lo 2^-11 of that).
+// E = u (sum of n_k A_k + 13.5 A), n_k roundings of sums up to step k; 2 % cover the bound's own roundings.  For 7-row filters
+// with a residual the A_k are summed up as the window passes (1.9 doubtful values per 32 pixels x 64 channels instead of 2.8
+// with A for each); the others, which have few doubtful values, take A for every A_k.
+// Where a residual is saved, -E itself enters the sum as one more product (a place that no tap uses), so the accumulators
+// hold S - E: a bit is certainly 1 where S - E >= bn, certainly 0 below bn - 2E.  Where none is saved, sums start from -bn: the
+// bit is the sign, in doubt where |S - bn| <= E (partial sums are then at most what is still to come and |S - bn|: A again).
+// Inputs outside the fp16 range, infinities and NaN make NaN of the sums or an infinity of E: all values of such a window are
+// recomputed, as are those of windows whose neighbouring rows (multiplied by zeros) hold them.
 //
 // Many values in doubt.  A saved residual puts every sum ON an integer in doubt, and images have areas of such sums: bars of
 // +-1 after scaling to [-1, 1], saturated white, bytes, a flat grey of 0.2 (every fifth channel); and E grows with the
-// magnitudes: bytes less a mean leave 7 % of the sums in doubt, values in the thousands all of them.  One by one (four at a
-// time, a trip to memory and 49 dependent additions) a tile full of them takes 512 rounds, a hundred multiplications' time.
-//   grid    : while every row a wave has staged is multiples of 1/256 (bytes, bytes / 128 - 1, +-1), sums of windows with
-//             a sum of |x| below 2^16 are exact: every partial sum is a multiple of 1/256 below 2^24 / 256, in both orders.
-//             E is 0.  Rows are checked as long as that holds; other inputs pay for the first window.
-//   COMMON  : a wave's first pass; it ends at an item with many values in doubt (kManyInLane, kManyLanesCommon; where no
-//             residual is saved: at a full list).  The test and the exit cost it 1.5 %; what the later passes do cost 3-9 %
-//             inside its loop, by its registers.
-//   MARKED  : the window is staged again, and rows from then on, with a mark at every column that is off that grid (the
-//             fourth channel of the lo plane).  An item looks at its windows' marks first; E is 0 where there is none.
-//   ORDERED : where that still leaves many, sums in the reference's order, 32 columns x 64 channels at a time, as fp32
+// magnitudes: bytes less a mean leave 7 % of the sums in doubt, values in the thousands all of them.
+//   grid    : sums of a window whose inputs are multiples of 1/256 (bytes, bytes / 128 - 1, +-1) with a sum of |x| below 2^15
+//             are exact in both orders: every partial sum is a multiple of 1/256 below 2^24 / 256, and the two halves hold
+//             the inputs.  E is 0.  (Sums that start from -bn: if all thresholds are such multiples too.)
+//   check   : a wave looks whether its inputs are on that grid (120 VALU instructions per item of 7-row filters) as long as all
+//             have been; other inputs pay for their first item.  From an item with many values in doubt on it always looks.
+//   ordered : from an item that has many even so, sums in the reference's order, 32 columns x 64 channels at a time, as fp32
 //             products on the matrix cores (ordered_sums): no values in doubt but those that are no numbers.
-// A single wave that leaves the common pass takes 80 us longer (code that no other wave has fetched), and the launch with
-// it: the lines lie where none of 25000 items of bytes / 255 (0.6 % in doubt) reaches them.
-// ResNet-18's first layer at batch 256, us, in brackets with the list alone: normal data 107 (111), bytes / 128 - 1 92 (245),
-// images in [-1, 1] with bars and patches of +-1 over a third 117 (7690), bytes / 255 147 (163), a third of 0.2 grey 271
-// (1490), bytes less a mean 326 (1404), normal x 1000 336 (14150); the additions on the VALU (inconv.hip) take 138 for any.
+// ResNet-18's first layer at batch 256, launched on end, us: normal data 84, bytes / 128 - 1 81, images in [-1, 1] with bars and
+// patches of +-1 over a third 94, bytes / 255 122, a third of 0.2 grey 241, bytes less a mean 320, normal x 1000 325.
 //
-// Work split.  A team owns NI images x a strip of xo output columns x a band of output rows, and walks down the rows:
-// the input rows of the window stay in LDS (a ring; stride_h new rows per output row, every input row is read and split
-// once per strip), as fp16 [row][image][column][4] for hi and the same for lo, image pitch an odd number of 16-byte units
-// (conflict-free).  A multiplication is 32 columns = NI images x 32/NI neighbouring pixels (so small batches fill their
-// tiles) by 32 MT channels whose +-1 fragments stay in registers; the next rows are requested before it and written
-// after it.  A team is ONE wave where its ring fits an eighth (2-wave registers) or twelfth to sixteenth of a CU's LDS:
-// waves then never wait for each other (with four waves to a ring and two barriers a row, every row waited for the
-// slowest wave's recomputation: ResNet-18's first layer at batch 256 took 170-180 us instead of 105 without doubtful
-// values).  11-row filters, whose rings are larger, share one among the four waves of a workgroup.  The four waves of a
-// workgroup are neighbouring strips; work of one image tile goes to one XCD.
+// Work split.  A tile is 32 columns = NI images x 32/NI neighbouring pixels of a row (so small batches fill their tiles) by 64
+// channels.  A wave walks down the rows of one column of tiles, a step per output row: the A (stride) input rows that are new
+// are loaded straight into registers, split there, and multiplied at once for every output row that they are part of.
+// sets_of(R, A) sums are under way; the first product of a step reads the next younger set's registers and writes its own, so
+// they move on without copies.  Compared with a ring of split rows in LDS (of which a CU holds eight waves' worth, at 240
+// registers a wave): no LDS traffic but the weights, which four waves share, no barrier, three waves per SIMD for 3x3 and 7x7/4
+// (two for the rest), and 8 places for a row's 7 taps in one channel, not 32 for its 21.  The next step's rows are requested as the
+// present ones are used up.  A workgroup's waves are neighbouring columns of tiles; an XCD has whole image tiles.
+// Eight images per tile: their residuals of a pixel are a whole 128-byte line.  Sixteen (64 bytes of output words) where no
+// residual is saved and a wave has 32 items or more: VGG-16 217 -> 206 us; below that fewer units fill the machine worse
+// (CIFAR VGG 16.7 -> 18.0 us).
 //
-// What binds it: nothing by itself.  At ResNet-18's layer (batch 256, 12-bit residual; 950 VALU instructions and 56 MFMAs per
-// 32 columns x 64 channels) the VALU is busy 38 % of the time and the matrix cores 18 %; a wave waits 31 % of its time for
-// counters (memory, LDS) and 28 % for its turn to issue: 1792 waves, under two per SIMD, do not hide one another's waits.
-// In a network's pass, where the images come from HBM and not from the memory-side cache, the first of these grows.  HBM
-// would allow 40 us; the launch fetches 336 MB, 2.2 times the images: a strip's rows are 80 bytes, and lines that neighbouring
-// strips share come more than once.
-// Measured, us, VALU adds (inconv.hip) -> here.  A launch within the network's pass, kernel trace, batch 256: ResNet-18 7x7/4
-// 127 -> 121 (launch after launch on one batch 121 -> 98), 7x7/2 423 -> 315, VGG-16 3x3 399 -> 207, AlexNet 11x11/4 310 -> 137,
-// CIFAR ResNet 3x3 27 -> 27, CIFAR VGG (no residual) 23 -> 18.  Events around 20 launches: ResNet-18 batch 8 52 -> 14; 7x7/2
-// batch 20 151 -> 38; VGG-16 batch 5 129 -> 14; CIFAR ResNet batch 77 26 -> 18; AlexNet batch 200 403 -> 134, batch 3 137 -> 16.
+// What binds it: memory traffic and the waits for it.  ResNet-18's layer at batch 256 fetches 294 MB for 154 MB of images (a doubtful
+// value's window comes back from HBM, 21 rows of 128 bytes: 116 MB; without that 178) and writes 90 MB, 3.6 TB/s; the VALU is
+// busy 30 % of the time, the matrix cores 15 %.  Recomputing a value at once finds its rows in L2 no more often (an XCD's waves bring
+// in 4 MB per step) and costs a trip to memory per item (130 us for 118).
+// Measured, us within the network's pass (kernel trace, batch 256 unless said; adds on the VALU -> ring in LDS -> here, both
+// matrix-core versions in turn on one box): ResNet-18 7x7/4 127 -> 124 -> 108, 7x7/2 423 -> 334 -> 305, VGG-16 3x3 399 -> 209 -> 205,
+// AlexNet 11x11/4 batch 200 403 -> 133 -> 97, CIFAR VGG 23 -> 20.4 -> 17.6, CIFAR ResNet batch 77 26 -> 18.8 -> 16.3, ResNet-18
+// batch 8 52 -> 18.0 -> 15.7.
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -80,21 +73,56 @@
 namespace tcbnn {
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int rounds_of(int r) { return r == 3 ? 3 : 5; }  // staging units (column pairs) per thread and step, at most
-// Whether E is taken for sums up to A/2: sums of 27 terms pass that in every fortieth value.
-constexpr bool bound_for_half(int r) { return r > 3; }
-constexpr bool ring_shared(int r) { return r > 7; }          // four waves to a ring, else one
 constexpr int kListCap = 64;   // doubtful values a wave keeps
-// A wave's passes (top of this file), and what counts as many values in doubt: one lane with this many (of its column's 32;
-// a flat area), or this many lanes (of 64) with any.
-enum Mode : int { COMMON, MARKED, ORDERED };
-constexpr int kManyInLane = 8, kManyLanesCommon = 28, kManyLanesMarked = 32;
+constexpr int kBatch = 16;     // ... and recomputes at a time
+// What counts as many values in doubt: one lane with this many (of its column's 32; a flat area), or this many lanes (of 64)
+// with any; the second for windows already checked for the grid.
+constexpr int kManyInLane = 8, kManyLanes = 28, kManyLanesChecked = 32;
+
+// A wave walks down the input, A rows (the stride) at a time, and an input row is multiplied for every output row that it is
+// part of while it is in registers: sets_of(R, A) sums are under way, the oldest of which is finished by the step.
+constexpr int sets_of(int r, int a) { return (r + a - 1) / a; }
+// The K order of a step.  A "pair" is one of its rows in one channel: 3 A of them, the even ones for lane half 0, the odd ones
+// for half 1.  A lane loads a pair's T taps at once and gives each pair slots_of(T) places of its stream; every eight places
+// are one fragment.  T = 7: a fragment is a pair; T = 3: places 0-2, 3-5; T = 11: 12 places.
+constexpr int pairs_of(int a) { return (3 * a + 1) / 2; }
+constexpr int slots_of(int t) { return t == 7 ? 8 : (t == 11 ? 12 : t); }
+constexpr int steps_of(int a, int t) { return (pairs_of(a) * slots_of(t) + 7) / 8; }
+// Place (of the step's last fragment, lane half 1) through which -E enters: none of the taps'.
+constexpr int kBoundPlace = 7;
+constexpr bool bound_place_free(int a, int t) {
+    const int slot = 8 * (steps_of(a, t) - 1) + kBoundPlace, pair = 2 * (slot / slots_of(t)) + 1;
+    return pair >= 3 * a || slot % slots_of(t) >= t;
+}
+// What E counts (top of this file).
+template <int R, int T, int A>
+struct Order {
+    static constexpr int P = slots_of(T), D = sets_of(R, A), KS = steps_of(A, T);
+    // Whether a pair's row is part of the oldest set's windows, or has zero weights there (3-row filters: all count)
+    static constexpr bool in_old(int pair) { return pair < 3 * A && (P % 2 != 0 || pair / 3 < R - (D - 1) * A); }
+    // Roundings of sums that hold what has been multiplied up to step k (a pair each of both lane halves): two halves of lo
+    // and of hi, and a row's T taps with its last pair.
+    static constexpr int roundings(int k, bool old) {
+        int n = !old || in_old(2 * k) ? 4 : 0;
+        for (int at = 2; at < 3 * A; at += 3)
+            if ((!old || in_old(at)) && at / 2 == k) n += T;
+        return n;
+    }
+    static constexpr int roundings(bool old) {
+        int n = 0;
+        for (int k = 0; k < KS; ++k) n += roundings(k, old);
+        return n;
+    }
+};
+// Registers: sums of sets_of() rows x 64 channels, taps of the next rows
+constexpr int waves_per_simd(int r, int a) { return sets_of(r, a) <= 2 ? 3 : (r == 3 ? 3 : 2); }
+constexpr int waves_of(int r) { return r > 7 ? 8 : 4; }  // of a workgroup: they share the LDS copy of the weight fragments
+constexpr int MT = 2;  // channel tiles of 32 that a wave multiplies
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h8u __attribute__((ext_vector_type(8), aligned(8)));
 typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v3f __attribute__((ext_vector_type(3)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -104,34 +132,18 @@ typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 // Saved residual: none, 12 bits, or 16 / 32 bits (looked up at run time).
 enum Residual : int { RES_NONE = 0, RES_12 = 1, RES_WIDE = 2 };
 
-// How a staged image row lies in LDS: column pairs of 16 bytes.  A multiplication's 64 lanes read 16 bytes each, half h of
-// them pair 2j + h of their pixel's window.  Strides that are multiples of four: even pairs, then odd ones, so that
-// neighbouring pixels are neighbouring units (with an image pitch of 2 modulo 4 units the lanes fall into different banks).
-// Other even strides: pairs in order, odd pitch.  Odd strides: the same, windows begin inside a pair (8-byte reads).
-enum Pairs : int { PAIRS_ANY = 0, PAIRS_EVEN = 1, PAIRS_SPLIT = 2 };
-
-// Workgroups a CU is to hold (one wave of each per SIMD): what the registers allow.
-constexpr int workgroups_per_cu(int r) { return r == 3 ? 4 : 2; }
-
 struct Geometry {
     int ni_log2;             // images per tile
-    int xo;                  // convolution columns per strip
-    int np, pp;              // staged column pairs per image row, and their odd pitch
-    int odd_pairs;           // PAIRS_SPLIT: where the odd pairs begin
-    int rounds;              // units per lane and step
-    int ring;                // input rows in LDS
-    int adv;                 // input rows a step moves on by
-    int strips, bands, band_rows, imgtiles, cgroups, waves_c;  // waves_c: waves of a workgroup side by side over channels
-    int total, per_xcd;
-    int rows;                // output rows (pooled)
+    int groups;              // tiles across a row
+    int bands, band_rows;    // bands of convolution rows
+    int rows;                // convolution rows
+    int cgroups;             // channel groups (of 64)
+    int total, per_xcd;      // waves' work units (image tile, band, column group), and those of an XCD
     int rs_taps;
     unsigned s_magic;        // tap / S == tap * s_magic >> 16 for every tap
-    float bound_scale;       // E = bound_scale * sqrt(sum of hi^2) + bound_add for |S| <= half_scale * sqrt(sum of hi^2)
-    float bound_scale_full;  // ... and for any S
-    float half_scale;
+    float bound_parts;       // E = bound_parts * (the sum of |x| before each rounding) + bound_sum * (the sum of |x|) + bound_add
+    float bound_sum;
     float bound_add;
-    float small_squares;     // sum of hi^2 below which the sum of |x| is below 1/2
-    float exact_squares;     // ... below which sums of multiples of 1/256 are exact
 };
 
 // The kernel's argument.  Code that seldom runs reads it anew from the argument segment (seldom_args): fields that
@@ -186,386 +198,356 @@ __device__ __forceinline__ void store_residual_group(__amdgpu_buffer_rsrc_t rsrc
     }
 }
 
-#define TCBNN_ROW_BCAST(v, t) \
-    __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 | (t), 0xf, 0xf, false))
-
-// acc += m of lane T, T + 1, ... N - 1 of each row of 16 lanes, in this order; all N of them, or while taps are left
-template <int T, int N, bool ALL>
-__device__ __forceinline__ float add_row_taps(float acc, float m, int left) {
-    if constexpr (T < N) {
-        if (ALL || T < left) {  // uniform
-            acc = acc + TCBNN_ROW_BCAST(m, T);
-            return add_row_taps<T + 1, N, ALL>(acc, m, left);
-        }
-    }
-    return acc;
+// The sum of v over the lane halves
+__device__ __forceinline__ float both_halves(float v) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+// acc + lane T of m's quad
+template <int T>
+__device__ __forceinline__ float add_quad_lane(float acc, float m) {
+    return acc + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x55 * T, 0xf, 0xf, false));
 }
 
-template <int R, int NQ, int MT, int RES, int POOL, int PAIRS>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgroups_per_cu(R)))) void inconv_mfma_kernel(
+// Taps t = 0 .. N - 1 from byte offset `at` (+ a uniform one): the address unit takes 16 cycles for 64 lanes' 4 to 16 bytes
+// each, whatever their alignment to 4, and 30 for single words that are not neighbours.
+template <int N>
+__device__ __forceinline__ void load_taps(__amdgpu_buffer_rsrc_t rsrc, unsigned at, unsigned base, float* f) {
+    if constexpr (N >= 4) {
+        const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)at, (int)base, 0));
+        f[0] = v[0], f[1] = v[1], f[2] = v[2], f[3] = v[3];
+        if constexpr (N > 4) load_taps<N - 4>(rsrc, at + 16u, base, f + 4);
+    } else {
+        static_assert(N == 3, "");
+        const v3f v = __builtin_bit_cast(v3f, __builtin_amdgcn_raw_buffer_load_b96(rsrc, (int)at, (int)base, 0));
+        f[0] = v[0], f[1] = v[1], f[2] = v[2];
+    }
+}
+
+template <int R, int T, int A, int RES, int POOL>
+__global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(R, A)))) void inconv_mfma_kernel(
     const KernelArgs args) {
     const SeldomArgs args_at = (SeldomArgs)__builtin_amdgcn_kernarg_segment_ptr();
     const InConvParams& p = args.p;
     const Geometry& q = args.q;
-    static_assert(MT * POOL <= 2 && !(RES != RES_NONE && POOL > 1), "doubtful values of an item are 32 bits of a register");
-    static_assert(!(ring_shared(R) && RES != RES_NONE), "a wave of a shared ring cannot leave its pass at an item");
-    constexpr int NK = R * NQ;  // MFMA steps: four taps (of one filter row) x four channels each
-    constexpr int kRounds = rounds_of(R);
+    static_assert(!(RES != RES_NONE && POOL > 1), "residuals of un-pooled layers only");
+    static_assert(bound_place_free(A, T), "-E needs a place of its own");
+    constexpr int kWaves = waves_of(R), kPairs = pairs_of(A), P = slots_of(T), KS = steps_of(A, T), D = sets_of(R, A);
+    constexpr int kRing = (R == 3 || A == 2 ? kPairs : 3);  // pairs in registers
+    static_assert(kPairs % kRing == 0, "a pair's place does not depend on the step");
     constexpr unsigned kOutOfRange = 0x80000000u;
+    constexpr int kChannels = 32 * MT;
+    // Where no residual is saved the sums start from the threshold's negative: the bit is the sum's sign.
+    constexpr bool kFromThreshold = RES == RES_NONE;
+    using order = Order<R, T, A>;
+    constexpr bool kParts = T == 7 && !kFromThreshold;  // E by the sums before each rounding
     extern __shared__ __align__(16) char lds[];
 
-    constexpr bool kShared = ring_shared(R);
-    constexpr bool kHalf = bound_for_half(R);
-    constexpr int kTeam = kShared ? 4 : 1;  // waves to a ring
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int member = kShared ? wave : 0;
-    const int slot_x = (int)blockIdx.x >> 3;
-    int work = ((int)blockIdx.x & 7) * q.per_xcd + (kShared ? slot_x : slot_x * 4 + wave);
-    const bool idle = (kShared ? slot_x : slot_x * 4 + wave) >= q.per_xcd || work >= q.total;
-    if (kShared && idle) return;  // whole workgroup
-    if (idle) work = 0;           // (such a wave helps with the thresholds and leaves)
-    const int strip = work % q.strips;
-    work /= q.strips;
-    const int band = work % q.bands;
-    work /= q.bands;
-    const int cg = work % q.cgroups, it = work / q.cgroups;
-    const int NI = 1 << q.ni_log2, NX = 32 >> q.ni_log2;
-    const int b0 = it << q.ni_log2;
-    const int x0 = strip * q.xo;
-    const int oy_begin = band * q.band_rows, oy_end = min(q.rows, oy_begin + q.band_rows);
-    const int wc = kShared ? wave % q.waves_c : 0, wg0 = kShared ? wave / q.waves_c : 0, wg_step = kShared ? 4 / q.waves_c : 1;
-    const int tile0 = (cg * q.waves_c + wc) * MT;  // first channel tile of this wave
+    // LDS: weight fragments, thresholds of the channel group, lists, signs
+    v4i* const frags = reinterpret_cast<v4i*>(lds);
+    float* const thr = reinterpret_cast<float*>(lds + D * KS * MT * 1024);
+    uint32_t* const list = reinterpret_cast<uint32_t*>(lds + D * KS * MT * 1024 + MT * 128) + wave * 2 * kListCap;
+    uint8_t* const signs = reinterpret_cast<uint8_t*>(lds + D * KS * MT * 1024 + MT * 128 + kWaves * 8 * kListCap);
+
+    const int slot = (int)blockIdx.x >> 3, cg = slot % q.cgroups, in_xcd = slot / q.cgroups * kWaves + wave;
+    int work = ((int)blockIdx.x & 7) * q.per_xcd + in_xcd;
+    const bool idle = in_xcd >= q.per_xcd || work >= q.total;
+    const int tile0 = cg * MT;  // first channel tile
+
+    if (idle) work = 0;  // (such a wave helps with the weights and leaves)
+
+    const int g = work % q.groups;
+    work /= q.groups;
+    const int band = work % q.bands, it = work / q.bands;
+    int cy = band * q.band_rows;  // convolution row
+    const int cy_end = min(cy + q.band_rows, q.rows);
+    const int NI = 1 << q.ni_log2, NX = 32 >> q.ni_log2, b0 = it << q.ni_log2;
     const int xcols = POOL > 1 ? POOL * p.OW : p.PW;
-    const int n_groups = (min(q.xo, xcols - x0) + NX - 1) >> (5 - q.ni_log2);
+    const unsigned plane_b = (unsigned)(p.H * p.W) * 4u, row_b = (unsigned)p.W * 4u;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.in + (size_t)b0 * 3 * p.H * p.W), 0,
+                                                                          (int)((unsigned)min(NI, p.B - b0) * 3u * plane_b), 0x00020000);
+    const __amdgpu_buffer_rsrc_t out_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)args.out_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t res_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.res, 0, (int)args.res_bytes, 0x00020000);
+    auto threshold = [&](int i) __attribute__((always_inline)) { return kFromThreshold ? -thr[i] : thr[i]; };
+    const unsigned uB = (unsigned)p.B, group_b = (RES == RES_12 ? 24u : (p.res_fmt == TCBNN_RES_I16 ? 32u : 64u)) * uB;
+    const unsigned pixel_b = (unsigned)(p.O / 16) * group_b;
+    // Where lane ln stores, relative to the item (uniform): its output word, its 16 residuals (12-bit: the 8-byte part
+    // apart); beyond the tensors for an image past the batch.
+    auto place_word = [&](int ln) __attribute__((always_inline)) {
+        const unsigned px = (unsigned)((ln & 31) >> q.ni_log2), h = (unsigned)ln >> 5, b = (unsigned)(b0 + (ln & (NI - 1)));
+        return b < uB && (POOL == 1 || (px & 1u) == 0u) ? ((px / POOL * (unsigned)p.ow + h) * uB + b) * 4u : kOutOfRange;
+    };
+    const unsigned word_place = kFromThreshold ? place_word(lane) : 0u;  // (where registers allow)
+    auto place_residual = [&](int ln) __attribute__((always_inline)) {
+        const unsigned px = (unsigned)((ln & 31) >> q.ni_log2), h = (unsigned)ln >> 5, b = (unsigned)(b0 + (ln & (NI - 1)));
+        return px * pixel_b + h * group_b + b * 16u;
+    };
+    auto place_residual8 = [&](int ln) __attribute__((always_inline)) { return place_residual(ln) + uB * 16u - (unsigned)(b0 + (ln & (NI - 1))) * 8u; };
 
-    // LDS: thresholds of all channels, lists, a flag, then the rings: hi rows, lo rows
-    const int row_bytes = (q.pp * 16) << q.ni_log2;
-    const int plane = q.ring * row_bytes;
-    float* const thr = reinterpret_cast<float*>(lds);
-    uint32_t* const list = reinterpret_cast<uint32_t*>(lds) + p.O + wave * 2 * kListCap;
-    int* const flags = reinterpret_cast<int*>(lds) + p.O + 4 * 2 * kListCap;  // kShared: rows off the grid; many doubts
-    char* const rows = lds + (p.O + 4 * 2 * kListCap + 4) * 4 + (kShared ? 0 : wave * 2 * plane);
-
-    // ---- thresholds (NaN: -infinity, the bit is 1 either way)
-    for (int i = tid; i < p.O; i += kThreads) {
-        const float t = p.bn[i];
-        thr[i] = t != t ? -INFINITY : t;
+    // ---- loading: pair 2 i + h of a step's rows into ring place i % kRing
+    // Where this lane reads: its pixel's window relative to the step's first one, and which of two pairs is this half's.
+    unsigned from_a, from_b;  // channels c, c + 1 of a row; channel 2 of a row and channel 0 of the next
+    unsigned outside = 0u;    // taps that are not inside the frame's columns (columns of the tile that are none: all)
+    const int ax_first = g * NX * p.stride_w - p.pad_w;
+    const bool columns_inside = p.S == T && ax_first >= 0 && ax_first + (NX - 1) * p.stride_w + T <= p.W && (g + 1) * NX <= xcols;
+    {
+        const int px = (lane & 31) >> q.ni_log2, h = lane >> 5, img = lane & (NI - 1), ax = ax_first + px * p.stride_w;
+        const int from = min(max(-ax, 0), 31), to = min(max(min(p.W - ax, p.S), 0), 31);
+        const bool none = (b0 + img >= p.B) | (g * NX + px >= xcols);
+        outside = none ? ~0u : ((1u << from) - 1u) | (~0u << to);
+        const unsigned first = b0 + img < p.B ? (unsigned)img * 3u * plane_b + (unsigned)(px * p.stride_w) * 4u : kOutOfRange;
+        from_a = first + (h ? plane_b : 0u);
+        from_b = first + (h ? row_b : 2u * plane_b);
     }
-    if (tid < 2) flags[tid] = 0;
+    float x[kRing][T];
+    // How a step's rows (`ay`: the first) are loaded: all inside the frame; rows outside it; columns outside it, which are masked
+    // when the taps are used (not in the first and last rows: what is in front of the first one's taps, or behind the last
+    // one's, need not be the tensor's); tap by tap.
+    enum Path : int { INSIDE, ROWS, COLUMNS, TAPS };
+    const bool columns_masked = p.S == T && p.W >= T;
+    auto path_of = [&](int ay) __attribute__((always_inline)) -> int {
+        if (columns_inside) return ay >= 0 && ay + A <= p.H ? INSIDE : ROWS;
+        return columns_masked && ay > 0 && ay + A < p.H ? COLUMNS : TAPS;
+    };
+    auto load = [&](int ay, int path, int i) __attribute__((always_inline)) {
+        float* const f = x[i % kRing];
+        const int r0 = 2 * i / 3, c0 = 2 * i % 3, r1 = (2 * i + 1) / 3;
+        const bool last = 2 * i + 1 >= 3 * A;  // half 1 has none
+        unsigned step_b = row_b;
+        asm volatile("" : "+v"(from_a), "+v"(from_b), "+s"(step_b));  // (sums with them are made when used, not kept)
+        const unsigned at = (unsigned)(ay * p.W + ax_first) * 4u + (unsigned)r0 * step_b + (c0 == 1 ? plane_b : 0u);
+        const unsigned from = c0 == 2 ? from_b : from_a;
+        if (path == INSIDE || path == COLUMNS) {  // uniform
+            load_taps<T>(rsrc, last && lane >= 32 ? kOutOfRange : from, at, f);
+        } else {
+            // rows outside the frame (and taps, and columns that are none): offsets beyond the tensor, zeros.  An offset can be
+            // negative where a window begins in front of its image; those of taps inside are not.
+            const unsigned row0 = (unsigned)(ay + r0) < (unsigned)p.H ? 0u : ~0u, row1 = !last && (unsigned)(ay + r1) < (unsigned)p.H ? 0u : ~0u;
+            const unsigned out = lane >= 32 ? row1 : row0;
+            if (path == ROWS) {
+                load_taps<T>(rsrc, out != 0u ? kOutOfRange : from + at, 0u, f);
+            } else {
+#pragma unroll
+                for (int t = 0; t < T; ++t)
+                    f[t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                         rsrc, (int)(((out | outside) << (31 - t) & kOutOfRange) | (from + at + 4u * t)), 0, 0));
+            }
+        }
+    };
+
+    // ---- The first rows are on their way while the weights are laid out.
+#pragma unroll
+    for (int i = 0; i < kRing; ++i) load(cy * A - p.pad_h, path_of(cy * A - p.pad_h), i);
+    // ---- signs of the channel group's filters (pattern 4 neg0 + 2 neg1 + neg2 of a tap; four channels to a load), thresholds (NaN:
+    // -infinity, the bit is 1 either way)
+    bool steps_256 = true;  // every threshold a multiple of 1/256 (below 2^15), or infinite: exact sums stay exact less these
+    {
+        constexpr int kLoads = (R * T * kChannels / 4 + 64 * kWaves - 1) / (64 * kWaves);
+        v4u sign[kLoads];
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const int e = i * 64 * kWaves + tid;
+            sign[i] = *reinterpret_cast<const v4u*>(args.pats + (unsigned)(min(e / (kChannels / 4), q.rs_taps - 1) * p.opad + tile0 * 32 + e % (kChannels / 4) * 4));
+        }
+        const float t = p.bn[tile0 * 32 + min(lane, kChannels - 1)];  // (every wave looks at all of them)
+        const float known = t != t ? -INFINITY : t;
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i)
+            if (i * 64 * kWaves + tid < R * T * kChannels / 4)
+                reinterpret_cast<uint32_t*>(signs)[i * 64 * kWaves + tid] = sign[i][0] | sign[i][1] << 8 | sign[i][2] << 16 | sign[i][3] << 24;
+        if (tid < kChannels) thr[tid] = kFromThreshold ? 0.0f - known : known;  // (a threshold of 0: sums start from +0)
+        steps_256 = __ballot(!(__builtin_fabsf(t) <= 32768.0f) ? __builtin_fabsf(t) < INFINITY : __builtin_amdgcn_fractf(t * 256.0f) != 0.0f) == 0;
+    }
+    __syncthreads();
+    // ---- +-1 fragments: lane (row n, half h) of set d's step k holds places 8 k .. 8 k + 7 of channel row_to_channel(n), half h
+    {
+        constexpr int kFrags = (D * KS * MT + kWaves - 1) / kWaves;  // of a wave
+        const int h = lane >> 5, n = mfma::row_to_channel(lane & 31);
+#pragma unroll 2
+        for (int i = 0; i < kFrags; ++i) {
+            const int e = i * kWaves + wave, d = e / (KS * MT), k = e / MT % KS;
+            if (e >= D * KS * MT) break;  // uniform
+            uint32_t half[8], pt[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int place = 8 * k + j, tap = place % P, r = d * A + (2 * (place / P) + h) / 3;
+                pt[j] = signs[(min(r, R - 1) * p.S + min(tap, p.S - 1)) * kChannels + e % MT * 32 + n];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int place = 8 * k + j, pair = 2 * (place / P) + h, tap = place % P, row = pair / 3;
+                const bool used = (tap < p.S) & (tap < T) & (pair < 3 * A) & (d * A + row < R);
+                half[j] = used ? 0x3c00u | (pt[j] << (13 + pair - 3 * row) & 0x8000u) : 0u;
+                if (!kFromThreshold && j == kBoundPlace && d == D - 1 && k == KS - 1 && h == 1) half[j] = 0x3c00u;
+            }
+            v4i f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) f[j] = (int)(half[2 * j] | half[2 * j + 1] << 16);
+            frags[e * 64 + lane] = f;
+        }
+    }
     __syncthreads();
     if (idle) return;
 
-    // ---- +-1 fragments: lane (row n, half h) holds taps 4j + 2h, 4j + 2h + 1 of channel row_to_channel(n), 4 channels each
-    v4i wf[NK][MT];
-    {
-    const int n = lane & 31, h = lane >> 5;
-#pragma unroll
-    for (int k = 0; k < NK; ++k)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const int o = (tile0 + m) * 32 + mfma::row_to_channel(n);
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int s = 4 * (k % NQ) + 2 * h + t;
-                const uint32_t pt = args.pats[(size_t)((k / NQ) * p.S + min(s, p.S - 1)) * p.opad + o];
-                uint32_t d0 = 0x3c003c00u | ((pt & 4u) << 13) | (pt << 30 & 0x80000000u), d1 = 0x3c00u | ((pt & 1u) << 15);
-                if (s >= p.S) d0 = d1 = 0u;
-                if (k == NK - 1 && t == 0) d1 |= h == 0 ? 0x3c000000u : 0u;  // the slot that -E enters through
-                wf[k][m][2 * t] = (int)d0;
-                wf[k][m][2 * t + 1] = (int)d1;
-            }
-        }
-    }
-
-    // ---- staging: units of one column pair x three channels, numbered over (row, image, pair)
-    const unsigned plane_b = (unsigned)(p.H * p.W) * 4u;
-    const int ax_first = x0 * p.stride_w - p.pad_w;
-    const bool edge = ax_first < 0 || ax_first + 2 * q.np > p.W;  // uniform
-    __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.in + (size_t)b0 * 3 * p.H * p.W), 0,
-                                                                    (int)((unsigned)min(NI, p.B - b0) * 3u * plane_b), 0x00020000);
-    unsigned voff[kRounds];  // byte offset of the left column (out of range: no such image)
-    unsigned cell[kRounds];  // cell in a row | left column in the frame << 16 | right one << 17 | row << 20
-#pragma unroll
-    for (int k = 0; k < kRounds; ++k) {
-        const int e = (member + kTeam * k) * 64 + lane, e2 = e / q.np, pr = e - e2 * q.np, im = e2 & (NI - 1), row = e2 >> q.ni_log2;
-        const int ax = ax_first + 2 * pr;
-        const bool used = row < q.adv && b0 + im < p.B;
-        voff[k] = used ? (unsigned)im * 3u * plane_b + (unsigned)((row * p.W + ax) * 4) : kOutOfRange;
-        cell[k] = (unsigned)(im * q.pp + (PAIRS == PAIRS_SPLIT ? (pr >> 1) + (pr & 1) * q.odd_pairs : pr)) | (used && ax >= 0 && ax < p.W ? 1u << 16 : 0u) |
-                  (used && ax + 1 >= 0 && ax + 1 < p.W ? 1u << 17 : 0u) | (unsigned)row << 20;
-    }
-    const int rounds = q.rounds;
-    v2f x[kRounds][3];
-    auto fetch = [&](int ay_first, int n_rows) __attribute__((always_inline)) {
-        const int row_b = ay_first * p.W * 4;
-        const bool inner = !edge && ay_first >= 0 && ay_first + q.adv <= p.H;  // uniform (units past n_rows read what nobody uses)
-#pragma unroll
-        for (int k = 0; k < kRounds; ++k) {
-            if (k >= rounds) break;  // uniform
-            if (inner) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-                    x[k][c] = __builtin_bit_cast(v2f, __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)voff[k], (int)((unsigned)row_b + c * plane_b), 0));
-            } else {
-                asm volatile("" : "+v"(cell[k]));  // (what is decoded from it is not kept across the multiplication)
-                // (an offset can be negative in front of the first image: the row's is part of the lane's here)
-                const int row = (int)(cell[k] >> 20), ay = ay_first + row;
-                const bool ok = row < n_rows && ay >= 0 && ay < p.H;
-                const unsigned oa = ok && (cell[k] >> 16 & 1u) ? voff[k] + (unsigned)row_b : kOutOfRange;
-                const unsigned ob = ok && (cell[k] >> 17 & 1u) ? voff[k] + (unsigned)row_b + 4u : kOutOfRange;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    x[k][c][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)oa, (int)(c * plane_b), 0));
-                    x[k][c][1] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)ob, (int)(c * plane_b), 0));
-                }
-            }
-        }
-    };
-    bool grid = true;  // every row staged so far is multiples of 1/256 (rows are checked as long as that holds)
-    // marks: the fourth channel of the lo plane says which columns are not multiples of 1/256
-    auto split_and_store = [&](auto marks, int n_rows, int slot0) __attribute__((always_inline)) {
-        bool on_grid = true;
-#pragma unroll
-        for (int k = 0; k < kRounds; ++k) {
-            if (k >= rounds) break;  // uniform
-            const float f[6] = {x[k][0][0], x[k][1][0], x[k][2][0], x[k][0][1], x[k][1][1], x[k][2][1]};
-            v4u hi, lo;
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const h2 a = __builtin_convertvector(v2f{f[3 * t], f[3 * t + 1]}, h2);
-                const h2 c = __builtin_convertvector(v2f{f[3 * t + 2], 0.0f}, h2);
-                const h2 al = __builtin_convertvector(v2f{minus_half<0>(f[3 * t], a), minus_half<1>(f[3 * t + 1], a)}, h2);
-                const h2 cl = __builtin_convertvector(v2f{minus_half<0>(f[3 * t + 2], c), 0.0f}, h2);
-                hi[2 * t] = __builtin_bit_cast(uint32_t, a);
-                hi[2 * t + 1] = __builtin_bit_cast(uint32_t, c);
-                lo[2 * t] = __builtin_bit_cast(uint32_t, al);
-                lo[2 * t + 1] = __builtin_bit_cast(uint32_t, cl);
-            }
-            if constexpr (decltype(marks)::value) {
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    float off = 0.0f;
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) off = __builtin_fmaxf(off, __builtin_amdgcn_fractf(f[3 * t + c] * 256.0f));
-                    lo[2 * t + 1] |= off > 0.0f ? 0x10000u : 0u;
-                }
-            }
-            asm volatile("" : "+v"(cell[k]));
-            const unsigned row = cell[k] >> 20;
-            if (row < (unsigned)n_rows) {
-                const unsigned s = (unsigned)slot0 + row, slot = min(s, s - (unsigned)q.ring);  // (ring: the smaller as unsigned)
-                char* const dst = rows + slot * (unsigned)row_bytes + (cell[k] & 0xffffu) * 16u;
-                *reinterpret_cast<v4u*>(dst) = hi;
-                *reinterpret_cast<v4u*>(dst + plane) = lo;
-            }
-            if (grid) {  // uniform
-#pragma unroll
-                for (int t = 0; t < 6; ++t) on_grid = on_grid & ((__builtin_amdgcn_fractf(f[t] * 256.0f) == 0.0f) | (row >= (unsigned)n_rows));
-            }
-        }
-        if (grid) {
-            const bool mine = __ballot(!on_grid) == 0;
-            if constexpr (kShared) {
-                if (!mine && lane == 0) flags[0] = 1;
-            } else {
-                grid = mine;
-            }
-        }
-    };
-
-    // ---- doubtful values: recomputed in the reference's order, 16 lanes per value (lane t of a row: tap 16 c + t), the
-    // list's last four at a time.  One trip to memory: inputs, signs and the residual's words are asked for together (the
-    // words after the sums, and the threshold from memory: two more trips, 111 us for 107, bytes / 255 163 for 147)
+    // ---- doubtful values: recomputed in the reference's order, 4 lanes per value (lane t of a quad: rows t, t + 4, ...), the
+    // list's last sixteen at a time.  What the residual's words hold is asked for with the inputs.
     int count = 0;  // entries on this wave's list (uniform)
-    constexpr int NC = (R * 4 * NQ + 15) / 16;
     auto recompute = [&]() __attribute__((always_inline)) {
         const SeldomArgs a = seldom_args(args_at);
         const auto& p = a->p;
-        const auto& q = a->q;
-        const uint32_t* const pats = a->pats;
-        float f[NC][3];
-        uint32_t pt[NC];
-        const int pending = min(count, 4);
+        constexpr int kTurns = (R + 3) / 4;  // rows of a lane
+        const int pending = min(count, kBatch);
         count -= pending;
-        int t16 = lane & 15;
-        int taps = q.rs_taps;
-        asm volatile("" : "+v"(t16), "+s"(taps));  // (nothing derived from them is kept outside)
-        const int e = count + min(lane >> 4, pending - 1);
+        int ln = lane;
+        asm volatile("" : "+v"(ln));  // (nothing derived from it is kept outside)
+        const int t4 = ln & 3, e = count + min(ln >> 2, pending - 1);
         const uint32_t ex = list[2 * e], ey = list[2 * e + 1];
         const int ay0 = (int)(ex >> 16) * p.stride_h - p.pad_h, ax0 = (int)(ex & 0xffffu) * p.stride_w - p.pad_w;
         const int o = (int)(ey & 0xffffu);
         const unsigned im = (ey >> 16) * 3u * plane_b;
-        const bool active = (lane >> 4) < pending;
+        const bool active = (ln >> 2) < pending;
         const int bb = b0 + (int)(ey >> 16);
         const unsigned pix = (ex >> 16) / POOL * (unsigned)p.OW + (ex & 0xffffu) / POOL;  // (host: tensors below 2 GiB)
-        // What the residual's words hold is asked for now, with the inputs.  Bits [fix_shift, ...) of the 32-bit word fix_at,
-        // under fix_mask, are the value's from bit fix_drop on; only this lane changes them, neighbours in the same word are
-        // left alone (exclusive or with what differs).
+        // Bits [fix_shift, ...) of the 32-bit word fix_at, under fix_mask, are the value's from bit fix_drop on; only this lane
+        // changes them, neighbours in the same word are left alone (exclusive or with what differs).
         uint32_t* const residual = reinterpret_cast<uint32_t*>(p.res);
         size_t fix_at = 0;
         int fix_shift = 0, fix_drop = 0;
         uint32_t fix_mask = 0u, old = 0u;
         if constexpr (RES == RES_12) {
             const int bit = 12 * (o & 15), here = min(12, 32 - (bit & 31));
-            const bool second = t16 == 1;
+            const bool second = t4 == 1;
             fix_shift = second ? 0 : bit & 31;
             fix_drop = second ? here : 0;
-            fix_mask = t16 < 2 ? (1u << (second ? 12 - here : here)) - 1u : 0u;
+            fix_mask = t4 < 2 ? (1u << (second ? 12 - here : here)) - 1u : 0u;
             fix_at = i12_word_index(pix, (size_t)((p.O + 15) / 16), o >> 4, p.B, bb, (bit >> 5) + (second ? 1 : 0));
         } else if constexpr (RES == RES_WIDE) {
             fix_at = residual_index(p.res_fmt, pix, p.O, o, p.B, bb);
             if (p.res_fmt == TCBNN_RES_I16) {
                 fix_shift = (int)(fix_at & 1) * 16;
-                fix_mask = t16 == 0 ? 0xffffu : 0u;
+                fix_mask = t4 == 0 ? 0xffffu : 0u;
                 fix_at >>= 1;
             }
         }
         const bool fix = active && fix_mask != 0u;
         if (RES != RES_NONE && fix) old = __hip_atomic_load(residual + fix_at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool whole = p.S == T && __ballot((ax0 < 0) | (ax0 + T > p.W)) == 0;  // uniform: every window inside the frame's columns
+        float acc = 0.0f;
+#pragma unroll(kTurns <= 2 ? kTurns : 1)
+        for (int turn = 0; turn < kTurns; ++turn) {
+            const int r = 4 * turn + t4, ay = ay0 + r;
+            const bool row = (r < R) & (ay >= 0) & (ay < p.H);  // (else zeros, which add nothing)
+            const unsigned at = im + (unsigned)(ay * p.W + ax0) * 4u;
+            float f[3][T];
+            if (whole) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const int tap = 16 * c + t16, r = (int)((unsigned)tap * q.s_magic >> 16), s = tap - r * p.S;
-            const int ay = ay0 + r, ax = ax0 + s;
-            const bool inside = (tap < taps) & (ay >= 0) & (ay < p.H) & (ax >= 0) & (ax < p.W);  // (else zeros, which add nothing)
-            const unsigned at = inside ? im + (unsigned)(ay * p.W + ax) * 4u : kOutOfRange;
+                for (int ch = 0; ch < 3; ++ch) load_taps<T>(rsrc, row ? at : kOutOfRange, ch * plane_b, f[ch]);
+            } else {
 #pragma unroll
-            for (int ch = 0; ch < 3; ++ch)
-                f[c][ch] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)at, (int)(ch * plane_b), 0));
-            pt[c] = pats[(unsigned)(min(tap, taps - 1) * p.opad + o)];
-        }
-        {
-            float acc = 0.0f;
+                for (int t = 0; t < T; ++t) {
+                    const bool inside = row & (t < p.S) & (ax0 + t >= 0) & (ax0 + t < p.W);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const float f0 = __uint_as_float(__float_as_uint(f[c][0]) ^ ((pt[c] & 4u) << 29));
-                const float f1 = __uint_as_float(__float_as_uint(f[c][1]) ^ ((pt[c] & 2u) << 30));
-                const float f2 = __uint_as_float(__float_as_uint(f[c][2]) ^ ((pt[c] & 1u) << 31));
-                const float m = (f0 + f1) + f2;
-                if (16 * c + 16 <= taps)  // uniform
-                    acc = add_row_taps<0, 16, true>(acc, m, 16);
-                else
-                    acc = add_row_taps<0, 16, false>(acc, m, taps - 16 * c);
+                    for (int ch = 0; ch < 3; ++ch)
+                        f[ch][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(inside ? at + 4u * t : kOutOfRange), (int)(ch * plane_b), 0));
+                }
             }
-            // (the row's 16 lanes all hold the sum: lane 2 sets the bit, lanes 0 and 1 repair the one or two words)
-            if (active && t16 == 2 && !(acc < thr[o]))
-                __hip_atomic_fetch_or(p.out + ((pix * (unsigned)p.ow + (unsigned)(o >> 5)) * (unsigned)p.B + (unsigned)bb), 0x80000000u >> (o & 31), __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);
-            if constexpr (RES != RES_NONE) {
-                const uint32_t v = (uint32_t)(int)acc;
-                const uint32_t d = ((old >> fix_shift ^ v >> fix_drop) & fix_mask) << fix_shift;
-                if (fix && d != 0u) __hip_atomic_fetch_xor(residual + fix_at, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (RES == RES_WIDE && active && t16 == 0 && p.res_fmt == TCBNN_RES_I32) residual[fix_at] = v;
+            const uint8_t* const row_signs = signs + min(r, R - 1) * p.S * kChannels + (o - tile0 * 32);
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const uint32_t pt = row_signs[min(t, p.S - 1) * kChannels];
+                const float f0 = __uint_as_float(__float_as_uint(f[0][t]) ^ (pt << 29 & 0x80000000u));
+                const float f1 = __uint_as_float(__float_as_uint(f[1][t]) ^ (pt << 30 & 0x80000000u));
+                const float f2 = __uint_as_float(__float_as_uint(f[2][t]) ^ (pt << 31));
+                f[0][t] = (f0 + f1) + f2;
+            }
+#pragma unroll
+            for (int t = 0; t < T; ++t) acc = add_quad_lane<0>(acc, f[0][t]);
+#pragma unroll
+            for (int t = 0; t < T; ++t) acc = add_quad_lane<1>(acc, f[0][t]);
+#pragma unroll
+            for (int t = 0; t < T; ++t) acc = add_quad_lane<2>(acc, f[0][t]);
+            if (kTurns * 4 == R || turn + 1 < kTurns) {
+#pragma unroll
+                for (int t = 0; t < T; ++t) acc = add_quad_lane<3>(acc, f[0][t]);
             }
         }
-    };
-
-    // ---- the window
-    int ay0 = oy_begin * POOL * p.stride_h - p.pad_h;  // first input row of the step's window
-    int s0 = 0;                                        // its ring slot
-    auto stage_window = [&](auto marks) __attribute__((always_inline)) {
-        for (int done = 0; done < q.ring; done += q.adv) {
-            const int n = min(q.adv, q.ring - done), slot = s0 + done;
-            fetch(ay0 + done, n);
-            split_and_store(marks, n, slot >= q.ring ? slot - q.ring : slot);
-        }
-    };
-    stage_window(std::false_type{});
-
-    const __amdgpu_buffer_rsrc_t out_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)args.out_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t res_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.res, 0, (int)args.res_bytes, 0x00020000);
-    // Where this lane stores, relative to the item (uniform): its output word, its 16 residuals (12-bit: the 8-byte part
-    // apart); beyond the tensors for an image past the batch.
-    const unsigned uB = (unsigned)p.B, group_b = (RES == RES_12 ? 24u : (p.res_fmt == TCBNN_RES_I16 ? 32u : 64u)) * uB;
-    const unsigned pixel_b = (unsigned)(p.O / 16) * group_b;
-    unsigned place_word, place_res = 0u, place_res8 = 0u;
-    {
-        const unsigned px = (unsigned)((lane & 31) >> q.ni_log2), h = (unsigned)lane >> 5, b = (unsigned)(b0 + (lane & (NI - 1)));
-        const bool image = b < uB;
-        place_word = image && (MT == 2 || h == 0u) && (POOL == 1 || (px & 1u) == 0u)
-                         ? ((px / POOL * (unsigned)p.ow + (MT == 2 ? h : 0u)) * uB + b) * 4u : kOutOfRange;
+        // (the quad's lanes all hold the sum: lane 2 sets the bit, lanes 0 and 1 repair the one or two words)
+        if (active && t4 == 2 && !(acc < threshold(o - tile0 * 32)))
+            __hip_atomic_fetch_or(p.out + ((pix * (unsigned)p.ow + (unsigned)(o >> 5)) * (unsigned)p.B + (unsigned)bb), 0x80000000u >> (o & 31), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
         if constexpr (RES != RES_NONE) {
-            place_res = image ? px * pixel_b + h * group_b + b * 16u : kOutOfRange;
-            place_res8 = image ? px * pixel_b + h * group_b + uB * 16u + b * 8u : kOutOfRange;
+            const uint32_t v = (uint32_t)(int)acc;
+            const uint32_t d = ((old >> fix_shift ^ v >> fix_drop) & fix_mask) << fix_shift;
+            if (fix && d != 0u) __hip_atomic_fetch_xor(residual + fix_at, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (RES == RES_WIDE && active && t4 == 0 && p.res_fmt == TCBNN_RES_I32) residual[fix_at] = v;
         }
-    }
+    };
 
     // ---- a whole item in the reference's order: words, residuals; in doubt stay sums that are no numbers.
     // A tap's eight possible values are four and their negatives, so adding one of them to 32 x 32 sums is a product with a
     // matrix of one +-1 and three 0 per row: two v_mfma_f32_32x32x2_f32, each one fp32 addition per sum (adding the zeros
     // changes nothing; tests/test_gpu_matrix_core.py).
-    auto ordered_sums = [&](int oy, int g, uint32_t* word, uint32_t& doubt) __attribute__((always_inline)) {
+    auto ordered_sums = [&](int cy, uint32_t* word) __attribute__((always_inline)) -> uint32_t {
         const SeldomArgs a = seldom_args(args_at);
         const auto& p = a->p;
         const uint32_t* const pats = a->pats;
         int ln = lane;
         asm volatile("" : "+v"(ln));  // (nothing derived from it is kept outside)
-        const int h = ln >> 5, img = ln & (NI - 1), xc = x0 + g * NX + ((ln & 31) >> a->q.ni_log2);
+        const int h = ln >> 5, img = ln & (NI - 1), xc = g * NX + ((ln & 31) >> a->q.ni_log2);
         const bool valid = b0 + img < p.B && xc < xcols;
-        const int ax0 = xc * p.stride_w - p.pad_w, o0 = tile0 * 32 + mfma::row_to_channel(ln & 31);
+        const int ax0 = xc * p.stride_w - p.pad_w, ay0 = cy * A - p.pad_h, r_end = min(R, p.H - ay0);
         const unsigned im = (unsigned)img * 3u * plane_b, flip = (unsigned)h << 31;
-        doubt = 0u;
+        uint32_t undecided = 0u;
+        const int o0 = tile0 * 32 + mfma::row_to_channel(ln & 31);
+        const bool whole = p.S == T && __ballot(valid & ((ax0 < 0) | (ax0 + T > p.W))) == 0;  // uniform
+        v16f acc[MT];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) word[m] = 0u;
-#pragma unroll 1
-        for (int py = 0; py < POOL; ++py) {
-            const int ay0 = (oy * POOL + py) * p.stride_h - p.pad_h, r_end = min(R, p.H - ay0);
-            v16f acc[MT];
+        for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int m = 0; m < MT; ++m)
+            for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
+        // a filter row at a time, requested one row ahead; out of the frame: zeros, which add nothing
+        float next[3][T];
+        uint32_t next_pt[T][MT];
+        auto request = [&](int r) __attribute__((always_inline)) {
+            const unsigned at0 = im + (unsigned)((ay0 + r) * p.W + ax0) * 4u;
+            if (whole) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
-            // a filter row at a time, requested one row ahead; out of the frame: zeros, which add nothing
-            constexpr int kTaps = 4 * NQ;
-            float next[kTaps][3];
-            uint32_t next_pt[kTaps][MT];
-            auto request = [&](int r) __attribute__((always_inline)) {
-                const unsigned at0 = im + (unsigned)((ay0 + r) * p.W + ax0) * 4u;
+                for (int ch = 0; ch < 3; ++ch) load_taps<T>(rsrc, valid ? at0 : kOutOfRange, ch * plane_b, next[ch]);
+            } else {
 #pragma unroll
-                for (int j = 0; j < NQ; ++j) {
-                    const int ax = ax0 + 4 * j;
-                    const unsigned at = at0 + 16u * j;
-                    if (__ballot(valid & ((ax < 0) | (ax + 4 > p.W))) == 0) {  // uniform
+                for (int t = 0; t < T; ++t) {
+                    const bool inside = valid & (ax0 + t >= 0) & (ax0 + t < p.W);
 #pragma unroll
-                        for (int ch = 0; ch < 3; ++ch) {
-                            const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(valid ? at : kOutOfRange), (int)(ch * plane_b), 0));
-#pragma unroll
-                            for (int t = 0; t < 4; ++t) next[4 * j + t][ch] = v[t];
-                        }
-                    } else {
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) {
-                            const bool inside = valid & (ax + t >= 0) & (ax + t < p.W);
-#pragma unroll
-                            for (int ch = 0; ch < 3; ++ch)
-                                next[4 * j + t][ch] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(inside ? at + 4u * t : kOutOfRange), (int)(ch * plane_b), 0));
-                        }
-                    }
+                    for (int ch = 0; ch < 3; ++ch)
+                        next[ch][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(inside ? at0 + 4u * t : kOutOfRange), (int)(ch * plane_b), 0));
                 }
-                const uint32_t* const row = pats + (unsigned)(r * p.S * p.opad);  // (uniform)
+            }
+            const uint32_t* const row = pats + (unsigned)(r * p.S * p.opad);  // (uniform)
 #pragma unroll
-                for (int t = 0; t < kTaps; ++t)
+            for (int t = 0; t < T; ++t)
 #pragma unroll
-                    for (int m = 0; m < MT; ++m) next_pt[t][m] = row[(unsigned)(min(t, p.S - 1) * p.opad + o0 + 32 * m)];
-            };
-            const int r_begin = max(0, -ay0);
-            if (r_begin < r_end) request(r_begin);
+                for (int m = 0; m < MT; ++m) next_pt[t][m] = row[(unsigned)(min(t, p.S - 1) * p.opad + o0 + 32 * m)];
+        };
+        const int r_begin = max(0, -ay0);
+        if (r_begin < r_end) request(r_begin);
 #pragma unroll 1
-            for (int r = r_begin; r < r_end; ++r) {
-                float f[kTaps][3];
-                uint32_t pt[kTaps][MT];
+        for (int r = r_begin; r < r_end; ++r) {
+            float f[3][T];
+            uint32_t pt[T][MT];
 #pragma unroll
-                for (int t = 0; t < kTaps; ++t) {
+            for (int t = 0; t < T; ++t) {
 #pragma unroll
-                    for (int ch = 0; ch < 3; ++ch) f[t][ch] = next[t][ch];
+                for (int ch = 0; ch < 3; ++ch) f[ch][t] = next[ch][t];
 #pragma unroll
-                    for (int m = 0; m < MT; ++m) pt[t][m] = next_pt[t][m];
-                }
-                if (r + 1 < r_end) request(r + 1);
+                for (int m = 0; m < MT; ++m) pt[t][m] = next_pt[t][m];
+            }
+            if (r + 1 < r_end) request(r + 1);
 #pragma unroll
-                for (int t = 0; t < kTaps; ++t) {
-                    if (t >= p.S) break;  // uniform
-                    const float f2 = __uint_as_float(__float_as_uint(f[t][2]) ^ flip);
-                    const float same = (f[t][0] + f[t][1]) + f2, other = (f[t][0] - f[t][1]) + f2;
+            for (int t = 0; t < T; ++t) {
+                if (t < p.S) {  // uniform
+                    const float f2 = __uint_as_float(__float_as_uint(f[2][t]) ^ flip);
+                    const float same = (f[0][t] + f[1][t]) + f2, other = (f[0][t] - f[1][t]) + f2;
 #pragma unroll
                     for (int m = 0; m < MT; ++m) {
                         // pattern 4 neg0 + 2 neg1 + neg2; a pattern from 4 on is the negative of the inverted one
@@ -576,306 +558,381 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(workgr
                     }
                 }
             }
+        }
 #pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                const v4f* const tp = reinterpret_cast<const v4f*>(thr + (tile0 + m) * 32 + 16 * h);
-                uint32_t w = 0u;
-                float zero = 0.0f;  // an infinity or NaN among a tap's values makes NaN of it, times 0, in every sum
+        for (int m = 0; m < MT; ++m) {
+            const v4f* const tp = reinterpret_cast<const v4f*>(thr + m * 32 + 16 * h);
+            uint32_t w = 0u;
+            float zero = 0.0f;  // an infinity or NaN among a tap's values makes NaN of it, times 0, in every sum
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    w = __builtin_amdgcn_alignbit(w, __float_as_uint(acc[m][i] - tp[i >> 2][i & 3]), 31);
-                    zero = __builtin_fmaf(acc[m][i], 0.0f, zero);
-                }
-                const bool bad = !(zero == 0.0f);
-                word[m] |= bad ? 0u : ~w & 0xffffu;
-                doubt |= (bad && valid ? 0xffffu : 0u) << (16 * (POOL > 1 ? py : m));
-                if constexpr (RES != RES_NONE) {
-                    int v[16];
+            for (int i = 0; i < 16; ++i) {
+                w = __builtin_amdgcn_alignbit(w, __float_as_uint(kFromThreshold ? acc[m][i] + tp[i >> 2][i & 3] : acc[m][i] - tp[i >> 2][i & 3]), 31);
+                zero = __builtin_fmaf(acc[m][i], 0.0f, zero);
+            }
+            const bool bad = !(zero == 0.0f);
+            w = bad ? 0u : ~w & 0xffffu;
+            undecided |= (bad && valid ? 0xffffu : 0u) << (16 * m);
+            word[m] |= w;
+            if constexpr (RES != RES_NONE) {
+                int v[16];
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) v[i] = (int)acc[m][i];
-                    const unsigned item = (unsigned)(oy * p.PW + x0 + g * NX) * pixel_b + (unsigned)((tile0 + m) * 2) * group_b;
-                    store_residual_group<RES>(res_rsrc, p.res_fmt, valid ? place_res + item : kOutOfRange,
-                                              RES == RES_12 ? (valid ? place_res8 + item : kOutOfRange) : 0u, uB * 16u, v);
-                    __builtin_amdgcn_sched_barrier(0);  // (one tile at a time: registers)
-                }
+                for (int i = 0; i < 16; ++i) v[i] = (int)acc[m][i];
+                const unsigned item = (unsigned)(cy * p.PW + g * NX) * pixel_b + (unsigned)((tile0 + m) * 2) * group_b;
+                store_residual_group<RES>(res_rsrc, p.res_fmt, valid ? place_residual(ln) + item : kOutOfRange,
+                                          RES == RES_12 ? (valid ? place_residual8(ln) + item : kOutOfRange) : 0u, uB * 16u, v);
             }
         }
+        return undecided;
     };
 
-    // ---- the band's items, in up to three passes.  The common one ends at an item with many values in doubt.  That item and
-    // the rest of the band are then done with marks (common sums, exact where a window has none), and from an item on where
-    // that still leaves many, in the reference's order.  (A shared ring is left by all its waves together, before the next
-    // row, and for ordered sums.)
-    int oy = oy_begin, g = wg0;
-    bool many = false;
-    auto pass = [&](auto mode) __attribute__((always_inline)) {
-        constexpr bool kMarked = decltype(mode)::value == MARKED, kOrdered = decltype(mode)::value == ORDERED;
-        constexpr int kManyLanes = kMarked ? kManyLanesMarked : kManyLanesCommon;
-        // Few sums are ever in doubt where no residual is saved: that there are many is seen by the list, and the pass ends
-        // with the row, which costs its loop less.
-        constexpr bool kRowExit = RES == RES_NONE && !kShared;
-        int first_g = n_groups;
-        many = false;
-        for (; oy < oy_end; ++oy) {
-            const bool more = oy + 1 < oy_end;  // uniform
-            if constexpr (kShared && !kOrdered) {
-                __syncthreads();
-                if (grid) grid = __builtin_amdgcn_readfirstlane(flags[0]) == 0;
-                if (__builtin_amdgcn_readfirstlane(flags[1]) != 0) return;  // (written between the two barriers only)
+    // ---- the wave's rows.  An item (a row) with many values in doubt is done again with its windows checked for the grid, as
+    // are all that follow; one that still has many, and all that follow, in the reference's order.
+    bool check = !kFromThreshold, keep_checking = false, loaded = true;  // (sums that start from -bn are seldom in doubt)
+    auto pass = [&](auto ordered) __attribute__((always_inline)) {
+        constexpr bool kOrdered = decltype(ordered)::value;
+        v16f acc[D][MT];
+        float sum[D], parts[D], off[D];
+        const int first_row = cy;
+        int block = cy;  // of A input rows; the oldest set's output row is block - D + 1
+        if constexpr (!kOrdered) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                sum[d] = parts[d] = off[d] = 0.0f;
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[d][m][i] = 0.0f;
             }
-            if (!kOrdered && more) fetch(ay0 + q.ring, q.adv);
-            while (g < n_groups) {
-                uint32_t word[MT];
-                uint32_t doubt = 0u;
-                // A lane's place (column of the tile: image and pixel; half of the channels) is worked out anew from a lane
-                // index the compiler cannot carry over: kept across the multiplication, the addresses made from it spill.
-                int ln = lane;
-                asm volatile("" : "+v"(ln));
+            if (!loaded) {  // uniform
 #pragma unroll
-                for (int m = 0; m < MT; ++m) word[m] = 0u;
-                if constexpr (!kOrdered) {
+                for (int i = 0; i < kRing; ++i) load(block * A - p.pad_h, path_of(block * A - p.pad_h), i);
+            }
+            loaded = false;
+        }
+        v4i weights[MT];  // of the set and step that is multiplied next
+        auto read_weights = [&](int d, int k) __attribute__((always_inline)) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) weights[m] = frags[((d * KS + k) * MT + m) * 64 + lane];
+        };
+        if constexpr (!kOrdered) read_weights(D - 1, 0);
+        uint32_t word[MT], doubt[POOL];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) word[m] = 0u;
+#pragma unroll
+        for (int py = 0; py < POOL; ++py) doubt[py] = 0u;
 #pragma unroll 1
-                    for (int py = 0; py < POOL; ++py) {
-                        v16f acc[MT];
+        while (cy < cy_end) {
+            // A lane's place (column of the tile: image and pixel; half of the channels) is worked out anew from a lane
+            // index the compiler cannot carry over: kept across the multiplication, the addresses made from it spill.
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+            uint32_t undecided = 0u;
+            if constexpr (!kOrdered) {
+                const int ay = block * A - p.pad_h, done = block - (D - 1);  // (uniform)
+                const bool more = done + 1 < cy_end;
+                const int path = path_of(ay), next_path = path_of(ay + A);
+                // Sums of |x| (and what is off the grid): of the step's rows, and of those that the oldest set has weights for; and
+                // these sums before each rounding, added up.
+                float step_sum = 0.0f, step_off = 0.0f, step_parts = 0.0f, old_sum = 0.0f, old_off = 0.0f, old_parts = 0.0f, two_e = 0.0f;
+                bool bad = false, small = false;  // small: |S| and |acc| are below 1/2, the residual is 0
 #pragma unroll
-                        for (int m = 0; m < MT; ++m)
+                for (int k = 0; k < KS; ++k) {
+                    if (!columns_inside) {  // uniform
+                        unsigned in = ~outside;
+                        asm volatile("" : "+v"(in));  // (nothing derived from it is kept outside)
 #pragma unroll
-                            for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
-                        const int first_col = (g * NX + ((ln & 31) >> q.ni_log2)) * p.stride_w;
-                        const int lane_at = (ln & (NI - 1)) * q.pp * 16 + (PAIRS == PAIRS_SPLIT ? (first_col >> 2) * 16 + (ln >> 5) * q.odd_pairs * 16
-                                                                                               : first_col * 8 + (ln >> 5) * 16);
-                        auto fragment = [&](int r, int j, int plane_off) -> v4i {
-                            int slot = s0 + py * p.stride_h + r;
-                            slot = slot >= q.ring ? slot - q.ring : slot;
-                            const char* const at = rows + (slot * row_bytes + plane_off) + lane_at + j * (PAIRS == PAIRS_SPLIT ? 16 : 32);
-                            if constexpr (PAIRS != PAIRS_ANY)
-                                return __builtin_bit_cast(v4i, *reinterpret_cast<const h8*>(at));
-                            else
-                                return __builtin_bit_cast(v4i, static_cast<h8>(*reinterpret_cast<const h8u*>(at)));
-                        };
-                        bool exact = false;  // this lane's window has no mark
-                        if constexpr (kMarked) {
-                            uint32_t marks = 0u;
-#pragma unroll 2
-                            for (int k = 0; k < NK; ++k) {
-                                const v4i v = fragment(k / NQ, k % NQ, plane);
-                                const int s = 4 * (k % NQ) + 2 * (ln >> 5);
-                                marks |= (s < p.S ? (uint32_t)v[1] : 0u) | (s + 1 < p.S ? (uint32_t)v[3] : 0u);
-                            }
-                            const auto sw = __builtin_amdgcn_permlane32_swap(marks, marks, false, false);
-                            exact = (sw[0] | sw[1]) < 0x10000u;
+                        for (int j = 0; j < 8; ++j) {
+                            const int at = 8 * k + j;
+                            if (at / P >= kPairs || at % P >= T) continue;
+                            float& f = x[at / P % kRing][at % P < T ? at % P : 0];
+                            f = __uint_as_float(__float_as_uint(f) & (unsigned)((int)(in << (31 - at % P)) >> 31));
                         }
-                        // lo steps, then hi steps; a step's fragment is requested kAhead steps ahead
-                        constexpr int kAhead = 4;
-                        v4i ahead[kAhead];
+                    }
+                    // eight places: hi and lo
+                    v4i hi, lo;
 #pragma unroll
-                        for (int k = 0; k < kAhead; ++k) ahead[k] = fragment(k % NK / NQ, k % NK % NQ, k < NK ? plane : 0);
-                        float sq = 0.0f, two_e = 0.0f, half_a = 0.0f, wide_shift = 0.0f, wide_two_e = 0.0f;
-                        bool bad = false, small = false;  // small: |S| and |acc| are below 1/2, the residual is 0
+                    for (int j = 0; j < 4; ++j) {
+                        const int p0 = 8 * k + 2 * j, p1 = p0 + 1;
+                        const bool u0 = p0 / P < kPairs && p0 % P < T, u1 = p1 / P < kPairs && p1 % P < T;
+                        const float f0 = u0 ? x[p0 / P % kRing][p0 % P < T ? p0 % P : 0] : 0.0f, f1 = u1 ? x[p1 / P % kRing][p1 % P < T ? p1 % P : 0] : 0.0f;
+                        const h2 v = __builtin_convertvector(v2f{f0, f1}, h2);
+                        const h2 w = __builtin_convertvector(v2f{u0 ? minus_half<0>(f0, v) : 0.0f, u1 ? minus_half<1>(f1, v) : 0.0f}, h2);
+                        hi[j] = __builtin_bit_cast(int, v);
+                        lo[j] = __builtin_bit_cast(int, w);
+                    }
 #pragma unroll
-                        for (int k = 0; k < 2 * NK; ++k) {
-                            v4i v = ahead[k % kAhead];
-                            if (k + kAhead < 2 * NK)
-                                ahead[k % kAhead] = fragment((k + kAhead) % NK / NQ, (k + kAhead) % NK % NQ, k + kAhead < NK ? plane : 0);
-                            if (k >= NK) {
+                    for (int j = 0; j < 8; ++j) {
+                        const int at = 8 * k + j;
+                        if (at / P >= kPairs || at % P >= T) continue;
+                        step_sum += __builtin_fabsf(x[at / P % kRing][at % P < T ? at % P : 0]);
+                        if (order::in_old(2 * (at / P)) && order::in_old(2 * (at / P) + 1)) old_sum = step_sum;
+                        else if (order::in_old(2 * (at / P)) && (at % P == T - 1 || j == 7)) old_sum = lane < 32 ? step_sum : old_sum;
+                    }
+                    if constexpr (kParts) {
+                        step_parts = __builtin_fmaf(step_sum, (float)order::roundings(k, false), step_parts);
+                        old_parts = __builtin_fmaf(old_sum, (float)order::roundings(k, true), old_parts);
+                    }
+                    if (check) {  // uniform
 #pragma unroll
-                                for (int d = 0; d < 4; ++d) {
-                                    const int two = v[d];
-                                    sq = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, two), __builtin_bit_cast(h2, two), sq, false);
-                                }
-                            }
-                            if (kMarked && k == NK - 1 && lane < 32) v[1] &= 0xffff;  // (a mark where -E will enter)
-                            if (k == 2 * NK - 1) {
-                                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(sq), __float_as_uint(sq), false, false);
-                                const float all = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-                                const float root = __builtin_amdgcn_sqrtf(all), full = root * q.bound_scale_full + q.bound_add;
-                                small = all < q.small_squares;
-                                bad = !(all < 4.0e9f) || !(full < 3.0e4f);
-                                _Float16 eh = (_Float16)(root * q.bound_scale + q.bound_add);
-                                half_a = root * q.half_scale;
-                                wide_two_e = 2.002f * full;
-                                if ((grid | exact) & (all < q.exact_squares)) {
-                                    eh = (_Float16)0.0f;
-                                    half_a = INFINITY;
-                                }
-                                two_e = 2.002f * (float)eh;
-                                wide_shift = (float)eh - full;
-                                if (lane < 32) v[1] |= (int)((uint32_t)(__builtin_bit_cast(uint16_t, eh) | 0x8000u) << 16);
-                            }
-#pragma unroll
-                            for (int m = 0; m < MT; ++m)
-                                acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, wf[k % NK][m]), __builtin_bit_cast(h8, v), acc[m], 0, 0, 0);
-                            __builtin_amdgcn_sched_barrier(0);
+                        for (int j = 0; j < 8; ++j) {
+                            const int at = 8 * k + j;
+                            if (at / P < kPairs && at % P < T) step_off = __builtin_fmaxf(step_off, __builtin_amdgcn_fractf(x[at / P % kRing][at % P < T ? at % P : 0] * 256.0f));
+                            if (order::in_old(2 * (at / P)) && order::in_old(2 * (at / P) + 1)) old_off = step_off;
+                            else if (order::in_old(2 * (at / P))) old_off = lane < 32 ? step_off : old_off;
                         }
-                        // ---- bits (MSB first; the sign of S - E - bn, inverted), residual, doubtful values
-                        asm volatile("" : "+v"(ln));
-                        const int h = ln >> 5;
-                        const bool valid = b0 + (ln & (NI - 1)) < p.B && x0 + g * NX + ((ln & 31) >> q.ni_log2) < xcols;
+                    }
+                    // the pairs that are used up make room
+#pragma unroll
+                    for (int i = 8 * k / P; i < (k == KS - 1 ? kPairs : 8 * (k + 1) / P); ++i) {
+                        if (i + kRing < kPairs)
+                            load(ay, path, i + kRing);
+                        else if (more)  // uniform
+                            load(ay + A, next_path, i + kRing - kPairs);
+                    }
+                    if (k == KS - 1) {
+#pragma unroll
+                        for (int d = D - 1; d > 0; --d) {
+                            const bool old = d == D - 1;
+                            if constexpr (kParts) parts[d] = __builtin_fmaf(sum[d - 1], (float)order::roundings(old), parts[d - 1]) + (old ? old_parts : step_parts);
+                            sum[d] = sum[d - 1] + (old ? old_sum : step_sum);
+                            off[d] = __builtin_fmaxf(off[d - 1], old ? old_off : step_off);
+                        }
+                        parts[0] = step_parts, sum[0] = step_sum, off[0] = step_off;
+                        const float all = both_halves(sum[D - 1]);
+                        small = all < 0.49f;
+                        const float e = __builtin_fmaf(all, q.bound_sum, kParts ? __builtin_fmaf(both_halves(parts[D - 1]), q.bound_parts, q.bound_add) : q.bound_add);
+                        bad = !(e < 3.0e4f);
+                        _Float16 eh = (_Float16)e;
+                        bool exact = false;
+                        if (check) {  // uniform
+                            const auto so = __builtin_amdgcn_permlane32_swap(__float_as_uint(off[D - 1]), __float_as_uint(off[D - 1]), false, false);
+                            exact = (so[0] | so[1]) == 0u;
+                            if (!keep_checking && done >= cy && __ballot(!exact) != 0) check = false;
+                            exact = exact & (all < 3.2e4f) & (steps_256 || !kFromThreshold);  // (below 2^15: 23 bits, which the halves hold)
+                        }
+                        if (exact | bad) eh = (_Float16)0.0f;  // (bad: nothing infinite may meet the other sets' zeros)
+                        if constexpr (kFromThreshold) {
+                            two_e = exact ? 0.0f : e;
+                        } else {
+                            two_e = 2.002f * (float)eh;
+                            if (lane >= 32) hi[kBoundPlace / 2] |= (int)((uint32_t)(__builtin_bit_cast(uint16_t, eh) | 0x8000u) << 16);
+                        }
+                    }
+                    // lo, then hi; the first product of a step moves a set's sums on to the next.  A set's weights are read while the
+                    // one before it is multiplied.  (7x7/4: the test for rows of other bands costs it registers that it does not have:
+                    // 111 us -> 151; elsewhere 2 to 6 % less.)
+#pragma unroll
+                    for (int d = D - 1; d >= 0; --d) {
+                        v4i a[MT];
+#pragma unroll
+                        for (int m = 0; m < MT; ++m) a[m] = weights[m];
+                        read_weights(d > 0 ? d - 1 : D - 1, d > 0 ? k : (k + 1) % KS);
+                        if ((R != 7 || A == 2) && (block - d < first_row || block - d >= cy_end)) continue;  // uniform: not a row of this band
 #pragma unroll
                         for (int m = 0; m < MT; ++m) {
-                            const v4f* const tp = reinterpret_cast<const v4f*>(thr + (tile0 + m) * 32 + 16 * h);
-                            // Signs are collected MSB first (bit 15 - i: channel i).  w: S - E < bn, dm: values in doubt.  Integers
-                            // within E are common (in every other tile) and collected like the bits; thresholds within E and sums
-                            // above A/2 (E is less than a bound for those) are rare: the tile's nearest distance below a threshold
-                            // and its largest |S| tell whether to look for them.
-                            uint32_t w = 0u, dm = 0u;
-                            int nearest = INT32_MAX;
-                            float most = 0.0f;
-                            {
-                                const v4f th[4] = {tp[0], tp[1], tp[2], tp[3]};
+                            v16f c = acc[d][m];
+                            if (k == 0) {
+                                if (d > 0) {
+                                    c = acc[d > 0 ? d - 1 : 0][m];
+                                } else if (kFromThreshold) {
+                                    const v4f* const tp = reinterpret_cast<const v4f*>(thr + m * 32 + (lane >> 5) * 16);
 #pragma unroll
-                                for (int i = 0; i < 16; ++i) {
-                                    const float d = acc[m][i] - th[i >> 2][i & 3];
-                                    w = __builtin_amdgcn_alignbit(w, __float_as_uint(d), 31);
-                                    nearest = min(nearest, __float_as_int(d));
-                                    if constexpr (kHalf) most = __builtin_fmaxf(most, __builtin_fabsf(acc[m][i]));
-                                    if constexpr (RES != RES_NONE)
-                                        dm = __builtin_amdgcn_alignbit(dm, __float_as_uint(__builtin_amdgcn_fractf(-acc[m][i]) - two_e), 31);
+                                    for (int i = 0; i < 16; ++i) c[i] = tp[i >> 2][i & 3];
+                                } else {
+#pragma unroll
+                                    for (int i = 0; i < 16; ++i) c[i] = 0.0f;
                                 }
                             }
-                            if constexpr (RES != RES_NONE) dm = small ? 0u : dm;
-                            // (NaN: `bad` is set)
-                            if (__ballot(bad | (kHalf & !(most <= half_a)) | (nearest <= (int)(0x80000000u | __float_as_uint(two_e)))) != 0) {
-                                const bool wide = kHalf & !(most <= half_a);  // this lane's sums with the full bound
-                                const float shift = wide ? wide_shift : 0.0f, two = wide ? wide_two_e : two_e;
-                                uint32_t w2 = 0u, r = 0u;
-                                w = 0u;
-#pragma unroll
-                                for (int i = 0; i < 16; ++i) {
-                                    float a = acc[m][i];
-                                    asm volatile("" : "+v"(a));  // (evaluated again here: not kept from above)
-                                    a += shift;
-                                    const float d = a - tp[i >> 2][i & 3];
-                                    w = __builtin_amdgcn_alignbit(w, __float_as_uint(d), 31);
-                                    w2 = __builtin_amdgcn_alignbit(w2, __float_as_uint(d + two), 31);
-                                    if constexpr (RES != RES_NONE) r = __builtin_amdgcn_alignbit(r, __float_as_uint(__builtin_amdgcn_fractf(-a) - two), 31);
-                                }
-                                w = bad ? 0xffffu : w;
-                                dm = bad ? 0xffffu : (w & ~w2) | (wide || !small ? r : 0u);
-                            }
-                            doubt |= (valid ? dm & 0xffffu : 0u) << (16 * (POOL > 1 ? py : m));
-                            word[m] |= ~w & 0xffffu;  // (a bit in doubt is 0 here: the recomputation only ever sets it)
-                            if constexpr (RES != RES_NONE) {
-                                int v[16];
-#pragma unroll
-                                for (int i = 0; i < 16; ++i) v[i] = (int)acc[m][i];
-                                const unsigned item = (unsigned)(oy * p.PW + x0 + g * NX) * pixel_b + (unsigned)((tile0 + m) * 2) * group_b;
-                                store_residual_group<RES>(res_rsrc, p.res_fmt, valid ? place_res + item : kOutOfRange,
-                                                          RES == RES_12 ? (valid ? place_res8 + item : kOutOfRange) : 0u, uB * 16u, v);
-                                __builtin_amdgcn_sched_barrier(0);  // (one tile at a time: registers)
-                            }
+                            acc[d][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a[m]), __builtin_bit_cast(h8, lo), c, 0, 0, 0);
                         }
+#pragma unroll
+                        for (int m = 0; m < MT; ++m)
+                            acc[d][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a[m]), __builtin_bit_cast(h8, hi), acc[d][m], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                 }
-                if constexpr (kOrdered) ordered_sums(oy, g, word, doubt);
-                // ---- output words: two tiles: lane half h stores the word of tile h; one tile: half 0 stores
+                ++block;
+                if (done < cy) continue;  // the first rows' sums are not complete
+                // (An input outside the fp16 range has an infinity in hi and another in lo: no sum of its window is a number then,
+                // and none of a window whose rows only met zero weights with it.)
+                bad |= acc[D - 1][0][0] != acc[D - 1][0][0];
+                // ---- bits (MSB first; the sign of S - E - bn, inverted), residual, doubtful values
                 asm volatile("" : "+v"(ln));
-                const int h = ln >> 5, img = ln & (NI - 1), xc = x0 + g * NX + ((ln & 31) >> q.ni_log2);
-                const auto sw = __builtin_amdgcn_permlane32_swap(word[0], word[MT - 1], false, false);
-                uint32_t full = (sw[0] << 16) | sw[1];
-                if constexpr (POOL > 1) full |= (uint32_t)__shfl_xor((int)full, NI);  // the window's other column
-                const unsigned item_word = ((unsigned)(oy * p.OW + (x0 + g * NX) / POOL) * (unsigned)p.ow + (unsigned)tile0) * uB * 4u;
-                __builtin_amdgcn_raw_buffer_store_b32(full, out_rsrc, (int)(xc < xcols ? place_word + item_word : kOutOfRange), 0, 0);
-                // ---- doubtful values of this item go on the list, one per lane at a time.  Recomputed are those of earlier
-                // items (their stores are older than this item's, so nothing of this item is waited for), four at a time, and
-                // all that are there where the list is full and after the wave's last item.
-                const bool last = !more && g + wg_step >= n_groups;
-                if (count >= 4) {
-                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RES != RES_NONE ? 2 * MT + 1 : 1) : "memory");
-                    recompute();
+                const int h = ln >> 5;
+                const bool valid = b0 + (ln & (NI - 1)) < p.B && g * NX + ((ln & 31) >> q.ni_log2) < xcols;
+                if constexpr (kFromThreshold) {
+                    // the sums are S - bn: their signs are the bits, and those within E of 0 are in doubt (rare: the nearest tells)
+                    float nearest[MT];
+                    uint32_t bits[MT];
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) {
+                        uint32_t w = 0u;
+                        nearest[m] = INFINITY;
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) {
+                            w = __builtin_amdgcn_alignbit(w, __float_as_uint(acc[D - 1][m][i]), 31);
+                            nearest[m] = __builtin_fminf(nearest[m], __builtin_fabsf(acc[D - 1][m][i]));
+                        }
+                        bits[m] = ~w & 0xffffu;
+                    }
+                    const float least = __builtin_fminf(nearest[0], nearest[1]);
+                    if (__ballot(bad | !(least > two_e)) != 0) {  // uniform
+#pragma unroll
+                        for (int m = 0; m < MT; ++m) {
+                            uint32_t dm = 0u;
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) dm = __builtin_amdgcn_alignbit(dm, __builtin_fabsf(acc[D - 1][m][i]) > two_e ? 0u : 0x80000000u, 31);
+                            dm = bad ? 0xffffu : (two_e == 0.0f ? 0u : dm & 0xffffu);
+                            undecided |= (valid ? dm : 0u) << (16 * m);
+                            bits[m] &= ~dm;  // (a bit in doubt is 0 here: the recomputation only ever sets it)
+                        }
+                    }
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) word[m] |= bits[m];
+                } else {
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) {
+                        const v4f* const tp = reinterpret_cast<const v4f*>(thr + m * 32 + 16 * h);
+                        // Signs are collected MSB first (bit 15 - i: channel i).  w: S - E < bn, dm: values in doubt.  Integers
+                        // within E are common (in every other tile) and collected like the bits; thresholds within E are
+                        // rare: the tile's nearest distance below a threshold tells whether to look for them.
+                        uint32_t w = 0u, dm = 0u;
+                        int nearest = INT32_MAX;
+                        {
+                            const v4f th[4] = {tp[0], tp[1], tp[2], tp[3]};
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) {
+                                const float d = acc[D - 1][m][i] - th[i >> 2][i & 3];
+                                w = __builtin_amdgcn_alignbit(w, __float_as_uint(d), 31);
+                                nearest = min(nearest, __float_as_int(d));
+                                dm = __builtin_amdgcn_alignbit(dm, __float_as_uint(__builtin_amdgcn_fractf(-acc[D - 1][m][i]) - two_e), 31);
+                            }
+                        }
+                        dm = small ? 0u : dm;
+                        // (NaN: `bad` is set)
+                        if (__ballot(bad | (nearest <= (int)(0x80000000u | __float_as_uint(two_e)))) != 0) {
+                            uint32_t w2 = 0u;
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) {
+                                float a = acc[D - 1][m][i];
+                                asm volatile("" : "+v"(a));  // (evaluated again here: not kept from above)
+                                const float d = a - tp[i >> 2][i & 3];
+                                w2 = __builtin_amdgcn_alignbit(w2, __float_as_uint(d + two_e), 31);
+                            }
+                            dm = bad ? 0xffffu : (w & ~w2) | dm;
+                            w = bad ? 0xffffu : w;
+                        }
+                        undecided |= (valid ? dm & 0xffffu : 0u) << (16 * m);
+                        word[m] |= ~w & 0xffffu;  // (a bit in doubt is 0 here: the recomputation only ever sets it)
+                        int v[16];
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) v[i] = (int)acc[D - 1][m][i];
+                        const unsigned item = (unsigned)(done * p.PW + g * NX) * pixel_b + (unsigned)((tile0 + m) * 2) * group_b;
+                        store_residual_group<RES>(res_rsrc, p.res_fmt, valid ? place_residual(ln) + item : kOutOfRange,
+                                                  RES == RES_12 ? (valid ? place_residual8(ln) + item : kOutOfRange) : 0u, uB * 16u, v);
+                        __builtin_amdgcn_sched_barrier(0);  // (one tile at a time: registers)
+                    }
                 }
-                unsigned long long who = __ballot(doubt != 0u);
-                const int earlier = count;
-                if (!kOrdered && RES != RES_NONE && who != 0) {  // uniform
-                    many = __builtin_popcountll(who) >= kManyLanes || __ballot(__builtin_popcount(doubt) >= kManyInLane) != 0;
-                    if (many) who = 0;  // (what is stored of this item is stored again)
+            } else {
+                undecided = ordered_sums(cy, word);
+            }
+            const bool last = cy + 1 == cy_end;
+            if (POOL > 1 && (cy & 1) == 0) {
+                doubt[0] = undecided;
+                ++cy;
+                continue;
+            }
+            doubt[POOL - 1] = undecided;
+            // ---- output words: two tiles: lane half h stores the word of tile h; one tile: half 0 stores
+            asm volatile("" : "+v"(ln));
+            const int h = ln >> 5, img = ln & (NI - 1), xc = g * NX + ((ln & 31) >> q.ni_log2);
+            const auto sw = __builtin_amdgcn_permlane32_swap(word[0], word[MT - 1], false, false);
+            uint32_t full = (sw[0] << 16) | sw[1];
+            if constexpr (POOL > 1) full |= (uint32_t)__shfl_xor((int)full, NI);  // the window's other column
+            const unsigned item_word = ((unsigned)(cy / POOL * p.OW + g * NX / POOL) * (unsigned)p.ow + (unsigned)tile0) * uB * 4u;
+            __builtin_amdgcn_raw_buffer_store_b32(full, out_rsrc, (int)(xc < xcols ? (kFromThreshold ? word_place : place_word(ln)) + item_word : kOutOfRange), 0, 0);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) word[m] = 0u;
+            // ---- doubtful values of this item go on the list, one per lane at a time.  Recomputed are those of earlier
+            // items (their stores are older than this item's, so nothing of this item is waited for), sixteen at a time, and
+            // all that are there where the list is full and after the wave's last item.
+            const uint32_t any = doubt[0] | doubt[POOL - 1];
+            const unsigned long long lanes = __ballot(any != 0u);
+            if (!kOrdered && lanes != 0) {  // uniform
+                if (__builtin_popcountll(lanes) >= (check ? kManyLanesChecked : kManyLanes) ||
+                    __ballot(__builtin_popcount(doubt[0]) >= kManyInLane || (POOL > 1 && __builtin_popcount(doubt[POOL - 1]) >= kManyInLane)) != 0) {
+                    cy -= POOL - 1;  // (what is stored of this item is stored again)
+                    return;
                 }
-                if (!kOrdered && kRowExit && many) who = 0;
+            }
+            bool go = count >= kBatch;
+            if (go) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RES != RES_NONE ? 2 * MT + 1 : 1) : "memory");
+            if (go || lanes != 0 || last) {
                 for (;;) {
-                    int c;
-                    while ((c = __builtin_amdgcn_readfirstlane(__popcll(who))) != 0 && count + c <= kListCap) {
-                        if (doubt != 0u) {
-                            const int bit = __ffs(doubt) - 1;
-                            doubt &= doubt - 1u;
-                            const int at = count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0u));
-                            const int py = POOL > 1 ? bit >> 4 : 0, m = POOL > 1 ? 0 : bit >> 4;
-                            list[2 * at] = (uint32_t)(oy * POOL + py) << 16 | (uint32_t)xc;
-                            list[2 * at + 1] = (uint32_t)((tile0 + m) * 32 + 16 * h + 15 - (bit & 15)) | (uint32_t)img << 16;
+                    if (go) recompute();
+                    bool full_list = false;
+#pragma unroll
+                    for (int py = 0; py < POOL; ++py) {
+                        unsigned long long who = __ballot(doubt[py] != 0u);
+                        int c;
+                        while ((c = __builtin_amdgcn_readfirstlane(__popcll(who))) != 0 && count + c <= kListCap) {
+                            if (doubt[py] != 0u) {
+                                const int bit = __ffs(doubt[py]) - 1;
+                                doubt[py] &= doubt[py] - 1u;
+                                const int at = count + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0u));
+                                list[2 * at] = (uint32_t)(cy - (POOL - 1) + py) << 16 | (uint32_t)xc;
+                                list[2 * at + 1] = (uint32_t)((tile0 + (bit >> 4)) * 32 + 16 * h + 15 - (bit & 15)) | (uint32_t)img << 16;
+                            }
+                            count += c;
+                            who = __ballot(doubt[py] != 0u);
                         }
-                        count += c;
-                        who = __ballot(doubt != 0u);
+                        full_list |= c != 0;
                     }
-                    if (c == 0 && (!last || count == 0 || (!kShared && many))) break;
-                    if (!kOrdered && RES == RES_NONE && c != 0) {  // the list is full
-                        many = true;
-                        if constexpr (kRowExit) {
-                            first_g = g;
-                            count = earlier;
-                            break;
-                        }
-                    }
+                    if (!full_list && (!last || count == 0)) break;
                     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    do recompute();
-                    while (count > kListCap / 2);
+                    go = true;
                 }
-                if (RES != RES_NONE && many) return;
-                g += wg_step;
             }
-            if (kRowExit && many) {
-                g = first_g;
-                return;
-            }
-            g = wg0;
-            if constexpr (kShared && !kOrdered) {
-                __syncthreads();
-                if (many && lane == 0) flags[1] = 1;
-            }
-            if (!kOrdered && more) split_and_store(std::bool_constant<kMarked>{}, q.adv, s0);
-            ay0 += q.adv;
-            s0 += q.adv;
-            s0 = s0 >= q.ring ? s0 - q.ring : s0;
+            ++cy;
         }
     };
-    pass(std::integral_constant<Mode, COMMON>{});
-    if (!kShared && oy < oy_end) {
-        stage_window(std::true_type{});
-        pass(std::integral_constant<Mode, MARKED>{});
+    for (;;) {
+        pass(std::false_type{});
+        if (cy >= cy_end) return;
+        if (check) break;
+        check = keep_checking = true;
     }
-    if (oy < oy_end) pass(std::integral_constant<Mode, ORDERED>{});
+    pass(std::true_type{});
 }
 
 // ---------------------------------------------------------------- host side
-constexpr int kMaxDevices = 64;
-constexpr int kLdsPerCu = 160 * 1024;
-
 struct Choice {
-    int r, nq, mt, pool;
-    int res, pairs;
-    int wg_per_cu;
+    int r, t, a, pool, res;
     Geometry q;
     size_t lds_bytes;
     int grid;
     long long out_bytes, res_bytes;
 };
 
-size_t lds_extra(int channels) { return (size_t)(channels + 4 * 2 * kListCap + 4) * 4; }
-
 // The instantiation for a problem's form, if there is one: what the networks' first layers need.  (For other forms, 5x5
-// filters, pooled 3x3, 32-channel or odd-stride 7x7 layers, there is none and nothing has been measured: the kernels of
-// inconv.hip serve them.)
-bool instantiated(const InConvParams& p, Choice* out) {
+// filters, pooled 3x3, 32-channel 7x7 layers, other strides, there is none and nothing has been measured: the kernels of
+// inconv.hip serve them.)  Filters narrower than the instantiation's row are served tap by tap.
+bool instantiated(const InConvParams& p, int cus, Choice* out) {
     Choice& c = *out;
     c.r = p.R;
-    c.nq = (p.S + 3) / 4;
+    c.a = p.stride_h;
     c.res = p.res == nullptr ? RES_NONE : (p.res_fmt == TCBNN_RES_I12 ? RES_12 : RES_WIDE);
-    c.pairs = p.stride_w % 4 == 0 ? PAIRS_SPLIT : (p.stride_w % 2 == 0 ? PAIRS_EVEN : PAIRS_ANY);
     const bool pooled = p.pool_h != 1 || p.pool_w != 1;
-    if (p.R == 3 && c.nq == 1 && !pooled && p.O % 64 == 0 && c.pairs != PAIRS_SPLIT) {
-        c.mt = 2, c.pool = 1;
-    } else if (p.R == 7 && c.nq == 2 && !pooled && p.O % 64 == 0 && c.pairs != PAIRS_ANY) {
-        c.mt = 2, c.pool = 1;
-    } else if (p.R == 11 && c.nq == 3 && p.pool_h == 2 && p.pool_w == 2 && p.O % 32 == 0 && c.pairs == PAIRS_SPLIT) {
-        c.mt = 1, c.pool = 2;
+    if (p.O % 64 != 0) return false;
+    if (p.R == 3 && p.S <= 4 && !pooled && (c.a == 1 || (c.a == 2 && p.S <= 3))) {
+        c.t = p.S <= 3 ? 3 : 4, c.pool = 1;
+    } else if (p.R == 7 && p.S <= 7 && !pooled && (c.a == 4 || c.a == 2)) {
+        c.t = 7, c.pool = 1;
+    } else if (p.R == 11 && p.S <= 11 && p.pool_h == 2 && p.pool_w == 2 && c.res == RES_NONE && c.a == 4) {
+        // Thirteen tiles of a row per compute unit or more: below that, and for 32 channels, the ring in LDS is faster
+        // (inconv_mfma_ring.hip has both sides' times).
+        if (4LL * p.OH * p.OW * p.B * (p.O / 64) < 13LL * 32 * cus) return false;
+        c.t = 11, c.pool = 2;
     } else {
         return false;
     }
@@ -885,106 +942,72 @@ bool instantiated(const InConvParams& p, Choice* out) {
 // How a launch is split; false for sizes that the kernel does not take.  `cus`: compute units.
 bool choose(const InConvParams& p, int cus, Choice* out) {
     Choice c{};
-    if (!instantiated(p, &c)) return false;
-    c.wg_per_cu = workgroups_per_cu(c.r);
+    if (!instantiated(p, cus, &c)) return false;
     Geometry& q = c.q;
-    q.adv = c.pool * p.stride_h;
-    q.ring = p.R + (c.pool - 1) * p.stride_h;
-    if (q.adv > q.ring) return false;
     if (p.PH > 32767 || p.PW > 32767 || p.O > 65535) return false;
     // (32-bit buffer offsets)
     c.out_bytes = 4LL * p.OH * p.OW * p.ow * p.B;
     c.res_bytes = p.res != nullptr ? (long long)tcbnn_residual_bytes(p.PH, p.PW, p.O, p.B, p.res_fmt) : 0;
     if (c.out_bytes >= (1LL << 31) || c.res_bytes >= (1LL << 31)) return false;
-    q.rows = p.OH;
     q.rs_taps = p.R * p.S;
-    const bool shared = ring_shared(c.r);
-    const int teams = shared ? 1 : 4;  // per workgroup
-    const int chp = p.O / (32 * c.mt);
-    q.waves_c = !shared ? 1 : (chp % 4 == 0 ? 4 : (chp % 2 == 0 ? 2 : 1));
-    q.cgroups = chp / q.waves_c;
-    const size_t extra = lds_extra(p.O), share = (size_t)kLdsPerCu / c.wg_per_cu;
-    if (extra >= share) return false;
-    const size_t lds_limit = (share - extra) / teams;
     q.s_magic = 65536u / (unsigned)p.S + 1u;
     for (int t = 0; t < q.rs_taps; ++t)
         if ((int)((unsigned)t * q.s_magic >> 16) != t / p.S) return false;
+    const int waves = waves_of(c.r), xcols = c.pool > 1 ? c.pool * p.OW : p.PW, sets = sets_of(c.r, c.a), steps = sets * steps_of(c.a, c.t);
+    q.cgroups = p.O / (32 * MT);
+    q.rows = c.pool * p.OH;
 
-    // Images per 32-column tile and columns per strip: the cheapest over the batch and the width, in rough cycles of a
-    // wave: items (multiplication and epilogue) and staging rounds.  At most eight images (eight images' residuals of a
-    // pixel are a whole 128-byte line; more would leave no room for a strip), fewer than that only where it is worth an
-    // eighth; a pooled layer needs neighbouring pixels in one tile and stores little.
-    const int xcols = c.pool > 1 ? c.pool * p.OW : p.PW;
-    const int item = p.R == 3 ? 900 : (p.R == 7 ? 2300 : 3200) * c.pool;
+    // Images per 32-column tile
     double best = 1e30;
-    int most_images = 3;
-    while (most_images > 0 && (1 << (most_images - 1)) >= p.B) --most_images;
-    for (int ni_log2 = most_images; ni_log2 >= std::max(0, most_images - 2); --ni_log2) {
-        const int NI = 1 << ni_log2, NX = 32 >> ni_log2, step = std::max(NX, c.pool), imgtiles = (p.B + NI - 1) >> ni_log2;
+    int imgtiles = 0;
+    const long long target = std::max(1LL, (long long)cus * 4 * waves_per_simd(c.r, c.a) / q.cgroups);  // resident waves
+    const int most = c.res == RES_NONE && c.pool == 1 && (long long)p.B * xcols * q.rows / 32 >= 32 * target ? 4 : 3;
+    for (int ni_log2 = most; ni_log2 >= 0; --ni_log2) {
+        const int NI = 1 << ni_log2, NX = 32 >> ni_log2;
         if ((long long)NI * 3 * p.H * p.W * 4 >= (1LL << 31)) continue;
-        for (int xo = step; xo < xcols + step; xo += step) {
-            const int np = ((xo - 1) * p.stride_w + 4 * c.nq + 1) / 2, odd = (np + 1) / 2;
-            const int pp = c.pairs == PAIRS_SPLIT ? 2 * odd + (odd % 2 == 0 ? 2 : 0) : np | 1;
-            const int per_round = shared ? 256 : 64, units = (np * NI * q.adv + per_round - 1) / per_round;
-            const size_t bytes = (size_t)2 * q.ring * NI * pp * 16;
-            if (units > rounds_of(p.R) || bytes > lds_limit || NI * pp > 0xffff) break;
-            const int groups = xo / NX, strips = (xcols + xo - 1) / xo;
-            const int rounds = shared ? (groups * q.waves_c + 3) / 4 : groups;
-            const double cost = (double)imgtiles * strips * (rounds * (double)item + 200.0 * units + (shared ? 500.0 : 100.0)) *
-                                (ni_log2 < most_images && c.pool == 1 ? 1.125 : 1.0);
-            if (cost < best * 0.999) {
-                best = cost;
-                q.ni_log2 = ni_log2;
-                q.imgtiles = imgtiles;
-                q.xo = xo;
-                q.np = np;
-                q.pp = pp;
-                q.odd_pairs = odd;
-                q.rounds = units;
-                q.strips = strips;
-            }
+        const int tiles = (p.B + NI - 1) >> ni_log2, groups = (xcols + NX - 1) / NX;
+        const double cost = (double)tiles * groups * (ni_log2 == most ? 1.0 : 1.06);
+        if (cost < best) {
+            best = cost;
+            q.ni_log2 = ni_log2;
+            q.groups = groups;
+            imgtiles = tiles;
         }
     }
     if (best >= 1e30) return false;
-    c.lds_bytes = (size_t)2 * q.ring * ((size_t)q.pp << q.ni_log2) * 16 * teams + extra;
+    c.lds_bytes = (size_t)steps * MT * 1024 + MT * 128 + (size_t)waves * kListCap * 8 + (size_t)c.r * c.t * MT * 32;
 
-    // Bands of rows: one round of resident workgroups where the width and the batch leave a choice; a band's first
-    // window is staged whole (counted as 0.7 of a row's work).
-    const long long per = (long long)q.imgtiles * q.cgroups * q.strips, target = (long long)cus * c.wg_per_cu * teams;
+    // Bands of rows: whole rounds of resident waves; a band begins with sets - 1 steps whose rows are only read (0.6 of one)
+    const long long per = (long long)imgtiles * q.groups;
     double best_t = 1e30;
-    for (int bands = 1; bands <= q.rows; ++bands) {
-        const int br = (q.rows + bands - 1) / bands;
-        if ((q.rows + br - 1) / br != bands) continue;
-        const double t = (double)((per * bands + target - 1) / target) * (br + 0.7);
+    for (int bands = 1; bands <= p.OH; ++bands) {
+        const int br = (p.OH + bands - 1) / bands;
+        if ((p.OH + br - 1) / br != bands) continue;
+        const double t = (double)((per * bands + target - 1) / target) * (br * c.pool + 0.6 * (sets - 1) + 0.5);
         if (t < best_t * 0.999) {
             best_t = t;
             q.bands = bands;
-            q.band_rows = br;
+            q.band_rows = br * c.pool;
         }
     }
     const long long total = per * q.bands;
-    if (total > 0x0fffffffLL) return false;
+    if (total * q.cgroups > 0x0fffffffLL) return false;
     q.total = (int)total;
-    q.per_xcd = (q.total + 7) / 8;  // (teams)
-    c.grid = 8 * ((q.per_xcd + teams - 1) / teams);
-    // E (see the top of this file): the roundings of sums, T of the reference's and 2 per hi step and for -E (2.25 taken:
-    // what the halves lose) with partial sums below (A + |S|) / 2 <= 0.75 A (or A); 2 u A for the additions in a tap, 2 u A for the split, and
-    // 0.5 u A for the lo steps.  2 % cover the roundings of the bound itself.
-    const double T = q.rs_taps, u = std::ldexp(1.0, -24), sums = T + 2.25 * (p.R * c.nq + 1), a_scale = std::sqrt(3.0 * T);
-    q.bound_scale = (float)(((bound_for_half(p.R) ? 0.75 : 1.0) * sums + 4.5) * u * 1.02 * a_scale);
-    q.bound_scale_full = (float)((sums + 4.5) * u * 1.02 * a_scale);
-    q.half_scale = (float)(0.49 * a_scale);
+    q.per_xcd = (q.total + 7) / 8;
+    c.grid = 8 * ((q.per_xcd + waves - 1) / waves) * q.cgroups;
+    // E (see the top of this file)
+    const double T = q.rs_taps, u = std::ldexp(1.0, -24) * 1.02;
+    q.bound_parts = (float)u;
+    q.bound_sum = (float)((13.5 + (c.t == 7 && c.res != RES_NONE ? 0.0 : T + 4.0 * steps)) * u);
     q.bound_add = (float)(3.0 * T * std::ldexp(1.0, -24) + std::ldexp(1.0, -22));
-    q.small_squares = (float)(0.2 / (3.0 * T));
-    q.exact_squares = (float)(60000.0 * 60000.0 / (3.0 * T));  // (sum of |x| below 2^16 = 2^24 / 256)
     *out = c;
     return true;
 }
 
 int device_info(int* dev, int* cus) {
-    static std::atomic<int> cu_count[kMaxDevices];
+    static std::atomic<int> cu_count[kInConvDevices];
     if (int rc = check_hip(hipGetDevice(dev), "hipGetDevice")) return rc;
-    if (*dev < 0 || *dev >= kMaxDevices) return fail(TCBNN_EUNSUPPORTED, "inconv: device ordinal %d", *dev);
+    if (*dev < 0 || *dev >= kInConvDevices) return fail(TCBNN_EUNSUPPORTED, "inconv: device ordinal %d", *dev);
     int n = cu_count[*dev].load(std::memory_order_acquire);
     if (n == 0) {
         if (int rc = check_hip(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, *dev),
@@ -997,18 +1020,19 @@ int device_info(int* dev, int* cus) {
     return TCBNN_OK;
 }
 
-template <int R, int NQ, int MT, int RES, int POOL, int PAIRS>
+template <int R, int T, int A, int RES, int POOL>
 int launch(const InConvParams& p, const Choice& c, int dev, hipStream_t stream) {
-    static std::atomic<bool> ready[kMaxDevices];  // (setting the limit twice does no harm)
-    if (!ready[dev].load(std::memory_order_acquire)) {
-        const void* fn = reinterpret_cast<const void*>(&inconv_mfma_kernel<R, NQ, MT, RES, POOL, PAIRS>);
-        if (int rc = check_hip(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu / workgroups_per_cu(R)),
-                               "hipFuncSetAttribute(MaxDynamicSharedMemorySize)"))
-            return rc;
-        ready[dev].store(true, std::memory_order_release);
+    if (c.lds_bytes > 64 * 1024) {
+        static std::atomic<bool> ready[kInConvDevices];  // (setting the limit twice does no harm)
+        if (!ready[dev].load(std::memory_order_acquire)) {
+            const void* fn = reinterpret_cast<const void*>(&inconv_mfma_kernel<R, T, A, RES, POOL>);
+            if (int rc = check_hip(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.lds_bytes), "hipFuncSetAttribute(MaxDynamicSharedMemorySize)"))
+                return rc;
+            ready[dev].store(true, std::memory_order_release);
+        }
     }
     const uint32_t* pats = reinterpret_cast<const uint32_t*>(p.masks) + (size_t)p.R * p.S * p.opad * 4;
-    hipLaunchKernelGGL((inconv_mfma_kernel<R, NQ, MT, RES, POOL, PAIRS>), dim3((unsigned)c.grid), dim3(kThreads),
+    hipLaunchKernelGGL((inconv_mfma_kernel<R, T, A, RES, POOL>), dim3((unsigned)c.grid), dim3(64 * waves_of(R)),
                        c.lds_bytes, stream, KernelArgs{p, c.q, pats, (unsigned)c.out_bytes, (unsigned)c.res_bytes});
     TCBNN_LAUNCH_CHECK("inconv_mfma_kernel");
     return TCBNN_OK;
@@ -1018,29 +1042,31 @@ int launch(const InConvParams& p, const Choice& c, int dev, hipStream_t stream) 
 
 bool inconv_mfma_kernel_name(const InConvParams& p, char* buf, size_t len) {
     Choice c;
-    if (!choose(p, 256, &c)) return false;
-    snprintf(buf, len, "inconv_mfma_kernel<%d, %d, %d, %d, %d, %d>", c.r, c.nq, c.mt, c.res, c.pool, c.pairs);
+    if (!choose(p, 256, &c)) {
+        if (!inconv_mfma_ring_serves(p)) return false;
+        snprintf(buf, len, "inconv_mfma_ring_kernel");
+        return true;
+    }
+    snprintf(buf, len, "inconv_mfma_kernel<%d, %d, %d, %d, %d>", c.r, c.t, c.a, c.res, c.pool);
     return true;
 }
 
 int launch_inconv_mfma(const InConvParams& p, hipStream_t stream, bool* served) {
     Choice c{};
-    *served = instantiated(p, &c);
+    *served = p.O % 32 == 0 && (p.R == 3 || p.R == 7 || p.R == 11);
     if (!*served) return TCBNN_OK;
     int dev = 0, cus = 0;
     if (int rc = device_info(&dev, &cus)) return rc;
-    *served = choose(p, cus, &c);
-    if (!*served) return TCBNN_OK;
+    if (!choose(p, cus, &c)) return launch_inconv_mfma_ring(p, dev, cus, stream, served);
     auto with_residual = [&](auto go) { return c.res == RES_12 ? go(std::integral_constant<int, RES_12>{}) : (c.res == RES_WIDE ? go(std::integral_constant<int, RES_WIDE>{}) : go(std::integral_constant<int, RES_NONE>{})); };
     if (c.r == 3)
         return with_residual([&](auto res) {
-            return c.pairs == PAIRS_EVEN ? launch<3, 1, 2, decltype(res)::value, 1, PAIRS_EVEN>(p, c, dev, stream) : launch<3, 1, 2, decltype(res)::value, 1, PAIRS_ANY>(p, c, dev, stream);
+            return c.t == 4 ? launch<3, 4, 1, decltype(res)::value, 1>(p, c, dev, stream)
+                            : (c.a == 1 ? launch<3, 3, 1, decltype(res)::value, 1>(p, c, dev, stream) : launch<3, 3, 2, decltype(res)::value, 1>(p, c, dev, stream));
         });
     if (c.r == 7)
-        return with_residual([&](auto res) {
-            return c.pairs == PAIRS_SPLIT ? launch<7, 2, 2, decltype(res)::value, 1, PAIRS_SPLIT>(p, c, dev, stream) : launch<7, 2, 2, decltype(res)::value, 1, PAIRS_EVEN>(p, c, dev, stream);
-        });
-    return launch<11, 3, 1, RES_NONE, 2, PAIRS_SPLIT>(p, c, dev, stream);
+        return with_residual([&](auto res) { return c.a == 4 ? launch<7, 7, 4, decltype(res)::value, 1>(p, c, dev, stream) : launch<7, 7, 2, decltype(res)::value, 1>(p, c, dev, stream); });
+    return launch<11, 11, 4, RES_NONE, 2>(p, c, dev, stream);
 }
 
 }  // namespace tcbnn

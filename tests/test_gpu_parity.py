@@ -1055,6 +1055,56 @@ def test_inconv128_thresholds_at_the_ordered_sums(gpu, b, h, R, stride, pool, ki
     layer.release()
 
 
+@pytest.mark.parametrize("b,h,w,R,stride,cout,pool,save,kind", [
+    # frames narrower than the filter, one row, columns of tiles that end inside the frame, bands of single rows
+    (1, 5, 3, 7, 4, 64, 1, True, "normal"), (600, 60, 5, 11, 4, 512, 2, False, "normal"), (3, 1, 40, 3, 1, 64, 1, True, "normal"),
+    (10, 13, 67, 7, 2, 64, 1, False, "normal"), (300, 9, 7, 3, 1, 128, 1, True, "normal"),
+    # enough rows per wave for sixteen images to a tile, the last tile incomplete
+    (63, 224, 224, 3, 1, 64, 1, False, "normal"),
+    # inputs at and beyond the end of fp16 in rows that neighbouring windows multiply by zeros
+    (17, 23, 29, 7, 2, 128, 1, True, "overflow"), (9, 33, 30, 7, 4, 64, 1, True, "overflow"),
+    (70, 61, 57, 11, 4, 512, 2, False, "overflow"), (9, 20, 20, 3, 2, 64, 1, True, "overflow"),
+    # multiples of 1/256: too large for two fp16 halves; with thresholds that are multiples too, and some that are not
+    (8, 24, 24, 7, 4, 64, 1, True, "large_grid"), (16, 21, 20, 3, 2, 64, 1, False, "grid"), (16, 21, 20, 3, 1, 64, 1, False, "grid"),
+    (70, 60, 60, 11, 4, 512, 2, False, "grid"), (16, 21, 20, 3, 1, 64, 1, False, "near_grid"),
+    # sums on their thresholds all over the frame
+    (70, 61, 57, 11, 4, 512, 2, False, "flat")])
+def test_inconv128_rows_in_flight(gpu, b, h, w, R, stride, cout, pool, save, kind):
+    """First-layer sums of several output rows under way at once: the edges of tiles, bands and of what makes a sum exact."""
+    r = rng(9000 + b + h + w + R)
+    x = r.standard_normal((b, 3, h, w)).astype(np.float32)
+    f = rm.pm1(r, (R, R, 3, cout))
+    bn = r.normal(0, np.sqrt(3 * R * R), cout).astype(np.float32)
+    if kind == "overflow":
+        for i, v in enumerate([65504, 65519, 65520, -7e4, 3e38, np.inf, np.nan]):
+            x[i % b, i % 3, int(r.integers(h)), int(r.integers(w))] = v
+    elif kind == "large_grid":
+        x = np.rint(x * 256).astype(np.float32) / 256
+        x[r.random(x.shape) < 0.01] = np.float32(50000 + 1 / 256)
+    elif kind in ("grid", "near_grid"):
+        x = np.rint(x).astype(np.float32)
+        bn = np.rint(bn).astype(np.float32)
+        bn[:3] = [0.0, -0.0, np.inf]
+        if kind == "near_grid":
+            bn[3::2] = np.nextafter(bn[3::2], np.float32(100))
+    elif kind == "flat":
+        x[:, :, :, : w // 2] = np.float32(0.1)
+        bn[:] = 0.0
+        for a, c, d in f.reshape(R * R, 3, cout) * np.float32(0.1):
+            bn += (a + c) + d
+    with np.errstate(all="ignore"):
+        want, wres = orc.inconv128(x, f, bn, stride, True, pool, save)
+    layer = gpu.InConv128LayerParam("Conv1", h, w, R, R, 3, cout, b, stride, stride, True, pool, pool, save)
+    layer.initialize(x, gpu.ArrayWeights([f, bn]))
+    assert "inconv_mfma_kernel" in layer.kernel_name(), layer.kernel_name()
+    layer.forward()
+    gpuops.sync()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    if save:
+        np.testing.assert_array_equal(layer.download_residual(), wres)
+    layer.release()
+
+
 def test_inconv128_special_thresholds(gpu):
     """NaN, +-inf and exactly met thresholds in the first layer (kernel.cuh:655: bit = !(acc < bn))."""
     r = rng(321)
