@@ -231,6 +231,13 @@ typedef struct tcbnn_out128_desc {
 } tcbnn_out128_desc;
 int tcbnn_out128_forward(const tcbnn_out128_desc* d, void* stream);
 
+/* In128 (or NULL), n_fc Fc128 layers and Out128 (or NULL), one after the other: the same results, in every layer's
+ * output, as the calls above in this order.  Layers that follow one another (each reads the output of the one before,
+ * same batch, at most 2048 inputs and outputs, the FP4 engine) go in one launch.  Allocates nothing and needs no
+ * workspace.  No counterpart in the reference (its network kernel runs all layers, kernel.cuh:153-280). */
+int tcbnn_fc_chain_forward(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out,
+                           void* stream);
+
 /* InConv128LayerFMT (kernel.cuh:578-672), fields of InConv128LayerParam
  * (param.h:841-869).  fp32 NCHW 3-channel input, +-1 filters, fp32 adds in the
  * reference order  acc += ((+-f0) + (+-f1)) + (+-f2)  per in-frame tap in (r,s)

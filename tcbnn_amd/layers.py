@@ -279,8 +279,11 @@ class In128LayerParam(_ReferenceLayoutIO):
     def get_output_gpu(self):
         return self.output_gpu
 
+    def _desc(self):
+        return _lib.In128Desc(self.input_gpu.ptr, self.output_gpu.ptr, self.input_height, self.input_width)
+
     def forward(self, stream=None):
-        d = _lib.In128Desc(self.input_gpu.ptr, self.output_gpu.ptr, self.input_height, self.input_width)
+        d = self._desc()
         check(lib.tcbnn_in128_forward(C.byref(d), _stream_handle(stream)))
 
     def download_packed(self):
@@ -461,6 +464,27 @@ class Out128LayerParam(_ReferenceLayoutIO):
             if b is not None:
                 b.free()
         self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = None
+
+
+def fc_run_end(layers, begin):
+    """Where the run of an In128 layer, Fc128 layers and an Out128 layer (all optional) at `begin` ends."""
+    end = begin
+    if type(layers[end]) is In128LayerParam:
+        end += 1
+    while end < len(layers) and type(layers[end]) is Fc128LayerParam:
+        end += 1
+    if end < len(layers) and type(layers[end]) is Out128LayerParam:
+        end += 1
+    return max(end, begin + 1)
+
+
+def forward_fc_run(layers, stream=None):
+    """forward() of the layers of such a run, one after the other, in as few launches as they allow."""
+    first, last = layers[0], layers[-1]
+    fc = [layer._desc() for layer in layers if type(layer) is Fc128LayerParam]
+    check(lib.tcbnn_fc_chain_forward(
+        C.byref(first._desc()) if type(first) is In128LayerParam else None, (_lib.Fc128Desc * len(fc))(*fc), len(fc),
+        C.byref(last._desc()) if type(last) is Out128LayerParam else None, _stream_handle(stream)))
 
 
 class _ConvGeometry(_ReferenceLayoutIO):

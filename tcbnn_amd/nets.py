@@ -11,7 +11,7 @@ import numpy as np
 
 from . import _lib
 from .layers import (ArrayWeights, AvgPoolFcLayerParam, Conv128LayerParam, Fc128LayerParam, In128LayerParam,
-                     InConv128LayerParam, Out128LayerParam, PAD128, Pool128LayerParam)
+                     InConv128LayerParam, Out128LayerParam, PAD128, Pool128LayerParam, fc_run_end, forward_fc_run)
 
 
 def _conv_out(h, r, s, padding=True, pool=1):
@@ -305,8 +305,14 @@ class Network:
         self.order[0].set_input(input)
 
     def forward(self, stream=None):
-        for layer in self.order:
-            layer.forward(stream)
+        order, i = self.order, 0
+        while i < len(order):
+            end = fc_run_end(order, i)
+            if end > i + 1:
+                forward_fc_run(order[i:end], stream)
+            else:
+                order[i].forward(stream)
+            i = end
 
     def logits(self):
         _lib.device_synchronize()

@@ -105,6 +105,49 @@ def test_out128(gpu, variant, b, k, n):
     np.testing.assert_array_equal(got, want)  # and in fact bit-identical
 
 
+@pytest.mark.parametrize("b,widths,with_in,with_out", [
+    # one image and neuron; ends of words, tiles and groups of K; a wave's second tiles and second round of tiles; activations
+    # of 2048 (two requests of weights ahead, 64 KB of LDS)
+    (1, (5, 3, 2), True, True), (33, (100, 33, 31, 10), True, True), (31, (1023, 544, 40), True, True),
+    (32, (1024, 512, 513, 96), True, True), (70, (257, 2048, 160, 1000), True, True), (64, (512, 2048, 129), True, True),
+    (257, (784, 1024, 1024, 1024, 10), True, True), (40, (2048, 96, 2048), False, True), (40, (300, 260, 64), True, False),
+    (9, (130, 70, 66), False, False),
+    # more layers than one launch takes; a layer that is too wide, or wide for so few images, between two that are not
+    (12, (64,) * 11 + (7,), True, True), (20, (96, 2080, 64, 64, 5), True, True), (20, (96, 2048, 1024, 64, 5), True, True)])
+def test_fc_chain(gpu, b, widths, with_in, with_out):
+    """A run of fully connected layers in one launch: every layer's output, thresholds met exactly and none."""
+    from tcbnn_amd.layers import forward_fc_run
+    r = rng(b + sum(widths))
+    x = r.standard_normal((b, widths[0])).astype(np.float32)
+    x[0, :3] = [0.0, -0.0, np.nan]
+    layers = [gpu.In128LayerParam("Fin", b, widths[0]).initialize(x)]
+    want = [orc.in128(x)]
+    for i, (k, n) in enumerate(zip(widths, widths[1:])):
+        w = rm.pm1(r, (k, n))
+        wl = orc.pack_fc_weight(w)
+        prev = layers[-1].get_output_gpu()
+        if with_out and i + 2 == len(widths):
+            scale, bias = r.normal(1, 0.1, n).astype(np.float32), r.normal(0, 1, n).astype(np.float32)
+            layers.append(gpu.Out128LayerParam("Fout", b, k, n).initialize(gpu.ArrayWeights([w, scale, bias]), prev))
+            want.append(orc.out128(want[-1], wl, scale, bias, k, n))
+            continue
+        bn = r.normal(0, np.sqrt(k), n).astype(np.float32)
+        _, acc = orc.fc128(want[-1], wl, bn, k, n, want_acc=True)
+        bn[: n // 2] = (k - 2 * acc)[b // 2, : n // 2]
+        bn[n // 2 : n // 2 + 5] = np.array([np.nan, np.inf, -np.inf, 3e38, -0.0], np.float32)[: n - n // 2]
+        layers.append(gpu.Fc128LayerParam("Fc%d" % i, b, k, n).initialize(gpu.ArrayWeights([w, bn]), prev))
+        want.append(orc.fc128(want[-1], wl, bn, k, n))
+    for layer in layers:
+        layer.get_output_gpu().fill(0x55)
+    if not with_in:
+        layers[0].forward()
+    forward_fc_run(layers if with_in else layers[1:])
+    gpuops.sync()
+    for layer, w in zip(layers, want):
+        np.testing.assert_array_equal(layer.download_packed() if hasattr(layer, "download_packed") else layer.download_output(), w)
+        layer.release()
+
+
 # --------------------------------------------------------------------------- standalone conv
 SWEEP = [(32, 128), (16, 256), (8, 512), (56, 64), (28, 128), (14, 256), (7, 512)]
 
