@@ -957,7 +957,12 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     q.cgroups = p.O / (32 * MT);
     q.rows = c.pool * p.OH;
 
-    // Images per 32-column tile
+    // Images per 32-column tile.  Fewer than eight are stored in pieces shorter than what memory takes at once, which shows where the
+    // launch's bytes are not at home in the memory-side cache with what the network does between two passes: VGG-16's layer
+    // within a pass, us: batch 148 in fours 178, 133 in ones 208, 150 in twos 239; in sixteens 125-150.  (Batch 100 in
+    // fours 94, in sixteens 95; the 7x7/2 layer at batch 28 in fours 42.3, in eights 47.8.)
+    constexpr double kFewer[4] = {2.2, 1.65, 1.25, 1.06};
+    const bool large = 12LL * p.H * p.W * p.B + c.out_bytes + c.res_bytes >= 96LL << 20;
     double best = 1e30;
     int imgtiles = 0;
     const long long target = std::max(1LL, (long long)cus * 4 * waves_per_simd(c.r, c.a) / q.cgroups);  // resident waves
@@ -966,7 +971,7 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
         const int NI = 1 << ni_log2, NX = 32 >> ni_log2;
         if ((long long)NI * 3 * p.H * p.W * 4 >= (1LL << 31)) continue;
         const int tiles = (p.B + NI - 1) >> ni_log2, groups = (xcols + NX - 1) / NX;
-        const double cost = (double)tiles * groups * (ni_log2 == most ? 1.0 : 1.06);
+        const double cost = (double)tiles * groups * (ni_log2 == most ? 1.0 : (large ? kFewer[ni_log2] : 1.06));
         if (cost < best) {
             best = cost;
             q.ni_log2 = ni_log2;
@@ -991,6 +996,9 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
         }
     }
     const long long total = per * q.bands;
+    // 11x11: a launch that leaves a third of the machine's waves out is slower than the ring in LDS too (AlexNet, batch 48 / 64, 1176 and
+    // 1568 of 2048 waves with two pooled rows: 44.0 / 46.4 us; there 40.7 / 49.7)
+    if (c.r == 11 && total * 10 < target * 7) return false;
     if (total * q.cgroups > 0x0fffffffLL) return false;
     q.total = (int)total;
     q.per_xcd = (q.total + 7) / 8;
