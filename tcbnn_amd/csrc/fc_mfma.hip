@@ -24,12 +24,14 @@ using namespace mfma;
 constexpr int kMaxWaves = 16;
 constexpr int FC_THRESH = 0, FC_AFFINE = 1;
 
-// PRE > 0: the wave's K slice is at most PRE groups and is requested whole before the first multiply.
-template <int MODE, int PRE>
+// PRE > 0: the wave's K slice is at most PRE groups and is requested whole before the first multiply.  STAGED: activations are
+// requested sixteen bytes a lane and turned in LDS (fc_plan says when).
+template <int MODE, int PRE, bool STAGED>
 __global__ __launch_bounds__(64 * kMaxWaves) void fc_mfma_f4_kernel(
     const BgemmParams p, const uint32_t* __restrict__ act, const uint32_t* __restrict__ wgt,
     const float* __restrict__ bnp, const float* __restrict__ bias, int n_tiles, int groups_per_wave) {
     __shared__ int red[16 * 64];
+    extern __shared__ __align__(16) v4i stage[];  // [wave][2][64]: a group's activations on their way from rows to lanes
     __shared__ float par[64];
 
     const int tid = threadIdx.x;
@@ -41,7 +43,6 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fc_mfma_f4_kernel(
     const int nt = blockIdx.x % n_tiles, bt = blockIdx.x / n_tiles;
     const int n0 = nt * 32, b0 = bt * 32;
     const int b = b0 + j;
-    const int bl = min(b, p.B - 1);
     const int cw = p.cw;  // words per image / per neuron; a multiple of 4
     // The weights in lane order (after the [NPAD32][cw] rows): a group is 64 lanes x 4 words, contiguous; rows >= N
     // and words >= cw hold zeros (their outputs are discarded / they multiply activation words that read as 0).
@@ -53,21 +54,36 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fc_mfma_f4_kernel(
     // (lanes 32-63) of both operands.
     const int g_begin = wave * groups_per_wave, g_end = min(groups, g_begin + groups_per_wave);
 
-    auto load_group = [&](int g, v4i& a, uint32_t (&bw)[4]) {
-        const int w0 = 8 * g + 4 * h;
+    // Activations.  STAGED: eight words of 32 images are one request of 16 bytes per lane (lane l: word l / 8, images 4 (l % 8) ..), a
+    // quarter of the address unit's time of four words per lane; through LDS each lane gets its image's words.  Past the tensor:
+    // zeros, images past the batch: whatever is there (discarded).
+    const __amdgpu_buffer_rsrc_t r_act = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(act), 0, cw * p.B * 4, 0x00020000);
+    const int act_lane = STAGED ? ((lane >> 3) * p.B + b0 + 4 * (lane & 7)) * 4 : (4 * h * p.B + min(b, p.B - 1)) * 4;
+    uint32_t* const mine = reinterpret_cast<uint32_t*>(stage + wave * 128);
+    auto load_group = [&](int g, v4i& a, v4i& bw) {
         a = wlane[(size_t)g * 64];  // (one contiguous 1 KB request per wave)
-        if (w0 < cw) {  // cw % 4 == 0: the lane's four activation words exist or none does
-#pragma unroll
-            for (int i = 0; i < 4; ++i) bw[i] = act[(size_t)(w0 + i) * p.B + bl];
+        const int at = act_lane + g * 32 * p.B;
+        if constexpr (STAGED) {
+            bw = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r_act, at, 0, 0));
         } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) bw[i] = 0;
+            for (int i = 0; i < 4; ++i) bw[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(r_act, at + i * 4 * p.B, 0, 0);
         }
     };
     v16f acc;
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-    auto compute_group = [&](int g, const v4i& a, const uint32_t (&bw)[4]) {
+    auto compute_group = [&](int g, int turn, const v4i& a, const v4i& words) {
+        uint32_t bw[4];
+        if constexpr (STAGED) {
+            uint32_t* const at = mine + turn * 256;
+            reinterpret_cast<v4i*>(at)[lane] = words;  // (written and read by this wave only)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bw[i] = at[(4 * h + i) * 32 + j];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bw[i] = (uint32_t)words[i];
+        }
         const int w0 = 8 * g + 4 * h;
         if (32 * (8 * g + 8) <= p.k_tap) {  // uniform: every bit of the group is a true input
 #pragma unroll
@@ -91,26 +107,26 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fc_mfma_f4_kernel(
     if constexpr (PRE > 0) {
         // short slice: every operand word of the wave is requested before the first multiply (one round trip)
         v4i a[PRE];
-        uint32_t bw[PRE][4];
+        v4i bw[PRE];
 #pragma unroll
         for (int u = 0; u < PRE; ++u)
             if (g_begin + u < g_end) load_group(g_begin + u, a[u], bw[u]);
 #pragma unroll
         for (int u = 0; u < PRE; ++u)
-            if (g_begin + u < g_end) compute_group(g_begin + u, a[u], bw[u]);
+            if (g_begin + u < g_end) compute_group(g_begin + u, u & 1, a[u], bw[u]);
     } else {
         // two groups (8 k-steps) per stage, double-buffered in registers
         v4i a0[2], a1[2];
-        uint32_t w0[2][4], w1[2][4];
-        auto load_stage = [&](int g, v4i (&a)[2], uint32_t (&bw)[2][4]) {
+        v4i w0[2], w1[2];
+        auto load_stage = [&](int g, v4i (&a)[2], v4i (&bw)[2]) {
 #pragma unroll
             for (int u = 0; u < 2; ++u)
                 if (g + u < g_end) load_group(g + u, a[u], bw[u]);
         };
-        auto compute_stage = [&](int g, v4i (&a)[2], uint32_t (&bw)[2][4]) {
+        auto compute_stage = [&](int g, v4i (&a)[2], v4i (&bw)[2]) {
 #pragma unroll
             for (int u = 0; u < 2; ++u)
-                if (g + u < g_end) compute_group(g + u, a[u], bw[u]);
+                if (g + u < g_end) compute_group(g + u, u, a[u], bw[u]);
         };
         int g = g_begin;
         if (g < g_end) load_stage(g, a0, w0);
@@ -192,7 +208,7 @@ bool fc_mfma_applicable(const BgemmParams& p) {
     if (!p.wgt_lane_copy) return false;
     if (p.PH * p.PW != 1 || p.R * p.S != 1 || p.res_in != nullptr || p.res_out != nullptr) return false;
     if (p.mode != EPI_THRESH && p.mode != EPI_AFFINE) return false;
-    if (p.cw % 4 != 0 || p.k_tap > 32 * p.cw) return false;
+    if (p.cw % 4 != 0 || p.k_tap > 32 * p.cw || 4LL * p.B * (p.cw + 4) >= (1LL << 31)) return false;
     // larger problems fill the machine with one wave per tile and are served by the generic kernel
     const long long tiles = (long long)((p.B + 31) / 32) * ((p.N + 31) / 32);
     return tiles <= 16384;
@@ -203,6 +219,7 @@ namespace {
 // kernel requests ahead of its first multiply (0: a streaming loop).
 struct FcPlan {
     int n_tiles, b_tiles, kwaves, gpw, pre;
+    bool staged;
 };
 FcPlan fc_plan(const BgemmParams& p) {
     FcPlan f;
@@ -215,27 +232,34 @@ FcPlan fc_plan(const BgemmParams& p) {
     f.gpw = (groups + kwaves - 1) / kwaves;
     f.kwaves = (groups + f.gpw - 1) / f.gpw;
     f.pre = f.gpw <= 2 ? 2 : (f.gpw <= 7 ? 7 : 0);
+    // Requests of sixteen bytes a lane where the address units are busy: long slices (25088 inputs, batch 256, 4096 outputs: 32.5 ->
+    // 27.7 us; 32768 inputs, 512 outputs, batch 77: 13.2 -> 12.3) and many waves (9216 inputs, 4096 outputs, batch 200, 8064 waves: 21.7 ->
+    // 21.1).  With few, the way through LDS only adds to the chain (8192 inputs, 1024 outputs, batch 256, 2048 waves: 8.2 -> 8.4).
+    f.staged = f.pre == 0 || (f.pre == 7 && (long long)f.n_tiles * f.b_tiles * f.kwaves >= 3072);
     return f;
 }
 }  // namespace
 
 void fc_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len) {
-    snprintf(buf, len, "fc_mfma_f4_kernel<%d, %d>", p.mode == EPI_AFFINE ? FC_AFFINE : FC_THRESH, fc_plan(p).pre);
+    const FcPlan f = fc_plan(p);
+    snprintf(buf, len, "fc_mfma_f4_kernel<%d, %d, %s>", p.mode == EPI_AFFINE ? FC_AFFINE : FC_THRESH, f.pre, f.staged ? "true" : "false");
 }
 
 int launch_fc_mfma(const BgemmParams& p, hipStream_t stream) {
     const FcPlan f = fc_plan(p);
     const int n_tiles = f.n_tiles, b_tiles = f.b_tiles, kwaves = f.kwaves, gpw = f.gpw;
     const dim3 grid((unsigned)(n_tiles * b_tiles)), block(64 * kwaves);
-    auto launch = [&](auto mode, auto pre) {
+    auto launch = [&](auto mode, auto pre, auto staged) {
         constexpr int MODE = decltype(mode)::value, PRE = decltype(pre)::value;
-        hipLaunchKernelGGL((fc_mfma_f4_kernel<MODE, PRE>), grid, block, 0, stream, p, p.act, p.wgt,
+        constexpr bool STAGED = decltype(staged)::value;
+        hipLaunchKernelGGL((fc_mfma_f4_kernel<MODE, PRE, STAGED>), grid, block, STAGED ? kwaves * 2048 : 0, stream, p, p.act, p.wgt,
                            MODE == FC_AFFINE ? p.bn_scale : p.bn, MODE == FC_AFFINE ? p.bn_bias : p.bn, n_tiles, gpw);
     };
     auto by_slice = [&](auto mode) {
-        if (f.pre == 2) launch(mode, std::integral_constant<int, 2>{});
-        else if (f.pre == 7) launch(mode, std::integral_constant<int, 7>{});
-        else launch(mode, std::integral_constant<int, 0>{});
+        if (f.pre == 2) launch(mode, std::integral_constant<int, 2>{}, std::false_type{});
+        else if (f.pre == 0) launch(mode, std::integral_constant<int, 0>{}, std::true_type{});
+        else if (f.staged) launch(mode, std::integral_constant<int, 7>{}, std::true_type{});
+        else launch(mode, std::integral_constant<int, 7>{}, std::false_type{});
     };
     if (p.mode == EPI_AFFINE) by_slice(std::integral_constant<int, FC_AFFINE>{});
     else by_slice(std::integral_constant<int, FC_THRESH>{});

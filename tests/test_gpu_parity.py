@@ -105,6 +105,26 @@ def test_out128(gpu, variant, b, k, n):
     np.testing.assert_array_equal(got, want)  # and in fact bit-identical
 
 
+@pytest.mark.parametrize("b,k,n", [(1, 32768, 40), (3, 30001, 32), (31, 29000, 33), (67, 32641, 96),  # long slices of K
+                                   (131, 9220, 4000), (98, 8161, 4096)])  # many waves; words that end inside a group
+def test_fc128_activations_through_lds(gpu, b, k, n):
+    """Requests of four images a lane: batches that are no multiple of four, groups that end past the last word."""
+    r = rng(b + k + n)
+    x = r.standard_normal((b, k)).astype(np.float32)
+    w = rm.pm1(r, (k, n))
+    bn = r.normal(0, np.sqrt(k), n).astype(np.float32)
+    want = orc.fc128(orc.in128(x), orc.pack_fc_weight(w), bn, k, n)
+    fin = gpu.In128LayerParam("Fin", b, k).initialize(x)
+    layer = gpu.Fc128LayerParam("Fc", b, k, n).initialize(gpu.ArrayWeights([w, bn]), fin.get_output_gpu())
+    assert layer.kernel_name().startswith("fc_mfma_f4_kernel") and layer.kernel_name().endswith("true>"), layer.kernel_name()
+    fin.forward()
+    layer.forward()
+    gpuops.sync()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    layer.release()
+    fin.release()
+
+
 @pytest.mark.parametrize("b,widths,with_in,with_out", [
     # one image and neuron; ends of words, tiles and groups of K; a wave's second tiles and second round of tiles; activations
     # of 2048 (two requests of weights ahead, 64 KB of LDS)
