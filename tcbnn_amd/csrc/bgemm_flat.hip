@@ -16,12 +16,17 @@
 //   small work: K is split over the waves of a workgroup (up to 8) so that a launch of few tiles still spreads over
 //               the machine; the partial sums, exact integers, meet in LDS.
 //
-// What bounds it, with counters: the small launches latency, one or two memory round trips and the launch itself (3x3 layers
-// at batch 8, 5.6-6.3 us: waves wait for memory 52-64 % of their time, VALU busy 20-33 %, matrix cores 4 %).  The larger ones
+// The finish of a tile stays in fp32 (whole numbers): sums start from minus what the pad bits add, a bit is the sign of sum -
+// threshold shifted in, and what lies past the last channel is masked once.  Small launches end with one wave's finish, and
+// with conversions, compares and selects per value it was a fifth of their time: ResNet-18 at batch 1 / 8 113.1 -> 105.3 / 117.4 ->
+// 112.3 us a pass, VGG-16 at batch 8 212 -> 180, AlexNet at batch 150 175 -> 168.  (Shared by two waves instead, eight channels of a
+// lane each: 1 % slower than by one.)
+//
+// What bounds it, with counters (from before that): the small launches latency, one or two memory round trips and the launch itself (3x3
+// layers at batch 8, 5.6-6.3 us: waves wait for memory 52-64 % of their time, VALU busy 20-33 %, matrix cores 4 %).  The larger ones
 // instruction issue: expanding the operands takes 7 VALU instructions per fragment, plus 5 per column tile and step for
 // address and border, against 32 cycles per MFMA (AlexNet's 5x5 layer at batch 256, 50 us: VALU 63 %, matrix cores 27 %, of
-// the same issue slots).  1x1 layers with a residual at batch 256 (19.5 us) their traffic: 40 % waiting, 54 % VALU, 3 %
-// matrix cores.
+// the same issue slots).
 #include <algorithm>
 #include <initializer_list>
 
@@ -32,6 +37,8 @@ namespace tcbnn {
 namespace {
 
 using namespace mfma;
+
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 // what happens to the sums
 constexpr int FM_BITS = 0;    // threshold, packed bits
@@ -85,7 +92,7 @@ __device__ __forceinline__ void fetch_one(T v) {
 }
 
 template <int MT, int NT, int FM, int RF, int WIN>
-__global__ __launch_bounds__(64 * max_waves(MT, NT)) __attribute__((amdgpu_waves_per_eu(MT * NT == 1 ? 4 : 2))) void
+__global__ __launch_bounds__(64 * max_waves(MT, NT)) __attribute__((amdgpu_waves_per_eu(MT * NT == 1 ? (FM == FM_RESPOOL ? 3 : 4) : 2))) void
 bgemm_flat_f4_kernel(const FlatArgs p) {
     static_assert(WIN == FW_NONE || (FM == FM_BITS && MT == (WIN == FW_TILES ? 4 : 1)), "see FW_*");
     static_assert(FM != FM_RESPOOL || MT == 1, "four source pixels per column");
@@ -114,7 +121,7 @@ bgemm_flat_f4_kernel(const FlatArgs p) {
     const int ct = live ? (int)div_by((unsigned)tile, p.by_groups) : 0, ng = live ? tile - ct * p.n_groups : 0;
     const int n0 = ng * (32 * NT);
 
-    v4i* red = lds_dyn;                                                           // [slices - 1][MT * NT][4][64]
+    v4f* red = reinterpret_cast<v4f*>(lds_dyn);                                   // [slices - 1][MT * NT][4][64]
     int* raw_area = reinterpret_cast<int*>(red + (size_t)(p.slices - 1) * MT * NT * 256);
     constexpr int kRawWords = FM == FM_RAW ? 32 * raw_pitch(NT) + 64 : 0;         // per tile of the workgroup
     int2* tab = reinterpret_cast<int2*>(raw_area + per_wg * kRawWords);           // [8 * groups]
@@ -251,13 +258,17 @@ bgemm_flat_f4_kernel(const FlatArgs p) {
     for (int d = 0; d < D; ++d)
         if (g_begin + d < g_end) request_b(d, g_begin + d);
 
+    // A tap's pad bits are 0 in both operands: each adds +1, which the sums (of the wave that finishes) start below 0 by.
     v16f acc[MT][NT];
+    const int padbits = 32 * p.cw - p.k_tap;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt) {
+        const float from = slice == 0 ? 0.0f - (float)(padbits * (p.R * p.S - __popc(inval[mt] & ((1u << (p.R * p.S)) - 1u)))) : 0.0f;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[mt][nt][v] = 0.0f;
+            for (int v = 0; v < 16; ++v) acc[mt][nt][v] = from;
+    }
 
     // +-1 in FP4 as in expand_f4, zero where the tap is invalid (its word was returned as 0)
     auto expand_col = [&](uint32_t x, unsigned c) __attribute__((always_inline)) {
@@ -322,8 +333,7 @@ bgemm_flat_f4_kernel(const FlatArgs p) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const v16f& s = acc[t / NT][t % NT];
-                    red[(((slice - 1) * MT * NT + t) * 4 + q) * 64 + lane] =
-                        v4i{(int)s[4 * q], (int)s[4 * q + 1], (int)s[4 * q + 2], (int)s[4 * q + 3]};
+                    red[(((slice - 1) * MT * NT + t) * 4 + q) * 64 + lane] = v4f{s[4 * q], s[4 * q + 1], s[4 * q + 2], s[4 * q + 3]};
                 }
         }
         __syncthreads();
@@ -331,36 +341,40 @@ bgemm_flat_f4_kernel(const FlatArgs p) {
     }
     if (!live) return;
 
-    const int padbits = 32 * p.cw - p.k_tap;  // a tap's pad bits are 0 in both operands: each adds +1
     const int ow = (p.N + 31) / 32;
+    const float never = p.nan_bit ? -INFINITY : INFINITY;  // (a threshold that is no number)
     uint32_t orw[NT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int k = WIN == FW_TILES ? 0 : mt;
         const int b = cb[k];
         const bool ok = cok[k];
-        const int corr = padbits * (p.R * p.S - __popc(inval[mt] & ((1u << (p.R * p.S)) - 1u)));
         const size_t pix = (size_t)cy[mt] * p.PW + cx[mt];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             const int cbase = n0 + nt * 32 + 16 * h;
-            int dot[16];
+            float sum[16];  // (whole numbers below 2^24)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) dot[v] = (int)acc[mt][nt][v] - corr;
+            for (int v = 0; v < 16; ++v) sum[v] = acc[mt][nt][v];
             for (int s = 1; s < p.slices; ++s)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const v4i o = red[(((s - 1) * MT * NT + mt * NT + nt) * 4 + q) * 64 + lane];
+                    const v4f o = red[(((s - 1) * MT * NT + mt * NT + nt) * 4 + q) * 64 + lane];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) dot[4 * q + e] += o[e];
+                    for (int e = 0; e < 4; ++e) sum[4 * q + e] += o[e];
                 }
             if constexpr (FM == FM_RAW) {
                 int* mine = raw_area + (p.slices > 1 ? 0 : wave) * kRawWords;
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     *reinterpret_cast<v4i*>(mine + j * raw_pitch(NT) + nt * 32 + 16 * h + 4 * q) =
-                        v4i{dot[4 * q], dot[4 * q + 1], dot[4 * q + 2], dot[4 * q + 3]};
+                        v4i{(int)sum[4 * q], (int)sum[4 * q + 1], (int)sum[4 * q + 2], (int)sum[4 * q + 3]};
                 continue;
+            }
+            int whole[16];
+            if constexpr (kRes && RF == TCBNN_RES_I32) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) whole[v] = (int)sum[v];
             }
             if constexpr (kRes) {
                 if (p.res_lim > 0) {
@@ -382,22 +396,30 @@ bgemm_flat_f4_kernel(const FlatArgs p) {
 #pragma unroll
                         for (int v = 0; v < 16; ++v) rv[v] = s == 0 ? t[v] : max(rv[v], t[v]);
                     }
+                    if (n0 + nt * 32 + 32 > p.res_lim)  // (uniform)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) dot[v] += cbase + v < p.res_lim ? rv[v] : 0;
+                        for (int v = 0; v < 16; ++v) rv[v] = cbase + v < p.res_lim ? rv[v] : 0;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        if constexpr (RF == TCBNN_RES_I32) whole[v] += rv[v], sum[v] = (float)whole[v];  // (any number)
+                        else sum[v] += (float)rv[v];
+                    }
                 }
             }
+            // bits, MSB first: the inverted sign of sum - threshold
             uint32_t hw = 0;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const uint32_t bit = cbase + v < p.N ? thresh_bit(dot[v], thr[nt][v], p.nan_bit) : 0u;
-                hw = hw + hw + bit;
-            }
+            for (int v = 0; v < 16; ++v) hw = __builtin_amdgcn_alignbit(hw, __float_as_uint(sum[v] - (thr[nt][v] == thr[nt][v] ? thr[nt][v] : never)), 31);
+            hw = ~hw & 0xffffu & (0xffff0000u >> min(max(p.N - cbase, 0), 16));
             if constexpr (kRes) {
                 if (p.res_out != nullptr) {
                     if (ok && cbase < p.N) {
                         int rs[16];
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) rs[v] = cbase + v < p.N ? dot[v] : 0;  // (0 past N inside a group)
+                        for (int v = 0; v < 16; ++v) rs[v] = RF == TCBNN_RES_I32 ? whole[v] : (int)sum[v];
+                        if (n0 + nt * 32 + 32 > p.N)  // (uniform)
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) rs[v] = cbase + v < p.N ? rs[v] : 0;  // (0 past N inside a group)
                         if (p.res_out_fmt == TCBNN_RES_I12) {
                             residual_store_group16(p.res_out, TCBNN_RES_I12, pix, p.N, cbase / 16, p.B, b, rs);
                         } else if (p.res_out_fmt == TCBNN_RES_I16) {

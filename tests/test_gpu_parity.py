@@ -1627,6 +1627,33 @@ def test_conv128_flat_columns(gpu, b, h, cin, cout, R, pool, res):
     layer.release()
 
 
+@pytest.mark.parametrize("b,h,cin,cout,R,res", [(3, 5, 512, 64, 3, None), (2, 5, 512, 64, 3, 2), (3, 5, 100, 40, 3, 1), (4, 1, 32, 7, 5, None),
+                                                (3, 6, 160, 70, 3, 0), (9, 64, 32, 250, 1, 0), (9, 64, 33, 250, 1, None)])
+def test_conv128_flat_thresholds(gpu, b, h, cin, cout, R, res):
+    """Bits from the sign of sum - threshold: met exactly, zeros, infinities, no number (kernel.cuh:795-796: the bit is then 1);
+    pad bits and taps outside the frame; 32-bit residuals beyond what fp32 holds exactly."""
+    r = rng(3 * b + h + cin + cout)
+    x = rm.pm1(r, (b, h, h, cin))
+    f = rm.pm1(r, (R, R, cin, cout))
+    inp, filt = orc.pack_conv_input_nhwc(x), orc.pack_conv_filter(f)
+    kw, okw = {}, {}
+    if res is not None:
+        most = {2: 900, 1: 20000, 0: 1 << 28}[res]
+        src = r.integers(-most, most, size=(h, h, b, cout)).astype(np.int32)
+        okw = dict(save_residual=True, inject_residual=True, residual_channels=cout, res_in=src)
+        kw = dict(okw, in_fmt=res, out_fmt=min(res, 1))
+    _, sums = orc.conv128(inp, filt, np.zeros(cout, np.float32), cin, cout, R, R, **dict(okw, save_residual=True))
+    bn = sums[h // 2, 0, b // 2].astype(np.float32)
+    bn[:6] = [np.nan, np.inf, -np.inf, 0.0, -0.0, sums[0, 0, 0, 5] + 0.5]
+    want, wres = orc.conv128(inp, filt, bn, cin, cout, R, R, **okw)
+    layer = _run_conv_layer(gpu, "mfma_f4", x, f, bn, **kw)
+    assert layer.kernel_name().startswith("bgemm_flat_f4_kernel<"), layer.kernel_name()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    if res is not None:
+        np.testing.assert_array_equal(layer.download_residual(), wres)
+    layer.release()
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 32, 32), (33, 64, 8192), (700, 2048, 160), (1025, 3072, 96),
                                    # the large kernel with an odd number of words per row
                                    (4100, 992, 32), (4100, 1056, 544), (8200, 1024, 7200)])
