@@ -631,7 +631,10 @@ bool bgemm_flat_preferred(const BgemmParams& p) {
     const double t_persistent = 4.0 + 0.02 * steps + std::max(item, all) + (res ? 1.2 : 0.0) + 0.24 * mib;
     // this kernel: full tiles, but operands expanded for every tile and a prologue per tile (the share of short K)
     const double mfmas = (double)(((long long)p.PH * p.PW * p.B + 31) / 32) * n_tiles * steps;
-    const double t_flat = 4.4 + 1e-6 * mfmas * (40.0 + 380.0 / steps) + 0.015 * steps + (res ? 0.5 : 0.0) + 0.16 * mib;
+    // (The fit is from before the finish in fp32, which launches of few tiles gain from by up to 1.2 us: with that, ResNet-18 at batch 8
+    // 111.9 -> 107.4 us a pass and at 10 117.0 -> 113.8.  As much for all launches: batch 25 of the textbook wiring 1.7 % slower.)
+    const double few = 1.2 * std::max(0.0, 1.0 - mfmas / 23000.0);
+    const double t_flat = 4.4 - few + 1e-6 * mfmas * (40.0 + 380.0 / steps) + 0.015 * steps + (res ? 0.5 : 0.0) + 0.16 * mib;
     return t_flat < t_persistent;
 }
 
