@@ -98,7 +98,9 @@ def layer_work(L, spec=(), res_bytes=None, pooled=()):
         if L["kind"] == "inconv":
             byts = B * 3 * L["h"] * L["w"] * 4 + out_bits + L["r"] * L["s"] * 3 * L["cout"] * 4
             # fp16 products of the matrix-core kernel: four taps of four channels to a step, high and low parts
-            mfma_flops = 2.0 * B * oh * ow * L["cout"] * 2 * 16 * L["r"] * -(-L["s"] // 4)
+            # sets of rows under way x fragments of a step (its rows' pairs, 8 / 12 places for 7 / 11 taps), high and low parts
+            pairs, places = (3 * L["stride"] + 1) // 2, {7: 8, 11: 12}.get(L["s"], L["s"])
+            mfma_flops = 2.0 * B * oh * ow * L["cout"] * 2 * 16 * -(-L["r"] // L["stride"]) * -(-pairs * places // 8)
             if L["save_residual"]:
                 byts += B * oh * ow * L["cout"] * res_bytes.get(L["name"], 4)
         else:
@@ -145,7 +147,7 @@ def roofline_of(name, g, variant):
         done = g["mfma_flops"] / secs / 1e12
         rec["matrix_fp16"] = {"flops_per_launch": round(g["mfma_flops"] / g["launches"]), "achieved": round(done, 1),
                               "peak": 2500.0, "unit": "TFLOP/s", "frac": round(done / 2500.0, 4)}
-        rec["binding"] = "waves waiting for memory and for issue slots, under two per SIMD; see matrix_fp16"
+        rec["binding"] = "waves waiting for the images and for issue slots, three per SIMD; see matrix_fp16"
     elif g.get("flops"):
         # The fp32 first layer on the VALU is far from the HBM roof because its additions bind it: one dependent fp32 add
         # per (tap, output channel, pixel, image) is the least the reference's summation order allows (its 2 flops per
