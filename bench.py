@@ -98,9 +98,9 @@ def layer_work(L, spec=(), res_bytes=None, pooled=()):
         if L["kind"] == "inconv":
             byts = B * 3 * L["h"] * L["w"] * 4 + out_bits + L["r"] * L["s"] * 3 * L["cout"] * 4
             # fp16 products of the matrix-core kernel: four taps of four channels to a step, high and low parts
-            # sets of rows under way x fragments of a step (its rows' pairs, 8 / 12 places for 7 / 11 taps), high and low parts
-            pairs, places = (3 * L["stride"] + 1) // 2, {7: 8, 11: 12}.get(L["s"], L["s"])
-            mfma_flops = 2.0 * B * oh * ow * L["cout"] * 2 * 16 * -(-L["r"] // L["stride"]) * -(-pairs * places // 8)
+            # counted as fragments of four taps x four channels per filter row, high and low parts (14 at 7x7; the kernel's
+            # order of K, pairs of a row and a channel, needs 12)
+            mfma_flops = 2.0 * B * oh * ow * L["cout"] * 2 * 16 * L["r"] * -(-L["s"] // 4)
             if L["save_residual"]:
                 byts += B * oh * ow * L["cout"] * res_bytes.get(L["name"], 4)
         else:
