@@ -205,44 +205,73 @@ struct HeadParams {
 };
 
 constexpr int kHeadImages = 8;     // images per workgroup
-constexpr int kHeadOutputs = 128;  // outputs per workgroup: a thread takes one of them for four of the images
+constexpr int kHeadOutputs = 128;  // outputs per workgroup: a thread takes one of them for two of the images
+constexpr int kHeadThreads = kHeadOutputs * kHeadImages / 2;
 constexpr int kHeadMaxC = 512;
-constexpr int kHeadChunk = 64;     // channels whose weights are in flight at a time
+constexpr int kHeadChunk = 32;     // channels whose weights are laid out in LDS at a time
+constexpr int kHeadAhead = 2;      // chunks requested ahead
+
+// Sixteen channels of a thread's output and four images: means lie one channel per lane of each row of 16 (all rows the same), and
+// a multiply-add takes its channel's by DPP.  (As asm because the compiler moves the lane's value first, in an instruction of
+// its own; the wait states are those between a write of m and a DPP read of it.)
+#define TCBNN_HEAD_CHANNEL(K, LANE)                                                        \
+    "v_fmac_f32_dpp %0, %2, %" #K " row_newbcast:" #LANE " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %1, %3, %" #K " row_newbcast:" #LANE " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void head_channels(const float2& m, const float (&w)[16], float (&acc)[2]) {
+    asm("s_nop 1\n\t" TCBNN_HEAD_CHANNEL(4, 0) TCBNN_HEAD_CHANNEL(5, 1) TCBNN_HEAD_CHANNEL(6, 2) TCBNN_HEAD_CHANNEL(7, 3)
+            TCBNN_HEAD_CHANNEL(8, 4) TCBNN_HEAD_CHANNEL(9, 5) TCBNN_HEAD_CHANNEL(10, 6) TCBNN_HEAD_CHANNEL(11, 7)
+                TCBNN_HEAD_CHANNEL(12, 8) TCBNN_HEAD_CHANNEL(13, 9) TCBNN_HEAD_CHANNEL(14, 10) TCBNN_HEAD_CHANNEL(15, 11)
+                    TCBNN_HEAD_CHANNEL(16, 12) TCBNN_HEAD_CHANNEL(17, 13) TCBNN_HEAD_CHANNEL(18, 14) TCBNN_HEAD_CHANNEL(19, 15)
+        : "+&v"(acc[0]), "+&v"(acc[1])
+        : "v"(m.x), "v"(m.y), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]),
+          "v"(w[10]), "v"(w[11]), "v"(w[12]), "v"(w[13]), "v"(w[14]), "v"(w[15]));
+}
 
 // Workgroup = 8 images x 128 outputs.  Phase 1: the means of the 8 images, all channels, into LDS.  Phase 2: a thread
-// takes one output of four images; per channel one coalesced weight load (the workgroup's other half finds it in L1) and
-// four fused multiply-adds on means that every lane reads from the same LDS address; channels in ascending order.
-// Everything here is latency: a dependent chain of C multiply-adds (8 k cycles for 512 channels and four images at one
-// wave per SIMD) behind two trips to memory and the fetch of the code itself, which runs once.  So the grid is as many
-// workgroups as CUs at batch 256, all pixels of a 7x7 map are requested together, weights run 64 channels ahead, LDS reads
-// eight; and addresses advance on the scalar unit (wave-uniform base + lane offset) to keep the unrolled code short.
-// (8 images per thread, 8 pixels and 16 channels ahead, 128 workgroups, sums in a dynamically indexed array: 67 us at batch
-// 256 and at batch 20 alike; now 22 and 21 us for 7x7x512 -> 1000.)
-// Workgroups of the same images are gridDim.x apart in launch order: for a multiple of 8 image groups they share an L2.
+// takes one output of two images: per channel a weight from LDS and two fused multiply-adds, channels in ascending order.
+// Everything here is latency: a chain of C multiply-adds behind the pixels' way from memory and the fetch of the code, which runs
+// once.  So the grid is as many workgroups as CUs at batch 256, two waves to a SIMD (with one, 256 threads and four images each,
+// the means took 10 us and the products 11), and the pixels' loop is rolled (all 49 of a 7x7 map unrolled: 27.7 us for 23.8).
+// Weights come from memory sixteen bytes a lane, two channels a request, two chunks of 32 channels ahead, and are shared through
+// LDS: the address unit takes 17 cycles for a request whatever its size, and eight waves that each ask for a channel's 256 bytes
+// at a time would keep it busy for 30 us.  A group of 16 channels' means is one read, a channel to a lane of each row of 16, and a
+// multiply-add takes its lane's by DPP: read per channel they would keep LDS busy for 7 us.
+// 7x7x512 -> 1000, events around one launch in a pass, us, 256 threads with weights straight from memory -> here: batch 1 23.6 -> 18.8,
+// 50 29.1 -> 22.4, 128 27.5 -> 21.0, 256 30.5 -> 23.8.
 template <int FMT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void avgpool_fc_kernel(const HeadParams p) {
+__global__ __launch_bounds__(kHeadThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void avgpool_fc_kernel(const HeadParams p) {
     constexpr int kPer = (int)residual_group_channels(FMT);
-    constexpr int kPixels = FMT == TCBNN_RES_I12 ? 25 : 49;  // requested together (integer sums: the order does not matter)
+    constexpr int kPixels = 17;  // requested together (integer sums: the order does not matter)
     __shared__ __align__(16) float mean[kHeadMaxC][kHeadImages];
     const int tid = threadIdx.x;
     const int b0 = blockIdx.x * kHeadImages;
-    const int n = blockIdx.y * kHeadOutputs + (tid & (kHeadOutputs - 1)), i0 = tid / kHeadOutputs * 4;
-    // Weights eight channels at a time: a wave-uniform base and eight lane offsets.
-    unsigned w_lane[8];
+    const int n = blockIdx.y * kHeadOutputs + (tid & (kHeadOutputs - 1)), i0 = tid / kHeadOutputs * 2;
+    __shared__ __align__(16) float weights[2][kHeadChunk][kHeadOutputs];
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    // A chunk: 32 threads to a channel's 128 outputs (past the last one: the next channel's, or zeros; not stored).  Past the last
+    // channel: zeros.  A buffer is one chunk (128 N bytes: 2^31 is out of reach of a grid's second dimension).
+    const int w_at = ((tid >> 5) * p.N + (int)blockIdx.y * kHeadOutputs + (tid & 31) * 4) * 4;
+    v4u ahead[kHeadAhead][2];
+    float* next = const_cast<float*>(p.w);
+    int left = p.C;
+    auto request = [&](int slot) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rsrc =
+            __builtin_amdgcn_make_buffer_rsrc(next, 0, min(kHeadChunk, max(0, left)) * p.N * 4, 0x00020000);
+        next += (size_t)kHeadChunk * p.N;
+        left -= kHeadChunk;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) w_lane[q] = ((unsigned)q * (unsigned)p.N + (unsigned)min(n, p.N - 1)) * 4u;
-    float w[kHeadChunk];
-    auto request = [&](int c, int slot) {  // channels c .. c + 7 (c uniform), of no use past the last chunk
-        const char* const row = reinterpret_cast<const char*>(p.w) + (size_t)min(c, max(0, p.C - 8)) * p.N * 4;
+        for (int q = 0; q < 2; ++q) ahead[slot][q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, w_at + q * 16 * p.N * 4, 0, 0);
+    };
+    auto lay_out = [&](int chunk, int slot) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < 8; ++q) w[slot + q] = *reinterpret_cast<const float*>(row + (p.C >= 8 ? w_lane[q] : w_lane[0]));
+        for (int q = 0; q < 2; ++q) *reinterpret_cast<v4u*>(&weights[chunk & 1][(tid >> 5) + 16 * q][(tid & 31) * 4]) = ahead[slot][q];
     };
 #pragma unroll
-    for (int q = 0; q < kHeadChunk; q += 8) request(q, q);
+    for (int k = 0; k < kHeadAhead; ++k) request(k);
 
     const float npix = (float)p.P;
     const size_t pixel_b = (size_t)p.groups * residual_group_bytes(FMT) * p.B;
-    for (int u = tid; u < p.groups * kHeadImages; u += kThreads) {
+    for (int u = tid; u < p.groups * kHeadImages; u += kHeadThreads) {
         const int g = u / kHeadImages, i = u % kHeadImages;  // image fastest: 128-byte runs
         const unsigned bb = (unsigned)min(b0 + i, p.B - 1);
         const unsigned lane = (unsigned)g * (unsigned)residual_group_bytes(FMT) * (unsigned)p.B + bb * 16u;
@@ -250,6 +279,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         int sum[kPer];
 #pragma unroll
         for (int k = 0; k < kPer; ++k) sum[k] = 0;
+#pragma unroll 1
         for (int pix0 = 0; pix0 < p.P; pix0 += kPixels) {
             uint4 v[kPixels];
             uint2 v2[FMT == TCBNN_RES_I12 ? kPixels : 1];
@@ -282,39 +312,38 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         for (int k = 0; k < kPer; ++k)
             if (g * kPer + k < p.C) mean[g * kPer + k][i] = (float)sum[k] / npix;
     }
-    __syncthreads();
-    if (b0 + i0 >= p.B) return;  // (a wave's lanes share i0)
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto channel = [&](const float4& m, float weight) {
-        acc[0] = __fmaf_rn(m.x, weight, acc[0]);
-        acc[1] = __fmaf_rn(m.y, weight, acc[1]);
-        acc[2] = __fmaf_rn(m.z, weight, acc[2]);
-        acc[3] = __fmaf_rn(m.w, weight, acc[3]);
-    };
-    int c0 = 0;
-    for (; c0 + kHeadChunk <= p.C; c0 += kHeadChunk) {
-        float4 m[2][8];
-        auto means = [&](int q0) {
+    float acc[2] = {0.0f, 0.0f};
+    const int col = tid & (kHeadOutputs - 1), chunks = (p.C + kHeadChunk - 1) / kHeadChunk;
+    for (int k0 = 0; k0 < chunks; k0 += kHeadAhead) {
 #pragma unroll
-            for (int q = 0; q < 8; ++q) m[q0 / 8 % 2][q] = *reinterpret_cast<const float4*>(&mean[c0 + q0 + q][i0]);
-        };
-        means(0);
+        for (int k = 0; k < kHeadAhead; ++k) {
+            const int chunk = k0 + k;
+            if (chunk >= chunks) break;  // uniform
+            lay_out(chunk, k);  // (the buffer's last readers have passed the barrier of the chunk before)
+            request(k);
+            __syncthreads();
 #pragma unroll
-        for (int q0 = 0; q0 < kHeadChunk; q0 += 8) {
-            if (q0 + 8 < kHeadChunk) means(q0 + 8);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int g = 0; g < kHeadChunk; g += 16) {
+                const int c0 = chunk * kHeadChunk + g;
+                if (c0 + 16 <= p.C) {  // uniform
+                    float w[16];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) channel(m[q0 / 8 % 2][q], w[q0 + q]);
-            __builtin_amdgcn_sched_barrier(0);
-            request(c0 + kHeadChunk + q0, q0);
+                    for (int c = 0; c < 16; ++c) w[c] = weights[chunk & 1][g + c][col];
+                    head_channels(*reinterpret_cast<const float2*>(&mean[c0 + (tid & 15)][i0]), w, acc);
+                } else {
+                    for (int c = c0; c < p.C; ++c) {
+                        const float weight = weights[chunk & 1][c - chunk * kHeadChunk][col];
+                        acc[0] = __fmaf_rn(mean[c][i0], weight, acc[0]);
+                        acc[1] = __fmaf_rn(mean[c][i0 + 1], weight, acc[1]);
+                    }
+                }
+            }
         }
     }
-    for (; c0 < p.C; ++c0)  // (what is left of a channel count that 64 does not divide)
-        channel(*reinterpret_cast<const float4*>(&mean[c0][i0]), p.w[(size_t)c0 * p.N + min(n, p.N - 1)]);
     if (n >= p.N) return;
     const float bias = p.bias[n];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i)
         if (b0 + i0 + i < p.B) p.out[(size_t)(b0 + i0 + i) * p.N + n] = __fadd_rn(acc[i], bias);
 }
 
@@ -407,7 +436,7 @@ extern "C" int tcbnn_avgpool_fc_forward(const tcbnn_avgpool_fc_desc* d, void* st
     const int per_group = (int)residual_group_channels(p.fmt);
     p.groups = (p.C + per_group - 1) / per_group;
     const dim3 grid((unsigned)((p.B + kHeadImages - 1) / kHeadImages), (unsigned)((p.N + kHeadOutputs - 1) / kHeadOutputs));
-    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, p); };
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kHeadThreads), 0, (hipStream_t)stream, p); };
     if (p.fmt == TCBNN_RES_I12)
         launch(avgpool_fc_kernel<TCBNN_RES_I12>);
     else if (p.fmt == TCBNN_RES_I16)
