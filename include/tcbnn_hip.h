@@ -233,7 +233,8 @@ int tcbnn_out128_forward(const tcbnn_out128_desc* d, void* stream);
 
 /* In128 (or NULL), n_fc Fc128 layers and Out128 (or NULL), one after the other: the same results, in every layer's
  * output, as the calls above in this order.  Layers that follow one another (each reads the output of the one before,
- * same batch, at most 2048 inputs and outputs, the FP4 engine) go in one launch.  Allocates nothing and needs no
+ * same batch, at most 2048 inputs and outputs, the FP4 engine) go in one launch, unless an output lies where another
+ * layer of the run reads or writes: what shares memory is launched one by one.  Allocates nothing and needs no
  * workspace.  No counterpart in the reference (its network kernel runs all layers, kernel.cuh:153-280). */
 int tcbnn_fc_chain_forward(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out,
                            void* stream);

@@ -294,10 +294,54 @@ bool pays(int launches, long long products, int batch) {
     return 1.7 * (launches - 1) >= (double)products / (1024 * 1024) * (2.2 - batch / 1024.0);
 }
 
+// The memory of a run's layers.  Launched one by one, a layer may write where an earlier one has read or written (two buffers in
+// turn); in one launch nothing orders the waves and workgroups of different layers but LDS, so every output has to be apart
+// from all else that the run reads and writes, except as the input of the layer that follows.
+class Memory {
+   public:
+    // A layer that reads `n` ranges besides the output of the one before it; false: it has to have a launch of its own
+    struct Range {
+        const void* at;
+        size_t bytes;
+    };
+    bool add(const Range* reads, int n, const Range& write) {
+        bool apart = true;
+        for (int i = 0; i < n; ++i) apart &= !meets(reads[i], writes_, n_writes_) && !meets(reads[i], &write, 1);
+        apart &= !meets(write, reads_, n_reads_) && !meets(write, writes_, n_writes_);
+        if (!apart) return false;
+        for (int i = 0; i < n; ++i) reads_[n_reads_++] = reads[i];
+        writes_[n_writes_++] = write;
+        return true;
+    }
+
+   private:
+    static bool meets(const Range& r, const Range* of, int n) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(r.at);
+        for (int i = 0; i < n; ++i) {
+            const uintptr_t b = reinterpret_cast<uintptr_t>(of[i].at);
+            if (a < b ? b - a < r.bytes : a - b < of[i].bytes) return true;
+        }
+        return false;
+    }
+    Range reads_[3 * kMaxLayers + 1], writes_[kMaxLayers + 1];
+    int n_reads_ = 0, n_writes_ = 0;
+};
+
 // The layers from fc[0] on that one launch can take (0: none, or the chain is not worth one)
 int chain_length(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out, bool* with_out) {
     *with_out = false;
     auto usable = [](const void* a, const void* b, const void* c, const void* d) { return a != nullptr && b != nullptr && c != nullptr && d != nullptr; };
+    auto bits = [](const void* at, int batch, int n) { return Memory::Range{at, 4 * tcbnn_fc_act_words(batch, n)}; };
+    auto weights = [](const void* at, int k, int n) { return Memory::Range{at, 4 * tcbnn_fc_weight_words(k, n)}; };
+    auto floats = [](const void* at, int rows, int n) { return Memory::Range{at, (size_t)4 * rows * n}; };
+    Memory memory;
+    if (in != nullptr) {
+        if (in->input == nullptr || in->output != fc[0].input || in->input_height != fc[0].input_height || in->input_width != fc[0].input_width ||
+            !fits(in->input_height, in->input_width, 1))
+            return 0;
+        const Memory::Range x = floats(in->input, in->input_height, in->input_width);
+        if (!memory.add(&x, 1, bits(in->output, in->input_height, in->input_width))) return 0;
+    }
     int n = 0;
     for (; n < n_fc && n < kMaxLayers; ++n) {
         const tcbnn_fc128_desc& f = fc[n];
@@ -305,14 +349,19 @@ int chain_length(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_f
             resolve_variant(f.variant) != TCBNN_VARIANT_MFMA_F4)
             break;
         if (n > 0 && (f.input != fc[n - 1].output || f.input_height != fc[0].input_height || f.input_width != fc[n - 1].weight_width)) break;
+        const Memory::Range reads[3] = {weights(f.weight, f.input_width, f.weight_width), floats(f.bn, 1, f.weight_width), bits(f.input, f.input_height, f.input_width)};
+        if (!memory.add(reads, n == 0 && in == nullptr ? 3 : 2, bits(f.output, f.input_height, f.weight_width))) break;
     }
     if (n == 0) return 0;
     long long products = 0;
     for (int i = 0; i < n; ++i) products += (long long)fc[i].input_width * fc[i].weight_width;
-    if (in != nullptr && (in->input == nullptr || in->output != fc[0].input || in->input_height != fc[0].input_height || in->input_width != fc[0].input_width)) return 0;
     *with_out = out != nullptr && n == n_fc && n < kMaxLayers && usable(out->input, out->weight, out->bn_scale, out->output) && out->bn_bias != nullptr &&
                 fits(out->input_height, out->input_width, out->weight_width) && resolve_variant(out->variant) == TCBNN_VARIANT_MFMA_F4 &&
                 out->input == fc[n - 1].output && out->input_height == fc[0].input_height && out->input_width == fc[n - 1].weight_width;
+    if (*with_out) {
+        const Memory::Range reads[3] = {weights(out->weight, out->input_width, out->weight_width), floats(out->bn_scale, 1, out->weight_width), floats(out->bn_bias, 1, out->weight_width)};
+        *with_out = memory.add(reads, 3, floats(out->output, out->input_height, out->weight_width));
+    }
     if (*with_out) products += (long long)out->input_width * out->weight_width;
     const int launches = n + (*with_out ? 1 : 0) + (in != nullptr ? 1 : 0);
     return launches >= 2 && pays(launches, products, fc[0].input_height) ? n : 0;

@@ -100,6 +100,38 @@ def test_large_products_test_for_odd_words_only_where_there_can_be_any():
     assert name.value == b"gemm_mfma_f4_kernel<2, 0, false>"
 
 
+@pytest.mark.parametrize("run,moved,to,apart", [
+    ("fc fc", None, None, True), ("in fc", None, None, True), ("fc out", None, None, True),
+    # neighbours in memory, and one byte's worth too near
+    ("fc fc", "output 1", ("input 0", 40 * 8 * 4), True), ("fc fc", "output 1", ("input 0", 40 * 8 * 4 - 4), False),
+    ("fc fc", "output 1", ("input 0", -40 * 4 * 4), True), ("fc fc", "output 1", ("input 0", -40 * 4 * 4 + 4), False),
+    # two buffers in turn; both outputs in one; an output over what a layer reads before or after it is written
+    ("fc fc", "output 1", ("input 0", 0), False), ("fc fc", "output 1", ("output 0", 0), False), ("fc fc", "output 1", ("output 0", 16), False),
+    ("fc fc", "weight 1", ("output 0", 64), False), ("fc fc", "scale 0", ("output 1", 4), False),
+    ("in fc", "output 0", ("x", 40 * 200 * 4 - 4), False), ("in fc", "output 0", ("x", 40 * 200 * 4), True), ("in fc", "scale 0", ("input 0", 0), False),
+    ("fc out", "output 1", ("input 0", 0), False), ("fc out", "output 1", ("output 0", -40 * 10 * 4 + 4), False),
+    ("fc out", "output 1", ("output 0", -40 * 10 * 4), True), ("fc out", "bias", ("output 1", 8), False)])
+def test_layers_that_share_memory_are_not_one_launch(run, moved, to, apart):
+    """Layers launched one by one may write where an earlier one has read or written; inside one launch of a run nothing
+    orders them, so such a run is not one.  Without a device the first launch fails, and its message names the kernel."""
+    import ctypes as C
+    from tcbnn_amd import _lib
+    L = _lib.lib
+    if _lib.device_count() > 0:
+        pytest.skip("made-up pointers")
+    b, widths = 40, (200, 100, 10 if "out" in run else 100)
+    at = {name: 0x10000000 * (1 + i) for i, name in enumerate(("x", "input 0", "weight 0", "scale 0", "output 0", "weight 1", "scale 1", "bias", "output 1"))}
+    if moved is not None:
+        at[moved] = at[to[0]] + to[1]
+    fc = (_lib.Fc128Desc * 2)()
+    fc[0] = _lib.Fc128Desc(at["input 0"], at["weight 0"], at["scale 0"], at["output 0"], b, widths[0], widths[1], _lib.VARIANT_MFMA_F4, None, 0)
+    fc[1] = _lib.Fc128Desc(at["output 0"], at["weight 1"], at["scale 1"], at["output 1"], b, widths[1], widths[2], _lib.VARIANT_MFMA_F4, None, 0)
+    fin = _lib.In128Desc(at["x"], at["input 0"], b, widths[0])
+    out = _lib.Out128Desc(at["output 0"], at["weight 1"], at["scale 1"], at["bias"], at["output 1"], b, widths[1], widths[2], _lib.VARIANT_MFMA_F4)
+    assert L.tcbnn_fc_chain_forward(C.byref(fin) if "in" in run else None, fc, 2 if run == "fc fc" else 1, C.byref(out) if "out" in run else None, None) == -3
+    assert (b"fc_chain" in L.tcbnn_last_error()) == apart, L.tcbnn_last_error()
+
+
 def test_network_specs_match_reference_wiring():
     from tcbnn_amd import nets
     spec = nets.imagenet_resnet_spec(batch=256)

@@ -168,6 +168,33 @@ def test_fc_chain(gpu, b, widths, with_in, with_out):
         layer.release()
 
 
+@pytest.mark.parametrize("widths,turns", [((300, 260, 100, 260, 10), 2), ((70, 70, 70, 70, 70, 70), 2), ((64, 96, 40, 33, 96, 5), 3)])
+def test_fc_run_with_outputs_in_shared_buffers(gpu, widths, turns):
+    """Layers that write `turns` buffers in turn: the last output, and what each buffer holds in the end."""
+    from tcbnn_amd._lib import lib
+    from tcbnn_amd.layers import forward_fc_run
+    b = 37
+    r = rng(sum(widths))
+    x = r.standard_normal((b, widths[0])).astype(np.float32)
+    layers, want = [gpu.In128LayerParam("Fin", b, widths[0]).initialize(x)], [orc.in128(x)]
+    own = []
+    shared = [gpuops.dev(np.zeros(lib.tcbnn_fc_act_words(b, max(widths)), np.uint32)) for _ in range(turns)]
+    for i, (k, n) in enumerate(zip(widths, widths[1:])):
+        w, bn = rm.pm1(r, (k, n)), r.normal(0, np.sqrt(k), n).astype(np.float32)
+        layers.append(gpu.Fc128LayerParam("Fc%d" % i, b, k, n).initialize(gpu.ArrayWeights([w, bn]), layers[-1].get_output_gpu()))
+        own.append(layers[-1].output_gpu)
+        layers[-1].output_gpu = shared[i % turns]
+        want.append(orc.fc128(want[-1], orc.pack_fc_weight(w), bn, k, n))
+    forward_fc_run(layers)
+    gpuops.sync()
+    for layer, w in list(zip(layers, want))[-turns:]:
+        np.testing.assert_array_equal(layer.download_packed(), w)
+    for layer, buf in zip(layers[1:], own):
+        layer.output_gpu = buf
+    for thing in layers:
+        thing.release()
+
+
 # --------------------------------------------------------------------------- standalone conv
 SWEEP = [(32, 128), (16, 256), (8, 512), (56, 64), (28, 128), (14, 256), (7, 512)]
 
