@@ -466,16 +466,21 @@ class Out128LayerParam(_ReferenceLayoutIO):
         self.weight_gpu = self.bn_scale_gpu = self.bn_bias_gpu = self.output_gpu = None
 
 
-def fc_run_end(layers, begin):
-    """Where the run of an In128 layer, Fc128 layers and an Out128 layer (all optional) at `begin` ends."""
-    end = begin
-    if type(layers[end]) is In128LayerParam:
-        end += 1
-    while end < len(layers) and type(layers[end]) is Fc128LayerParam:
-        end += 1
-    if end < len(layers) and type(layers[end]) is Out128LayerParam:
-        end += 1
-    return max(end, begin + 1)
+def fc_runs(layers):
+    """`layers` cut into runs: an In128 layer, Fc128 layers and an Out128 layer (each optional), other layers alone."""
+    runs, begin = [], 0
+    while begin < len(layers):
+        end = begin
+        if type(layers[end]) is In128LayerParam:
+            end += 1
+        while end < len(layers) and type(layers[end]) is Fc128LayerParam:
+            end += 1
+        if end < len(layers) and type(layers[end]) is Out128LayerParam:
+            end += 1
+        end = max(end, begin + 1)
+        runs.append(layers[begin:end])
+        begin = end
+    return runs
 
 
 def forward_fc_run(layers, stream=None):

@@ -11,7 +11,7 @@ import numpy as np
 
 from . import _lib
 from .layers import (ArrayWeights, AvgPoolFcLayerParam, Conv128LayerParam, Fc128LayerParam, In128LayerParam,
-                     InConv128LayerParam, Out128LayerParam, PAD128, Pool128LayerParam, fc_run_end, forward_fc_run)
+                     InConv128LayerParam, Out128LayerParam, PAD128, Pool128LayerParam, fc_runs, forward_fc_run)
 
 
 def _conv_out(h, r, s, padding=True, pool=1):
@@ -265,6 +265,7 @@ class Network:
         self.spec = spec
         self.layers = {}
         self.order = []
+        self._plan = ([], [])  # an order of layers, and its runs (forward_fc_run)
         src = weights if hasattr(weights, "launch_array") else ArrayWeights(weights)
         for L in spec:
             k = L["kind"]
@@ -305,14 +306,15 @@ class Network:
         self.order[0].set_input(input)
 
     def forward(self, stream=None):
-        order, i = self.order, 0
-        while i < len(order):
-            end = fc_run_end(order, i)
-            if end > i + 1:
-                forward_fc_run(order[i:end], stream)
+        planned, runs = self._plan
+        if planned != self.order:  # (a comparison of identities; the runs themselves take four times the loop below)
+            runs = fc_runs(self.order)
+            self._plan = (list(self.order), runs)
+        for run in runs:
+            if len(run) == 1:
+                run[0].forward(stream)
             else:
-                order[i].forward(stream)
-            i = end
+                forward_fc_run(run, stream)
 
     def logits(self):
         _lib.device_synchronize()

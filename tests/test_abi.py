@@ -151,6 +151,43 @@ def test_network_specs_match_reference_wiring():
     assert abs(bops / 1e9 - 314.1) < 0.5
 
 
+def test_network_plans_its_runs_of_layers_once(monkeypatch):
+    """forward() works out which layers go in one call when their order is new, not on every pass."""
+    from tcbnn_amd import layers, nets
+    calls, planned, plan = [], [], layers.fc_runs
+
+    class Conv:
+        def forward(self, stream=None):
+            calls.append(self)
+
+    def counted(order):
+        planned.append(len(order))
+        return plan(order)
+
+    def together(run, stream=None):
+        calls.extend(run)
+
+    monkeypatch.setattr(nets, "fc_runs", counted)
+    monkeypatch.setattr(nets, "forward_fc_run", together)
+    fc = [layers.Fc128LayerParam("Fc%d" % i, 8, 64, 64) for i in range(2)]
+    out = layers.Out128LayerParam("Fout", 8, 64, 10)
+    alone = layers.Out128LayerParam("Aux", 8, 64, 10)
+    monkeypatch.setattr(alone, "forward", lambda stream=None: calls.append(alone), raising=False)
+    net = nets.Network([], [], None)
+    net.order = [Conv(), Conv()] + fc + [out, alone]
+    for _ in range(3):
+        net.forward()
+    assert planned == [6] and calls == 3 * net.order
+    assert [len(run) for run in plan(net.order)] == [1, 1, 3, 1]
+    del calls[:], planned[:]
+    net.order.insert(1, Conv())  # in place
+    net.forward()
+    net.order = net.order[2:]
+    net.forward()
+    net.forward()
+    assert planned == [7, 5] and len(calls) == 7 + 2 * 5
+
+
 def test_residual_formats_sizes_and_choice():
     """Host-only helpers of the residual storage formats: bytes per tensor, and the narrowest format a bound allows
     (12 bits need an even batch: the format's 128-bit accesses are aligned only then)."""
