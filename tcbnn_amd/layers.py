@@ -483,12 +483,16 @@ def fc_runs(layers):
     return runs
 
 
+_fc_arrays = {}  # array types by length: ctypes makes one again (27 us) once nothing holds it and a collection has passed
+
+
 def forward_fc_run(layers, stream=None):
     """forward() of the layers of such a run, one after the other, in as few launches as they allow."""
     first, last = layers[0], layers[-1]
     fc = [layer._desc() for layer in layers if type(layer) is Fc128LayerParam]
+    array = _fc_arrays.get(len(fc)) or _fc_arrays.setdefault(len(fc), _lib.Fc128Desc * len(fc))
     check(lib.tcbnn_fc_chain_forward(
-        C.byref(first._desc()) if type(first) is In128LayerParam else None, (_lib.Fc128Desc * len(fc))(*fc), len(fc),
+        C.byref(first._desc()) if type(first) is In128LayerParam else None, array(*fc), len(fc),
         C.byref(last._desc()) if type(last) is Out128LayerParam else None, _stream_handle(stream)))
 
 

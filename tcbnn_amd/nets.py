@@ -265,7 +265,6 @@ class Network:
         self.spec = spec
         self.layers = {}
         self.order = []
-        self._plan = ([], [])  # an order of layers, and its runs (forward_fc_run)
         src = weights if hasattr(weights, "launch_array") else ArrayWeights(weights)
         for L in spec:
             k = L["kind"]
@@ -301,6 +300,7 @@ class Network:
                 raise ValueError(k)
             self.layers[L["name"]] = layer
             self.order.append(layer)
+        self._plan = (list(self.order), fc_runs(self.order))  # an order of layers, and its runs (forward_fc_run)
 
     def set_input(self, input):
         self.order[0].set_input(input)

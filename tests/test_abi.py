@@ -173,7 +173,9 @@ def test_network_plans_its_runs_of_layers_once(monkeypatch):
     out = layers.Out128LayerParam("Fout", 8, 64, 10)
     alone = layers.Out128LayerParam("Aux", 8, 64, 10)
     monkeypatch.setattr(alone, "forward", lambda stream=None: calls.append(alone), raising=False)
-    net = nets.Network([], [], None)
+    net = nets.Network([], [], None)  # (plans the order that it makes: nothing here)
+    assert planned == [0]
+    del planned[:]
     net.order = [Conv(), Conv()] + fc + [out, alone]
     for _ in range(3):
         net.forward()
@@ -186,6 +188,29 @@ def test_network_plans_its_runs_of_layers_once(monkeypatch):
     net.forward()
     net.forward()
     assert planned == [7, 5] and len(calls) == 7 + 2 * 5
+
+
+def test_a_run_of_layers_makes_no_types_of_its_own(monkeypatch):
+    """The descriptors' array type outlives the call and a collection: a new network's first pass does not make it again."""
+    import gc
+    import weakref
+    from tcbnn_amd import layers
+    made = []
+
+    class Lib:
+        @staticmethod
+        def tcbnn_fc_chain_forward(first, array, n, last, stream):
+            made.append(weakref.ref(type(array)))
+            return 0
+
+    run = [layers.Fc128LayerParam("Fc%d" % i, 8, 64, 64) for i in range(3)] + [layers.Out128LayerParam("Fout", 8, 64, 10)]
+    for layer in run:
+        layer._desc = layers._lib.Out128Desc if layer is run[-1] else layers._lib.Fc128Desc
+    monkeypatch.setattr(layers, "lib", Lib)
+    for _ in range(2):
+        layers.forward_fc_run(run)
+        gc.collect()
+    assert made[0]() is not None and made[0]() is made[1]()
 
 
 def test_residual_formats_sizes_and_choice():
