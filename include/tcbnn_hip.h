@@ -238,6 +238,10 @@ int tcbnn_out128_forward(const tcbnn_out128_desc* d, void* stream);
  * workspace.  No counterpart in the reference (its network kernel runs all layers, kernel.cuh:153-280). */
 int tcbnn_fc_chain_forward(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out,
                            void* stream);
+/* The launches that tcbnn_fc_chain_forward makes of such a run: their number, and how many layers each takes (n_fc + 2
+ * entries at most).  Several layers are joined where that is faster.  Launches nothing. */
+int tcbnn_fc_chain_plan(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out,
+                        int* layers, int* n_launches);
 
 /* InConv128LayerFMT (kernel.cuh:578-672), fields of InConv128LayerParam
  * (param.h:841-869).  fp32 NCHW 3-channel input, +-1 filters, fp32 adds in the

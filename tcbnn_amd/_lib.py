@@ -121,6 +121,7 @@ ABI = {
     "tcbnn_fc128_forward_static_scratch": (c_int, [C.POINTER(Fc128Desc), c_void_p]),
     "tcbnn_out128_forward": (c_int, [C.POINTER(Out128Desc), c_void_p]),
     "tcbnn_fc_chain_forward": (c_int, [C.POINTER(In128Desc), C.POINTER(Fc128Desc), c_int, C.POINTER(Out128Desc), c_void_p]),
+    "tcbnn_fc_chain_plan": (c_int, [C.POINTER(In128Desc), C.POINTER(Fc128Desc), c_int, C.POINTER(Out128Desc), C.POINTER(c_int), C.POINTER(c_int)]),
     "tcbnn_inconv128_forward": (c_int, [C.POINTER(InConv128Desc), c_void_p]),
     "tcbnn_inconv_packed_input_floats": (c_size_t, [c_int] * 8),
     "tcbnn_inconv_pack_input": (c_int, [c_void_p, c_void_p] + [c_int] * 8 + [c_void_p]),

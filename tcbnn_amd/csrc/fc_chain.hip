@@ -283,15 +283,27 @@ __global__ __launch_bounds__(64 * kWaves) void fc_chain_kernel(const ChainArgs a
 
 bool fits(int batch, int k, int n) { return batch > 0 && k > 0 && n > 0 && k <= kMaxWidth && n <= kMaxWidth; }
 
-// Whether one launch is faster than `launches`.  A launch costs 1.7 us more than a layer's share of this one; a workgroup does a
-// layer's products for its 32 images on one compute unit, 2.2 us longer for 1024 x 1024 of them than all units together where
-// there are few images, and less where there are many.  The MLP, us, in a launch per layer and here: 512 wide, batch 1: 17.6 and
-// 12.7; 1024 wide, batch 1 / 256 / 8192: 18.9 / 20.4 / 44.6 and 17.6 / 18.0 / 21.1; 1152 wide, batch 64 / 256 / 1024: 20.8 / 22.2 /
-// 25.7 and 21.9 / 22.0 / 22.4; 1408 wide, batch 256 / 512 / 1024: 24.0 / 24.4 / 28.0 and 25.6 / 25.6 / 25.9; 2048 wide, batch
-// 256 / 1536 / 2048 / 8192: 22.6 / 37.7 / 40.4 / 75.3 and 36.5 / 37.4 / 38.0 / 47.4.  The last two layers of CIFAR VGG (1024 x 1024,
-// 1024 x 10), batch 256, are 1 us faster in two launches.
-bool pays(int launches, long long products, int batch) {
-    return 1.7 * (launches - 1) >= (double)products / (1024 * 1024) * (2.2 - batch / 1024.0);
+// Whether one launch is faster than one per layer, by what it saves (us), fitted to both sides' times of 380 runs (1 to 5 layers,
+// 10 to 2048 wide, batch 1 to 16384, launched on end).  A launch of its own costs a layer 1.75 us more than its share of this one, the
+// input's signs 0.7 and more where there is more to read, and this launch has 3.6 of its own.  A workgroup does a layer's products
+// for its 32 images on one compute unit, 1.85 us longer for 1024 x 1024 of them than all units together where there are few images, and
+// less where there are many; a layer of 4096 tiles or more is 2.4 us slower by itself; an output layer stores a number at a
+// time (14 us for 1000 of 32 images); and beyond 8192 images workgroups wait for a compute unit.
+// us, a launch per layer and here: the MLP, batch 1 / 256 / 8192: 17.5 / 19.5 / 45.1 and 17.6 / 18.0 / 20.5; 1408 wide, batch 256 /
+// 1024 / 1536: 21.5 / 25.1 / 28.5 and 25.4 / 25.4 / 25.5; 2048 wide, batch 256 / 1536 / 2048: 21.2 / 32.2 / 40.6 and 36.3 / 36.6 / 37.0;
+// the last two layers of CIFAR VGG (1024 x 1024, 1024 x 10), batch 256 / 1024 / 2048 / 4096: 7.2 / 7.4 / 8.1 / 12.6 and 8.8 / 8.9 / 9.0 / 9.2.
+struct Work {
+    int inputs;           // of the signs; 0: none
+    int layers;           // besides the signs
+    double products;      // in 1024 x 1024
+    int large;            // layers of 4096 tiles or more
+    int numbers;          // outputs that are numbers
+};
+bool pays(const Work& w, int batch) {
+    const double x = std::min(batch, 8192) / 1024.0, read = (double)w.inputs * batch / (1024 * 1024);
+    const double saved = 1.75 * w.layers + (w.inputs > 0 ? 0.7 + 0.0029 * w.inputs : 0.0) - 3.6 + w.products * (0.48 * x - 1.85) + 2.4 * w.large -
+                         0.014 * w.numbers * std::min(batch, 16) / 16 * std::max(0.0, 1.0 - x / 6);
+    return saved + (batch > 8192 ? 1.1 * read - 7.0 : 0.0) >= 0.0;
 }
 
 // The memory of a run's layers.  Launched one by one, a layer may write where an earlier one has read or written (two buffers in
@@ -353,8 +365,14 @@ int chain_length(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_f
         if (!memory.add(reads, n == 0 && in == nullptr ? 3 : 2, bits(f.output, f.input_height, f.weight_width))) break;
     }
     if (n == 0) return 0;
-    long long products = 0;
-    for (int i = 0; i < n; ++i) products += (long long)fc[i].input_width * fc[i].weight_width;
+    const int batch = fc[0].input_height;
+    Work work{in != nullptr ? in->input_width : 0, 0, 0.0, 0, 0};
+    auto count = [&](int k, int outputs) {
+        ++work.layers;
+        work.products += (double)k * outputs / (1024 * 1024);
+        work.large += (long long)((batch + 31) / 32) * ((outputs + 31) / 32) >= 4096;
+    };
+    for (int i = 0; i < n; ++i) count(fc[i].input_width, fc[i].weight_width);
     *with_out = out != nullptr && n == n_fc && n < kMaxLayers && usable(out->input, out->weight, out->bn_scale, out->output) && out->bn_bias != nullptr &&
                 fits(out->input_height, out->input_width, out->weight_width) && resolve_variant(out->variant) == TCBNN_VARIANT_MFMA_F4 &&
                 out->input == fc[n - 1].output && out->input_height == fc[0].input_height && out->input_width == fc[n - 1].weight_width;
@@ -362,9 +380,11 @@ int chain_length(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_f
         const Memory::Range reads[3] = {weights(out->weight, out->input_width, out->weight_width), floats(out->bn_scale, 1, out->weight_width), floats(out->bn_bias, 1, out->weight_width)};
         *with_out = memory.add(reads, 3, floats(out->output, out->input_height, out->weight_width));
     }
-    if (*with_out) products += (long long)out->input_width * out->weight_width;
-    const int launches = n + (*with_out ? 1 : 0) + (in != nullptr ? 1 : 0);
-    return launches >= 2 && pays(launches, products, fc[0].input_height) ? n : 0;
+    if (*with_out) {
+        count(out->input_width, out->weight_width);
+        work.numbers = out->weight_width;
+    }
+    return work.layers + (in != nullptr ? 1 : 0) >= 2 && pays(work, batch) ? n : 0;
 }
 
 int launch_chain(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out, hipStream_t stream) {
@@ -401,31 +421,59 @@ int launch_chain(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_f
     return TCBNN_OK;
 }
 
-}  // namespace
-}  // namespace tcbnn
-
-using namespace tcbnn;
-
-extern "C" int tcbnn_fc_chain_forward(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out, void* stream) {
+// The launches of a run, in order: chain(in, fc, n_fc, out) for one of several layers, single(in, fc, out), one of them not null
+template <typename Chain, typename Single>
+int each_launch(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out, const Chain& chain, const Single& single) {
     TCBNN_REQUIRE(n_fc >= 0 && (n_fc == 0 || fc != nullptr), "fc_chain: no layers");
     bool with_out = false;
     for (int i = 0; i <= n_fc;) {
         const tcbnn_in128_desc* const first = i == 0 ? in : nullptr;
         const int n = i < n_fc ? chain_length(first, fc + i, n_fc - i, out, &with_out) : 0;
         if (n > 0) {
-            if (int rc = launch_chain(first, fc + i, n, with_out ? out : nullptr, (hipStream_t)stream)) return rc;
+            if (int rc = chain(first, fc + i, n, with_out ? out : nullptr)) return rc;
             i += n;
             if (with_out) return TCBNN_OK;
             continue;
         }
         if (first != nullptr)
-            if (int rc = tcbnn_in128_forward(first, stream)) return rc;
+            if (int rc = single(first, nullptr, nullptr)) return rc;
         if (i < n_fc) {
-            if (int rc = tcbnn_fc128_forward(fc + i, stream)) return rc;
+            if (int rc = single(nullptr, fc + i, nullptr)) return rc;
         } else if (out != nullptr) {
-            return tcbnn_out128_forward(out, stream);
+            return single(nullptr, nullptr, out);
         }
         ++i;
     }
     return TCBNN_OK;
+}
+
+}  // namespace
+}  // namespace tcbnn
+
+using namespace tcbnn;
+
+extern "C" int tcbnn_fc_chain_forward(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out, void* stream) {
+    return each_launch(
+        in, fc, n_fc, out,
+        [&](const tcbnn_in128_desc* i, const tcbnn_fc128_desc* f, int n, const tcbnn_out128_desc* o) { return launch_chain(i, f, n, o, (hipStream_t)stream); },
+        [&](const tcbnn_in128_desc* i, const tcbnn_fc128_desc* f, const tcbnn_out128_desc* o) {
+            return i != nullptr ? tcbnn_in128_forward(i, stream) : (f != nullptr ? tcbnn_fc128_forward(f, stream) : tcbnn_out128_forward(o, stream));
+        });
+}
+
+extern "C" int tcbnn_fc_chain_plan(const tcbnn_in128_desc* in, const tcbnn_fc128_desc* fc, int n_fc, const tcbnn_out128_desc* out, int* layers, int* n_launches) {
+    TCBNN_REQUIRE(layers != nullptr && n_launches != nullptr, "fc_chain: NULL pointer");
+    int n = 0;
+    const int rc = each_launch(
+        in, fc, n_fc, out,
+        [&](const tcbnn_in128_desc* i, const tcbnn_fc128_desc*, int n_layers, const tcbnn_out128_desc* o) {
+            layers[n++] = n_layers + (i != nullptr) + (o != nullptr);
+            return (int)TCBNN_OK;
+        },
+        [&](const tcbnn_in128_desc*, const tcbnn_fc128_desc*, const tcbnn_out128_desc*) {
+            layers[n++] = 1;
+            return (int)TCBNN_OK;
+        });
+    *n_launches = n;
+    return rc;
 }

@@ -15,6 +15,7 @@ Conv128LayerParam.  Differences forced by the redesign:
 All compute goes through the C ABI of libtcbnn_hip.so.
 """
 import ctypes as C
+import itertools
 
 import numpy as np
 
@@ -486,14 +487,27 @@ def fc_runs(layers):
 _fc_arrays = {}  # array types by length: ctypes makes one again (27 us) once nothing holds it and a collection has passed
 
 
-def forward_fc_run(layers, stream=None):
-    """forward() of the layers of such a run, one after the other, in as few launches as they allow."""
+def _fc_run_args(layers):
     first, last = layers[0], layers[-1]
     fc = [layer._desc() for layer in layers if type(layer) is Fc128LayerParam]
     array = _fc_arrays.get(len(fc)) or _fc_arrays.setdefault(len(fc), _lib.Fc128Desc * len(fc))
-    check(lib.tcbnn_fc_chain_forward(
-        C.byref(first._desc()) if type(first) is In128LayerParam else None, array(*fc), len(fc),
-        C.byref(last._desc()) if type(last) is Out128LayerParam else None, _stream_handle(stream)))
+    return (C.byref(first._desc()) if type(first) is In128LayerParam else None, array(*fc), len(fc),
+            C.byref(last._desc()) if type(last) is Out128LayerParam else None)
+
+
+def fc_launches(run):
+    """A run of fc_runs() cut into the layers that one launch takes."""
+    if len(run) == 1:
+        return [run]
+    counts, n = (C.c_int * len(run))(), C.c_int()
+    check(lib.tcbnn_fc_chain_plan(*_fc_run_args(run), counts, C.byref(n)))
+    ends = list(itertools.accumulate(counts[:n.value]))
+    return [run[begin:end] for begin, end in zip([0] + ends, ends)]
+
+
+def forward_fc_run(layers, stream=None):
+    """forward() of the layers of such a run, one after the other, in as few launches as is fastest."""
+    check(lib.tcbnn_fc_chain_forward(*_fc_run_args(layers), _stream_handle(stream)))
 
 
 class _ConvGeometry(_ReferenceLayoutIO):

@@ -11,7 +11,7 @@ import numpy as np
 
 from . import _lib
 from .layers import (ArrayWeights, AvgPoolFcLayerParam, Conv128LayerParam, Fc128LayerParam, In128LayerParam,
-                     InConv128LayerParam, Out128LayerParam, PAD128, Pool128LayerParam, fc_runs, forward_fc_run)
+                     InConv128LayerParam, Out128LayerParam, PAD128, Pool128LayerParam, fc_launches, fc_runs, forward_fc_run)
 
 
 def _conv_out(h, r, s, padding=True, pool=1):
@@ -300,16 +300,19 @@ class Network:
                 raise ValueError(k)
             self.layers[L["name"]] = layer
             self.order.append(layer)
-        self._plan = (list(self.order), fc_runs(self.order))  # an order of layers, and its runs (forward_fc_run)
+        self._plan = self._plan_order()
 
     def set_input(self, input):
         self.order[0].set_input(input)
 
+    def _plan_order(self):
+        """The order of layers, and what is launched together: layers that have launches of their own go one by one."""
+        return list(self.order), [launch for run in fc_runs(self.order) for launch in fc_launches(run)]
+
     def forward(self, stream=None):
         planned, runs = self._plan
-        if planned != self.order:  # (a comparison of identities; the runs themselves take four times the loop below)
-            runs = fc_runs(self.order)
-            self._plan = (list(self.order), runs)
+        if planned != self.order:  # (a comparison of identities; the plan itself takes four times the loop below)
+            planned, runs = self._plan = self._plan_order()
         for run in runs:
             if len(run) == 1:
                 run[0].forward(stream)

@@ -100,36 +100,65 @@ def test_large_products_test_for_odd_words_only_where_there_can_be_any():
     assert name.value == b"gemm_mfma_f4_kernel<2, 0, false>"
 
 
+_B = 8192  # (a batch at which two layers are faster together)
+
+
 @pytest.mark.parametrize("run,moved,to,apart", [
     ("fc fc", None, None, True), ("in fc", None, None, True), ("fc out", None, None, True),
     # neighbours in memory, and one byte's worth too near
-    ("fc fc", "output 1", ("input 0", 40 * 8 * 4), True), ("fc fc", "output 1", ("input 0", 40 * 8 * 4 - 4), False),
-    ("fc fc", "output 1", ("input 0", -40 * 4 * 4), True), ("fc fc", "output 1", ("input 0", -40 * 4 * 4 + 4), False),
+    ("fc fc", "output 1", ("input 0", _B * 16 * 4), True), ("fc fc", "output 1", ("input 0", _B * 16 * 4 - 4), False),
+    ("fc fc", "output 1", ("input 0", -_B * 12 * 4), True), ("fc fc", "output 1", ("input 0", -_B * 12 * 4 + 4), False),
     # two buffers in turn; both outputs in one; an output over what a layer reads before or after it is written
     ("fc fc", "output 1", ("input 0", 0), False), ("fc fc", "output 1", ("output 0", 0), False), ("fc fc", "output 1", ("output 0", 16), False),
     ("fc fc", "weight 1", ("output 0", 64), False), ("fc fc", "scale 0", ("output 1", 4), False),
-    ("in fc", "output 0", ("x", 40 * 200 * 4 - 4), False), ("in fc", "output 0", ("x", 40 * 200 * 4), True), ("in fc", "scale 0", ("input 0", 0), False),
-    ("fc out", "output 1", ("input 0", 0), False), ("fc out", "output 1", ("output 0", -40 * 10 * 4 + 4), False),
-    ("fc out", "output 1", ("output 0", -40 * 10 * 4), True), ("fc out", "bias", ("output 1", 8), False)])
+    ("in fc", "output 0", ("x", _B * 500 * 4 - 4), False), ("in fc", "output 0", ("x", _B * 500 * 4), True), ("in fc", "scale 0", ("input 0", 0), False),
+    ("fc out", "output 1", ("input 0", 0), False), ("fc out", "output 1", ("output 0", -_B * 10 * 4 + 4), False),
+    ("fc out", "output 1", ("output 0", -_B * 10 * 4), True), ("fc out", "bias", ("output 1", 8), False)])
 def test_layers_that_share_memory_are_not_one_launch(run, moved, to, apart):
     """Layers launched one by one may write where an earlier one has read or written; inside one launch of a run nothing
-    orders them, so such a run is not one.  Without a device the first launch fails, and its message names the kernel."""
+    orders them, so such a run is not one."""
     import ctypes as C
     from tcbnn_amd import _lib
-    L = _lib.lib
-    if _lib.device_count() > 0:
-        pytest.skip("made-up pointers")
-    b, widths = 40, (200, 100, 10 if "out" in run else 100)
+    widths = (500, 500, 10 if "out" in run else 380)
     at = {name: 0x10000000 * (1 + i) for i, name in enumerate(("x", "input 0", "weight 0", "scale 0", "output 0", "weight 1", "scale 1", "bias", "output 1"))}
     if moved is not None:
         at[moved] = at[to[0]] + to[1]
     fc = (_lib.Fc128Desc * 2)()
-    fc[0] = _lib.Fc128Desc(at["input 0"], at["weight 0"], at["scale 0"], at["output 0"], b, widths[0], widths[1], _lib.VARIANT_MFMA_F4, None, 0)
-    fc[1] = _lib.Fc128Desc(at["output 0"], at["weight 1"], at["scale 1"], at["output 1"], b, widths[1], widths[2], _lib.VARIANT_MFMA_F4, None, 0)
-    fin = _lib.In128Desc(at["x"], at["input 0"], b, widths[0])
-    out = _lib.Out128Desc(at["output 0"], at["weight 1"], at["scale 1"], at["bias"], at["output 1"], b, widths[1], widths[2], _lib.VARIANT_MFMA_F4)
-    assert L.tcbnn_fc_chain_forward(C.byref(fin) if "in" in run else None, fc, 2 if run == "fc fc" else 1, C.byref(out) if "out" in run else None, None) == -3
-    assert (b"fc_chain" in L.tcbnn_last_error()) == apart, L.tcbnn_last_error()
+    fc[0] = _lib.Fc128Desc(at["input 0"], at["weight 0"], at["scale 0"], at["output 0"], _B, widths[0], widths[1], _lib.VARIANT_MFMA_F4, None, 0)
+    fc[1] = _lib.Fc128Desc(at["output 0"], at["weight 1"], at["scale 1"], at["output 1"], _B, widths[1], widths[2], _lib.VARIANT_MFMA_F4, None, 0)
+    fin = _lib.In128Desc(at["x"], at["input 0"], _B, widths[0])
+    out = _lib.Out128Desc(at["output 0"], at["weight 1"], at["scale 1"], at["bias"], at["output 1"], _B, widths[1], widths[2], _lib.VARIANT_MFMA_F4)
+    layers, n = (C.c_int * 4)(), C.c_int()
+    _lib.check(_lib.lib.tcbnn_fc_chain_plan(C.byref(fin) if "in" in run else None, fc, 2 if run == "fc fc" else 1, C.byref(out) if "out" in run else None, layers, C.byref(n)))
+    assert layers[:n.value] == ([2] if apart else [1, 1])
+
+
+@pytest.mark.parametrize("batch,widths,with_in,with_out,launches", [
+    # the MLP, at every batch; layers too wide for one compute unit until there are many images
+    (1, (784, 1024, 1024, 1024, 10), True, True, [5]), (8192, (784, 1024, 1024, 1024, 10), True, True, [5]),
+    (16384, (784, 1024, 1024, 1024, 10), True, True, [5]),
+    (1024, (784, 2048, 2048, 2048, 10), True, True, [1] * 5), (2048, (784, 2048, 2048, 2048, 10), True, True, [5]),
+    # two layers: where few images leave most compute units without work, launches of their own are faster
+    (256, (1024, 1024, 10), False, True, [1, 1]), (768, (1024, 1024, 10), False, True, [1, 1]), (2048, (1024, 1024, 10), False, True, [1, 1]),
+    (4096, (1024, 1024, 10), False, True, [2]), (8192, (64, 64, 10), False, True, [1, 1]), (1024, (512, 512, 10), False, True, [1, 1]),
+    # many numbers to store; little to multiply for many images
+    (64, (512, 1024, 1000), False, True, [1, 1]), (8, (256, 512, 512, 1000), True, True, [1] * 4), (16384, (200, 100, 50, 10), True, True, [1] * 4),
+    (9000, (784, 128, 10), True, True, [3]), (12000, (64, 64, 64, 64, 64, 10), False, True, [1] * 5), (12000, (512, 512, 512, 10), False, True, [3]),
+    # the input's signs and one layer
+    (1, (784, 256), True, False, [2]), (64, (100, 50), True, False, [1, 1]), (1024, (512, 512), True, False, [1, 1]), (8192, (512, 512), True, False, [2])])
+def test_which_layers_of_a_run_are_one_launch(batch, widths, with_in, with_out, launches):
+    """The choice between one launch and one per layer, where both sides were timed."""
+    import ctypes as C
+    from tcbnn_amd import _lib
+    n = len(widths) - 1 - int(with_out)
+    fc, at = (_lib.Fc128Desc * n)(), [0x100000000 * (1 + i) for i in range(16)]
+    for i in range(n):
+        fc[i] = _lib.Fc128Desc(at[i], at[14] + 0x1000000 * i, at[15] + 0x1000000 * i, at[i + 1], batch, widths[i], widths[i + 1], _lib.VARIANT_MFMA_F4, None, 0)
+    fin = _lib.In128Desc(at[13], at[0], batch, widths[0])
+    out = _lib.Out128Desc(at[n], at[12], at[11], at[10], at[9], batch, widths[-2], widths[-1], _lib.VARIANT_MFMA_F4)
+    layers, got = (C.c_int * 16)(), C.c_int()
+    _lib.check(_lib.lib.tcbnn_fc_chain_plan(C.byref(fin) if with_in else None, fc, n, C.byref(out) if with_out else None, layers, C.byref(got)))
+    assert layers[:got.value] == launches
 
 
 def test_network_specs_match_reference_wiring():
@@ -168,6 +197,7 @@ def test_network_plans_its_runs_of_layers_once(monkeypatch):
         calls.extend(run)
 
     monkeypatch.setattr(nets, "fc_runs", counted)
+    monkeypatch.setattr(nets, "fc_launches", lambda run: [run])
     monkeypatch.setattr(nets, "forward_fc_run", together)
     fc = [layers.Fc128LayerParam("Fc%d" % i, 8, 64, 64) for i in range(2)]
     out = layers.Out128LayerParam("Fout", 8, 64, 10)

@@ -125,18 +125,19 @@ def test_fc128_activations_through_lds(gpu, b, k, n):
     fin.release()
 
 
-@pytest.mark.parametrize("b,widths,with_in,with_out", [
+@pytest.mark.parametrize("b,widths,with_in,with_out,launches", [
     # one image and neuron; ends of words, tiles and groups of K; a wave's second tiles and second round of tiles; activations
-    # of 2048 (two requests of weights ahead, 64 KB of LDS)
-    (1, (5, 3, 2), True, True), (33, (100, 33, 31, 10), True, True), (31, (1023, 544, 40), True, True),
-    (32, (1024, 512, 513, 96), True, True), (70, (257, 2048, 160, 1000), True, True), (64, (512, 2048, 129), True, True),
-    (257, (784, 1024, 1024, 1024, 10), True, True), (40, (2048, 96, 2048), False, True), (40, (300, 260, 64), True, False),
-    (9, (130, 70, 66), False, False),
-    # more layers than one launch takes; a layer that is too wide, or wide for so few images, between two that are not
-    (12, (64,) * 11 + (7,), True, True), (20, (96, 2080, 64, 64, 5), True, True), (20, (96, 2048, 1024, 64, 5), True, True)])
-def test_fc_chain(gpu, b, widths, with_in, with_out):
-    """A run of fully connected layers in one launch: every layer's output, thresholds met exactly and none."""
-    from tcbnn_amd.layers import forward_fc_run
+    # of 2048 (two requests of weights ahead, 64 KB of LDS); outputs of several rounds of tiles
+    (1, (5, 3, 2), True, True, [3]), (33, (100, 33, 31, 10), True, True, [4]), (31, (1023, 544, 40), True, True, [3]),
+    (32, (1024, 512, 513, 96), True, True, [4]), (4097, (257, 2048, 160, 1000), True, True, [4]), (2050, (512, 2048, 129), True, True, [3]),
+    (257, (784, 1024, 1024, 1024, 10), True, True, [5]), (8191, (2048, 96, 2048), False, True, [2]), (40, (300, 260, 64), True, False, [3]),
+    (9, (130, 70, 66, 40), False, False, [3]),
+    # more layers than one launch takes; a layer that is too wide, or wide for so few images, in front of some that are not
+    (12, (64,) * 11 + (7,), True, True, [9, 3]), (20, (96, 2080, 64, 64, 64, 5), True, True, [1, 1, 1, 3]),
+    (20, (96, 2048, 2048, 2048, 64, 64, 5), True, True, [1, 1, 1, 1, 3])])
+def test_fc_chain(gpu, b, widths, with_in, with_out, launches):
+    """A run of fully connected layers in few launches: every layer's output, thresholds met exactly and none."""
+    from tcbnn_amd.layers import fc_launches, forward_fc_run
     r = rng(b + sum(widths))
     x = r.standard_normal((b, widths[0])).astype(np.float32)
     x[0, :3] = [0.0, -0.0, np.nan]
@@ -161,7 +162,9 @@ def test_fc_chain(gpu, b, widths, with_in, with_out):
         layer.get_output_gpu().fill(0x55)
     if not with_in:
         layers[0].forward()
-    forward_fc_run(layers if with_in else layers[1:])
+    run = layers if with_in else layers[1:]
+    assert [len(part) for part in fc_launches(run)] == launches
+    forward_fc_run(run)
     gpuops.sync()
     for layer, w in zip(layers, want):
         np.testing.assert_array_equal(layer.download_packed() if hasattr(layer, "download_packed") else layer.download_output(), w)
