@@ -9,7 +9,7 @@
 //
 // The layers of the networks go to the matrix cores (inconv_mfma.hip, inconv_mfma_ring.hip, same bits and residuals); the kernels here serve what
 // that file has no instantiation for (other filter heights and poolings, channels that are no multiple of 64 or, at 11x11,
-// of 32, strides outside its forms, tensors of 2 GiB) and packed input:
+// of 32, strides other than 4 at 11x11, tensors of 2 GiB) and packed input:
 //   inconv_tiled_kernel (pool 1x1, or a pool_w of at most 2 without a residual): workgroup = one output row y, 4 consecutive output
 //     columns, 64 images (lane = image); a wave owns two of the columns and 32 of the 64 output
 //     channels of a pass.  For each filter row the needed

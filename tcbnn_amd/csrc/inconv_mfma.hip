@@ -80,7 +80,8 @@ constexpr int kBatch = 16;     // ... and recomputes at a time
 constexpr int kManyInLane = 8, kManyLanes = 28, kManyLanesChecked = 32;
 
 // A wave walks down the input, A rows (the stride) at a time, and an input row is multiplied for every output row that it is
-// part of while it is in registers: sets_of(R, A) sums are under way, the oldest of which is finished by the step.
+// part of while it is in registers: sets_of(R, A) sums are under way, the oldest of which is finished by the step.  A = R: a step
+// loads the window of its output row whole, and the next one's begins a stride (of any size) further down.
 constexpr int sets_of(int r, int a) { return (r + a - 1) / a; }
 // The K order of a step.  A "pair" is one of its rows in one channel: 3 A of them, the even ones for lane half 0, the odd ones
 // for half 1.  A lane loads a pair's T taps at once and gives each pair slots_of(T) places of its stream; every eight places
@@ -115,7 +116,7 @@ struct Order {
     }
 };
 // Registers: sums of sets_of() rows x 64 channels, taps of the next rows
-constexpr int waves_per_simd(int r, int a) { return sets_of(r, a) <= 2 ? 3 : (r == 3 ? 3 : 2); }
+constexpr int waves_per_simd(int r, int t, int a) { return r == 3 || (t == 7 && sets_of(r, a) == 2) ? 3 : 2; }
 constexpr int waves_of(int r) { return r > 7 ? 8 : 4; }  // of a workgroup: they share the LDS copy of the weight fragments
 constexpr int MT = 2;  // channel tiles of 32 that a wave multiplies
 
@@ -225,20 +226,20 @@ __device__ __forceinline__ void load_taps(__amdgpu_buffer_rsrc_t rsrc, unsigned 
 }
 
 template <int R, int T, int A, int RES, int POOL>
-__global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(R, A)))) void inconv_mfma_kernel(
+__global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(R, T, A)))) void inconv_mfma_kernel(
     const KernelArgs args) {
     const SeldomArgs args_at = (SeldomArgs)__builtin_amdgcn_kernarg_segment_ptr();
     const InConvParams& p = args.p;
     const Geometry& q = args.q;
     static_assert(!(RES != RES_NONE && POOL > 1), "residuals of un-pooled layers only");
-    static_assert(bound_place_free(A, T), "-E needs a place of its own");
     constexpr int kWaves = waves_of(R), kPairs = pairs_of(A), P = slots_of(T), KS = steps_of(A, T), D = sets_of(R, A);
-    constexpr int kRing = (R == 3 || A == 2 ? kPairs : 3);  // pairs in registers
+    constexpr int kRing = (R == 3 || A == 2 || D == 1 ? kPairs : 3);  // pairs in registers
     static_assert(kPairs % kRing == 0, "a pair's place does not depend on the step");
     constexpr unsigned kOutOfRange = 0x80000000u;
     constexpr int kChannels = 32 * MT;
     // Where no residual is saved the sums start from the threshold's negative: the bit is the sum's sign.
     constexpr bool kFromThreshold = RES == RES_NONE;
+    constexpr bool kBoundInSum = !kFromThreshold && bound_place_free(A, T);  // (else -E is added at the end)
     using order = Order<R, T, A>;
     constexpr bool kParts = T == 7 && !kFromThreshold;  // E by the sums before each rounding
     extern __shared__ __align__(16) char lds[];
@@ -259,6 +260,7 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
 
     const int g = work % q.groups;
     work /= q.groups;
+    const int advance = D == 1 ? p.stride_h : A;  // input rows from one output row's to the next one's
     const int band = work % q.bands, it = work / q.bands;
     int cy = band * q.band_rows;  // convolution row
     const int cy_end = min(cy + q.band_rows, q.rows);
@@ -338,7 +340,7 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
 
     // ---- The first rows are on their way while the weights are laid out.
 #pragma unroll
-    for (int i = 0; i < kRing; ++i) load(cy * A - p.pad_h, path_of(cy * A - p.pad_h), i);
+    for (int i = 0; i < kRing; ++i) load(cy * advance - p.pad_h, path_of(cy * advance - p.pad_h), i);
     // ---- signs of the channel group's filters (pattern 4 neg0 + 2 neg1 + neg2 of a tap; four channels to a load), thresholds (NaN:
     // -infinity, the bit is 1 either way)
     bool steps_256 = true;  // every threshold a multiple of 1/256 (below 2^15), or infinite: exact sums stay exact less these
@@ -379,7 +381,7 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
                 const int place = 8 * k + j, pair = 2 * (place / P) + h, tap = place % P, row = pair / 3;
                 const bool used = (tap < p.S) & (tap < T) & (pair < 3 * A) & (d * A + row < R);
                 half[j] = used ? 0x3c00u | (pt[j] << (13 + pair - 3 * row) & 0x8000u) : 0u;
-                if (!kFromThreshold && j == kBoundPlace && d == D - 1 && k == KS - 1 && h == 1) half[j] = 0x3c00u;
+                if (kBoundInSum && j == kBoundPlace && d == D - 1 && k == KS - 1 && h == 1) half[j] = 0x3c00u;
             }
             v4i f;
 #pragma unroll
@@ -496,7 +498,7 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
         asm volatile("" : "+v"(ln));  // (nothing derived from it is kept outside)
         const int h = ln >> 5, img = ln & (NI - 1), xc = g * NX + ((ln & 31) >> a->q.ni_log2);
         const bool valid = b0 + img < p.B && xc < xcols;
-        const int ax0 = xc * p.stride_w - p.pad_w, ay0 = cy * A - p.pad_h, r_end = min(R, p.H - ay0);
+        const int ax0 = xc * p.stride_w - p.pad_w, ay0 = cy * advance - p.pad_h, r_end = min(R, p.H - ay0);
         const unsigned im = (unsigned)img * 3u * plane_b, flip = (unsigned)h << 31;
         uint32_t undecided = 0u;
         const int o0 = tile0 * 32 + mfma::row_to_channel(ln & 31);
@@ -605,7 +607,7 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
             }
             if (!loaded) {  // uniform
 #pragma unroll
-                for (int i = 0; i < kRing; ++i) load(block * A - p.pad_h, path_of(block * A - p.pad_h), i);
+                for (int i = 0; i < kRing; ++i) load(block * advance - p.pad_h, path_of(block * advance - p.pad_h), i);
             }
             loaded = false;
         }
@@ -628,12 +630,13 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
             asm volatile("" : "+v"(ln));
             uint32_t undecided = 0u;
             if constexpr (!kOrdered) {
-                const int ay = block * A - p.pad_h, done = block - (D - 1);  // (uniform)
+                const int ay = block * advance - p.pad_h, done = block - (D - 1);  // (uniform)
                 const bool more = done + 1 < cy_end;
-                const int path = path_of(ay), next_path = path_of(ay + A);
+                const int path = path_of(ay), next_path = path_of(ay + advance);
                 // Sums of |x| (and what is off the grid): of the step's rows, and of those that the oldest set has weights for; and
                 // these sums before each rounding, added up.
                 float step_sum = 0.0f, step_off = 0.0f, step_parts = 0.0f, old_sum = 0.0f, old_off = 0.0f, old_parts = 0.0f, two_e = 0.0f;
+                [[maybe_unused]] float lowered = 0.0f;  // E, where it is not one of the products
                 bool bad = false, small = false;  // small: |S| and |acc| are below 1/2, the residual is 0
 #pragma unroll
                 for (int k = 0; k < KS; ++k) {
@@ -687,7 +690,7 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
                         if (i + kRing < kPairs)
                             load(ay, path, i + kRing);
                         else if (more)  // uniform
-                            load(ay + A, next_path, i + kRing - kPairs);
+                            load(ay + advance, next_path, i + kRing - kPairs);
                     }
                     if (k == KS - 1) {
 #pragma unroll
@@ -714,8 +717,9 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
                         if constexpr (kFromThreshold) {
                             two_e = exact ? 0.0f : e;
                         } else {
-                            two_e = 2.002f * (float)eh;
-                            if (lane >= 32) hi[kBoundPlace / 2] |= (int)((uint32_t)(__builtin_bit_cast(uint16_t, eh) | 0x8000u) << 16);
+                            lowered = (float)eh;
+                            two_e = 2.002f * lowered;
+                            if (kBoundInSum && lane >= 32) hi[kBoundPlace / 2] |= (int)((uint32_t)(__builtin_bit_cast(uint16_t, eh) | 0x8000u) << 16);
                         }
                     }
                     // lo, then hi; the first product of a step moves a set's sums on to the next.  A set's weights are read while the
@@ -727,7 +731,7 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
 #pragma unroll
                         for (int m = 0; m < MT; ++m) a[m] = weights[m];
                         read_weights(d > 0 ? d - 1 : D - 1, d > 0 ? k : (k + 1) % KS);
-                        if ((R != 7 || A == 2) && (block - d < first_row || block - d >= cy_end)) continue;  // uniform: not a row of this band
+                        if (D > 1 && (R != 7 || (A == 2 && T == 7)) && (block - d < first_row || block - d >= cy_end)) continue;  // uniform: not a row of this band
 #pragma unroll
                         for (int m = 0; m < MT; ++m) {
                             v16f c = acc[d][m];
@@ -756,6 +760,12 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
                 // (An input outside the fp16 range has an infinity in hi and another in lo: no sum of its window is a number then,
                 // and none of a window whose rows only met zero weights with it.)
                 bad |= acc[D - 1][0][0] != acc[D - 1][0][0];
+                if constexpr (!kFromThreshold && !kBoundInSum) {
+#pragma unroll
+                    for (int m = 0; m < MT; ++m)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) acc[D - 1][m][i] -= lowered;
+                }
                 // ---- bits (MSB first; the sign of S - E - bn, inverted), residual, doubtful values
                 asm volatile("" : "+v"(ln));
                 const int h = ln >> 5;
@@ -914,9 +924,14 @@ struct Choice {
     long long out_bytes, res_bytes;
 };
 
-// The instantiation for a problem's form, if there is one: what the networks' first layers need.  (For other forms, 5x5
-// filters, pooled 3x3, 32-channel 7x7 layers, other strides, there is none and nothing has been measured: the kernels of
-// inconv.hip serve them.)  Filters narrower than the instantiation's row are served tap by tap.
+// The instantiation for a problem's form, if there is one: what the networks' first layers need (3- and 7-row filters with strides of 1
+// and 2, 2 and 4), and for other strides of such filters one that loads each window whole.  (For other forms, 5x5 filters, pooled
+// 3x3, 32-channel 7x7 layers, there is none and nothing has been measured: the kernels of inconv.hip serve them.)  Filters
+// narrower than the instantiation's row are served tap by tap.
+// Windows loaded whole, 64 channels, 224x224, batch 64, us, inconv.hip -> here, without and with a residual: 3x3/3 26.1 -> 13.8, 29.5 ->
+// 21.4; 3x3/5 16.1 -> 8.9, 17.6 -> 13.8; 3x4/2 44 -> 24.7, 52 -> 41.2; 7x7/3 82 -> 41.7, 84 -> 52; 7x7/1 400 -> 274, 415 -> 327; 7x8/3 91 -> 43,
+// 93 -> 56; batch 8, 3x3/3 29.8 -> 6.2.  7x8 filters at strides 2 and 4 share rows: 152 -> 64, 155 -> 90 and 53 -> 25.6, 56 -> 37 (windows
+// loaded whole 83, 107, 30, 41).
 bool instantiated(const InConvParams& p, int cus, Choice* out) {
     Choice& c = *out;
     c.r = p.R;
@@ -924,10 +939,12 @@ bool instantiated(const InConvParams& p, int cus, Choice* out) {
     c.res = p.res == nullptr ? RES_NONE : (p.res_fmt == TCBNN_RES_I12 ? RES_12 : RES_WIDE);
     const bool pooled = p.pool_h != 1 || p.pool_w != 1;
     if (p.O % 64 != 0) return false;
-    if (p.R == 3 && p.S <= 4 && !pooled && (c.a == 1 || (c.a == 2 && p.S <= 3))) {
+    if (p.R == 3 && p.S <= 4 && !pooled) {
         c.t = p.S <= 3 ? 3 : 4, c.pool = 1;
-    } else if (p.R == 7 && p.S <= 7 && !pooled && (c.a == 4 || c.a == 2)) {
-        c.t = 7, c.pool = 1;
+        if (c.a > 2 || (c.a == 2 && c.t == 4)) c.a = 3;
+    } else if (p.R == 7 && p.S <= 8 && !pooled) {
+        c.t = p.S <= 7 ? 7 : 8, c.pool = 1;
+        if (c.a != 2 && c.a != 4) c.a = 7;
     } else if (p.R == 11 && p.S <= 11 && p.pool_h == 2 && p.pool_w == 2 && c.res == RES_NONE && c.a == 4) {
         // Thirteen tiles of a row per compute unit or more: below that, and for 32 channels, the ring in LDS is faster
         // (inconv_mfma_ring.hip has both sides' times).
@@ -965,7 +982,7 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     const bool large = 12LL * p.H * p.W * p.B + c.out_bytes + c.res_bytes >= 96LL << 20;
     double best = 1e30;
     int imgtiles = 0;
-    const long long target = std::max(1LL, (long long)cus * 4 * waves_per_simd(c.r, c.a) / q.cgroups);  // resident waves
+    const long long target = std::max(1LL, (long long)cus * 4 * waves_per_simd(c.r, c.t, c.a) / q.cgroups);  // resident waves
     const int most = c.res == RES_NONE && c.pool == 1 && (long long)p.B * xcols * q.rows / 32 >= 32 * target ? 4 : 3;
     for (int ni_log2 = most; ni_log2 >= 0; --ni_log2) {
         const int NI = 1 << ni_log2, NX = 32 >> ni_log2;
@@ -1006,7 +1023,7 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     // E (see the top of this file)
     const double T = q.rs_taps, u = std::ldexp(1.0, -24) * 1.02;
     q.bound_parts = (float)u;
-    q.bound_sum = (float)((13.5 + (c.t == 7 && c.res != RES_NONE ? 0.0 : T + 4.0 * steps)) * u);
+    q.bound_sum = (float)((13.5 + (bound_place_free(c.a, c.t) ? 0.0 : 1.0) + (c.t == 7 && c.res != RES_NONE ? 0.0 : T + 4.0 * steps)) * u);
     q.bound_add = (float)(3.0 * T * std::ldexp(1.0, -24) + std::ldexp(1.0, -22));
     *out = c;
     return true;
@@ -1069,11 +1086,16 @@ int launch_inconv_mfma(const InConvParams& p, hipStream_t stream, bool* served) 
     auto with_residual = [&](auto go) { return c.res == RES_12 ? go(std::integral_constant<int, RES_12>{}) : (c.res == RES_WIDE ? go(std::integral_constant<int, RES_WIDE>{}) : go(std::integral_constant<int, RES_NONE>{})); };
     if (c.r == 3)
         return with_residual([&](auto res) {
-            return c.t == 4 ? launch<3, 4, 1, decltype(res)::value, 1>(p, c, dev, stream)
-                            : (c.a == 1 ? launch<3, 3, 1, decltype(res)::value, 1>(p, c, dev, stream) : launch<3, 3, 2, decltype(res)::value, 1>(p, c, dev, stream));
+            constexpr int RES = decltype(res)::value;
+            if (c.t == 4) return c.a == 1 ? launch<3, 4, 1, RES, 1>(p, c, dev, stream) : launch<3, 4, 3, RES, 1>(p, c, dev, stream);
+            return c.a == 1 ? launch<3, 3, 1, RES, 1>(p, c, dev, stream) : (c.a == 2 ? launch<3, 3, 2, RES, 1>(p, c, dev, stream) : launch<3, 3, 3, RES, 1>(p, c, dev, stream));
         });
     if (c.r == 7)
-        return with_residual([&](auto res) { return c.a == 4 ? launch<7, 7, 4, decltype(res)::value, 1>(p, c, dev, stream) : launch<7, 7, 2, decltype(res)::value, 1>(p, c, dev, stream); });
+        return with_residual([&](auto res) {
+            constexpr int RES = decltype(res)::value;
+            if (c.t == 8) return c.a == 4 ? launch<7, 8, 4, RES, 1>(p, c, dev, stream) : (c.a == 2 ? launch<7, 8, 2, RES, 1>(p, c, dev, stream) : launch<7, 8, 7, RES, 1>(p, c, dev, stream));
+            return c.a == 4 ? launch<7, 7, 4, RES, 1>(p, c, dev, stream) : (c.a == 2 ? launch<7, 7, 2, RES, 1>(p, c, dev, stream) : launch<7, 7, 7, RES, 1>(p, c, dev, stream));
+        });
     return launch<11, 11, 4, RES_NONE, 2>(p, c, dev, stream);
 }
 

@@ -1081,6 +1081,34 @@ def test_inconv128_areas_in_doubt(gpu, b, h, w, R, S, stride, cout, pool, save, 
         layer.release()
 
 
+@pytest.mark.parametrize("kind", ["random", "quantised", "grey", "special"])
+@pytest.mark.parametrize("b,h,w,R,S,stride,cout,save", [
+    # strides that rows are not shared at; a tap more than the other forms have; frames as wide as a window, and narrower
+    (9, 31, 34, 3, 3, 3, 64, True), (33, 22, 22, 3, 3, 3, 128, False), (5, 40, 37, 3, 4, 2, 64, True), (70, 9, 4, 3, 4, 3, 64, True),
+    (3, 30, 50, 7, 8, 2, 64, True), (17, 33, 8, 7, 8, 4, 64, True), (2, 60, 45, 7, 8, 4, 128, False), (40, 16, 5, 7, 8, 2, 64, False),
+    (3, 40, 41, 7, 7, 6, 64, True), (9, 30, 33, 7, 7, 3, 64, False), (5, 30, 33, 7, 8, 3, 64, True), (4, 12, 12, 7, 7, 1, 64, True),
+    (6, 25, 26, 3, 3, 5, 64, True), (6, 40, 40, 7, 7, 9, 64, True), (2, 3, 9, 7, 8, 3, 64, True)])
+def test_inconv128_windows_loaded_whole(gpu, b, h, w, R, S, stride, cout, save, kind):
+    """First layers whose rows are loaded anew for every output row, on the matrix cores too."""
+    r = rng(8000 + b + h + w + S)
+    x = r.standard_normal((b, 3, h, w)).astype(np.float32) if kind == "random" else _flat_images(r, b, h, w, kind)
+    f = rm.pm1(r, (R, S, 3, cout))
+    bn = r.normal(0, np.sqrt(3 * R * S), cout).astype(np.float32)
+    bn[:8] = [0.0, -0.0, np.nan, np.inf, -np.inf, 1.0, -2.0, 0.5]
+    with np.errstate(all="ignore"):
+        want, wres = orc.inconv128(x, f, bn, stride, True, 1, save)
+    for fmt in ([None, gpu._lib.RES_I32] if save else [None]):
+        layer = gpu.InConv128LayerParam("Conv1", h, w, R, S, 3, cout, b, stride, stride, True, 1, 1, save, residual_format=fmt)
+        layer.initialize(x, gpu.ArrayWeights([f, bn]))
+        assert layer.kernel_name().startswith("inconv_mfma_kernel<%d, %d, " % (R, S)), layer.kernel_name()
+        layer.forward()
+        gpuops.sync()
+        np.testing.assert_array_equal(layer.download_packed(), want)
+        if save:
+            np.testing.assert_array_equal(layer.download_residual(), wres)
+        layer.release()
+
+
 def test_inconv128_time_does_not_hang_on_the_images(gpu):
     """Bars and patches of +-1 over a third of the images cost next to nothing over random ones, and images of which every
     sum is in doubt a small factor (one by one, sums in doubt took 70 and 130 times as long)."""
