@@ -141,7 +141,6 @@ struct Geometry {
     int cgroups;             // channel groups (of 64)
     int total, per_xcd;      // waves' work units (image tile, band, column group), and those of an XCD
     int rs_taps;
-    unsigned s_magic;        // tap / S == tap * s_magic >> 16 for every tap
     float bound_parts;       // E = bound_parts * (the sum of |x| before each rounding) + bound_sum * (the sum of |x|) + bound_add
     float bound_sum;
     float bound_add;
@@ -307,7 +306,7 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
     // when the taps are used (not in the first and last rows: what is in front of the first one's taps, or behind the last
     // one's, need not be the tensor's); tap by tap.
     enum Path : int { INSIDE, ROWS, COLUMNS, TAPS };
-    const bool columns_masked = p.S == T && p.W >= T;
+    const bool columns_masked = p.W >= T;
     auto path_of = [&](int ay) __attribute__((always_inline)) -> int {
         if (columns_inside) return ay >= 0 && ay + A <= p.H ? INSIDE : ROWS;
         return columns_masked && ay > 0 && ay + A < p.H ? COLUMNS : TAPS;
@@ -927,7 +926,8 @@ struct Choice {
 // The instantiation for a problem's form, if there is one: what the networks' first layers need (3- and 7-row filters with strides of 1
 // and 2, 2 and 4), and for other strides of such filters one that loads each window whole.  (For other forms, 5x5 filters, pooled
 // 3x3, 32-channel 7x7 layers, there is none and nothing has been measured: the kernels of inconv.hip serve them.)  Filters
-// narrower than the instantiation's row are served tap by tap.
+// narrower than the instantiation's row have the taps beyond masked, like columns outside the frame (loaded tap by tap the
+// 7x6/4 layer took 32.6 us for 26.3, 7x5/2 58 for 52).
 // Windows loaded whole, 64 channels, 224x224, batch 64, us, inconv.hip -> here, without and with a residual: 3x3/3 26.1 -> 13.8, 29.5 ->
 // 21.4; 3x3/5 16.1 -> 8.9, 17.6 -> 13.8; 3x4/2 44 -> 24.7, 52 -> 41.2; 7x7/3 82 -> 41.7, 84 -> 52; 7x7/1 400 -> 274, 415 -> 327; 7x8/3 91 -> 43,
 // 93 -> 56; batch 8, 3x3/3 29.8 -> 6.2.  7x8 filters at strides 2 and 4 share rows: 152 -> 64, 155 -> 90 and 53 -> 25.6, 56 -> 37 (windows
@@ -967,9 +967,6 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     c.res_bytes = p.res != nullptr ? (long long)tcbnn_residual_bytes(p.PH, p.PW, p.O, p.B, p.res_fmt) : 0;
     if (c.out_bytes >= (1LL << 31) || c.res_bytes >= (1LL << 31)) return false;
     q.rs_taps = p.R * p.S;
-    q.s_magic = 65536u / (unsigned)p.S + 1u;
-    for (int t = 0; t < q.rs_taps; ++t)
-        if ((int)((unsigned)t * q.s_magic >> 16) != t / p.S) return false;
     const int waves = waves_of(c.r), xcols = c.pool > 1 ? c.pool * p.OW : p.PW, sets = sets_of(c.r, c.a), steps = sets * steps_of(c.a, c.t);
     q.cgroups = p.O / (32 * MT);
     q.rows = c.pool * p.OH;
