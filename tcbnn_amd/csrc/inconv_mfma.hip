@@ -32,9 +32,11 @@
 // Many values in doubt.  A saved residual puts every sum ON an integer in doubt, and images have areas of such sums: bars of
 // +-1 after scaling to [-1, 1], saturated white, bytes, a flat grey of 0.2 (every fifth channel); and E grows with the
 // magnitudes: bytes less a mean leave 7 % of the sums in doubt, values in the thousands all of them.
-//   grid    : sums of a window whose inputs are multiples of 1/256 (bytes, bytes / 128 - 1, +-1) with a sum of |x| below 2^15
+//   grid    : sums of a window whose inputs are multiples of 1/256 (bytes, bytes / 128 - 1, +-1) with a sum of |x| below 2^16
 //             are exact in both orders: every partial sum is a multiple of 1/256 below 2^24 / 256, and the two halves hold
-//             the inputs.  E is 0.  (Sums that start from -bn: if all thresholds are such multiples too.)
+//             inputs below 2^15 (a lane's |x| of a step add up to less than that).  E is 0.  (Sums that start from -bn: below 2^15,
+//             if all thresholds are such multiples too.  With 2^15 for all, windows of bytes above 223 were in doubt: 7x7/4
+//             293 us for 113, 7x7/2 1110 for 351.)
 //   check   : a wave looks whether its inputs are on that grid (120 VALU instructions per item of 7-row filters) as long as all
 //             have been; other inputs pay for their first item.  From an item with many values in doubt on it always looks.
 //   ordered : from an item that has many even so, sums in the reference's order, 32 columns x 64 channels at a time, as fp32
@@ -692,6 +694,10 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
                             load(ay + advance, next_path, i + kRing - kPairs);
                     }
                     if (k == KS - 1) {
+                        if (check) {  // uniform; an input of 2^15 or more can have more bits than the halves hold
+                            step_off = step_sum < 32768.0f ? step_off : 1.0f;
+                            old_off = old_sum < 32768.0f ? old_off : 1.0f;
+                        }
 #pragma unroll
                         for (int d = D - 1; d > 0; --d) {
                             const bool old = d == D - 1;
@@ -710,7 +716,7 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
                             const auto so = __builtin_amdgcn_permlane32_swap(__float_as_uint(off[D - 1]), __float_as_uint(off[D - 1]), false, false);
                             exact = (so[0] | so[1]) == 0u;
                             if (!keep_checking && done >= cy && __ballot(!exact) != 0) check = false;
-                            exact = exact & (all < 3.2e4f) & (steps_256 || !kFromThreshold);  // (below 2^15: 23 bits, which the halves hold)
+                            exact = exact & (kFromThreshold ? (all < 3.2e4f) & steps_256 : all < 6.5e4f);  // (with a threshold: below 2^16 together)
                         }
                         if (exact | bad) eh = (_Float16)0.0f;  // (bad: nothing infinite may meet the other sets' zeros)
                         if constexpr (kFromThreshold) {

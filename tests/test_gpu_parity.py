@@ -1189,7 +1189,11 @@ def test_inconv128_thresholds_at_the_ordered_sums(gpu, b, h, R, stride, pool, ki
     (8, 24, 24, 7, 4, 64, 1, True, "large_grid"), (16, 21, 20, 3, 2, 64, 1, False, "grid"), (16, 21, 20, 3, 1, 64, 1, False, "grid"),
     (62, 60, 60, 11, 4, 512, 2, False, "grid"), (16, 21, 20, 3, 1, 64, 1, False, "near_grid"),
     # sums on their thresholds all over the frame
-    (62, 61, 57, 11, 4, 512, 2, False, "flat")])
+    (62, 61, 57, 11, 4, 512, 2, False, "flat"),
+    # bytes whose windows add up to more than 2^15, and single inputs of 23 and 24 bits in windows on either side of 2^16
+    (8, 30, 26, 7, 4, 64, 1, True, "bright"), (5, 26, 31, 7, 2, 64, 1, True, "bright"), (5, 26, 31, 7, 3, 64, 1, True, "bright"),
+    (8, 30, 26, 7, 4, 64, 1, True, "heavy_grid"), (5, 26, 31, 7, 2, 64, 1, True, "heavy_grid"), (16, 21, 20, 3, 1, 64, 1, True, "heavy_grid"),
+    (16, 21, 20, 3, 1, 64, 1, False, "heavy_grid")])
 def test_inconv128_rows_in_flight(gpu, b, h, w, R, stride, cout, pool, save, kind):
     """First-layer sums of several output rows under way at once: the edges of tiles, bands and of what makes a sum exact."""
     r = rng(9000 + b + h + w + R)
@@ -1202,6 +1206,12 @@ def test_inconv128_rows_in_flight(gpu, b, h, w, R, stride, cout, pool, save, kin
     elif kind == "large_grid":
         x = np.rint(x * 256).astype(np.float32) / 256
         x[r.random(x.shape) < 0.01] = np.float32(50000 + 1 / 256)
+    elif kind == "bright":
+        x = np.rint(255 - 60 * r.random(x.shape)).astype(np.float32)
+    elif kind == "heavy_grid":
+        x = np.rint(x * 256).astype(np.float32) / 256
+        heavy = r.random(x.shape) < 0.01
+        x[heavy] = (r.integers(-2 ** 24, 2 ** 24, int(heavy.sum())) // r.choice([1, 2, 4], int(heavy.sum())) / 256).astype(np.float32)
     elif kind in ("grid", "near_grid"):
         x = np.rint(x).astype(np.float32)
         bn = np.rint(bn).astype(np.float32)
