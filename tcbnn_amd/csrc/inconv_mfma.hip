@@ -40,7 +40,9 @@
 //   check   : a wave looks whether its inputs are on that grid (120 VALU instructions per item of 7-row filters) as long as all
 //             have been; other inputs pay for their first item.  From an item with many values in doubt on it always looks.
 //   ordered : from an item that has many even so, sums in the reference's order, 32 columns x 64 channels at a time, as fp32
-//             products on the matrix cores (ordered_sums): no values in doubt but those that are no numbers.
+//             products on the matrix cores (ordered_sums): no values in doubt but those that are no numbers.  It lasts to the
+//             end of the wave's rows (left as soon as few would be in doubt, the common pass is reached from two places, and
+//             the registers that takes cost 7x7/2 288 -> 328 us on ordinary images).
 // ResNet-18's first layer at batch 256, launched on end, us: normal data 84, bytes / 128 - 1 81, images in [-1, 1] with bars and
 // patches of +-1 over a third 94, bytes / 255 122, a third of 0.2 grey 241, bytes less a mean 320, normal x 1000 325.
 //
@@ -494,7 +496,6 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
     auto ordered_sums = [&](int cy, uint32_t* word) __attribute__((always_inline)) -> uint32_t {
         const SeldomArgs a = seldom_args(args_at);
         const auto& p = a->p;
-        const uint32_t* const pats = a->pats;
         int ln = lane;
         asm volatile("" : "+v"(ln));  // (nothing derived from it is kept outside)
         const int h = ln >> 5, img = ln & (NI - 1), xc = g * NX + ((ln & 31) >> a->q.ni_log2);
@@ -502,62 +503,69 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
         const int ax0 = xc * p.stride_w - p.pad_w, ay0 = cy * advance - p.pad_h, r_end = min(R, p.H - ay0);
         const unsigned im = (unsigned)img * 3u * plane_b, flip = (unsigned)h << 31;
         uint32_t undecided = 0u;
-        const int o0 = tile0 * 32 + mfma::row_to_channel(ln & 31);
         const bool whole = p.S == T && __ballot(valid & ((ax0 < 0) | (ax0 + T > p.W))) == 0;  // uniform
         v16f acc[MT];
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
-        // a filter row at a time, requested one row ahead; out of the frame: zeros, which add nothing
-        float next[3][T];
-        uint32_t next_pt[T][MT];
-        auto request = [&](int r) __attribute__((always_inline)) {
+        // a filter row at a time, requested two rows ahead; out of the frame: zeros, which add nothing
+        float next[2][3][T];
+        auto request = [&](int r, int slot) __attribute__((always_inline)) {
             const unsigned at0 = im + (unsigned)((ay0 + r) * p.W + ax0) * 4u;
             if (whole) {
 #pragma unroll
-                for (int ch = 0; ch < 3; ++ch) load_taps<T>(rsrc, valid ? at0 : kOutOfRange, ch * plane_b, next[ch]);
+                for (int ch = 0; ch < 3; ++ch) load_taps<T>(rsrc, valid ? at0 : kOutOfRange, ch * plane_b, next[slot][ch]);
             } else {
 #pragma unroll
                 for (int t = 0; t < T; ++t) {
-                    const bool inside = valid & (ax0 + t >= 0) & (ax0 + t < p.W);
+                    const bool inside = valid & (t < p.S) & (ax0 + t >= 0) & (ax0 + t < p.W);
 #pragma unroll
                     for (int ch = 0; ch < 3; ++ch)
-                        next[ch][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(inside ? at0 + 4u * t : kOutOfRange), (int)(ch * plane_b), 0));
+                        next[slot][ch][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(inside ? at0 + 4u * t : kOutOfRange), (int)(ch * plane_b), 0));
                 }
             }
-            const uint32_t* const row = pats + (unsigned)(r * p.S * p.opad);  // (uniform)
-#pragma unroll
-            for (int t = 0; t < T; ++t)
-#pragma unroll
-                for (int m = 0; m < MT; ++m) next_pt[t][m] = row[(unsigned)(min(t, p.S - 1) * p.opad + o0 + 32 * m)];
         };
         const int r_begin = max(0, -ay0);
-        if (r_begin < r_end) request(r_begin);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            if (r_begin + u < r_end) request(r_begin + u, u);
 #pragma unroll 1
-        for (int r = r_begin; r < r_end; ++r) {
-            float f[3][T];
-            uint32_t pt[T][MT];
+        for (int r0 = r_begin; r0 < r_end; r0 += 2) {
 #pragma unroll
-            for (int t = 0; t < T; ++t) {
+            for (int u = 0; u < 2; ++u) {
+                const int r = r0 + u;
+                if (r >= r_end) break;  // uniform
+                float f[3][T];
+                uint32_t pt[T][MT];
+                const uint8_t* const row_signs = signs + (unsigned)(r * p.S * kChannels) + mfma::row_to_channel(ln & 31);
 #pragma unroll
-                for (int ch = 0; ch < 3; ++ch) f[ch][t] = next[ch][t];
+                for (int t = 0; t < T; ++t) {
 #pragma unroll
-                for (int m = 0; m < MT; ++m) pt[t][m] = next_pt[t][m];
-            }
-            if (r + 1 < r_end) request(r + 1);
+                    for (int m = 0; m < MT; ++m) pt[t][m] = row_signs[min(t, p.S - 1) * kChannels + 32 * m];
 #pragma unroll
-            for (int t = 0; t < T; ++t) {
-                if (t < p.S) {  // uniform
-                    const float f2 = __uint_as_float(__float_as_uint(f[2][t]) ^ flip);
-                    const float same = (f[0][t] + f[1][t]) + f2, other = (f[0][t] - f[1][t]) + f2;
+                    for (int ch = 0; ch < 3; ++ch) f[ch][t] = next[u][ch][t];
+                }
+                if (r + 2 < r_end) request(r + 2, u);
 #pragma unroll
-                    for (int m = 0; m < MT; ++m) {
+                for (int t = 0; t < T; ++t) {
+                    if (T == 3 || t < T - 2 || t < p.S) {  // uniform (narrower filters than that: zeros)
+                        const float f2 = __uint_as_float(__float_as_uint(f[2][t]) ^ flip);
+                        const float same = (f[0][t] + f[1][t]) + f2, other = (f[0][t] - f[1][t]) + f2;
                         // pattern 4 neg0 + 2 neg1 + neg2; a pattern from 4 on is the negative of the inverted one
-                        const uint32_t neg = (uint32_t)((int)(pt[t][m] << 29) >> 31), c = (pt[t][m] ^ neg) & 3u;
-                        const uint32_t one = 0x3f800000u | (neg & 0x80000000u);
-                        acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(c == (uint32_t)h ? one : 0u), same, acc[m], 0, 0, 0);
-                        acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(c == (uint32_t)h + 2u ? one : 0u), other, acc[m], 0, 0, 0);
+                        uint32_t c[MT], one[MT];
+#pragma unroll
+                        for (int m = 0; m < MT; ++m) {
+                            const uint32_t neg = (uint32_t)((int)(pt[t][m] << 29) >> 31);
+                            c[m] = (pt[t][m] ^ neg) & 3u;
+                            one[m] = 0x3f800000u | (neg & 0x80000000u);
+                        }
+#pragma unroll
+                        for (int m = 0; m < MT; ++m)
+                            acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(c[m] == (uint32_t)h ? one[m] : 0u), same, acc[m], 0, 0, 0);
+#pragma unroll
+                        for (int m = 0; m < MT; ++m)
+                            acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(c[m] == (uint32_t)h + 2u ? one[m] : 0u), other, acc[m], 0, 0, 0);
                     }
                 }
             }
