@@ -137,6 +137,9 @@ typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 // Saved residual: none, 12 bits, or 16 / 32 bits (looked up at run time).
 enum Residual : int { RES_NONE = 0, RES_12 = 1, RES_WIDE = 2 };
 
+// What neighbouring work units differ in (after the first: in this order), and whether a workgroup's waves go down their rows in step
+enum Units : int { COLUMNS_BANDS_IMAGES = 0, IMAGES_COLUMNS_BANDS_IN_STEP = 1, IMAGES_BANDS_COLUMNS_IN_STEP = 2 };
+
 struct Geometry {
     int ni_log2;             // images per tile
     int groups;              // tiles across a row
@@ -144,6 +147,8 @@ struct Geometry {
     int rows;                // convolution rows
     int cgroups;             // channel groups (of 64)
     int total, per_xcd;      // waves' work units (image tile, band, column group), and those of an XCD
+    Units units;             // their order
+    int img_tiles;
     int rs_taps;
     float bound_parts;       // E = bound_parts * (the sum of |x| before each rounding) + bound_sum * (the sum of |x|) + bound_add
     float bound_sum;
@@ -261,10 +266,20 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
 
     if (idle) work = 0;  // (such a wave helps with the weights and leaves)
 
-    const int g = work % q.groups;
-    work /= q.groups;
+    constexpr bool kOrders = R == 3 && A == 1 && RES != RES_NONE;  // units in other orders (choose())
+    const bool in_step = kOrders && q.units != COLUMNS_BANDS_IMAGES;  // uniform
+    int g, band, it;
+    if (in_step) {
+        it = work % q.img_tiles;
+        work /= q.img_tiles;
+        if (q.units == IMAGES_COLUMNS_BANDS_IN_STEP) g = work % q.groups, band = work / q.groups;
+        else band = work % q.bands, g = work / q.bands;
+    } else {
+        g = work % q.groups;
+        work /= q.groups;
+        band = work % q.bands, it = work / q.bands;
+    }
     const int advance = D == 1 ? p.stride_h : A;  // input rows from one output row's to the next one's
-    const int band = work % q.bands, it = work / q.bands;
     int cy = band * q.band_rows;  // convolution row
     const int cy_end = min(cy + q.band_rows, q.rows);
     const int NI = 1 << q.ni_log2, NX = 32 >> q.ni_log2, b0 = it << q.ni_log2;
@@ -638,6 +653,8 @@ __global__ __launch_bounds__(64 * waves_of(R)) __attribute__((amdgpu_waves_per_e
             int ln = lane;
             asm volatile("" : "+v"(ln));
             uint32_t undecided = 0u;
+            // (Waves that have ended are not waited for, and every wave gets on without the others or ends.)
+            if (in_step) __builtin_amdgcn_s_barrier();
             if constexpr (!kOrdered) {
                 const int ay = block * advance - p.pad_h, done = block - (D - 1);  // (uniform)
                 const bool more = done + 1 < cy_end;
@@ -980,6 +997,7 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     c.out_bytes = 4LL * p.OH * p.OW * p.ow * p.B;
     c.res_bytes = p.res != nullptr ? (long long)tcbnn_residual_bytes(p.PH, p.PW, p.O, p.B, p.res_fmt) : 0;
     if (c.out_bytes >= (1LL << 31) || c.res_bytes >= (1LL << 31)) return false;
+    const long long bytes = 12LL * p.H * p.W * p.B + c.out_bytes + c.res_bytes;
     q.rs_taps = p.R * p.S;
     const int waves = waves_of(c.r), xcols = c.pool > 1 ? c.pool * p.OW : p.PW, sets = sets_of(c.r, c.a), steps = sets * steps_of(c.a, c.t);
     q.cgroups = p.O / (32 * MT);
@@ -990,7 +1008,7 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     // within a pass, us: batch 148 in fours 178, 133 in ones 208, 150 in twos 239; in sixteens 125-150.  (Batch 100 in
     // fours 94, in sixteens 95; the 7x7/2 layer at batch 28 in fours 42.3, in eights 47.8.)
     constexpr double kFewer[4] = {2.2, 1.65, 1.25, 1.06};
-    const bool large = 12LL * p.H * p.W * p.B + c.out_bytes + c.res_bytes >= 96LL << 20;
+    const bool large = bytes >= 96LL << 20;
     double best = 1e30;
     int imgtiles = 0;
     const long long target = std::max(1LL, (long long)cus * 4 * waves_per_simd(c.r, c.t, c.a) / q.cgroups);  // resident waves
@@ -1029,6 +1047,19 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     if (c.r == 11 && total * 10 < target * 7) return false;
     if (total * q.cgroups > 0x0fffffffLL) return false;
     q.total = (int)total;
+    q.img_tiles = imgtiles;
+    q.units = COLUMNS_BANDS_IMAGES;
+    // Large residuals of 3x3 filters.  Waves that drift apart scatter the 128-byte lines that they write over memory; four tiles of images
+    // that go down the same rows in step write 512 bytes side by side.  Worth it where the launch's bytes nearly fill the
+    // memory-side cache (256 MiB; us within the network's pass, 32x32, 128 channels, batch 768 / 800 / 896 / 1024 / 1100: 64.6 / 72 / 79.6 /
+    // 87.5 / 88 -> 65.6 / 69 / 76.5 / 79.6 / 87), beyond it where the 512 bytes are whole pieces of memory (batch 1600 / 2048: 131 / 172 -> 120 /
+    // 158; others there have no rule: 1200 / 1300 / 3000: 110 / 102 / 244 -> 113.5 / 113 / 247), and, with the bands in front of the
+    // columns, beyond it where frames are wide (on end, 64 channels, 224x224, batch 64 / 128: 150 / 284 -> 131 / 255, 112x112, batch 512:
+    // 289 -> 250, 64x64, batch 1024: 192 -> 177; below it 64x64, batch 512 85 -> 90).
+    if (c.r == 3 && c.a == 1 && c.res != RES_NONE) {
+        if (q.groups < 16 && bytes >= 170LL << 20 && (bytes <= 256LL << 20 || p.B % 32 == 0)) q.units = IMAGES_COLUMNS_BANDS_IN_STEP;
+        if (q.groups >= 16 && bytes > 256LL << 20) q.units = IMAGES_BANDS_COLUMNS_IN_STEP;
+    }
     q.per_xcd = (q.total + 7) / 8;
     c.grid = 8 * ((q.per_xcd + waves - 1) / waves) * q.cgroups;
     // E (see the top of this file)

@@ -1182,6 +1182,9 @@ def test_inconv128_thresholds_at_the_ordered_sums(gpu, b, h, R, stride, pool, ki
     (10, 13, 67, 7, 2, 64, 1, False, "normal"), (300, 9, 7, 3, 1, 128, 1, True, "normal"),
     # enough rows per wave for sixteen images to a tile, the last tile incomplete
     (63, 224, 224, 3, 1, 64, 1, False, "normal"),
+    # residuals so large that waves take neighbouring images and go down the rows in step: narrow and wide frames, last tiles
+    # incomplete, values that make waves take their rows again
+    (803, 32, 32, 3, 1, 128, 1, True, "normal"), (850, 32, 32, 3, 1, 128, 1, True, "flat_third"), (37, 224, 224, 3, 1, 64, 1, True, "flat_third"),
     # inputs at and beyond the end of fp16 in rows that neighbouring windows multiply by zeros
     (17, 23, 29, 7, 2, 128, 1, True, "overflow"), (9, 33, 30, 7, 4, 64, 1, True, "overflow"),
     (62, 61, 57, 11, 4, 512, 2, False, "overflow"), (9, 20, 20, 3, 2, 64, 1, True, "overflow"),
@@ -1206,6 +1209,8 @@ def test_inconv128_rows_in_flight(gpu, b, h, w, R, stride, cout, pool, save, kin
     elif kind == "large_grid":
         x = np.rint(x * 256).astype(np.float32) / 256
         x[r.random(x.shape) < 0.01] = np.float32(50000 + 1 / 256)
+    elif kind == "flat_third":
+        x[::3, :, : h // 2, : w // 2] = np.float32(0.2)
     elif kind == "bright":
         x = np.rint(255 - 60 * r.random(x.shape)).astype(np.float32)
     elif kind == "heavy_grid":
