@@ -998,6 +998,10 @@ bool choose(const InConvParams& p, int cus, Choice* out) {
     c.res_bytes = p.res != nullptr ? (long long)tcbnn_residual_bytes(p.PH, p.PW, p.O, p.B, p.res_fmt) : 0;
     if (c.out_bytes >= (1LL << 31) || c.res_bytes >= (1LL << 31)) return false;
     const long long bytes = 12LL * p.H * p.W * p.B + c.out_bytes + c.res_bytes;
+    // Residuals of more than the memory-side cache holds (256 MiB with the rest) at few products a byte: the VALU kernel, whose waves
+    // store 64 images side by side (3x3/3 at 224x224, batch 128 / 256 / 512: there 43 / 78 / 158 us, here 36 / 93 / 182; 3x4/2, batch 256: 162
+    // and 201; 3x3/4, batch 512: 90 and 119).
+    if (c.r == 3 && sets_of(c.r, c.a) == 1 && c.res != RES_NONE && bytes > 256LL << 20 && p.B % 64 == 0) return false;
     q.rs_taps = p.R * p.S;
     const int waves = waves_of(c.r), xcols = c.pool > 1 ? c.pool * p.OW : p.PW, sets = sets_of(c.r, c.a), steps = sets * steps_of(c.a, c.t);
     q.cgroups = p.O / (32 * MT);
