@@ -356,7 +356,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ROWS &
 #pragma unroll
                 for (int k = 0; k < NST; ++k) {
                     const int e = tid + k * kThreads;
-                    const int bc = (int)(((unsigned)e * (unsigned)div_magic) >> 16);
+                    const int bc = (int)(((unsigned)e * (unsigned)div_magic) >> 20);
                     const int col = e - bc * ncols;
                     const int ax = ax_base + col;
                     const int bb = min(b0 + (bc & 63), p.B - 1);
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ROWS &
 #pragma unroll
                 for (int k = 0; k < NST; ++k) {
                     const int e = tid + k * kThreads;
-                    const int bc = (int)(((unsigned)e * (unsigned)div_magic) >> 16);
+                    const int bc = (int)(((unsigned)e * (unsigned)div_magic) >> 20);
                     const int col = e - bc * ncols;
                     if (e < n_stage) tile[(col * 3 + (bc >> 6)) * kLB + (bc & 63)] = stg[k];
                 }
@@ -838,11 +838,12 @@ static int inconv128_run(const tcbnn_inconv128_desc* d, void* stream, char* name
         return TCBNN_OK;
     }
     if (tiled) {
-        // e / ncols == (e * magic) >> 16 for every e the staging loop uses
+        // e / ncols == (e * magic) >> 20 for every e that the staging loop uses: with ncols at most kMaxCols, e is at most 6143, e * magic
+        // below 2^32 and the magic's excess times e below 2^20 / kMaxCols.  (Sixteen bits do not do for 25 columns, 7x7 filters at stride 6.)
         const int ncols = (kXT - 1) * p.stride_w + p.S;
-        const int div_magic = 65536 / ncols + 1;
+        const int div_magic = (1 << 20) / ncols + 1;
         for (int e = 0; e < 3 * 64 * ncols; ++e)
-            TCBNN_REQUIRE((int)(((unsigned)e * (unsigned)div_magic) >> 16) == e / ncols,
+            TCBNN_REQUIRE((int)(((unsigned)e * (unsigned)div_magic) >> 20) == e / ncols,
                           "inconv128: internal error (division constant)");
         const InConvOrder o = inconv_order(p, pooled, rows_out);
         TCBNN_REQUIRE(o.ok, "inconv128: grid too large");

@@ -1109,6 +1109,23 @@ def test_inconv128_windows_loaded_whole(gpu, b, h, w, R, S, stride, cout, save, 
         layer.release()
 
 
+@pytest.mark.parametrize("R,S,stride", [(7, 7, 6), (7, 8, 6), (5, 7, 6), (3, 11, 7), (1, 4, 9), (5, 5, 9)])
+def test_inconv128_columns_of_every_number(gpu, R, S, stride):
+    """First layers that go to the VALU kernel (no multiple of 64 channels), whatever number of input columns it stages."""
+    r = rng(R + S + stride)
+    b, h, w, cout = 66, 30, 41, 40
+    x = r.standard_normal((b, 3, h, w)).astype(np.float32)
+    f, bn = rm.pm1(r, (R, S, 3, cout)), r.normal(0, np.sqrt(3 * R * S), cout).astype(np.float32)
+    want, wres = orc.inconv128(x, f, bn, stride, True, 1, True)
+    layer = gpu.InConv128LayerParam("Conv1", h, w, R, S, 3, cout, b, stride, stride, True, 1, 1, True)
+    layer.initialize(x, gpu.ArrayWeights([f, bn]))
+    layer.forward()
+    gpuops.sync()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    np.testing.assert_array_equal(layer.download_residual(), wres)
+    layer.release()
+
+
 def test_inconv128_time_does_not_hang_on_the_images(gpu):
     """Bars and patches of +-1 over a third of the images cost next to nothing over random ones, and images of which every
     sum is in doubt a small factor (one by one, sums in doubt took 70 and 130 times as long)."""
