@@ -4,15 +4,17 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--net imagenet_resnet] [--batch 256]
                     [--variant auto|popc|mfma_i8|mfma_f4] [--no-cpu] [--layers]
 
-A step is one forward pass of the whole network (every layer, one launch each, one stream) over
+A step is one forward pass of the whole network (every layer, one stream; a launch per layer, or per run of fully connected layers) over
 one batch of seeded synthetic input that is already resident in HBM; weight packing and host
 copies are outside the timed region (the reference times only its network kernel,
 imagenet_resnet.cu:358-363).  Prints ONE JSON line.
 """
 import argparse
 import ctypes as C
+import functools
 import json
 import os
+import re
 import sys
 import time
 
@@ -67,14 +69,27 @@ def load_measured_traffic():
 MEASURED_TRAFFIC_BYTES, TRAFFIC_STALE, TRAFFIC_NOTE = {}, True, "not loaded"
 
 
-def layer_work(L, spec=(), res_bytes=None, pooled=()):
+def first_layer_fragments(kernel, r, s):
+    """Fragments of sixteen fp16 products that the first layer's matrix-core kernel multiplies per output value and part (high,
+    low) of the inputs: inconv_mfma_kernel<R, T, A, ...> has ceil(R / A) rows' sums under way and for each as many as the 3 A
+    pairs of a row and a channel need, T taps in 8 (7), 12 (11) or T places, two pairs side by side; the kernel with a ring in
+    LDS has one for four taps of a filter row."""
+    form = re.match(r"inconv_mfma_kernel<(\d+), (\d+), (\d+),", kernel)
+    if not form:
+        return r * -(-s // 4) if kernel == "inconv_mfma_ring_kernel" else 0
+    rows, taps, step = (int(v) for v in form.groups())
+    places = {7: 8, 11: 12}.get(taps, taps)
+    return -(-rows // step) * -(-((3 * step + 1) // 2 * places) // 8)
+
+
+def layer_work(L, spec=(), res_bytes=None, pooled=(), kernel=""):
     """Algorithmic work of one layer launch: binary ops (2 per +-1 multiply-accumulate, border taps
     included), fp32 adds of the first layer, and the HBM bytes the launch has to move once
     (inputs + outputs + weights, packed activations at 1 bit per value, residuals at the width
     they are stored in: res_bytes[layer name] = 1.5, 2 or 4 bytes per value of that layer's saved
     residual, 4 = the reference's int32 when not given; `pooled` = names of the layers whose saved residual
     is stored as its maximum over 2x2 windows of pixels, a quarter of the tensor, because only pooling
-    consumers read it)."""
+    consumers read it).  mfma_flops: fp16 products of a first layer that `kernel` multiplies on the matrix cores."""
     res_bytes = res_bytes or {}
     from tcbnn_amd import nets
     bops, flops = nets.binary_ops([L])
@@ -97,10 +112,7 @@ def layer_work(L, spec=(), res_bytes=None, pooled=()):
         out_bits = B * poh * pow_ * L["cout"] / 8
         if L["kind"] == "inconv":
             byts = B * 3 * L["h"] * L["w"] * 4 + out_bits + L["r"] * L["s"] * 3 * L["cout"] * 4
-            # fp16 products of the matrix-core kernel: four taps of four channels to a step, high and low parts
-            # counted as fragments of four taps x four channels per filter row, high and low parts (14 at 7x7; the kernel's
-            # order of K, pairs of a row and a channel, needs 12)
-            mfma_flops = 2.0 * B * oh * ow * L["cout"] * 2 * 16 * L["r"] * -(-L["s"] // 4)
+            mfma_flops = 2.0 * B * oh * ow * L["cout"] * 2 * 16 * first_layer_fragments(kernel, L["r"], L["s"])
             if L["save_residual"]:
                 byts += B * oh * ow * L["cout"] * res_bytes.get(L["name"], 4)
         else:
@@ -114,6 +126,18 @@ def layer_work(L, spec=(), res_bytes=None, pooled=()):
                 src_pixels = 4 if L["residual_pool"] and L.get("res_src") not in pooled else 1
                 byts += B * oh * ow * src_pixels * ch * res_bytes.get(L.get("res_src"), 4)
     return dict(bops=bops, flops=flops, bytes=float(byts), mfma_flops=mfma_flops)
+
+
+def launch_work(layers, spec=(), res_bytes=None, pooled=(), kernel=""):
+    """layer_work of a launch: of its layer, or of a run of fully connected ones, whose activations in between are written
+    (every layer's output is a result) but not read from memory."""
+    total = dict(bops=0.0, flops=0.0, bytes=0.0, mfma_flops=0.0)
+    for i, L in enumerate(layers):
+        for key, amount in layer_work(L, spec, res_bytes, pooled, kernel).items():
+            total[key] += amount
+        if i > 0:
+            total["bytes"] -= L["batch"] * L["inp"] / 8
+    return total
 
 
 def roofline_of(name, g, variant):
@@ -147,7 +171,7 @@ def roofline_of(name, g, variant):
         done = g["mfma_flops"] / secs / 1e12
         rec["matrix_fp16"] = {"flops_per_launch": round(g["mfma_flops"] / g["launches"]), "achieved": round(done, 1),
                               "peak": 2500.0, "unit": "TFLOP/s", "frac": round(done / 2500.0, 4)}
-        rec["binding"] = "waves waiting for the images and for issue slots, three per SIMD; see matrix_fp16"
+        rec["binding"] = "waves waiting for the images and for issue slots; see matrix_fp16"
     elif g.get("flops"):
         # The fp32 first layer on the VALU is far from the HBM roof because its additions bind it: one dependent fp32 add
         # per (tap, output channel, pixel, image) is the least the reference's summation order allows (its 2 flops per
@@ -269,6 +293,7 @@ def main():
     import tcbnn_amd
     from tcbnn_amd import _lib, nets
     from tcbnn_amd.device import Event, Stream
+    from tcbnn_amd.layers import forward_fc_run
 
     if _lib.device_count() < 1:
         sys.exit("bench.py: no HIP device visible")
@@ -375,18 +400,28 @@ def main():
     # every output word is rewritten by each launch.  One pass over the layers first, so that each layer finds its
     # inputs as the forward leaves them.
     R = 10
-    per_layer = {L["name"]: [] for L in spec}
+    # What the step launches: a layer each, or a run of fully connected layers that go together.
+    spec_of = dict(zip(map(id, net.order), spec))
+    step_launches = []
+    for layers in net.launches():
+        single = layers[0]
+        step_launches.append(dict(
+            spec=[spec_of[id(layer)] for layer in layers],
+            forward=single.forward if len(layers) == 1 else functools.partial(forward_fc_run, layers),
+            kernel="fc_chain_kernel" if len(layers) > 1 else
+            single.kernel_name() if hasattr(single, "kernel_name") else {"in": "in128_kernel"}[spec_of[id(single)]["kind"]], ms=[]))
     e0, e1 = Event(), Event()
     net.forward(stream)
     for _ in range(3):
-        for L, layer in zip(spec, net.order):
+        for launch in step_launches:
             e0.record(stream)
             for _r in range(R):
-                layer.forward(stream)
+                launch["forward"](stream)
             e1.record(stream)
             stream.synchronize()
-            per_layer[L["name"]].append(e0.elapsed_ms(e1) / R)
-    layer_ms = {k: float(np.median(v)) for k, v in per_layer.items()}
+            launch["ms"].append(e0.elapsed_ms(e1) / R)
+    for launch in step_launches:
+        launch["ms"] = float(np.median(launch["ms"]))
 
     # ------------------------------------------------------------------ packed first-layer input (a request,
     # never the default): the upload also makes a zero-padded, batch-innermost copy of the input on the device and
@@ -444,16 +479,12 @@ def main():
     pooled = {name for name in res_bytes if net.layers[name].output_residual_gpu.pooled}
     # group launches by device kernel, as a profiler does
     groups = {}
-    for L, layer in zip(spec, net.order):
-        name = layer.kernel_name() if hasattr(layer, "kernel_name") else \
-            {"in": "in128_kernel"}[L["kind"]]
-        w = layer_work(L, spec, res_bytes, pooled)
-        g = groups.setdefault(name, dict(bops=0.0, flops=0.0, mfma_flops=0.0, bytes=0.0, ms=0.0, launches=0))
-        g["bops"] += w["bops"]
-        g["flops"] += w["flops"]
-        g["mfma_flops"] += w["mfma_flops"]
-        g["bytes"] += w["bytes"]
-        g["ms"] += layer_ms[L["name"]]
+    for launch in step_launches:
+        g = groups.setdefault(launch["kernel"], dict(bops=0.0, flops=0.0, mfma_flops=0.0, bytes=0.0, ms=0.0, launches=0))
+        launch["work"] = launch_work(launch["spec"], spec, res_bytes, pooled, launch["kernel"])
+        for key, amount in launch["work"].items():
+            g[key] += amount
+        g["ms"] += launch["ms"]
         g["launches"] += 1
     by_time = sorted(groups.items(), key=lambda kv: -kv[1]["ms"])
     global MEASURED_TRAFFIC_BYTES, TRAFFIC_STALE, TRAFFIC_NOTE
@@ -507,14 +538,11 @@ def main():
 
     if args.layers:
         sys.stderr.write("%-8s %-34s %10s %10s %9s\n" % ("layer", "kernel", "ms", "TOP/s", "GB/s"))
-        for L, layer in zip(spec, net.order):
-            ops = nets.binary_ops([L])[0]
-            kn = layer.kernel_name() if hasattr(layer, "kernel_name") else L["kind"]
-            byts = layer_work(L, spec, res_bytes, pooled)["bytes"]
-            ms = layer_ms[L["name"]]
-            sys.stderr.write("%-8s %-34s %10.4f %10.1f %9.0f\n" % (L["name"], kn, ms, ops / (ms * 1e-3) / 1e12,
-                                                                   byts / (ms * 1e-3) / 1e9))
-        sys.stderr.write("sum of layers: %.4f ms; step: %.4f ms\n" % (sum(layer_ms.values()), ms_per_step))
+        for launch in step_launches:
+            ms, w = launch["ms"], launch["work"]
+            sys.stderr.write("%-8s %-34s %10.4f %10.1f %9.0f\n" % ("+".join(L["name"] for L in launch["spec"]), launch["kernel"], ms,
+                                                                   w["bops"] / (ms * 1e-3) / 1e12, w["bytes"] / (ms * 1e-3) / 1e9))
+        sys.stderr.write("sum of layers: %.4f ms; step: %.4f ms\n" % (sum(launch["ms"] for launch in step_launches), ms_per_step))
 
     # ------------------------------------------------------------------ CPU baseline (bounded sample)
     cpu = None

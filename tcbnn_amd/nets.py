@@ -309,6 +309,10 @@ class Network:
         """The order of layers, and what is launched together: layers that have launches of their own go one by one."""
         return list(self.order), [launch for run in fc_runs(self.order) for launch in fc_launches(run)]
 
+    def launches(self):
+        """The layers of a pass in order, by what one launch takes: one layer, or a run of fully connected ones."""
+        return self._plan_order()[1]
+
     def forward(self, stream=None):
         planned, runs = self._plan
         if planned != self.order:  # (a comparison of identities; the plan itself takes four times the loop below)
