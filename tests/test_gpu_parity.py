@@ -995,7 +995,9 @@ def test_inconv128_linear_staging(gpu):
     (16, 40, 40, 7, 7, 4, 64, 1, True, None, "special"), (34, 60, 60, 11, 11, 4, 64, 2, False, None, "special"),
     (34, 40, 40, 7, 7, 4, 64, 1, True, None, "whole"), (34, 33, 31, 3, 3, 1, 64, 1, True, None, "whole"),
     (16, 40, 40, 7, 7, 4, 64, 1, True, None, "zeros"), (16, 40, 40, 7, 7, 4, 64, 1, True, None, "positive"),
-    (16, 20, 20, 3, 3, 1, 64, 1, False, None, "positive"), (16, 60, 60, 11, 11, 4, 64, 2, False, None, "positive")])
+    (16, 20, 20, 3, 3, 1, 64, 1, False, None, "positive"), (16, 60, 60, 11, 11, 4, 64, 2, False, None, "positive"),
+    # sums of bytes on both sides of 2^15 and 2^16, inputs of up to 24 bits, few rows of 11x11 filters
+    (8, 90, 70, 11, 11, 4, 64, 2, False, None, "bytes"), (8, 90, 70, 11, 11, 4, 96, 2, False, None, "heavy_grid")])
 def test_inconv128_matrix_cores(gpu, b, h, w, R, S, stride, cout, pool, save, fmt, kind):
     """The first layer's matrix-core kernel gives the bits and residuals of the reference's order of additions."""
     r = rng(b + h + R + cout)
@@ -1011,6 +1013,13 @@ def test_inconv128_matrix_cores(gpu, b, h, w, R, S, stride, cout, pool, save, fm
         x[0, 0, h // 2, w // 2], x[-1, 2, 0, 0], x[b // 2, 1, h - 1, w - 1] = np.nan, np.inf, -1e30
     elif kind == "whole":
         x = np.rint(x * 80).clip(-255, 255).astype(np.float32)
+    elif kind == "bytes":
+        x = np.rint(r.random(x.shape) * np.linspace(100, 255, w)).astype(np.float32)
+        bn = np.rint(bn * 100).astype(np.float32)
+    elif kind == "heavy_grid":
+        x = np.rint(x * 256).astype(np.float32) / 256
+        heavy = r.random(x.shape) < 0.002
+        x[heavy] = (r.integers(-2 ** 24, 2 ** 24, int(heavy.sum())) // r.choice([1, 2, 4], int(heavy.sum())) / 256).astype(np.float32)
     elif kind == "zeros":
         x[:, :, :h // 2] = 0
     elif kind == "positive":
