@@ -14,7 +14,7 @@
 // expanded as its counterpart, and a sum starts from the negative of the image's constant.
 // What binds it: the matrix and vector pipes of a SIMD in turn (they overlap little here).  A 1024 x 1024 layer's 512 products and
 // as many expansions per workgroup are 2.6 us, epilogues and starts of tiles 1.2 us more; the signs of the input take 4 us from
-// the launch on.  MLP, batch 8192: 44.6 -> 21.1 us (256 workgroups, one per compute unit; 257, at batch 8200: 59.4 -> 36.6).
+// the launch on.  MLP, batch 8192: 42.6 -> 21.4 us a pass (256 workgroups, one per compute unit; 257, at batch 8200: 60.3 -> 36.8).
 #include <algorithm>
 #include <atomic>
 

@@ -23,8 +23,8 @@
 // E = u (sum of n_k A_k + 13.5 A), n_k roundings of sums up to step k; 2 % cover the bound's own roundings.  For 7-row filters
 // with a residual the A_k are summed up as the window passes (1.9 doubtful values per 32 pixels x 64 channels instead of 2.8
 // with A for each); the others, which have few doubtful values, take A for every A_k.
-// Where a residual is saved, -E itself enters the sum as one more product (a place that no tap uses), so the accumulators
-// hold S - E: a bit is certainly 1 where S - E >= bn, certainly 0 below bn - 2E.  Where none is saved, sums start from -bn: the
+// Where a residual is saved, -E itself enters the sum as one more product (a place that no tap uses; 7x8 at strides 2 and 4 has none:
+// taken off at the end, one more rounding), so the accumulators hold S - E: a bit is certainly 1 where S - E >= bn, certainly 0 below bn - 2E.  Where none is saved, sums start from -bn: the
 // bit is the sign, in doubt where |S - bn| <= E (partial sums are then at most what is still to come and |S - bn|: A again).
 // Inputs outside the fp16 range, infinities and NaN make NaN of the sums or an infinity of E: all values of such a window are
 // recomputed, as are those of windows whose neighbouring rows (multiplied by zeros) hold them.
@@ -43,8 +43,9 @@
 //             products on the matrix cores (ordered_sums): no values in doubt but those that are no numbers.  It lasts to the
 //             end of the wave's rows (left as soon as few would be in doubt, the common pass is reached from two places, and
 //             the registers that takes cost 7x7/2 288 -> 328 us on ordinary images).
-// ResNet-18's first layer at batch 256, launched on end, us: normal data 84, bytes / 128 - 1 81, images in [-1, 1] with bars and
-// patches of +-1 over a third 94, bytes / 255 122, a third of 0.2 grey 241, bytes less a mean 320, normal x 1000 325.
+// ResNet-18's first layer at batch 256, launched on end, us: normal data 83, bytes and bytes / 128 - 1 73, images in [-1, 1] with a bar
+// and patches of +-1 87, bytes of 195 to 255 113, bytes / 255 119, a bar and patches of 0.2 grey 360, bytes less a mean 313, normal x
+// 1000 320.
 //
 // Work split.  A tile is 32 columns = NI images x 32/NI neighbouring pixels of a row (so small batches fill their tiles) by 64
 // channels.  A wave walks down the rows of one column of tiles, a step per output row: the A (stride) input rows that are new
@@ -53,19 +54,19 @@
 // they move on without copies.  Compared with a ring of split rows in LDS (of which a CU holds eight waves' worth, at 240
 // registers a wave): no LDS traffic but the weights, which four waves share, no barrier, three waves per SIMD for 3x3 and 7x7/4
 // (two for the rest), and 8 places for a row's 7 taps in one channel, not 32 for its 21.  The next step's rows are requested as the
-// present ones are used up.  A workgroup's waves are neighbouring columns of tiles; an XCD has whole image tiles.
+// present ones are used up.  A workgroup's waves are neighbouring columns of tiles; an XCD has whole image tiles (3x3 with large
+// residuals: neighbouring image tiles, see choose()).
 // Eight images per tile: their residuals of a pixel are a whole 128-byte line.  Sixteen (64 bytes of output words) where no
 // residual is saved and a wave has 32 items or more: VGG-16 217 -> 206 us; below that fewer units fill the machine worse
 // (CIFAR VGG 16.7 -> 18.0 us).
 //
-// What binds it: memory traffic and the waits for it.  ResNet-18's layer at batch 256 fetches 294 MB for 154 MB of images (a doubtful
-// value's window comes back from HBM, 21 rows of 128 bytes: 116 MB; without that 178) and writes 90 MB, 3.6 TB/s; the VALU is
+// What binds it: memory traffic and the waits for it.  ResNet-18's layer at batch 256 fetches 289 MB for 154 MB of images (a doubtful
+// value's window comes back from HBM, 21 rows of 128 bytes; without the recomputations 178 MB) and writes 90 MB, 3.7 TB/s; the VALU is
 // busy 30 % of the time, the matrix cores 15 %.  Recomputing a value at once finds its rows in L2 no more often (an XCD's waves bring
-// in 4 MB per step) and costs a trip to memory per item (130 us for 118).
-// Measured, us within the network's pass (kernel trace, batch 256 unless said; adds on the VALU -> ring in LDS -> here, both
-// matrix-core versions in turn on one box): ResNet-18 7x7/4 127 -> 124 -> 108, 7x7/2 423 -> 334 -> 305, VGG-16 3x3 399 -> 209 -> 205,
-// AlexNet 11x11/4 batch 200 403 -> 133 -> 97, CIFAR VGG 23 -> 20.4 -> 17.6, CIFAR ResNet batch 77 26 -> 18.8 -> 16.3, ResNet-18
-// batch 8 52 -> 18.0 -> 15.7.
+// in 4 MB per step) and costs a trip to memory per item (a tenth slower).
+// Measured, us within the network's pass at batch 256 (kernel trace, medians; adds on the VALU -> ring in LDS -> here): ResNet-18 7x7/4
+// 127 -> 121 -> 103, 7x7/2 423 -> 315 -> 296, VGG-16 3x3 399 -> 207 -> 200, AlexNet 11x11/4 310 -> 137 -> 102, CIFAR VGG 23 -> 18.0 -> 14.8,
+// CIFAR ResNet 27.4 -> 27.1 -> 25.9.
 #include <algorithm>
 #include <atomic>
 #include <cmath>

@@ -211,7 +211,7 @@ constexpr int kHeadMaxC = 512;
 constexpr int kHeadChunk = 32;     // channels whose weights are laid out in LDS at a time
 constexpr int kHeadAhead = 2;      // chunks requested ahead
 
-// Sixteen channels of a thread's output and four images: means lie one channel per lane of each row of 16 (all rows the same), and
+// Sixteen channels of a thread's output and two images: means lie one channel per lane of each row of 16 (all rows the same), and
 // a multiply-add takes its channel's by DPP.  (As asm because the compiler moves the lane's value first, in an instruction of
 // its own; the wait states are those between a write of m and a DPP read of it.)
 #define TCBNN_HEAD_CHANNEL(K, LANE)                                                        \
