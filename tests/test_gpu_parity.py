@@ -1202,6 +1202,39 @@ def test_inconv128_thresholds_at_the_ordered_sums(gpu, b, h, R, stride, pool, ki
     layer.release()
 
 
+@pytest.mark.parametrize("R,S,stride", [(7, 7, 6), (7, 7, 3), (3, 3, 3), (3, 4, 2), (7, 8, 2), (7, 8, 4), (7, 8, 3), (7, 6, 4)])
+@pytest.mark.parametrize("kind,save", [("mixed", True), ("spikes", True), ("mixed", False), ("spikes", False)])
+def test_inconv128_other_forms_with_thresholds_at_the_ordered_sums(gpu, R, S, stride, kind, save):
+    """The same for windows that are loaded whole, -E taken off at the end, and filters narrower than their form."""
+    r = rng(1100 + R + S + stride + len(kind))
+    b, h, w, cout = 9, 40, 37, 64
+    x = r.standard_normal((b, 3, h, w)).astype(np.float32)
+    x = x * (10.0 ** r.uniform(-3, 4, x.shape)).astype(np.float32) if kind == "mixed" else np.where(r.random(x.shape) < 0.3, x * np.float32(4096), x * np.float32(2e-4)).astype(np.float32)
+    f = rm.pm1(r, (R, S, 3, cout))
+    pad_h, _, out_h = rm.conv_pad_out(h, R, stride, True, 1)
+    pad_w, _, out_w = rm.conv_pad_out(w, S, stride, True, 1)
+    bn = np.empty(cout, np.float32)
+    for o in range(cout):
+        i, y0, x0 = int(r.integers(b)), int(r.integers(1, out_h - 1)) * stride - pad_h, int(r.integers(1, out_w - 1)) * stride - pad_w
+        acc = np.float32(0)
+        for t in range(R):
+            for s in range(S):
+                if 0 <= y0 + t < h and 0 <= x0 + s < w:
+                    v = x[i, :, y0 + t, x0 + s] * f[t, s, :, o]
+                    acc = acc + ((v[0] + v[1]) + v[2])
+        bn[o] = [acc, np.nextafter(acc, np.float32(np.inf)), np.nextafter(acc, np.float32(-np.inf))][o % 3]
+    want, wres = orc.inconv128(x, f, bn, stride, True, 1, save)
+    layer = gpu.InConv128LayerParam("Conv1", h, w, R, S, 3, cout, b, stride, stride, True, 1, 1, save)
+    layer.initialize(x, gpu.ArrayWeights([f, bn]))
+    assert "inconv_mfma_kernel" in layer.kernel_name(), layer.kernel_name()
+    layer.forward()
+    gpuops.sync()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    if save:
+        np.testing.assert_array_equal(layer.download_residual(), wres)
+    layer.release()
+
+
 @pytest.mark.parametrize("b,h,w,R,stride,cout,pool,save,kind", [
     # frames narrower than the filter, one row, columns of tiles that end inside the frame, bands of single rows
     (1, 5, 3, 7, 4, 64, 1, True, "normal"), (600, 60, 5, 11, 4, 512, 2, False, "normal"), (3, 1, 40, 3, 1, 64, 1, True, "normal"),
