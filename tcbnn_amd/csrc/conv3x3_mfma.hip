@@ -116,6 +116,7 @@ conv3x3_mfma_f4_kernel(
                   "the window maximum is taken on 16-bit pairs in the epilogue of full tiles with a narrow injected residual");
     static_assert(!PSAVE || (MT == 1 && waves_of(SPT, NT, WIN) == 4), "one wave per pixel of the window, one image tile each");
     constexpr bool kTwoPhase = PSAVE && win_two_phase(SPT, NT);
+    constexpr bool kStartMagic = kRes && FULLT && (RF == TCBNN_RES_I16 || RF == TCBNN_RES_I12);  // (see kMagic)
     constexpr int TPC = SPT >= 3 ? 3 : 9;  // taps per prefetch chunk (a filter row, or all of it)
     constexpr int NCH = 9 / TPC;           // chunks per tile
     constexpr int NQ = 9 * SPT;            // k-steps per tile
@@ -188,7 +189,7 @@ conv3x3_mfma_f4_kernel(
 
     // start values of a lane's 16 channels per channel tile (zeros when a residual is added first); filled once
     // the thresholds are staged
-    v16f acc0[NT];
+    v16f acc0[NT];  // (layers of one chunk per tile)
 
     // a wave's work items: output pixels, or 2x2 windows of them (row width `roww`)
     const int roww = kWin ? p.PW / 2 : p.PW;
@@ -292,6 +293,23 @@ conv3x3_mfma_f4_kernel(
     };
 
     v16f acc[MT][NT];
+    // Where a tile starts from: with one chunk per tile the first MFMAs take it as their operand C, in registers; with three
+    // the accumulators are set from the staged thresholds (or to a constant) at the tile's start, one instruction in 70 of its
+    // time, and its 32 registers go to the operands in flight.
+    constexpr bool kStartInLds = NCH > 1;
+    auto start_value = [&](int nt, int v) __attribute__((always_inline)) {
+        return RM == RM_NONE ? lds_thr[nt * 32 + 16 * h + v] : (kStartMagic ? __uint_as_float(0x4B400000u) : 0.0f);
+    };
+    auto start_tile = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float from = start_value(nt, v);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) acc[mt][nt][v] = from;
+            }
+    };
 
     // One k-step (64 input channels of one tap): the expanded activation words `bfrag` times the NT
     // weight fragments `a`.  FIRST: the accumulators start from acc0 instead of their old value.
@@ -376,16 +394,18 @@ conv3x3_mfma_f4_kernel(
     };
     auto compute_chunk = [&](int chunk, uint32_t (*buf)[MT], uint32_t mask, bool fused, uint32_t (*nbuf)[MT],
                              unsigned nsoff) __attribute__((always_inline)) {
-        if constexpr (SPT <= 2) {
-            if (fused) {  // uniform; NCH == 1: the chunk is a whole tile
+        if constexpr (kStartInLds) {
+            if (chunk == 0) start_tile();  // uniform
+            if (fused)                     // uniform
+                compute_chunk_as(std::false_type{}, std::true_type{}, chunk, buf, mask, nbuf, nsoff);
+            else
+                compute_chunk_as(std::false_type{}, std::false_type{}, chunk, buf, mask, nbuf, nsoff);
+        } else {
+            if (fused)  // uniform; the chunk is a whole tile
                 compute_chunk_as(std::true_type{}, std::true_type{}, chunk, buf, mask, nbuf, nsoff);
-                return;
-            }
+            else
+                compute_chunk_as(std::true_type{}, std::false_type{}, chunk, buf, mask, nbuf, nsoff);
         }
-        if (NCH == 1 || chunk == 0)  // uniform: the tile starts here
-            compute_chunk_as(std::true_type{}, std::false_type{}, chunk, buf, mask, nbuf, nsoff);
-        else
-            compute_chunk_as(std::false_type{}, std::false_type{}, chunk, buf, mask, nbuf, nsoff);
     };
 
     // ---- residual operand (kernel.cuh:770-794).  A lane owns channels n0 + 32 nt + 16 h + v of
@@ -1029,11 +1049,12 @@ conv3x3_mfma_f4_kernel(
         lds_thr[tid] = t;
     }
     __syncthreads();
+    if constexpr (!kStartInLds) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-            acc0[nt][v] = RM == RM_NONE ? lds_thr[nt * 32 + 16 * h + v] : (kMagic ? __uint_as_float(kMagicBits) : 0.0f);
+            for (int v = 0; v < 16; ++v) acc0[nt][v] = start_value(nt, v);
+    }
     if constexpr (kAhead && RM == RM_POOLED) {  // (one tile ahead: the first tile's operand)
         if (cc.pi < npix) finish_residual(rv[0]);
     }
@@ -1048,7 +1069,7 @@ conv3x3_mfma_f4_kernel(
         unsigned nsoff = 0;
         const bool ahead = lc.pi < npix;  // (uniform) there is a chunk LOOK steps ahead
         if (ahead) {
-            if (SPT <= 2 && msk[I] == kAllTaps && chunk_interior(pix_y(lc), pix_x(lc), lc.chunk, nsoff)) {
+            if (msk[I] == kAllTaps && chunk_interior(pix_y(lc), pix_x(lc), lc.chunk, nsoff)) {
                 fused = true;
                 msk[J] = kAllTaps;
             } else {
