@@ -50,15 +50,25 @@ constexpr int kResStoreAux = 0x11;
 // ... and of the output words: written through as well (the next launch reads them from every XCD); another 0.5 % of
 // that step (0.4633 -> 0.4610 ms, three runs each; non-temporal stores instead: 0.4693 ms).
 constexpr int kBitsStoreAux = 0x11;
+// Residual mode of an instantiation.
+constexpr int RM_NONE = 0;    // threshold only
+constexpr int RM_PLAIN = 1;   // residual injected from a source of the same size and / or saved
+constexpr int RM_POOLED = 2;  // residual injected as the 2x2 max of a source twice the size
+constexpr int RM_RAW = 3;     // no threshold: the +-1 dot products are stored as int32 (tcbnn_bconv)
+
 // Waves per workgroup: four, sharing the staged weights of their channel group; eight where the FP4 fragments of
 // two channel tiles (18 KB per tile and 64 input channels) leave room for only one workgroup in a CU's 160 KB of
 // LDS (Cin >= 384), and already at Cin = 256, where two four-wave workgroups would fit: the CU then still runs two
 // waves per SIMD, each expanded activation fragment still feeds two MFMAs, the weights are staged once per CU
-// instead of twice, and which waves share a SIMD is known (waves w and w + 4), which the numbering of the work
+// instead of twice, and which waves share a SIMD is known (waves w, w + 4, ...), which the numbering of the work
 // items uses (ResNet-18 at batch 256: L3B2C1 14.6 -> 13.2 us, L3B1C2 17.1 -> 16.1 us).
+// Twelve where a wave has one image tile and no 2x2 maximum to take: 168 registers hold that, and a third wave on
+// each SIMD covers what the other two wait for.  512 channels: 7 x 7, batch 256 16.3 / 15.8 -> 15.0 / 14.5 us,
+// 8 x 8, batch 77 12.1 -> 11.1, 28 x 28, batch 256 144.1 -> 140.2.
 constexpr int WIN_NONE = 0, WIN_ORPOOL = 1, WIN_MAXSAVE = 2;  // (see the kernel)
-constexpr int waves_of(int spt, int nt, int win) {
-    return win != WIN_MAXSAVE && 9 * spt * nt * 1024 > (nt == 2 ? 64 : 80) * 1024 ? 8 : 4;  // (WIN_MAXSAVE: a wave per pixel)
+constexpr int waves_of(int spt, int rm, int mt, int nt, int win) {
+    const bool alone = win != WIN_MAXSAVE && 9 * spt * nt * 1024 > (nt == 2 ? 64 : 80) * 1024;  // (WIN_MAXSAVE: a wave per pixel)
+    return alone ? (mt == 1 && (rm == RM_NONE || rm == RM_PLAIN) ? 12 : 8) : 4;
 }
 // WIN_MAXSAVE: where the four waves' sums of a window meet in LDS.  All channel tiles at once ([wave][NT][2][64]
 // 128-bit words) where that leaves room for two workgroups per CU next to the staged weights; else one channel tile
@@ -66,12 +76,6 @@ constexpr int waves_of(int spt, int nt, int win) {
 // price of two more barriers per window.
 constexpr bool win_two_phase(int spt, int nt) { return 9 * spt * nt * 1024 + nt * 128 + 4 * nt * 2 * 64 * 16 > 80 * 1024; }
 constexpr int win_area_bytes(int spt, int nt) { return win_two_phase(spt, nt) ? 3 * 2 * 64 * 16 : 4 * nt * 2 * 64 * 16; }
-// Residual mode of an instantiation.
-constexpr int RM_NONE = 0;    // threshold only
-constexpr int RM_PLAIN = 1;   // residual injected from a source of the same size and / or saved
-constexpr int RM_POOLED = 2;  // residual injected as the 2x2 max of a source twice the size
-constexpr int RM_RAW = 3;     // no threshold: the +-1 dot products are stored as int32 (tcbnn_bconv)
-
 // RM_RAW: a wave's sums are transposed through a private LDS area of [32 images][32 NT + 4] words, so that every store
 // writes whole contiguous channel runs, wherever that area leaves room for two workgroups in a CU's 160 KB of LDS
 // next to the staged weights (9 SPT NT KB).  (The pitch, an odd multiple of 4 words, keeps both directions free of
@@ -86,7 +90,9 @@ constexpr bool raw_transposed(int spt, int rm, int nt, bool fullt) {
 constexpr int kWavesPerSimd = 2;
 // ... except where a fourth wave per SIMD is two registers away (one register spilled): Cin = 64 layers that save
 // the window maximum
-constexpr int waves_per_simd(int spt, int rm, int win) { return spt == 1 && rm == 1 && win == 2 ? 4 : kWavesPerSimd; }
+constexpr int waves_per_simd(int spt, int rm, int mt, int nt, int win) {
+    return spt == 1 && rm == 1 && win == 2 ? 4 : (waves_of(spt, rm, mt, nt, win) == 12 ? 3 : kWavesPerSimd);
+}
 
 // SPT = k-steps (64 bits) per filter tap = Cin / 64; MT = 32-image tiles per wave (2 for plain
 // layers, 1 for residual layers); NT = 32-channel tiles per wave; RF = TCBNN_RES_* format of the
@@ -103,7 +109,7 @@ constexpr int waves_per_simd(int spt, int rm, int win) { return spt == 1 && rm =
 // tests of partial tiles are then not even compiled (they cost scalar registers and set-up instructions in
 // every launch, and the networks' channel counts are multiples of 64).
 template <int SPT, int RM, int MT, int NT, int RF, int WIN, bool FULLT>
-__global__ __launch_bounds__(64 * waves_of(SPT, NT, WIN)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(SPT, RM, WIN)))) void
+__global__ __launch_bounds__(64 * waves_of(SPT, RM, MT, NT, WIN)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(SPT, RM, MT, NT, WIN)))) void
 conv3x3_mfma_f4_kernel(
     const BgemmParams p, const uint32_t* __restrict__ act, const uint32_t* __restrict__ wgt,
     const float* __restrict__ bnp, const int32_t* __restrict__ rin, int32_t* __restrict__ rout, int res_lim,
@@ -114,13 +120,13 @@ conv3x3_mfma_f4_kernel(
     static_assert(RM == RM_NONE || !POOL, "residuals are defined for un-pooled layers only");
     static_assert(!PSAVE || (RM == RM_PLAIN && FULLT && (RF == TCBNN_RES_I16 || RF == TCBNN_RES_I12)),
                   "the window maximum is taken on 16-bit pairs in the epilogue of full tiles with a narrow injected residual");
-    static_assert(!PSAVE || (MT == 1 && waves_of(SPT, NT, WIN) == 4), "one wave per pixel of the window, one image tile each");
+    static_assert(!PSAVE || (MT == 1 && waves_of(SPT, RM, MT, NT, WIN) == 4), "one wave per pixel of the window, one image tile each");
     constexpr bool kTwoPhase = PSAVE && win_two_phase(SPT, NT);
     constexpr bool kStartMagic = kRes && FULLT && (RF == TCBNN_RES_I16 || RF == TCBNN_RES_I12);  // (see kMagic)
     constexpr int TPC = SPT >= 3 ? 3 : 9;  // taps per prefetch chunk (a filter row, or all of it)
     constexpr int NCH = 9 / TPC;           // chunks per tile
     constexpr int NQ = 9 * SPT;            // k-steps per tile
-    constexpr int kWaves = waves_of(SPT, NT, WIN);
+    constexpr int kWaves = waves_of(SPT, RM, MT, NT, WIN);
     // A tile of one chunk is shorter than the memory latency: its residual operand is then
     // requested a whole tile ahead (double-buffered); otherwise with the tile's first chunk.
     constexpr bool kAhead = kRes && NCH == 1;
@@ -199,7 +205,7 @@ conv3x3_mfma_f4_kernel(
     // waves 0-3 (one per SIMD) are numbered before the waves 4-7 of ANY workgroup, so that the left-over items fall
     // one to a SIMD over all CUs instead of two to a SIMD in the first CUs and none in the others.
     int pi = PSAVE ? stream  // (a window is taken by the whole workgroup)
-                   : (kWaves == 8 ? (wave >> 2) * (pix_streams * 4) + stream * 4 + (wave & 3) : stream * kWaves + wave);
+                   : (kWaves >= 8 ? (wave >> 2) * (pix_streams * 4) + stream * 4 + (wave & 3) : stream * kWaves + wave);
     const int dpi = PSAVE ? pix_streams : pix_streams * kWaves;
     // Item pi stands for row pi / roww and column (pi % roww + row) % roww.  The skew by the row keeps
     // a wave from staying in one column when its stride is a multiple of the row width (then the waves
@@ -966,11 +972,11 @@ conv3x3_mfma_f4_kernel(
 
     // ---- persistent loop over this wave's tiles.  The activation chunks rotate through NB register
     // buffers: the chunk that will be multiplied NB-1 steps from now is requested before the current
-    // one is multiplied (two steps of lookahead for Cin >= 192, where one chunk of MFMAs is shorter
+    // one is multiplied, or with it (two steps of lookahead for Cin >= 192, where one chunk of MFMAs is shorter
     // than the memory latency and few waves share a SIMD).
     // (Two tiles of lookahead for the short residual tiles, with a third buffer for words and operand, measured no
     // faster on ResNet-18's first two stages and cost the Cin = 128 layers their third wave per SIMD.)
-    constexpr int NB = kAhead ? 2 : (SPT >= 3 && !(kRes && MT == 2 && SPT >= 6) ? 3 : 2);  // (registers)
+    constexpr int NB = kAhead ? 2 : (SPT >= 3 && !(kRes && SPT >= 6 && (MT == 2 || kWaves == 12)) ? 3 : 2);  // (registers)
     constexpr int LOOK = NB - 1;
     struct Cursor {
         int pi, y, x, chunk, sub;  // item index, row and (skewed) column, chunk of the tile, pixel of the window
@@ -1158,7 +1164,7 @@ TensorBytes tensor_bytes(const BgemmParams& p) {
 template <int SPT, int RM, int MT, int NT, int RF, int WIN, bool FULLT>
 int launch_f(const BgemmParams& p, hipStream_t stream) {
     constexpr int NQ = 9 * SPT;
-    constexpr int kWaves = waves_of(SPT, NT, WIN), kThreads = 64 * kWaves;
+    constexpr int kWaves = waves_of(SPT, RM, MT, NT, WIN), kThreads = 64 * kWaves;
     constexpr bool kRawTranspose = raw_transposed(SPT, RM, NT, FULLT);
     constexpr bool kWgItems = WIN == WIN_MAXSAVE;  // a work item (window) is taken by a whole workgroup
     const size_t lds_bytes = (size_t)NQ * NT * 64 * 16 + NT * 32 * sizeof(float) +
@@ -1188,7 +1194,7 @@ int launch_f(const BgemmParams& p, hipStream_t stream) {
     const int items = WIN != WIN_NONE ? (p.PH / 2) * (p.PW / 2) : p.PH * p.PW;  // pixels, or 2x2 windows of them
     // streams worth launching: one per item for workgroup-wide items; else one per kWaves items, or per 4 for
     // eight-wave workgroups, whose waves 0-3 (one per SIMD) are served first (see the kernel's first item)
-    constexpr int kServedFirst = kWaves == 8 ? 4 : kWaves;
+    constexpr int kServedFirst = kWaves >= 8 ? 4 : kWaves;
     const int quads = kWgItems ? items : (items + kServedFirst - 1) / kServedFirst;
     // Persistent workgroups, all resident at once: two per CU (three for residual layers), fewer
     // when registers or LDS hold fewer.  Measured on every layer of ResNet-18 at batch 256: more, shorter-lived
@@ -1200,9 +1206,12 @@ int launch_f(const BgemmParams& p, hipStream_t stream) {
     // Residual layers with one image tile per wave are bound by memory and by their epilogue's latency chains: a third
     // workgroup per CU, where registers and LDS hold one (`resident`), keeps more requests in flight (stage-1 and
     // stage-2 layers of ResNet-18: -3 to -8 %); a fourth where the kernel was compiled for it (L1B2C2 at batch 256:
-    // 28.0 -> 26.5 us).
+    // 28.0 -> 26.5 us).  The plain layers of 64 channels as well, whose products are few to
+    // a tile's other instructions (112 x 112, 128 outputs, batch 256 87.7 -> 84.8 us; 56 x 56, 64 outputs
+    // 15.5 -> 14.8); pooled ones do not fit 168 registers (175 -> 186 us with that limit).
     constexpr bool kResLayer = RM == RM_PLAIN || RM == RM_POOLED;
-    const int wg_want = wg_env > 0 ? wg_env : (kResLayer && MT == 1 ? (waves_per_simd(SPT, RM, WIN) == 4 ? 4 : 3) : 2);
+    constexpr bool kPlainShort = RM == RM_NONE && SPT == 1 && WIN == WIN_NONE;
+    const int wg_want = wg_env > 0 ? wg_env : ((kResLayer && MT == 1) || kPlainShort ? (waves_per_simd(SPT, RM, MT, NT, WIN) == 4 ? 4 : 3) : 2);
     const int wg_per_cu = std::max(1, std::min(wg_want, resident));
     const int best = std::max(1, std::min(cus * wg_per_cu / (n_groups * b_groups), quads));
     // channels that receive an injected residual: o < residual_channels, and only those the
@@ -1248,6 +1257,7 @@ int launch_t(const BgemmParams& p, hipStream_t stream) {
 // accumulators).
 struct Pick {
     int rm, mt, nt, r16, win;  // r16: TCBNN_RES_* format of the injected residual; win: WIN_*
+    int fitted;                // image tiles by the rules that bgemm_flat_preferred's estimate was fitted with
 };
 constexpr int pick_nt(int spt, int rm) {
     return rm == RM_POOLED ? (spt >= 6 ? 1 : 2) : (rm == RM_RAW ? (spt >= 3 && spt < 8 ? 1 : 2) : 2);
@@ -1281,7 +1291,16 @@ Pick pick(const BgemmParams& p) {
         const long long tiles = (long long)p.PH * p.PW * ((p.B + 63) / 64) * ((p.N + 32 * nt - 1) / (32 * nt));
         if (device_info(&dev, &cus) == TCBNN_OK && tiles < 4LL * 4 * cus) mt = 1;
     }
-    return {rm, mt, nt, fmt, p.pool_h == 2 ? WIN_ORPOOL : (p.res_out_pool ? WIN_MAXSAVE : WIN_NONE)};
+    const int fitted = mt;
+    // A pooled layer with fewer windows than waves leaves waves without work: one image tile each, and twelve waves
+    // a compute unit (256 -> 256 channels at 16 x 16, batch 128 / 256 19.0 / 20.2 -> 13.3 / 18.4 us).  With items for
+    // every wave the two tiles that share a weight fragment win (un-pooled, 256 channels at 56 x 56: 148 us against 161).
+    if (rm == RM_NONE && p.pool_h == 2 && mt == 2 && p.cw >= 8) {
+        int dev = 0, cus = 0;
+        const long long items = (long long)(p.PH / 2) * (p.PW / 2) * ((p.B + 63) / 64) * ((p.N + 32 * nt - 1) / (32 * nt));
+        if (device_info(&dev, &cus) == TCBNN_OK && items < 8LL * cus) mt = 1;
+    }
+    return {rm, mt, nt, fmt, p.pool_h == 2 ? WIN_ORPOOL : (p.res_out_pool ? WIN_MAXSAVE : WIN_NONE), fitted};
 }
 
 template <int SPT>
@@ -1350,7 +1369,7 @@ bool conv3x3_mfma_applicable(const BgemmParams& p) {
            (long long)p.PH * p.PW < (1 << 24) && within_2gib(p);
 }
 
-int conv3x3_mfma_image_tiles(const BgemmParams& p) { return pick(p).mt; }
+int conv3x3_mfma_image_tiles(const BgemmParams& p) { return pick(p).fitted; }
 
 void conv3x3_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len) {
     const Pick k = pick(p);

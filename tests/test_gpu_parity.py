@@ -422,6 +422,24 @@ def test_conv128_layer(gpu, variant, b, h, cin, cout, stride, pool, ahead_fc):
     layer.release()
 
 
+@pytest.mark.parametrize("b,h,cin,cout,pool,image_tiles", [
+    (33, 1, 256, 64, 1, 1), (40, 5, 384, 96, 1, 1), (65, 3, 512, 160, 1, 1),  # fewer items than waves; partial tiles
+    (520, 7, 256, 512, 1, 1),  # one workgroup per pair of tile and channel group: four items a wave and one left over
+    (290, 12, 256, 384, 2, 1), (200, 16, 256, 512, 2, 2),  # windows for fewer and for as many waves as two per SIMD
+])
+def test_conv128_waves_of_a_workgroup(gpu, b, h, cin, cout, pool, image_tiles):
+    """Plain layers whose weights fill a compute unit's LDS: twelve waves with one image tile, eight with two."""
+    r = rng(b + h + cin + cout + pool)
+    x, f = rm.pm1(r, (b, h, h, cin)), rm.pm1(r, (3, 3, cin, cout))
+    bn = r.normal(0, np.sqrt(9 * cin), cout).astype(np.float32)
+    want, _ = orc.conv128(orc.pack_conv_input_nhwc(x), orc.pack_conv_filter(f), bn, cin, cout, 3, 3, 1, True, pool)
+    layer = _run_conv_layer(gpu, "mfma_f4", x, f, bn, 1, pool)
+    name = layer.kernel_name()
+    assert "conv3x3_mfma_f4_kernel<%d, 0, %d, " % (cin // 64, image_tiles) in name, name
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    layer.release()
+
+
 # (cin, cout): the persistent 3x3 kernel's instantiations (Cin 64 .. 512), a channel count that is not a
 # multiple of 32 and an odd one (half-filled last 16-bit pair); formats of the injected and saved tensors
 RES_SHAPES = [(64, 96), (128, 64), (256, 35), (512, 64), (192, 64), (384, 40), (96, 35)]
