@@ -6,11 +6,15 @@
 //
 //   workgroup = 4 waves = (4 x MT x 32 rows of the batch / of A) x 64 output columns;
 //   wave      = MT image tiles x 2 column tiles: 2 MT MFMAs (32 x 32 x 64, FP4) per k-step;
-//   weights   : the 64 columns' words are expanded to MFMA "A" fragments in LDS, 16 k-steps at a time,
-//               double-buffered: the words of the next block are requested before the current block is
-//               multiplied and expanded into the other buffer after it, one barrier per block;
-//   rows      : a lane's words come straight from memory through buffer addressing (one per-lane constant
-//               offset per image tile, the k-step in the scalar offset), four k-steps ahead of their use.
+//   weights   : the 64 columns' words are expanded to MFMA "A" fragments in LDS, 8 or 16 k-steps at a time,
+//               double-buffered: the words of the next block, 16 bytes a thread with four threads to a row, are
+//               requested before the current block is multiplied and expanded into the other buffer after it, one
+//               barrier per block;
+//   rows      : a lane's words, of MT neighbouring images in one request, come straight from memory through buffer
+//               addressing (a per-lane constant offset, the k-step in the scalar offset), eight k-steps ahead of their use.
+// Bound by the matrix pipe and by power: with operands like these the MFMA alone reaches 8.1 P (constants: 9.8), this kernel 5.8
+// on 8 192^3, of whose time a tenth is the output's.  Before (a row of the weights per lane, a request per image tile, one block
+// size): 8 192^3 214 us, 5 000 x 3 104 x 7 200 69, 3 072 x 3 072 x 8 192 51, 1 500 x 8 192 x 4 096 31.8; now 190, 56.5, 38.2, 25.0.
 // Operand roles, fragment order and the accumulator layout are those of bgemm_mfma.hip.
 #include "common.h"
 #include "mfma_util.h"
@@ -23,20 +27,27 @@ using namespace mfma;
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kNT = 2;     // 32-column tiles per wave
-constexpr int kBlk = 16;   // k-steps of weights per LDS buffer (16 * kNT KiB)
-constexpr int kAhead = 8;  // k-steps a row word is requested ahead of its use; divides kBlk
-constexpr int kFrags = kBlk * kNT / kWaves;  // fragments a wave stages per block
+// k-steps of weights per LDS buffer (kNT KiB each): with two image tiles per wave the registers hold three workgroups in a CU, and
+// so does the LDS
+constexpr int blk_of(int mt) { return mt == 2 ? 8 : 16; }
+constexpr int kAhead = 8;  // k-steps a row word is requested ahead of its use; divides blk_of()
+constexpr int kOutOfRange = (int)0x80000000u;  // (a request there touches no memory and returns 0)
+static_assert(kThreads == 4 * 32 * kNT, "four threads stage a column");
+typedef int v2i __attribute__((ext_vector_type(2)));
 
 // Row words are expanded without shifts (expand_rows_f4 in mfma_util.h): the accumulator ends as the dot product
 // plus a per-column constant, which the staging lanes count as they go and the epilogue takes off.
-// ODD: an odd number of words per row (the stand-alone product alone can have one; a fully connected layer's rows are whole
-// 128-bit units): the last k-step's upper words do not exist.  As a test in every staging it cost the MLP, whose hidden
-// layers' whole K is one staging block, 1.2 % (43.2 us for 42.7 at batch 8192).
-template <int MT, int EPI, bool ODD>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_mfma_f4_kernel(
+// TAIL: rows that are no whole 128-bit units (the stand-alone product alone has them): the last unit's words past the row
+// are the next row's.
+template <int MT, int EPI, bool TAIL>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 2 ? 3 : 2))) void gemm_mfma_f4_kernel(
     const BgemmParams p, const uint32_t* __restrict__ act, const uint32_t* __restrict__ wgt,
     const float* __restrict__ bnp, const float* __restrict__ bias, int n_groups) {
-    __shared__ v4i lds_w[2][kBlk * kNT * 64];
+    constexpr int kBlk = blk_of(MT);
+    constexpr int kUnits = kBlk / 8;  // 16-byte units of a column's row that a thread stages per block: two k-steps each, four threads
+    constexpr int kRawInts = kNT * 32 + kWaves * 32 * (32 * kNT + 4);  // int32 output on its way (below)
+    __shared__ v4i lds_all[(2 * kBlk * kNT * 64 * 4 > kRawInts || EPI != EPI_RAW ? 2 * kBlk * kNT * 64 * 4 : kRawInts) / 4];
+    v4i(*const lds_w)[kBlk * kNT * 64] = reinterpret_cast<v4i(*)[kBlk * kNT * 64]>(lds_all);
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -52,37 +63,49 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     // both sides, so each such position adds exactly +1 to the dot product, and the known count is taken off in the
     // epilogue.
     const int steps = (p.cw + 2 * kAhead - 1) / (2 * kAhead) * kAhead;
-    const int corr = 64 * steps - p.k_tap;
+    const int corr = 64 * steps - p.k_tap + 2 * steps * class_sum(0u);  // (with what a column of zeros adds, see set0)
 
-    // ---- weights: this wave stages fragments f = wave + 4 i = (k-step ql = wave/2 + 2 i, column tile wave % 2)
-    const int snt = wave & 1, sq = wave >> 1;
+    // ---- weights: this thread stages 16-byte units sc and sc + 4 (two k-steps each) of one of the 64 columns' rows.  Fragments
+    // lie in LDS with the low bits of their lane exchanged by the unit, so eight neighbouring threads (two columns, four
+    // units) write to different banks; a reading wave covers whole runs of 64 slots either way.
+    const int sj = tid >> 2 & 31, snt = tid >> 7, sc = tid & 3;
     // a row past N (stand-alone product: the rows do not exist) reads the last row; its results are discarded
-    const uint32_t* __restrict__ wrow = wgt + (size_t)min(n0 + snt * 32 + row_to_channel(j), p.N - 1) * p.cw + h;
-    uint32_t wx[kFrags];
+    const int srow = min(n0 + snt * 32 + row_to_channel(sj), p.N - 1) - n0;
+    const __amdgpu_buffer_rsrc_t r_wgt = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t*>(wgt + (size_t)n0 * p.cw), 0, min(32 * kNT, p.N - n0) * p.cw * 4, 0x00020000);
+    const int woff = (srow * p.cw + 4 * sc) * 4;
+    v4i wx[kUnits];
     auto stage_load = [&](int q0) {
 #pragma unroll
-        for (int i = 0; i < kFrags; ++i) {
-            const int q = q0 + sq + 2 * i;
-            wx[i] = 0u;
-            if (ODD ? 2 * q + h < p.cw : 2 * q < p.cw) wx[i] = wrow[2 * q];  // (not ODD: uniform)
+        for (int i = 0; i < kUnits; ++i) {
+            const int w = 2 * q0 + 16 * i + 4 * sc;  // the unit's first word
+            wx[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r_wgt, w < p.cw ? woff + (2 * q0 + 16 * i) * 4 : kOutOfRange, 0, 0));
         }
     };
-    int csum = 0;  // this lane's share of its column's constant C: the words it stages, pad steps included
+    // this thread's share of its column's constant C, counted by class (words past K are zeros and count nothing)
+    int set0 = 0, set1 = 0, set2 = 0;
     auto stage_store = [&](int buf, int q0) {
 #pragma unroll
-        for (int i = 0; i < kFrags; ++i) {
-            lds_w[buf][((sq + 2 * i) * kNT + snt) * 64 + lane] = expand_weights_f4(wx[i]);
-            if (q0 + sq + 2 * i < steps) csum += class_sum(wx[i]);
-        }
-    };
-
-    // ---- rows: words [cw][B]; lane (j, h) of image tile mt reads word 2 q + h of image b0 + 32 mt + j
-    int bimg[MT], voff[MT];
+        for (int i = 0; i < kUnits; ++i)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        bimg[mt] = b0 + mt * 32 + j;
-        voff[mt] = (h * p.B + min(bimg[mt], p.B - 1)) * 4;
-    }
+            for (int t = 0; t < 4; ++t) {
+                const int ql = 8 * i + 2 * sc + (t >> 1);
+                uint32_t word = (uint32_t)wx[i][t];
+                if (TAIL && 2 * (q0 + ql) + (t & 1) >= p.cw) word = 0u;
+                lds_w[buf][(ql * kNT + snt) * 64 + ((32 * (t & 1) + sj) ^ (sc << 1))] = expand_weights_f4(word);
+                set0 += __popc(word & 0x11111111u);
+                set1 += __popc(word & 0x22222222u);
+                set2 += __popc(word & 0x44444444u);
+            }
+    };
+    int rlane[4];  // where the lane's fragment of k-step q lies in its run of 64: rlane[q / 2 % 4]
+#pragma unroll
+    for (int c = 0; c < 4; ++c) rlane[c] = lane ^ (c << 1);
+
+    // ---- rows: words [cw][B]; lane (j, h) reads word 2 q + h of its MT neighbouring images in one request.  Images past B:
+    // the next word's, or 0 behind the tensor; their results are discarded.
+    const int b_lane = b0 + MT * j;
+    const int voff = (h * p.B + b_lane) * 4;
     const __amdgpu_buffer_rsrc_t r_act =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(act), 0, p.cw * p.B * 4, 0x00020000);
     const int step_bytes = 2 * p.B * 4;
@@ -91,9 +114,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     // no test for the end of K: a request past it lies outside the descriptor's range, touches no memory and
     // returns 0 (such words are never multiplied), and the k-steps stay free of branches
     auto request = [&](uint32_t* dst) {
+        static_assert(MT == 2 || MT == 4, "one request holds the lane's images");
+        if constexpr (MT == 4) {
+            const v4i v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r_act, voff, lq * step_bytes, 0));
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-            dst[mt] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r_act, voff[mt], lq * step_bytes, 0);
+            for (int mt = 0; mt < 4; ++mt) dst[mt] = (uint32_t)v[mt];
+        } else {
+            const v2i v = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(r_act, voff, lq * step_bytes, 0));
+            dst[0] = (uint32_t)v[0];
+            dst[1] = (uint32_t)v[1];
+        }
         ++lq;
     };
 
@@ -108,6 +138,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 #pragma unroll
     for (int d = 0; d < kAhead; ++d) request(ring[d]);
     stage_load(0);
+    __builtin_amdgcn_sched_barrier(0);  // (everything is requested before anything is waited for)
     stage_store(0, 0);
     __syncthreads();
 
@@ -119,59 +150,68 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     for (int mt = 0; mt < MT; ++mt) bnext[mt] = expand_rows_f4(ring[0][mt]);
     request(ring[0]);
 
-    int buf = 0;
-    for (int q0 = 0; q0 < steps; q0 += kBlk) {
-        const bool more = q0 + kBlk < steps;  // uniform
-        if (more) stage_load(q0 + kBlk);
-        const int cnt = min(kBlk, steps - q0);  // a multiple of kAhead
-        const v4i* __restrict__ wl = lds_w[buf];
+    auto run = [&](const v4i* __restrict__ wl, int ql) __attribute__((always_inline)) {  // kAhead steps of a block
 #pragma unroll
-        for (int nt = 0; nt < kNT; ++nt) anext[nt] = wl[nt * 64 + lane];
-        for (int ql = 0; ql < cnt; ql += kAhead) {
+        for (int d = 0; d < kAhead; ++d) {
+            v4i acur[kNT], bcur[MT];
 #pragma unroll
-            for (int d = 0; d < kAhead; ++d) {
-                v4i acur[kNT], bcur[MT];
+            for (int nt = 0; nt < kNT; ++nt) acur[nt] = anext[nt];
 #pragma unroll
-                for (int nt = 0; nt < kNT; ++nt) acur[nt] = anext[nt];
+            for (int mt = 0; mt < MT; ++mt) bcur[mt] = bnext[mt];
+            const int qn = min(ql + d + 1, kBlk - 1);  // after a block's last step: read again, not used
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) bcur[mt] = bnext[mt];
-                const int qn = min(ql + d + 1, kBlk - 1);  // after a block's last step: read again, not used
+            for (int nt = 0; nt < kNT; ++nt) anext[nt] = wl[(qn * kNT + nt) * 64 + rlane[(d + 1) / 2 % 4]];
+            const int dn = (d + 1) % kAhead;  // a constant once the loop over d is unrolled
 #pragma unroll
-                for (int nt = 0; nt < kNT; ++nt) anext[nt] = wl[(qn * kNT + nt) * 64 + lane];
-                const int dn = (d + 1) % kAhead;  // a constant once the loop over d is unrolled
+            for (int mt = 0; mt < MT; ++mt) bnext[mt] = expand_rows_f4(ring[dn][mt]);
+            request(ring[dn]);
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) bnext[mt] = expand_rows_f4(ring[dn][mt]);
-                request(ring[dn]);
+            for (int nt = 0; nt < kNT; ++nt)
 #pragma unroll
-                for (int nt = 0; nt < kNT; ++nt)
+                for (int mt = 0; mt < MT; ++mt)
+                    acc[mt][nt] = Acc<FMT_F4>::mma(acur[nt], bcur[mt], acc[mt][nt]);
+            // issue order of the step: fragment reads first, then each MFMA followed by a few of the next
+            // step's expansion instructions (they run while the matrix pipeline is busy), the row requests
+            // in the middle
+            __builtin_amdgcn_sched_group_barrier(0x100, kNT, 0);  // LDS reads
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        acc[mt][nt] = Acc<FMT_F4>::mma(acur[nt], bcur[mt], acc[mt][nt]);
-                // issue order of the step: fragment reads first, then each MFMA followed by a few of the next
-                // step's expansion instructions (they run while the matrix pipeline is busy), the row requests
-                // in the middle
-                __builtin_amdgcn_sched_group_barrier(0x100, kNT, 0);  // LDS reads
-#pragma unroll
-                for (int i = 0; i < kNT * MT; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x002, (4 * MT + kNT * MT - 1) / (kNT * MT), 0);  // VALU
-                    if (i == kNT * MT / 2) __builtin_amdgcn_sched_group_barrier(0x020, MT, 0);  // row requests
-                }
-                __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < kNT * MT; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, (4 * MT + kNT * MT - 1) / (kNT * MT), 0);  // VALU
+                if (i == kNT * MT / 2) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // row request
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    auto first_fragments = [&](const v4i* __restrict__ wl) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < kNT; ++nt) anext[nt] = wl[nt * 64 + rlane[0]];
+    };
+    // Whole blocks that another one follows, without a branch from the next weights' request to their staging: with one (a
+    // request only where there are more, a loop over the block's steps) the compiler cannot count what is outstanding
+    // and waits for every row request twice a block (8 192 x 448 x 8 192 23.1 us, so 19.1; 200 x 8 192 x 8 192 18.7 / 16.5;
+    // 2 048 x 4 096 x 8 192 31.9 / 30.5; level where two workgroups in a CU cover for each other).
+    int buf = 0, q0 = 0;
+    for (; q0 + kBlk < steps; q0 += kBlk) {
+        stage_load(q0 + kBlk);
+        first_fragments(lds_w[buf]);
+#pragma unroll
+        for (int ql = 0; ql < kBlk; ql += kAhead) run(lds_w[buf], ql);
         // the other buffer was last read in the previous block, which every wave left before the barrier below
-        if (more) stage_store(buf ^ 1, q0 + kBlk);
+        stage_store(buf ^ 1, q0 + kBlk);
         __syncthreads();
         buf ^= 1;
     }
+    first_fragments(lds_w[buf]);
+    for (int ql = 0; ql < steps - q0; ql += kAhead) run(lds_w[buf], ql);
+    __syncthreads();
 
-    // ---- the columns' constants: four lanes (two k-halves of two waves) staged each column's words.  The weight
+    // ---- the columns' constants: four threads staged each column's words.  The weight
     // buffers are free now (every wave has passed the loop's last barrier).
     int* colc = reinterpret_cast<int*>(&lds_w[0][0]);  // [kNT * 32]
     if (tid < kNT * 32) colc[tid] = 0;
     __syncthreads();
-    atomicAdd(&colc[snt * 32 + row_to_channel(j)], csum);
+    atomicAdd(&colc[snt * 32 + row_to_channel(sj)], 2 * (5 * set0 + 3 * set1 + set2));
     __syncthreads();
 
     // int32 output, all 64 columns of the group exist and every row's run of them is 16-byte aligned (uniform): the
@@ -179,7 +219,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     const bool raw_rows = EPI == EPI_RAW && n0 + 32 * kNT <= p.N && p.raw_b_stride % 4 == 0 &&
                           (reinterpret_cast<uintptr_t>(p.out_i32) & 15) == 0;
 
-    // ---- epilogue: the lane holds columns cbase + v of image bimg[mt]
+    // ---- epilogue: the lane holds columns cbase + v of image b_lane + mt
 #pragma unroll
     for (int nt = 0; nt < kNT; ++nt) {
         const int cbase = n0 + nt * 32 + 16 * h;
@@ -196,7 +236,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const int b = bimg[mt];
+            const int b = b_lane + mt;
             const bool b_ok = b < p.B;
             if constexpr (EPI == EPI_THRESH) {
                 uint32_t hw = 0;
@@ -272,7 +312,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
                                 (int)acc[mt][nt][4 * g + 2] - off[4 * g + 2], (int)acc[mt][nt][4 * g + 3] - off[4 * g + 3]};
                 }
                 // (same wave writes and reads: program order and the wait for LDS are all the synchronisation)
-                const int row0 = b0 + mt * 32;
 #pragma unroll
                 for (int part = 0; part < 2; ++part) {
                     v4i q[4];
@@ -280,7 +319,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
                     for (int k = 0; k < 4; ++k) q[k] = *reinterpret_cast<const v4i*>(mine + (16 * part + 4 * k + rl) * kPitch + 4 * cl);
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
-                        const int row = row0 + 16 * part + 4 * k + rl;
+                        const int row = b0 + MT * (16 * part + 4 * k + rl) + mt;
                         if (row < p.B)
                             *reinterpret_cast<v4i*>(p.out_i32 + (size_t)row * p.raw_b_stride + n0 + 4 * cl) = q[k];
                     }
@@ -290,10 +329,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     }
 }
 
-// image tiles per wave: 4 when that still gives every CU two workgroups
+// Image tiles per wave: two, whose smaller workgroups leave less of a last round empty and of which a compute unit runs three
+// (3 072 x 3 072 x 8 192 39.5 us against 45.0 with four, 8 000 x 2 080 x 6 016 51.8 / 56.9, 1 500 x 8 192 x 4 096 26.2 / 28.7); four, which multiply
+// every weight fragment twice as often, where they come out even over the compute units, at two workgroups in each or more,
+// and K is long (5 000 x 3 104 x 7 200 62 us with two, 58.6 with four; 8 192^3 217 / 201; 8 192 x 8 192 x 512 45.0 / 48.2).
 int gemm_mt(const BgemmParams& p) {
+    constexpr int kCus = 256, kLongK = 64;  // (words)
     const long long n_groups = (p.N + 32 * kNT - 1) / (32 * kNT);
-    return ((p.B + 32 * 4 * kWaves - 1) / (32 * 4 * kWaves)) * n_groups >= 512 ? 4 : 2;
+    auto a_cu = [&](int mt) {  // image tiles that the busiest compute unit's waves take
+        return mt * ((((p.B + 32 * mt * kWaves - 1) / (32 * mt * kWaves)) * n_groups + kCus - 1) / kCus);
+    };
+    return p.cw >= kLongK && a_cu(4) >= 8 && a_cu(4) <= a_cu(2) ? 4 : 2;
 }
 
 }  // namespace
@@ -302,16 +348,20 @@ bool gemm_mfma_applicable(const BgemmParams& p) {
     if (p.PH * p.PW != 1 || p.R * p.S != 1 || p.pool_h * p.pool_w != 1) return false;
     if (p.res_in != nullptr || p.res_out != nullptr) return false;
     if (p.mode != EPI_THRESH && p.mode != EPI_AFFINE && p.mode != EPI_RAW) return false;
-    if (p.k_tap > 32 * p.cw || (p.cw % 2 != 0 && p.mode != EPI_RAW)) return false;
-    if ((long long)p.cw * p.B * 4 >= (1LL << 31)) return false;          // 32-bit buffer offsets
-    // large enough to give every CU a workgroup with two image tiles per wave; smaller problems are bound by
-    // launch and fill and stay with the kernels written for them
+    if (p.k_tap > 32 * p.cw || (p.cw % 4 != 0 && p.mode != EPI_RAW)) return false;
+    // 32-bit buffer offsets: all rows' words, 64 columns' words
+    if ((long long)p.cw * p.B * 4 >= (1LL << 31) || (long long)p.cw * 32 * kNT * 4 >= (1LL << 31)) return false;
+    // Large enough to give every CU a workgroup with two image tiles per wave; smaller problems are bound by launch and fill and
+    // stay with the kernels written for them, but for int32 products of many 32 x 32 tiles and a long K (8 192 x 448 x 8 192
+    // 30.3 us there, 19.5 here; 200 x 8 192 x 8 192 24.6 / 17.0; 1 500 x 1 504 x 1 504 8.4 / 7.7; below the line 512 x 3 072 x 2 048
+    // 7.8 / 7.9, 2 048 x 1 024 x 1 024 6.2 / 6.8, 33 x 8 192 x 4 096 6.7 / 10.0).
     const long long wgs = (long long)((p.B + 32 * 2 * kWaves - 1) / (32 * 2 * kWaves)) * ((p.N + 32 * kNT - 1) / (32 * kNT));
-    return wgs >= 256;
+    const long long tiles = (long long)((p.B + 31) / 32) * ((p.N + 31) / 32);
+    return wgs >= 256 || (p.mode == EPI_RAW && tiles >= 1200 && tiles * p.cw >= 100000);
 }
 
 void gemm_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len) {
-    snprintf(buf, len, "gemm_mfma_f4_kernel<%d, %d, %s>", gemm_mt(p), p.mode, p.cw % 2 != 0 ? "true" : "false");
+    snprintf(buf, len, "gemm_mfma_f4_kernel<%d, %d, %s>", gemm_mt(p), p.mode, p.cw % 4 != 0 ? "true" : "false");
 }
 
 template <int MT>
@@ -321,8 +371,8 @@ static int launch_gemm_mt(const BgemmParams& p, hipStream_t stream) {
     const long long blocks = row_blocks * n_groups;
     if (blocks <= 0 || blocks > 0x7fffffffLL) return fail(TCBNN_EINVAL, "gemm grid too large");
     const dim3 grid((unsigned)blocks), block(kThreads);
-    const bool odd = p.cw % 2 != 0;
-    TCBNN_REQUIRE(!odd || p.mode == EPI_RAW, "gemm: an odd number of words per row");
+    const bool tail = p.cw % 4 != 0;
+    TCBNN_REQUIRE(!tail || p.mode == EPI_RAW, "gemm: rows that are no whole 128-bit units");
     switch (p.mode) {
         case EPI_THRESH:
             hipLaunchKernelGGL((gemm_mfma_f4_kernel<MT, EPI_THRESH, false>), grid, block, 0, stream, p, p.act, p.wgt, p.bn,
@@ -333,7 +383,7 @@ static int launch_gemm_mt(const BgemmParams& p, hipStream_t stream) {
                                p.bn_scale, p.bn_bias, n_groups);
             break;
         default:
-            if (odd)
+            if (tail)
                 hipLaunchKernelGGL((gemm_mfma_f4_kernel<MT, EPI_RAW, true>), grid, block, 0, stream, p, p.act, p.wgt, p.bn,
                                    p.bn, n_groups);
             else

@@ -40,6 +40,20 @@ def test_bmm(gpu, variant, m, n, k):
     np.testing.assert_array_equal(got, orc.bmm(a, b, k))
 
 
+@pytest.mark.parametrize("m,n,k", [
+    # few rows or columns and a long K: both sides of the line between the kernels for small and for large products
+    (300, 4096, 4128), (257, 4128, 2624), (1220, 1056, 2624), (1184, 1024, 4096),
+    # two and four image tiles per wave: rows past the last one, a last column group of 32, rows of the weights that are
+    # no whole 128-bit units (1 to 3 words more), K that ends with a block, after one group of k-steps, within one
+    (3070, 2112, 1024), (3070, 2080, 1088), (2049, 3104, 544), (4095, 4064, 2080), (4097, 4096, 2528), (5000, 3104, 2112),
+])
+def test_bmm_wide_requests(gpu, m, n, k):
+    r = rng(m + n + k)
+    a = r.integers(0, 2 ** 32, size=(m, k // 32), dtype=np.uint64).astype(np.uint32)
+    b = r.integers(0, 2 ** 32, size=(n, k // 32), dtype=np.uint64).astype(np.uint32)
+    np.testing.assert_array_equal(gpuops.bmm(a, b, m, n, k, _variant(gpu, "mfma_f4")), orc.bmm(a, b, k))
+
+
 # --------------------------------------------------------------------------- In / Fc / Out layers
 @pytest.mark.parametrize("b,k", [(8, 784), (100, 128), (8192, 784), (3, 1000)])
 def test_in128(gpu, b, k):
