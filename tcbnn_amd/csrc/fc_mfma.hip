@@ -214,6 +214,7 @@ bool fc_mfma_applicable(const BgemmParams& p) {
 }
 
 namespace {
+constexpr int kCus = 256, kCuWaves = 16;  // compute units, and waves of these kernels that one holds (120 registers)
 // Split of K over the waves of a workgroup: waves per tile, 8-word groups per wave, and how many groups the
 // kernel requests ahead of its first multiply (0: a streaming loop).
 struct FcPlan {
@@ -225,16 +226,24 @@ FcPlan fc_plan(const BgemmParams& p) {
     f.n_tiles = (p.N + 31) / 32;
     f.b_tiles = (p.B + 31) / 32;
     const int groups = (p.cw + 7) / 8;
-    // waves per tile: at least 4 groups (16 k-steps) each, no more than fill the machine a few times
+    // Waves per tile: at least 4 groups (16 k-steps) each, and no more than let every workgroup be resident at once (the kernels hold
+    // four waves per SIMD): a second round of workgroups pays for its start and its sums again, while four waves a SIMD keep the VALU
+    // busy, which is what binds (14 of its instructions to a product).  Four waves are taken all the same: they end at different times
+    // and follow one another.  9216 inputs, 4096 outputs, batch 200: 9 waves in four rounds 13.6 us, 4 in one 9.3 (batch 128: 7.9 ->
+    // 5.9, 384: 16.1 -> 12.2 with four waves in two rounds, 14.8 with two in one); 25088 -> 4096, batch 224: 27.0 -> 19.3;
+    // 32768 -> 512, batch 544: 16.0 -> 13.7; 16384 -> 2048, batch 256: 10.4 -> 8.9.
+    const long long tiles = (long long)f.n_tiles * f.b_tiles;
     int kwaves = std::max(1, std::min(kMaxWaves, groups / 4));
-    while (kwaves > 1 && (long long)f.n_tiles * f.b_tiles * kwaves > 8192) --kwaves;
+    while (kwaves > 4 && tiles > kCus * (kCuWaves / kwaves)) --kwaves;
+    while (kwaves > 1 && tiles * kwaves > 8192) --kwaves;
     f.gpw = (groups + kwaves - 1) / kwaves;
     f.kwaves = (groups + f.gpw - 1) / f.gpw;
     f.pre = f.gpw <= 2 ? 2 : (f.gpw <= 7 ? 7 : 0);
     // Requests of sixteen bytes a lane where the address units are busy: long slices (25088 inputs, batch 256, 4096 outputs: 32.5 ->
-    // 27.7 us; 32768 inputs, 512 outputs, batch 77: 13.2 -> 12.3) and many waves (9216 inputs, 4096 outputs, batch 200, 8064 waves: 21.7 ->
-    // 21.1).  With few, the way through LDS only adds to the chain (8192 inputs, 1024 outputs, batch 256, 2048 waves: 8.2 -> 8.4).
-    f.staged = f.pre == 0 || (f.pre == 7 && (long long)f.n_tiles * f.b_tiles * f.kwaves >= 3072);
+    // 27.7 us; 32768 inputs, 512 outputs, batch 77: 13.2 -> 12.3) and many waves in large workgroups (16384 inputs, 2048 outputs, batch
+    // 128, 4096 waves: 5.65 -> 5.5).  With few, the way through LDS only adds to the chain (8192 inputs, 1024 outputs, batch 256, 2048
+    // waves: 8.2 -> 8.4), and four workgroups of four waves a CU hide it less (4096 inputs and outputs, batch 200: 5.5 -> 5.8).
+    f.staged = f.pre == 0 || (f.pre == 7 && f.kwaves > 4 && tiles * f.kwaves >= 3072);
     return f;
 }
 }  // namespace

@@ -139,6 +139,29 @@ def test_fc128_activations_through_lds(gpu, b, k, n):
     fin.release()
 
 
+@pytest.mark.parametrize("b,k,n,name", [
+    (255, 16001, 1024, "<0, 7, true>"),   # as many tiles as compute units
+    (255, 16001, 1056, "<0, 0, true>"),   # one column of tiles more: eight waves
+    (200, 9000, 4096, "<0, 0, true>"),    # four waves, all at once, the last with a part of a slice
+    (257, 4100, 3000, "<0, 7, false>")])  # four waves, short slices, images past the batch
+def test_fc128_workgroups_at_once(gpu, b, k, n, name):
+    """Waves per tile by how many workgroups a compute unit holds: around the lines between them."""
+    r = rng(b + k + n)
+    x = r.standard_normal((b, k)).astype(np.float32)
+    w = rm.pm1(r, (k, n))
+    bn = r.normal(0, np.sqrt(k), n).astype(np.float32)
+    want = orc.fc128(orc.in128(x), orc.pack_fc_weight(w), bn, k, n)
+    fin = gpu.In128LayerParam("Fin", b, k).initialize(x)
+    layer = gpu.Fc128LayerParam("Fc", b, k, n).initialize(gpu.ArrayWeights([w, bn]), fin.get_output_gpu())
+    assert layer.kernel_name() == "fc_mfma_f4_kernel" + name, layer.kernel_name()
+    fin.forward()
+    layer.forward()
+    gpuops.sync()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    layer.release()
+    fin.release()
+
+
 @pytest.mark.parametrize("b,widths,with_in,with_out,launches", [
     # one image and neuron; ends of words, tiles and groups of K; a wave's second tiles and second round of tiles; activations
     # of 2048 (two requests of weights ahead, 64 KB of LDS); outputs of several rounds of tiles
