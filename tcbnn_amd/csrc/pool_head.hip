@@ -111,88 +111,115 @@ __device__ __forceinline__ void i12_from_pairs(const uint32_t* q, uint32_t& w0, 
     i12_pack8(v, w0, w1, w2);
 }
 
-// A thread takes one unit (word of bits, or residual group) of one image and walks down `rows` output pixels of a
-// column: of the three input rows of a window the last is the next window's first, so an output costs six loads and not
-// nine, all of them in flight together.  417 MB at 112x112, 64 channels, 12 bits, batch 256, in 86 us (104 us with nine
-// loads and a 64-bit division per output): three quarters of the copy rate; a wave waits for memory (44 % of its time) and
-// for the other waves' unpacking, maxima and packing (47 %).
+// A thread takes one unit (word of bits, or residual group) of one image and two output pixels of a column: of the three input
+// rows of a window the last is the next window's first.  A pixel's address is scalar and a lane's place in it 32 bits.
+// Neighbouring windows share a column and pairs of outputs a row, so workgroups are dealt in runs of neighbours to an XCD, whose L2
+// then has what the windows share: asked for by several XCDs it came from memory again.  With that, two outputs a thread are as
+// good as any number or better at every size (many rows a thread: fewer, longer chains).  64 channels at 112x112 in 12 bits, us,
+// eight rows a thread and workgroups dealt in turn -> here: batch 256 91 -> 80 (417 MB, 5.2 TB/s), 64 27.3 -> 21.5, 32 14.4 -> 10.3,
+// 4 7.2 -> 6.6; 128 channels at 56x56 in 16 bits, batch 77 22 -> 15.3.  (Asking for the next output's words while one is reduced: 3 %
+// slower below batch 256, 4 % faster there.)  What binds it at batch 256: memory.
+constexpr int kPoolRows = 2;
 template <int FMT>
-__global__ __launch_bounds__(kThreads) void pool3x3s2_kernel(const PoolParams p, int rows) {
-    const int rem = (int)(blockIdx.x * kThreads + threadIdx.x);
-    if (rem >= (p.cw + p.groups) * p.B) return;
-    const int u = rem / p.B, b = rem - u * p.B;
-    const int ox = blockIdx.y, x0 = ox * 2 - p.pad;
-    const int oy0 = blockIdx.z * rows, oy1 = min(p.OH, oy0 + rows);
+__global__ __launch_bounds__(kThreads) void pool3x3s2_kernel(const PoolParams p) {
+    // units, then columns, then pairs of rows; workgroups go to the 8 XCDs in turn
+    auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const int units = (int)gridDim.x, wgs = units * p.OW * (int)gridDim.z, dealt = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+    const int xcd = dealt & 7, wg = xcd * (wgs >> 3) + min(xcd, wgs & 7) + (dealt >> 3);
+    const int col = uniform(wg / units), bx = wg - col * units, pair = uniform(col / p.OW), ox = col - pair * p.OW;
+    const int oy0 = pair * kPoolRows, oy1 = min(p.OH, oy0 + kPoolRows);
+    const unsigned rem = (unsigned)bx * kThreads + threadIdx.x;
+    if (rem >= (unsigned)((p.cw + p.groups) * p.B)) return;
+    const unsigned u = rem / (unsigned)p.B, b = rem - u * (unsigned)p.B;
+    const int x0 = ox * 2 - p.pad;
     // columns outside the frame repeat one inside it (padding < window: there is one)
     int xs[3];
 #pragma unroll
     for (int s = 0; s < 3; ++s) xs[s] = min(max(x0 + s, max(x0, 0)), min(x0 + 2, p.W - 1));
-    auto row_of = [&](int y) { return (size_t)y * p.W; };
-    if (u < p.cw) {  // OR of the window's words
-        const uint32_t* __restrict__ const src = p.in + (size_t)u * p.B + b;
+    if (u < (unsigned)p.cw) {  // OR of the window's words
+        const unsigned at = u * (unsigned)p.B + b;
         const size_t px = (size_t)p.cw * p.B;
         auto row = [&](int y) {
             uint32_t v = 0u;
             if (y >= 0 && y < p.H)
 #pragma unroll
-                for (int s = 0; s < 3; ++s) v |= src[(row_of(y) + xs[s]) * px];
+                for (int s = 0; s < 3; ++s) v |= (p.in + ((size_t)y * p.W + xs[s]) * px)[at];
             return v;
         };
         uint32_t last = row(oy0 * 2 - p.pad);
         for (int oy = oy0; oy < oy1; ++oy) {
             const int y = oy * 2 - p.pad;
             const uint32_t mid = row(y + 1), next = row(y + 2);
-            p.out[(((size_t)oy * p.OW + ox) * p.cw + u) * p.B + b] = last | mid | next;
+            (p.out + ((size_t)oy * p.OW + ox) * px)[at] = last | mid | next;
             last = next;
         }
         return;
     }
-    const int g = u - p.cw;
-    constexpr int kQ = FMT == TCBNN_RES_I12 ? 8 : 4;  // registers of a group: pairs, or the four words
+    const unsigned g = u - (unsigned)p.cw;
+    constexpr bool kI12 = FMT == TCBNN_RES_I12;
+    constexpr int kQ = kI12 ? 8 : 4;  // registers of a group: pairs, or the four words
+    // a lane's bytes of a pixel: sixteen, and eight more of twelve-bit groups
+    const unsigned at = kI12 ? (g * 6u * (unsigned)p.B + b * 4u) * 4u : (g * (unsigned)p.B + b) * 16u;
+    const unsigned at8 = (g * 6u * (unsigned)p.B + (unsigned)p.B * 4u + b * 2u) * 4u;
+    const size_t px = (size_t)p.groups * p.B * (kI12 ? 24 : 16);
+    struct Words {  // three pixels of a row, as they lie in memory
+        uint4 a[3];
+        uint2 c[kI12 ? 3 : 1];
+    };
     struct Group {
         uint32_t q[kQ];
     };
-    auto most = [](const Group& a, const Group& c) {
+    auto most = [](const Group& a, const Group& c) __attribute__((always_inline)) {
         Group m;
 #pragma unroll
         for (int k = 0; k < kQ; ++k)
             m.q[k] = FMT == TCBNN_RES_I32 ? (uint32_t)max((int)a.q[k], (int)c.q[k]) : max2x16(a.q[k], c.q[k]);
         return m;
     };
-    auto load = [&](size_t pix) {
-        Group r;
-        if constexpr (FMT == TCBNN_RES_I12) {
-            const uint32_t* const w = reinterpret_cast<const uint32_t*>(p.rin);
-            const uint4 a = *reinterpret_cast<const uint4*>(w + i12_word_index(pix, (size_t)p.groups, g, p.B, b, 0));
-            const uint2 c = *reinterpret_cast<const uint2*>(w + i12_word_index(pix, (size_t)p.groups, g, p.B, b, 4));
-            i12_to_pairs(a.x, a.y, a.z, r.q);
-            i12_to_pairs(a.w, c.x, c.y, r.q + 4);
-        } else {
-            const uint4 a = reinterpret_cast<const uint4*>(p.rin)[(pix * p.groups + g) * p.B + b];
-            r.q[0] = a.x, r.q[1] = a.y, r.q[2] = a.z, r.q[3] = a.w;
-        }
-        return r;
-    };
-    auto row = [&](int y) { return most(most(load(row_of(y) + xs[0]), load(row_of(y) + xs[1])), load(row_of(y) + xs[2])); };
     // (rows outside the frame repeat the nearest row inside, which is in the window: padding < window)
-    auto clamped = [&](int y, int oy) { return min(max(y, max(0, oy * 2 - p.pad)), min(p.H - 1, oy * 2 - p.pad + 2)); };
-    Group last = row(clamped(oy0 * 2 - p.pad, oy0));
+    auto request = [&](int y, int oy, Words& w) __attribute__((always_inline)) {
+        const int yc = min(max(y, max(0, oy * 2 - p.pad)), min(p.H - 1, oy * 2 - p.pad + 2));
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const char* const pix = reinterpret_cast<const char*>(p.rin) + ((size_t)yc * p.W + xs[s]) * px;
+            w.a[s] = *reinterpret_cast<const uint4*>(pix + at);
+            if constexpr (kI12) w.c[s] = *reinterpret_cast<const uint2*>(pix + at8);
+        }
+    };
+    auto reduce = [&](const Words& w) __attribute__((always_inline)) {
+        Group r[3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            if constexpr (kI12) {
+                i12_to_pairs(w.a[s].x, w.a[s].y, w.a[s].z, r[s].q);
+                i12_to_pairs(w.a[s].w, w.c[s].x, w.c[s].y, r[s].q + 4);
+            } else {
+                r[s].q[0] = w.a[s].x, r[s].q[1] = w.a[s].y, r[s].q[2] = w.a[s].z, r[s].q[3] = w.a[s].w;
+            }
+        }
+        return most(most(r[0], r[1]), r[2]);
+    };
+    Words first;
+    request(oy0 * 2 - p.pad, oy0, first);
+    Group last = reduce(first);
     for (int oy = oy0; oy < oy1; ++oy) {
         const int y = oy * 2 - p.pad;
-        const Group mid = row(clamped(y + 1, oy)), next = row(clamped(y + 2, oy));
-        const Group m = most(most(last, mid), next);
-        const size_t pix = (size_t)oy * p.OW + ox;
-        if constexpr (FMT == TCBNN_RES_I12) {
-            uint32_t* const w = reinterpret_cast<uint32_t*>(p.rout);
+        Words mid, next;
+        request(y + 1, oy, mid);
+        request(y + 2, oy, next);
+        const Group upper = most(last, reduce(mid));
+        last = reduce(next);
+        const Group m = most(upper, last);
+        char* const pix = reinterpret_cast<char*>(p.rout) + ((size_t)oy * p.OW + ox) * px;
+        if constexpr (kI12) {
             uint32_t d[6];
             i12_from_pairs(m.q, d[0], d[1], d[2]);
             i12_from_pairs(m.q + 4, d[3], d[4], d[5]);
-            *reinterpret_cast<uint4*>(w + i12_word_index(pix, (size_t)p.groups, g, p.B, b, 0)) = make_uint4(d[0], d[1], d[2], d[3]);
-            *reinterpret_cast<uint2*>(w + i12_word_index(pix, (size_t)p.groups, g, p.B, b, 4)) = make_uint2(d[4], d[5]);
+            *reinterpret_cast<uint4*>(pix + at) = make_uint4(d[0], d[1], d[2], d[3]);
+            *reinterpret_cast<uint2*>(pix + at8) = make_uint2(d[4], d[5]);
         } else {
-            reinterpret_cast<uint4*>(p.rout)[(pix * p.groups + g) * p.B + b] = make_uint4(m.q[0], m.q[1], m.q[2], m.q[3]);
+            *reinterpret_cast<uint4*>(pix + at) = make_uint4(m.q[0], m.q[1], m.q[2], m.q[3]);
         }
-        last = next;
     }
 }
 
@@ -391,12 +418,14 @@ extern "C" int tcbnn_pool128_forward(const tcbnn_pool128_desc* d, void* stream) 
     const long long total = (long long)(p.cw + p.groups) * p.B * p.OH * p.OW;
     const long long blocks = (total + kThreads - 1) / kThreads;
     TCBNN_REQUIRE(blocks <= 0x7fffffffLL, "pool128: grid too large");
-    if (p.window == 3 && p.stride == 2 && p.OW <= 65535 && p.OH <= 65535 && (long long)(p.cw + p.groups) * p.B < (1LL << 31) - kThreads) {
-        // output rows per thread: eight, fewer while that leaves the chip's 1024 SIMDs under eight waves each
-        const long long columns = (long long)(p.cw + p.groups) * p.B * p.OW;
-        const int rows = (int)std::min(8LL, std::max(1LL, columns * p.OH / (8192LL * 64)));
-        const dim3 grid((unsigned)(((long long)(p.cw + p.groups) * p.B + kThreads - 1) / kThreads), (unsigned)p.OW, (unsigned)((p.OH + rows - 1) / rows));
-        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, p, rows); };
+    const long long per_pixel = (long long)(p.cw + p.groups) * p.B;
+    const long long units = (per_pixel + kThreads - 1) / kThreads;
+    const int pairs = (p.OH + kPoolRows - 1) / kPoolRows;
+    // (32 bits hold a lane's bytes within a pixel and a workgroup's number)
+    if (p.window == 3 && p.stride == 2 && p.OW <= 65535 && pairs <= 65535 && per_pixel * 24 < (1LL << 32) - 24 * kThreads &&
+        units * p.OW * pairs < (1LL << 31)) {
+        const dim3 grid((unsigned)units, (unsigned)p.OW, (unsigned)pairs);
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, p); };
         if (p.fmt == TCBNN_RES_I12)
             launch(pool3x3s2_kernel<TCBNN_RES_I12>);
         else if (p.fmt == TCBNN_RES_I16)

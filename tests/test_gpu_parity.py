@@ -1877,7 +1877,8 @@ def test_uploads_through_pinned_memory(gpu, n):
 
 
 @pytest.mark.parametrize("fmt", [0, 1, 2])
-@pytest.mark.parametrize("b,h,c,pad", [(2, 5, 16, 0), (6, 8, 33, 2), (66, 4, 64, 1), (4, 3, 130, 2)])
+@pytest.mark.parametrize("b,h,c,pad", [(2, 5, 16, 0), (6, 8, 33, 2), (66, 4, 64, 1), (4, 3, 130, 2),
+                                        (300, 9, 40, 1)])  # several workgroups a pixel, their number no multiple of eight
 def test_pool3x3_stride2(gpu, b, h, c, pad, fmt):
     """The rolling 3x3 / stride 2 kernel at the frame's edges: every padding, odd and even frames, channel tails."""
     test_pool128(gpu, b, h, c, 3, 2, pad, fmt)
