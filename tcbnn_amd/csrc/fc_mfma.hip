@@ -200,6 +200,105 @@ __global__ __launch_bounds__(64 * kMaxWaves) void fc_mfma_f4_kernel(
     }
 }
 
+// A tile of 16 images x 16 neurons, for launches that leave compute units out (thresholds and bits only; fc_plan says when): four
+// times the workgroups of the kernel above, each with half the expansions, which are what its waves wait for each other with
+// (14 VALU instructions to a product of 32 cycles there, to two of 16 here).  Operands are the same words: lane (i, q) multiplies
+// words 8g + 4 (q & 1) + 2 (q >> 1) + s of group g in step s, of neuron and image i of the tile.  A workgroup writes half words.
+template <int PRE>
+__global__ __launch_bounds__(64 * kMaxWaves) void fc_mfma_f4_small_kernel(
+    const BgemmParams p, const uint32_t* __restrict__ act, const uint32_t* __restrict__ wgt, const float* __restrict__ bnp, int n_tiles,
+    int groups_per_wave) {
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    typedef int v2i __attribute__((ext_vector_type(2)));
+    __shared__ int red[4 * 64];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, i = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = blockIdx.x & 1, nt = (blockIdx.x >> 1) % n_tiles, bt = (blockIdx.x >> 1) / n_tiles;
+    const int n0 = nt * 32 + 16 * half, b = bt * 16 + i;
+    const int cw = p.cw, groups = (cw + 7) / 8;
+    // neuron 16 half + i of the tile is row 8 (i / 4) + 4 half + i % 4 of the lane order (row_to_channel)
+    const int row = 32 * (q & 1) + 8 * (i >> 2) + 4 * half + (i & 3), first = 4 * (q & 1) + 2 * (q >> 1);
+    const v2i* __restrict__ wlane = reinterpret_cast<const v2i*>(wgt + fc_weight_row_words(n_tiles * 32, cw)) +
+                                    ((size_t)nt * groups * 64 + row) * 2 + (q >> 1);
+    const __amdgpu_buffer_rsrc_t r_act = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(act), 0, cw * p.B * 4, 0x00020000);
+    const int act_lane = (first * p.B + min(b, p.B - 1)) * 4;
+    const int g_begin = wave * groups_per_wave, g_end = min(groups, g_begin + groups_per_wave);
+
+    // every word of the wave is requested before the first multiply
+    v2i a[PRE];
+    uint32_t x[PRE][2];
+#pragma unroll
+    for (int u = 0; u < PRE; ++u)
+        if (g_begin + u < g_end) {
+            a[u] = wlane[(size_t)(g_begin + u) * 128];
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                x[u][s] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r_act, act_lane + ((g_begin + u) * 8 + s) * 4 * p.B, 0, 0);
+        }
+    float thr[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) thr[v] = bnp[min(n0 + 4 * q + v, p.N - 1)];
+    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto product = [&](v4i w, v4i y) __attribute__((always_inline)) {
+        const v8i w8 = {w[0], w[1], w[2], w[3], 0, 0, 0, 0}, y8 = {y[0], y[1], y[2], y[3], 0, 0, 0, 0};
+        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w8, y8, acc, 4, 4, 0, 0, 0, 0);
+    };
+#pragma unroll
+    for (int u = 0; u < PRE; ++u)
+        if (g_begin + u < g_end) {
+            const int g = g_begin + u;
+            if (32 * (8 * g + 8) <= p.k_tap) {  // (uniform)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) product(expand_f4((uint32_t)a[u][s]), expand_f4(x[u][s]));
+            } else {  // K tail: pad bits (and words past cw) must multiply as 0, not as +1
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const int nbits = p.k_tap - 32 * (8 * g + first + s);
+                    const uint32_t valid = nbits >= 32 ? 0xffffffffu : (nbits <= 0 ? 0u : 0xffffffffu << (32 - nbits));
+                    product(expand_f4_masked((uint32_t)a[u][s], valid), expand_f4(x[u][s]));
+                }
+            }
+        }
+
+    // ---- sum the slices (exact integers) in LDS
+    int dot[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) dot[v] = (int)acc[v];
+    if (blockDim.x > 64) {
+        if (wave == 0) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) red[v * 64 + lane] = dot[v];
+        }
+        __syncthreads();
+        if (wave != 0) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) atomicAdd(&red[v * 64 + lane], dot[v]);
+        }
+        __syncthreads();
+        if (wave != 0) return;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dot[v] = red[v * 64 + lane];
+    }
+    // ---- lane (i, q) holds neurons n0 + 4q + v of image b: its four bits, then the half word of the four lanes of an image
+    uint32_t bits = 0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const float t = thr[v] != thr[v] ? (p.nan_bit ? -INFINITY : INFINITY) : thr[v];
+        bits = __builtin_amdgcn_alignbit(bits, __float_as_uint((float)dot[v] - t), 31);
+    }
+    bits = (~bits & 15u) << (12 - 4 * q);
+    bits |= (uint32_t)__shfl_xor((int)bits, 16);
+    bits |= (uint32_t)__shfl_xor((int)bits, 32);
+    bits &= 0xffff0000u >> min(max(p.N - n0, 0), 16);
+    if (q == 0 && b < p.B) {
+        if (nt < p.bits_row_words) reinterpret_cast<uint16_t*>(p.out_bits + (size_t)nt * p.B + b)[1 - half] = (uint16_t)bits;
+        if (nt == n_tiles - 1 && half == 0)  // padding words of the 128-padded feature axis
+            for (int w = n_tiles; w < p.bits_row_words; ++w) p.out_bits[(size_t)w * p.B + b] = 0;
+    }
+}
+
 }  // namespace
 
 bool fc_mfma_applicable(const BgemmParams& p) {
@@ -219,13 +318,29 @@ constexpr int kCus = 256, kCuWaves = 16;  // compute units, and waves of these k
 // kernel requests ahead of its first multiply (0: a streaming loop).
 struct FcPlan {
     int n_tiles, b_tiles, kwaves, gpw, pre;
-    bool staged;
+    bool staged, small;
 };
 FcPlan fc_plan(const BgemmParams& p) {
     FcPlan f;
     f.n_tiles = (p.N + 31) / 32;
     f.b_tiles = (p.B + 31) / 32;
     const int groups = (p.cw + 7) / 8;
+    // Tiles of 16 x 16 while a compute unit has no more than one of them, slices as long as a wave requests whole, at least three
+    // groups each (13 waves are faster than 16 where both hold: sums of fewer).  us, tiles of 32 x 32 -> 16 x 16: 25088 inputs, 512
+    // outputs, batch 1 .. 64 7.4 -> 5.1, 128 7.3 -> 5.3, above the line 192 7.3 -> 7.3, 256 7.6 -> 7.7; 32768 -> 512, batch 77 8.3 ->
+    // 6.3; 9216 -> 4096, batch 16 4.6 -> 3.9, above 17 4.6 -> 4.7; 8192 -> 1024, batch 64 4.1 -> 3.6, above 100 4.1 -> 4.2.  Under 32
+    // such tiles (fewer than 512 outputs at batches to 16) nothing was measured and the kernel of 32 x 32 stays.
+    const long long small_tiles = 2LL * f.n_tiles * ((p.B + 15) / 16);
+    f.small = p.mode == EPI_THRESH && small_tiles >= 32 && small_tiles <= kCus && groups <= 8 * kMaxWaves;
+    if (f.small) {
+        f.b_tiles = (p.B + 15) / 16;
+        f.gpw = std::max(3, (groups + 12) / 13);
+        if (f.gpw > 8) f.gpw = (groups + kMaxWaves - 1) / kMaxWaves;
+        f.kwaves = (groups + f.gpw - 1) / f.gpw;
+        f.pre = f.gpw <= 4 ? 4 : 8;
+        f.staged = false;
+        return f;
+    }
     // Waves per tile: at least 4 groups (16 k-steps) each, and no more than let every workgroup be resident at once (the kernels hold
     // four waves per SIMD): a second round of workgroups pays for its start and its sums again, while four waves a SIMD keep the VALU
     // busy, which is what binds (14 of its instructions to a product).  Four waves are taken all the same: they end at different times
@@ -250,13 +365,21 @@ FcPlan fc_plan(const BgemmParams& p) {
 
 void fc_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len) {
     const FcPlan f = fc_plan(p);
-    snprintf(buf, len, "fc_mfma_f4_kernel<%d, %d, %s>", p.mode == EPI_AFFINE ? FC_AFFINE : FC_THRESH, f.pre, f.staged ? "true" : "false");
+    if (f.small) snprintf(buf, len, "fc_mfma_f4_small_kernel<%d>", f.pre);
+    else snprintf(buf, len, "fc_mfma_f4_kernel<%d, %d, %s>", p.mode == EPI_AFFINE ? FC_AFFINE : FC_THRESH, f.pre, f.staged ? "true" : "false");
 }
 
 int launch_fc_mfma(const BgemmParams& p, hipStream_t stream) {
     const FcPlan f = fc_plan(p);
     const int n_tiles = f.n_tiles, b_tiles = f.b_tiles, kwaves = f.kwaves, gpw = f.gpw;
-    const dim3 grid((unsigned)(n_tiles * b_tiles)), block(64 * kwaves);
+    const dim3 grid((unsigned)(n_tiles * b_tiles * (f.small ? 2 : 1))), block(64 * kwaves);
+    if (f.small) {
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, p, p.act, p.wgt, p.bn, n_tiles, gpw); };
+        if (f.pre == 4) launch(fc_mfma_f4_small_kernel<4>);
+        else launch(fc_mfma_f4_small_kernel<8>);
+        TCBNN_LAUNCH_CHECK("fc_mfma_f4_small_kernel");
+        return TCBNN_OK;
+    }
     auto launch = [&](auto mode, auto pre, auto staged) {
         constexpr int MODE = decltype(mode)::value, PRE = decltype(pre)::value;
         constexpr bool STAGED = decltype(staged)::value;

@@ -162,6 +162,33 @@ def test_fc128_workgroups_at_once(gpu, b, k, n, name):
     fin.release()
 
 
+@pytest.mark.parametrize("b,k,n,name", [
+    (1, 100, 2000, "small_kernel<4>"), (16, 1537, 4096, "small_kernel<4>"),   # one wave and a part of a group; as many tiles as compute units
+    (17, 8193, 1000, "small_kernel<4>"), (77, 25001, 520, "small_kernel<8>"),  # half a tile without neurons, images past the batch
+    (128, 32768, 512, "small_kernel<8>"), (15, 26800, 513, "small_kernel<8>"),  # the longest slices, fifteen waves
+    (129, 4096, 512, "kernel<0, 7, false>"), (16, 32769, 512, "kernel<0, 0, true>")])  # a tile, a slice too many
+def test_fc128_small_tiles(gpu, b, k, n, name):
+    """Tiles of 16 x 16: ends of K, of the neurons and of the batch, half words, thresholds that are no numbers or met exactly."""
+    r = rng(b + k + n)
+    x = r.standard_normal((b, k)).astype(np.float32)
+    w = rm.pm1(r, (k, n))
+    bn = r.normal(0, np.sqrt(k), n).astype(np.float32)
+    bn[::7] = np.nan
+    bn[3::7] = ((np.where(x[0] >= 0, 1, -1) @ w.astype(np.int64)))[3::7]
+    want = orc.fc128(orc.in128(x), orc.pack_fc_weight(w), bn, k, n)
+    fin = gpu.In128LayerParam("Fin", b, k).initialize(x)
+    layer = gpu.Fc128LayerParam("Fc", b, k, n).initialize(gpu.ArrayWeights([w, bn]), fin.get_output_gpu())
+    assert layer.kernel_name() == "fc_mfma_f4_" + name, layer.kernel_name()
+    layer_out = layer.get_output_gpu()
+    layer_out.fill(0xAB)  # every half word and padding word is written
+    fin.forward()
+    layer.forward()
+    gpuops.sync()
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    layer.release()
+    fin.release()
+
+
 @pytest.mark.parametrize("b,widths,with_in,with_out,launches", [
     # one image and neuron; ends of words, tiles and groups of K; a wave's second tiles and second round of tiles; activations
     # of 2048 (two requests of weights ahead, 64 KB of LDS); outputs of several rounds of tiles
