@@ -51,17 +51,6 @@ constexpr int FW_NONE = 0, FW_LANES = 1, FW_TILES = 2;
 constexpr int kTapNone = 31;  // tap number of a word past K: its mask bit is always "invalid"
 constexpr int kMaxWords = 4096;
 
-// n / d for n < 2^31 by multiplication (Granlund and Montgomery's round-up method)
-struct FastDiv {
-    uint32_t mul, shift, d;
-};
-FastDiv fast_div(uint32_t d) {
-    uint32_t s = 0;
-    while ((1ull << s) < d) ++s;
-    return {(uint32_t)((((1ull << s) - d) << 32) / d + 1), s, d};
-}
-__device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv& f) { return (__umulhi(n, f.mul) + n) >> f.shift; }
-
 // Everything the kernel reads, and nothing else: it is fetched in one go at the start (see fetch_now).
 struct FlatArgs {
     const uint32_t* act;

@@ -234,6 +234,9 @@ void bgemm_flat_kernel_name(const BgemmParams& p, char* buf, size_t len);
 bool gemm_mfma_applicable(const BgemmParams& p);
 int launch_gemm_mfma(const BgemmParams& p, hipStream_t stream);
 void gemm_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len);
+bool conv1x1_mfma_applicable(const BgemmParams& p);
+int launch_conv1x1_mfma(const BgemmParams& p, hipStream_t stream);
+void conv1x1_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len);
 bool fc_mfma_applicable(const BgemmParams& p);
 int launch_fc_mfma(const BgemmParams& p, hipStream_t stream);
 void fc_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len);

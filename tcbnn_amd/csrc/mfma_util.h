@@ -110,6 +110,17 @@ __device__ __forceinline__ int class_sum(uint32_t x) {
     return 2 * (5 * __popc(x & 0x11111111u) + 3 * __popc(x & 0x22222222u) + __popc(x & 0x44444444u)) - 8 * (5 + 3 + 1);
 }
 
+// n / d for n < 2^31 by multiplication (Granlund and Montgomery's round-up method)
+struct FastDiv {
+    uint32_t mul, shift, d;
+};
+inline FastDiv fast_div(uint32_t d) {
+    uint32_t s = 0;
+    while ((1ull << s) < d) ++s;
+    return {(uint32_t)((((1ull << s) - d) << 32) / d + 1), s, d};
+}
+__device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv& f) { return (__umulhi(n, f.mul) + n) >> f.shift; }
+
 template <int FMT>
 struct Acc;
 template <>

@@ -504,6 +504,29 @@ def test_conv128_waves_of_a_workgroup(gpu, b, h, cin, cout, pool, image_tiles):
     layer.release()
 
 
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("b,h,cin,cout,stride,ahead_fc,served", [
+    (2, 1, 64, 64, 1, False, True), (6, 5, 128, 192, 2, False, True),      # a part of a tile; an odd number of channel groups
+    (70, 9, 256, 128, 2, True, True), (34, 8, 64, 320, 3, False, True),    # tiles across pixels, rows that no window reaches
+    (514, 8, 64, 128, 1, False, True), (258, 12, 256, 256, 1, False, True),  # more tiles than waves, by a few and many
+    (40, 6, 512, 64, 2, False, False), (40, 6, 128, 96, 2, False, False)])  # other forms: the kernel for all of them
+def test_conv128_1x1_saving_a_residual(gpu, b, h, cin, cout, stride, ahead_fc, served, fmt):
+    r = rng(b + h + cin + cout + stride)
+    x, f = rm.pm1(r, (b, h, h, cin)), rm.pm1(r, (1, 1, cin, cout))
+    inp, filt = orc.pack_conv_input_nhwc(x), orc.pack_conv_filter(f)
+    bn = r.normal(0, np.sqrt(cin), cout).astype(np.float32)
+    _, res = orc.conv128(inp, filt, bn, cin, cout, 1, 1, stride, True, 1, save_residual=True)
+    bn[:5] = res[0, 0, 0, :5]  # met exactly
+    bn[5:13] = [np.nan, np.inf, -np.inf, 3e38, -3e38, 0.0, -0.0, -0.5]
+    want, res = orc.conv128(inp, filt, bn, cin, cout, 1, 1, stride, True, 1, ahead_fc, save_residual=True)
+    layer = _run_conv_layer(gpu, "mfma_f4", x, f, bn, stride, 1, ahead_fc, True, out_fmt=fmt)
+    name = layer.kernel_name()
+    assert name == "conv1x1_mfma_f4_kernel<%d, %d>" % (cin // 64, fmt) if served else "flat" in name, name
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    np.testing.assert_array_equal(layer.download_residual(), res)
+    layer.release()
+
+
 # (cin, cout): the persistent 3x3 kernel's instantiations (Cin 64 .. 512), a channel count that is not a
 # multiple of 32 and an odd one (half-filled last 16-bit pair); formats of the injected and saved tensors
 RES_SHAPES = [(64, 96), (128, 64), (256, 35), (512, 64), (192, 64), (384, 40), (96, 35)]
