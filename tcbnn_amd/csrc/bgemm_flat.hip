@@ -29,6 +29,7 @@
 // the same issue slots).
 #include <algorithm>
 #include <initializer_list>
+#include <utility>
 
 #include "common.h"
 #include "mfma_util.h"
@@ -78,6 +79,19 @@ constexpr int ring_depth(int mt, int nt, int fm) { return mt * nt >= 8 ? 1 : (mt
 template <typename T>
 __device__ __forceinline__ void fetch_one(T v) {
     asm volatile("" ::"s"(v));
+}
+
+// Sixteen sums less their thresholds, the signs shifted in (MSB first).  Lane l of each row of 16 holds threshold l of its half: one
+// request for all of them, and a subtraction takes its threshold by DPP.  (Every lane of the wave is active here.)
+template <int V>
+__device__ __forceinline__ float row_lane(float t) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0x150 + V, 0xf, 0xf, true));  // row_newbcast:V
+}
+template <int... V>
+__device__ __forceinline__ uint32_t signs(const float (&sum)[16], float t, std::integer_sequence<int, V...>) {
+    uint32_t hw = 0;
+    ((hw = __builtin_amdgcn_alignbit(hw, __float_as_uint(sum[V] - row_lane<V>(t)), 31)), ...);
+    return hw;
 }
 
 template <int MT, int NT, int FM, int RF, int WIN>
@@ -170,15 +184,13 @@ bgemm_flat_f4_kernel(const FlatArgs p) {
 
     // ---- operands of the epilogue, requested ahead of K
     const bool fin = live && slice == 0;  // (uniform) this wave finishes the tile
-    float thr[NT][16];
+    float thr[NT];
     constexpr int NRAW = RF == TCBNN_RES_I12 ? 6 : (RF == TCBNN_RES_I16 ? 8 : 16);
     constexpr int NSRC = FM == FM_RESPOOL ? 4 : 1;
     int rraw[kRes ? MT * NT : 1][NSRC][NRAW];
     if (FM != FM_RAW && fin) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) thr[nt][v] = p.bn[min(n0 + nt * 32 + 16 * h + v, p.N - 1)];
+        for (int nt = 0; nt < NT; ++nt) thr[nt] = p.bn[min(n0 + nt * 32 + 16 * h + (lane & 15), p.N - 1)];
     }
     if constexpr (kRes) {
         if (fin && p.res_lim > 0) {
@@ -396,9 +408,7 @@ bgemm_flat_f4_kernel(const FlatArgs p) {
                 }
             }
             // bits, MSB first: the inverted sign of sum - threshold
-            uint32_t hw = 0;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) hw = __builtin_amdgcn_alignbit(hw, __float_as_uint(sum[v] - (thr[nt][v] == thr[nt][v] ? thr[nt][v] : never)), 31);
+            uint32_t hw = signs(sum, thr[nt] == thr[nt] ? thr[nt] : never, std::make_integer_sequence<int, 16>{});
             hw = ~hw & 0xffffu & (0xffff0000u >> min(max(p.N - cbase, 0), 16));
             if constexpr (kRes) {
                 if (p.res_out != nullptr) {
