@@ -1934,6 +1934,12 @@ def test_pool3x3_stride2(gpu, b, h, c, pad, fmt):
     test_pool128(gpu, b, h, c, 3, 2, pad, fmt)
 
 
+@pytest.mark.parametrize("b,h,c,fmt", [(70, 93, 64, 0), (130, 91, 64, 0)])
+def test_pool3x3_stride2_beyond_the_memory_side_cache(gpu, b, h, c, fmt):
+    """Launches whose XCDs share the rows: from the first (152 MiB of input) and from the last (271)."""
+    test_pool128(gpu, b, h, c, 3, 2, 1, fmt)
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2])
 @pytest.mark.parametrize("b,h,c,n", [(2, 7, 4, 3), (9, 8, 64, 129), (12, 5, 200, 128), (5, 2, 512, 1)])
 def test_avgpool_fc_tails(gpu, b, h, c, n, fmt):
