@@ -94,7 +94,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(res
         }
     }
     // One request for the thresholds of 64 channels, and through LDS (written and read by this wave only) to the lanes' sixteen
-    // of each channel tile: the address unit takes 17 cycles for a request, and 32 of them a wave were 3 us of a launch.
+    // of each channel tile: the address unit takes 17 cycles for a request (a channel at a time, 32 requests a wave: 11.3 us for 9.9,
+    // 8.7 for 7.4; weights by the word instead of the row's part: 8.9 for 6.2 at 256 channels).
     __shared__ __align__(16) float par[kWaves][32 * kNT];
     float* const mine = par[threadIdx.x >> 6];
     const float t = p.bn[n0 + lane];
