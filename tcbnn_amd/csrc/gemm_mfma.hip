@@ -349,6 +349,9 @@ bool gemm_mfma_applicable(const BgemmParams& p) {
     if (p.res_in != nullptr || p.res_out != nullptr) return false;
     if (p.mode != EPI_THRESH && p.mode != EPI_AFFINE && p.mode != EPI_RAW) return false;
     if (p.k_tap > 32 * p.cw || (p.cw % 4 != 0 && p.mode != EPI_RAW)) return false;
+    // The sums hold up to 13/4 of a count for each position of K, words past it included (1, 2, 4 and 6 on the four classes of
+    // expand_rows_f4), and fp32 is exact to 2^24: to K = 5.1 million.  A longer one goes to the kernels that multiply +-1.
+    if (13LL * 64 / 4 * ((p.cw + 2 * kAhead - 1) / (2 * kAhead) * kAhead) > (1LL << 24)) return false;
     // 32-bit buffer offsets: all rows' words, 64 columns' words
     if ((long long)p.cw * p.B * 4 >= (1LL << 31) || (long long)p.cw * 32 * kNT * 4 >= (1LL << 31)) return false;
     // Large enough to give every CU a workgroup with two image tiles per wave; smaller problems are bound by launch and fill and

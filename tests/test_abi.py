@@ -100,6 +100,31 @@ def test_large_products_test_for_odd_words_only_where_there_can_be_any():
     assert name.value == b"gemm_mfma_f4_kernel<2, 0, false>"
 
 
+def _fc_kernel(batch, k, n, out=False):
+    import ctypes as C
+    from tcbnn_amd import _lib
+    name = C.create_string_buffer(128)
+    if out:
+        d = _lib.Out128Desc(1, 1, 1, 1, 1, batch, k, n, _lib.VARIANT_MFMA_F4)
+        _lib.check(_lib.lib.tcbnn_out128_kernel_name(C.byref(d), name, 128))
+    else:
+        d = _lib.Fc128Desc(1, 1, 1, 1, batch, k, n, _lib.VARIANT_MFMA_F4, None, 0)
+        _lib.check(_lib.lib.tcbnn_fc128_kernel_name(C.byref(d), name, 128))
+    return name.value.decode()
+
+
+@pytest.mark.parametrize("out", [False, True])
+def test_large_products_only_where_their_sums_are_exact(out):
+    """The large-product kernel's rows are values of 0 .. 6 (13/4 on average where all signs agree), summed in fp32: taken
+    while that stays below 2^24, over K rounded up to groups of sixteen words."""
+    batch, n = 64, 16384  # 256 workgroups; 2 GiB of rows lie beyond the longest K
+    served = [k for k in range(128 * 39000, 1 << 24, 128) if _fc_kernel(batch, k, n, out).startswith("gemm_mfma")]
+    assert served, "the longest products that are exact stay with this kernel"
+    sums = 13 * (-(-max(served) // 512) * 512) // 4
+    assert (1 << 24) - 13 * 512 // 4 < sums <= 1 << 24, max(served)
+    assert "gemm_mfma" not in _fc_kernel(batch, (1 << 24) - 1, n, out)
+
+
 _B = 8192  # (a batch at which two layers are faster together)
 
 

@@ -54,6 +54,26 @@ def test_bmm_wide_requests(gpu, m, n, k):
     np.testing.assert_array_equal(gpuops.bmm(a, b, m, n, k, _variant(gpu, "mfma_f4")), orc.bmm(a, b, k))
 
 
+@pytest.mark.parametrize("k", [5161984, 5162016, 12000000])
+def test_bmm_longest_k(gpu, k):
+    """The last K that the large-product kernel takes (its sums reach 2^24), the next, and one at which its sums would lose
+    the last bit: ones all over but for up to 33 bits of a row, so that the sums are at their largest and every one differs."""
+    m, n = 1056, 1184  # 1221 tiles
+    first = np.full((2, m), 0xFFFFFFFF, np.uint32)
+    flips = np.arange(m) % 34  # leading bits of the row that are 0
+    first[0] = [(1 << 32) - 1 >> min(f, 32) for f in flips]
+    first[1] = [0x7FFFFFFF if f > 32 else 0xFFFFFFFF for f in flips]
+    a, b, c = (gpuops.DeviceBuffer(size) for size in (k // 8 * m, k // 8 * n, 4 * m * n))
+    a.fill(0xFF), b.fill(0xFF), c.fill(0xAB)
+    a.upload(first)
+    gpuops.check(gpuops.lib.tcbnn_bmm(a.ptr, b.ptr, c.ptr, m, n, k, _variant(gpu, "mfma_f4"), None))
+    gpuops.sync()
+    got = c.to_numpy(np.int32, (m, n))
+    for buf in (a, b, c):
+        buf.free()
+    np.testing.assert_array_equal(got, np.broadcast_to((k - 2 * flips)[:, None], (m, n)))
+
+
 # --------------------------------------------------------------------------- In / Fc / Out layers
 @pytest.mark.parametrize("b,k", [(8, 784), (100, 128), (8192, 784), (3, 1000)])
 def test_in128(gpu, b, k):
