@@ -346,6 +346,9 @@ int gemm_mt(const BgemmParams& p) {
 
 bool gemm_mfma_applicable(const BgemmParams& p) {
     if (p.PH * p.PW != 1 || p.R * p.S != 1 || p.pool_h * p.pool_w != 1) return false;
+    // the rows are the frame's first pixel: with a padding the one output pixel lies elsewhere in the frame (a stride beyond
+    // the frame makes it negative) or outside
+    if (p.pad_h != 0 || p.pad_w != 0) return false;
     if (p.res_in != nullptr || p.res_out != nullptr) return false;
     if (p.mode != EPI_THRESH && p.mode != EPI_AFFINE && p.mode != EPI_RAW) return false;
     if (p.k_tap > 32 * p.cw || (p.cw % 4 != 0 && p.mode != EPI_RAW)) return false;

@@ -125,6 +125,20 @@ def test_large_products_only_where_their_sums_are_exact(out):
     assert "gemm_mfma" not in _fc_kernel(batch, (1 << 24) - 1, n, out)
 
 
+@pytest.mark.parametrize("frame,stride,served", [(1, 1, True), (2, 2, True), (5, 8, False), (3, 7, False)])
+def test_large_products_read_the_first_pixel(frame, stride, served):
+    """One output pixel of a 1x1 filter is the frame's first one only without padding: ((5 + 8 - 5)/8 - 1)*8 + 1 - 5 = -4,
+    halved: the pixel at (2, 2) of a 5x5 frame."""
+    import ctypes as C
+    from tcbnn_amd import _lib
+    d = _lib.Conv128Desc(1, 1, 1, 1, None, None, frame, frame, 256, 1, 1, 1024, 8192, stride, stride, 1, 1, 1, 0, 0, 0, 0, 0, 0,
+                         _lib.VARIANT_MFMA_F4, 0, 0, 0)
+    name = C.create_string_buffer(128)
+    _lib.check(_lib.lib.tcbnn_conv128_kernel_name(C.byref(d), name, 128))
+    assert (_lib.lib.tcbnn_conv_pad(frame, 1, stride, 1) == 0) == served
+    assert name.value.decode().startswith("gemm_mfma") == served, name.value
+
+
 _B = 8192  # (a batch at which two layers are faster together)
 
 

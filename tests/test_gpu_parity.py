@@ -524,6 +524,30 @@ def test_conv128_waves_of_a_workgroup(gpu, b, h, cin, cout, pool, image_tiles):
     layer.release()
 
 
+@pytest.mark.parametrize("b,h,cin,cout,stride", [(4100, 5, 128, 1024, 8), (4100, 3, 128, 1024, 7), (4100, 2, 128, 1024, 2)])
+def test_conv128_1x1_of_one_output_pixel(gpu, b, h, cin, cout, stride):
+    """A stride beyond the frame: the one pixel is not the first; many images, so that the large-product kernel is near."""
+    r = rng(b + h)
+    x, f = rm.pm1(r, (b, h, h, cin)), rm.pm1(r, (1, 1, cin, cout))
+    bn = r.normal(0, np.sqrt(cin), cout).astype(np.float32)
+    want, _ = orc.conv128(orc.pack_conv_input_nhwc(x), orc.pack_conv_filter(f), bn, cin, cout, 1, 1, stride, True, 1)
+    layer = _run_conv_layer(gpu, "mfma_f4", x, f, bn, stride)
+    np.testing.assert_array_equal(layer.download_packed(), want)
+    layer.release()
+
+
+@pytest.mark.parametrize("pad,height", [(1, 1), (1, 5), (0, 3)])
+def test_bconv_of_one_padded_pixel(gpu, pad, height):
+    """The one output pixel lies in the padding: zeros; without a padding it is the frame's first."""
+    r = rng(pad + height)
+    b, cin, cout = 4100, 128, 1024
+    x, f = rm.pm1(r, (b, height, height, cin)), rm.pm1(r, (1, 1, cin, cout))
+    got = gpuops.bconv(gpuops.pack_conv_input(x), gpuops.pack_conv_filter(f), b, height, height, cin, cout, 1, 1, 1, pad, 1, 1,
+                       _variant(gpu, "mfma_f4"))
+    want = np.zeros((b, cout), np.int32) if pad else x[:, 0, 0].astype(np.int32) @ f[0, 0].astype(np.int32)
+    np.testing.assert_array_equal(got.reshape(b, cout), want)
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2])
 @pytest.mark.parametrize("b,h,cin,cout,stride,ahead_fc,served", [
     (2, 1, 64, 64, 1, False, True), (6, 5, 128, 192, 2, False, True),      # a part of a tile; an odd number of channel groups
