@@ -62,13 +62,18 @@ constexpr int RM_RAW = 3;     // no threshold: the +-1 dot products are stored a
 // waves per SIMD, each expanded activation fragment still feeds two MFMAs, the weights are staged once per CU
 // instead of twice, and which waves share a SIMD is known (waves w, w + 4, ...), which the numbering of the work
 // items uses (ResNet-18 at batch 256: L3B2C1 14.6 -> 13.2 us, L3B1C2 17.1 -> 16.1 us).
-// Twelve where a wave has one image tile and no 2x2 maximum to take: 168 registers hold that, and a third wave on
-// each SIMD covers what the other two wait for.  512 channels: 7 x 7, batch 256 16.3 / 15.8 -> 15.0 / 14.5 us,
-// 8 x 8, batch 77 12.1 -> 11.1, 28 x 28, batch 256 144.1 -> 140.2.
+// Twelve where a wave has one image tile and no 2x2 maximum to take and 168 registers hold it: a third wave on each SIMD
+// covers what the other two wait for.  512 channels: 7 x 7, batch 256 16.3 / 15.8 -> 15.0 / 14.5 us,
+// 8 x 8, batch 77 12.1 -> 11.1, 28 x 28, batch 256 144.1 -> 140.2.  Residual layers of partial channel tiles and, at 512
+// channels, with an int32 residual do not fit (up to 51 registers spilled: 512 -> 100 channels at 14 x 14, batch 256,
+// int32 / 16-bit / 12-bit residual 29.0 / 25.7 / 25.0 us for 20.6 / 19.0 / 18.8 with eight waves).
 constexpr int WIN_NONE = 0, WIN_ORPOOL = 1, WIN_MAXSAVE = 2;  // (see the kernel)
-constexpr int waves_of(int spt, int rm, int mt, int nt, int win) {
+constexpr bool fits_168_registers(int spt, int rm, int mt, int rf, bool fullt) {
+    return mt == 1 && (rm == RM_NONE || (rm == RM_PLAIN && fullt && (spt < 8 || rf != TCBNN_RES_I32)));
+}
+constexpr int waves_of(int spt, int rm, int mt, int nt, int rf, int win, bool fullt) {
     const bool alone = win != WIN_MAXSAVE && 9 * spt * nt * 1024 > (nt == 2 ? 64 : 80) * 1024;  // (WIN_MAXSAVE: a wave per pixel)
-    return alone ? (mt == 1 && (rm == RM_NONE || rm == RM_PLAIN) ? 12 : 8) : 4;
+    return alone ? (fits_168_registers(spt, rm, mt, rf, fullt) ? 12 : 8) : 4;
 }
 // WIN_MAXSAVE: where the four waves' sums of a window meet in LDS.  All channel tiles at once ([wave][NT][2][64]
 // 128-bit words) where that leaves room for two workgroups per CU next to the staged weights; else one channel tile
@@ -90,8 +95,8 @@ constexpr bool raw_transposed(int spt, int rm, int nt, bool fullt) {
 constexpr int kWavesPerSimd = 2;
 // ... except where a fourth wave per SIMD is two registers away (one register spilled): Cin = 64 layers that save
 // the window maximum
-constexpr int waves_per_simd(int spt, int rm, int mt, int nt, int win) {
-    return spt == 1 && rm == 1 && win == 2 ? 4 : (waves_of(spt, rm, mt, nt, win) == 12 ? 3 : kWavesPerSimd);
+constexpr int waves_per_simd(int spt, int rm, int mt, int nt, int rf, int win, bool fullt) {
+    return spt == 1 && rm == 1 && win == 2 ? 4 : (waves_of(spt, rm, mt, nt, rf, win, fullt) == 12 ? 3 : kWavesPerSimd);
 }
 
 // SPT = k-steps (64 bits) per filter tap = Cin / 64; MT = 32-image tiles per wave (2 for plain
@@ -109,7 +114,7 @@ constexpr int waves_per_simd(int spt, int rm, int mt, int nt, int win) {
 // tests of partial tiles are then not even compiled (they cost scalar registers and set-up instructions in
 // every launch, and the networks' channel counts are multiples of 64).
 template <int SPT, int RM, int MT, int NT, int RF, int WIN, bool FULLT>
-__global__ __launch_bounds__(64 * waves_of(SPT, RM, MT, NT, WIN)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(SPT, RM, MT, NT, WIN)))) void
+__global__ __launch_bounds__(64 * waves_of(SPT, RM, MT, NT, RF, WIN, FULLT)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(SPT, RM, MT, NT, RF, WIN, FULLT)))) void
 conv3x3_mfma_f4_kernel(
     const BgemmParams p, const uint32_t* __restrict__ act, const uint32_t* __restrict__ wgt,
     const float* __restrict__ bnp, const int32_t* __restrict__ rin, int32_t* __restrict__ rout, int res_lim,
@@ -120,13 +125,13 @@ conv3x3_mfma_f4_kernel(
     static_assert(RM == RM_NONE || !POOL, "residuals are defined for un-pooled layers only");
     static_assert(!PSAVE || (RM == RM_PLAIN && FULLT && (RF == TCBNN_RES_I16 || RF == TCBNN_RES_I12)),
                   "the window maximum is taken on 16-bit pairs in the epilogue of full tiles with a narrow injected residual");
-    static_assert(!PSAVE || (MT == 1 && waves_of(SPT, RM, MT, NT, WIN) == 4), "one wave per pixel of the window, one image tile each");
+    static_assert(!PSAVE || (MT == 1 && waves_of(SPT, RM, MT, NT, RF, WIN, FULLT) == 4), "one wave per pixel of the window, one image tile each");
     constexpr bool kTwoPhase = PSAVE && win_two_phase(SPT, NT);
     constexpr bool kStartMagic = kRes && FULLT && (RF == TCBNN_RES_I16 || RF == TCBNN_RES_I12);  // (see kMagic)
     constexpr int TPC = SPT >= 3 ? 3 : 9;  // taps per prefetch chunk (a filter row, or all of it)
     constexpr int NCH = 9 / TPC;           // chunks per tile
     constexpr int NQ = 9 * SPT;            // k-steps per tile
-    constexpr int kWaves = waves_of(SPT, RM, MT, NT, WIN);
+    constexpr int kWaves = waves_of(SPT, RM, MT, NT, RF, WIN, FULLT);
     // A tile of one chunk is shorter than the memory latency: its residual operand is then
     // requested a whole tile ahead (double-buffered); otherwise with the tile's first chunk.
     constexpr bool kAhead = kRes && NCH == 1;
@@ -1164,7 +1169,7 @@ TensorBytes tensor_bytes(const BgemmParams& p) {
 template <int SPT, int RM, int MT, int NT, int RF, int WIN, bool FULLT>
 int launch_f(const BgemmParams& p, hipStream_t stream) {
     constexpr int NQ = 9 * SPT;
-    constexpr int kWaves = waves_of(SPT, RM, MT, NT, WIN), kThreads = 64 * kWaves;
+    constexpr int kWaves = waves_of(SPT, RM, MT, NT, RF, WIN, FULLT), kThreads = 64 * kWaves;
     constexpr bool kRawTranspose = raw_transposed(SPT, RM, NT, FULLT);
     constexpr bool kWgItems = WIN == WIN_MAXSAVE;  // a work item (window) is taken by a whole workgroup
     const size_t lds_bytes = (size_t)NQ * NT * 64 * 16 + NT * 32 * sizeof(float) +
@@ -1211,7 +1216,7 @@ int launch_f(const BgemmParams& p, hipStream_t stream) {
     // 15.5 -> 14.8); pooled ones do not fit 168 registers (175 -> 186 us with that limit).
     constexpr bool kResLayer = RM == RM_PLAIN || RM == RM_POOLED;
     constexpr bool kPlainShort = RM == RM_NONE && SPT == 1 && WIN == WIN_NONE;
-    const int wg_want = wg_env > 0 ? wg_env : ((kResLayer && MT == 1) || kPlainShort ? (waves_per_simd(SPT, RM, MT, NT, WIN) == 4 ? 4 : 3) : 2);
+    const int wg_want = wg_env > 0 ? wg_env : ((kResLayer && MT == 1) || kPlainShort ? (waves_per_simd(SPT, RM, MT, NT, RF, WIN, FULLT) == 4 ? 4 : 3) : 2);
     const int wg_per_cu = std::max(1, std::min(wg_want, resident));
     const int best = std::max(1, std::min(cus * wg_per_cu / (n_groups * b_groups), quads));
     // channels that receive an injected residual: o < residual_channels, and only those the

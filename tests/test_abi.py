@@ -139,6 +139,38 @@ def test_large_products_read_the_first_pixel(frame, stride, served):
     assert name.value.decode().startswith("gemm_mfma") == served, name.value
 
 
+def _device_kernels():
+    """Name -> record of every kernel in the library, as its code objects describe them (their AMDGPU metadata notes)."""
+    import struct
+    msgpack = pytest.importorskip("msgpack")
+    blob = open(os.path.join(ROOT, "tcbnn_amd", "libtcbnn_hip.so"), "rb").read()
+    kernels, at = {}, blob.find(b"\x7fELF")
+    while at >= 0:
+        machine, = struct.unpack_from("<H", blob, at + 18)
+        if machine == 224:  # EM_AMDGPU
+            headers, = struct.unpack_from("<Q", blob, at + 32)
+            size, count = struct.unpack_from("<HH", blob, at + 54)
+            for i in range(count):
+                kind, _, offset, _, _, length = struct.unpack_from("<IIQQQQ", blob, at + headers + i * size)
+                note, end = at + offset, at + offset + length
+                while kind == 4 and note < end:  # PT_NOTE
+                    name, desc, which = struct.unpack_from("<III", blob, note)
+                    body = note + 12 + (name + 3) // 4 * 4
+                    if which == 32:  # NT_AMDGPU_METADATA
+                        for k in msgpack.unpackb(blob[body:body + desc])["amdhsa.kernels"]:
+                            kernels[k[".name"]] = k
+                    note = body + (desc + 3) // 4 * 4
+        at = blob.find(b"\x7fELF", at + 4)
+    return kernels
+
+
+def test_twelve_waves_of_the_3x3_kernel_do_not_spill():
+    """Twelve waves a workgroup leave a wave 168 registers: taken only by the instantiations that fit them."""
+    twelve = {name: k for name, k in _device_kernels().items() if "conv3x3_mfma" in name and k[".max_flat_workgroup_size"] == 768}
+    assert len(twelve) >= 10
+    assert not {name: k[".vgpr_spill_count"] for name, k in twelve.items() if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]}
+
+
 _B = 8192  # (a batch at which two layers are faster together)
 
 
