@@ -132,6 +132,12 @@ conv3x3_mfma_f4_kernel(
     constexpr int NCH = 9 / TPC;           // chunks per tile
     constexpr int NQ = 9 * SPT;            // k-steps per tile
     constexpr int kWaves = waves_of(SPT, RM, MT, NT, RF, WIN, FULLT);
+    // The next chunk's words are asked for between the present one's products (compute_chunk_as): everywhere with one chunk a
+    // tile; with three in plain layers (256 channels, 56 x 56, batch 256 153.7 -> 147.0 us) and with twelve waves.  Elsewhere
+    // the wave's registers or its few neighbours cost more than the burst: geometric means of 17 .. 28 shapes, in a burst ->
+    // between, pooled residual 192 / 256 / 384 / 512 channels in 12 bits +2.5 / 2.3 / 2.3 / 2.1 %, window maximum of 192 / 384
+    // / 512 +2.8 / 1.5 / 0.4 %, 192 channels with a 16-bit / 12-bit residual +0.8 / 1.3 %, int32 output +-1 %.
+    constexpr bool kThreeBetween = NCH > 1 && (RM == RM_NONE || kWaves == 12), kBetween = NCH == 1 || kThreeBetween;
     // A tile of one chunk is shorter than the memory latency: its residual operand is then
     // requested a whole tile ahead (double-buffered); otherwise with the tile's first chunk.
     constexpr bool kAhead = kRes && NCH == 1;
@@ -304,10 +310,10 @@ conv3x3_mfma_f4_kernel(
     };
 
     v16f acc[MT][NT];
-    // Where a tile starts from: with one chunk per tile the first MFMAs take it as their operand C, in registers; with three
-    // the accumulators are set from the staged thresholds (or to a constant) at the tile's start, one instruction in 70 of its
-    // time, and its 32 registers go to the operands in flight.
-    constexpr bool kStartInLds = NCH > 1;
+    // Where a tile starts from: the first MFMAs take it as their operand C, in registers; where three chunks' requests go
+    // between the products the accumulators are set from the staged thresholds (or to a constant) at the tile's start, one
+    // instruction in 70 of its time, and its 32 registers go to the operands in flight.
+    constexpr bool kStartInLds = kThreeBetween;
     auto start_value = [&](int nt, int v) __attribute__((always_inline)) {
         return RM == RM_NONE ? lds_thr[nt * 32 + 16 * h + v] : (kStartMagic ? __uint_as_float(0x4B400000u) : 0.0f);
     };
@@ -412,10 +418,16 @@ conv3x3_mfma_f4_kernel(
             else
                 compute_chunk_as(std::false_type{}, std::false_type{}, chunk, buf, mask, nbuf, nsoff);
         } else {
-            if (fused)  // uniform; the chunk is a whole tile
-                compute_chunk_as(std::true_type{}, std::true_type{}, chunk, buf, mask, nbuf, nsoff);
-            else
+            if constexpr (kBetween) {
+                if (fused) {  // uniform; the chunk is a whole tile
+                    compute_chunk_as(std::true_type{}, std::true_type{}, chunk, buf, mask, nbuf, nsoff);
+                    return;
+                }
+            }
+            if (NCH == 1 || chunk == 0)  // uniform: the tile starts here
                 compute_chunk_as(std::true_type{}, std::false_type{}, chunk, buf, mask, nbuf, nsoff);
+            else
+                compute_chunk_as(std::false_type{}, std::false_type{}, chunk, buf, mask, nbuf, nsoff);
         }
     };
 
@@ -1080,7 +1092,7 @@ conv3x3_mfma_f4_kernel(
         unsigned nsoff = 0;
         const bool ahead = lc.pi < npix;  // (uniform) there is a chunk LOOK steps ahead
         if (ahead) {
-            if (msk[I] == kAllTaps && chunk_interior(pix_y(lc), pix_x(lc), lc.chunk, nsoff)) {
+            if (kBetween && msk[I] == kAllTaps && chunk_interior(pix_y(lc), pix_x(lc), lc.chunk, nsoff)) {
                 fused = true;
                 msk[J] = kAllTaps;
             } else {

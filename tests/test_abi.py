@@ -171,6 +171,13 @@ def test_twelve_waves_of_the_3x3_kernel_do_not_spill():
     assert not {name: k[".vgpr_spill_count"] for name, k in twelve.items() if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]}
 
 
+def test_long_3x3_tiles_keep_their_operands_in_registers():
+    """192 channels and more (three chunks a tile): requests between the products must not push operands out of registers."""
+    spills = {name: k[".vgpr_spill_count"] for name, k in _device_kernels().items()
+              if re.search(r"conv3x3_mfma_f4_kernelILi[3468]E", name) and k[".vgpr_spill_count"] > 1}
+    assert not spills
+
+
 _B = 8192  # (a batch at which two layers are faster together)
 
 
