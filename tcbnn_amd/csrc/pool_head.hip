@@ -111,33 +111,47 @@ __device__ __forceinline__ void i12_from_pairs(const uint32_t* q, uint32_t& w0, 
     i12_pack8(v, w0, w1, w2);
 }
 
-// A thread takes one unit (word of bits, or residual group) of one image and two output pixels of a column: of the three input
+// A thread takes one unit (word of bits, or residual group) of one image and a few output pixels of a column: of the three input
 // rows of a window the last is the next window's first.  A pixel's address is scalar and a lane's place in it 32 bits.
-// Neighbouring windows share a column and pairs of outputs a row, so workgroups are dealt in runs of neighbours to an XCD, whose L2
-// then has what the windows share: asked for by several XCDs it came from memory again.  With that, two outputs a thread are as
-// good as any number or better at every size (many rows a thread: fewer, longer chains).  What a run is:
-//   ROWS          whole rows of outputs: an XCD reads what no other one does;
+// Neighbouring windows share a column and runs of outputs a row, and an XCD's L2 has what they share where the XCD takes them all:
+// asked for by several XCDs it came from memory again.  Workgroups are dealt
+//   TURN          in turn, an output pixel's units first, as many rows a thread as leave every SIMD eight waves (8 at most).  With a
+//                 multiple of eight workgroups a pixel an XCD has the same units of every pixel, all that they share with it: us, dealt
+//                 as below -> in turn, 256 channels at 27x27, batch 256, 16-bit 23.4 -> 20.4, 56x56 in 32 bits 215 -> 205.  Few
+//                 outputs (under four waves a SIMD), whose input the caches have: 32 channels in 12 bits at 56x56, batch 8 5.9 -> 3.9.
+//                 Bits alone, a word a thread, to which the division of the shares and a short walk cost more than they save: 64
+//                 channels at 112x112, batch 256 10.6 -> 8.2;
+//   ROWS          the others in runs of neighbours to an XCD, two rows a thread (more: fewer, longer chains): whole rows of outputs,
+//                 an XCD reads what no other one does;
 //   COLUMNS       a part of each row, all XCDs at the same row: better where the launch's bytes are more than the memory-side cache has
 //                 room for beside its producer's (us in the textbook wiring's pass, batch 64 / 90 / 110 / 128 / 200 / 256: 17.7 / 28.4 / 39.1 /
 //                 45.6 / 74.1 / 99.0 in ROWS, 19.7 / 29.7 / 37.9 / 42.3 / 69.7 / 94.0 in COLUMNS);
 //   COLUMNS_BACK  the same, last rows first, where the input alone is more than that cache (256 MiB): what was written last is still
 //                 in it (batch 256 91.3; 200, whose input fits, 70.7).
-// In the pass, with eight rows a thread and workgroups dealt in turn -> here: batch 32 14.8 -> 10.2, 64 26.3 -> 17.7, 128 49.4 -> 42.3, 256
+// (The lines between the last three are from that pass: 64 channels, 12 bits, a producer that goes down the rows.)
+// In the pass, with eight rows a thread and all dealt in turn -> here: batch 32 14.8 -> 10.2, 64 26.3 -> 17.7, 128 49.4 -> 42.3, 256
 // 97.8 -> 91.3 (417 MB, while the producer's last stores are on their way: on its own 79, 5.3 TB/s).  What binds it: memory.
 // (Asking for the next output's words while one is reduced: 3 % slower below batch 256, 4 % faster there.)
-constexpr int kPoolRows = 2;
-enum PoolOrder : int { ROWS = 0, COLUMNS = 1, COLUMNS_BACK = 2 };
+enum PoolOrder : int { ROWS = 0, COLUMNS = 1, COLUMNS_BACK = 2, TURN = 3 };
+constexpr int kPoolRows = 2;             // output rows a thread takes in the orders but TURN
+constexpr long long kPoolFew = 1 << 18;  // outputs' units: four waves for each of 1024 SIMDs
 template <int FMT>
-__global__ __launch_bounds__(kThreads) void pool3x3s2_kernel(const PoolParams p, int units, int per_xcd, PoolOrder order) {
+__global__ __launch_bounds__(kThreads) void pool3x3s2_kernel(const PoolParams p, int units, int per_xcd, PoolOrder order, int rows) {
     auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
-    // workgroup i of an XCD's share of turn z (a row of the grid's last dimension); units, then columns, then pairs of rows
-    const int xcd = (int)blockIdx.x & 7, i = (int)(blockIdx.x >> 3) + (int)(gridDim.x >> 3) * (int)blockIdx.y, z = (int)blockIdx.z;
-    if (i >= per_xcd) return;
-    const int pairs = (int)gridDim.z, share = (order == ROWS ? xcd * pairs + z : xcd) * per_xcd + i;
-    const int col = uniform(share / units), bx = share - col * units, row = order == ROWS ? uniform(col / p.OW) : 0, ox = col - row * p.OW;
-    const int pair = order == ROWS ? row : (order == COLUMNS ? z : pairs - 1 - z);
-    if (ox >= p.OW || pair >= pairs) return;  // (shares are rounded up)
-    const int oy0 = pair * kPoolRows, oy1 = min(p.OH, oy0 + kPoolRows);
+    int bx, ox, pair;  // workgroup of a pixel, column, run of rows
+    if (order == TURN) {
+        bx = (int)blockIdx.x, ox = (int)blockIdx.y, pair = (int)blockIdx.z;
+    } else {
+        // workgroup i of an XCD's share of turn z (a row of the grid's last dimension); units, then columns, then pairs of rows
+        const int xcd = (int)blockIdx.x & 7, i = (int)(blockIdx.x >> 3) + (int)(gridDim.x >> 3) * (int)blockIdx.y, z = (int)blockIdx.z;
+        if (i >= per_xcd) return;
+        const int pairs = (int)gridDim.z, share = (order == ROWS ? xcd * pairs + z : xcd) * per_xcd + i;
+        const int col = uniform(share / units), row = order == ROWS ? uniform(col / p.OW) : 0;
+        bx = share - col * units, ox = col - row * p.OW;
+        pair = order == ROWS ? row : (order == COLUMNS ? z : pairs - 1 - z);
+        if (ox >= p.OW || pair >= pairs) return;  // (shares are rounded up)
+    }
+    const int oy0 = pair * rows, oy1 = min(p.OH, oy0 + rows);
     const unsigned rem = (unsigned)bx * kThreads + threadIdx.x;
     if (rem >= (unsigned)((p.cw + p.groups) * p.B)) return;
     const unsigned u = rem / (unsigned)p.B, b = rem - u * (unsigned)p.B;
@@ -430,16 +444,21 @@ extern "C" int tcbnn_pool128_forward(const tcbnn_pool128_desc* d, void* stream) 
     TCBNN_REQUIRE(blocks <= 0x7fffffffLL, "pool128: grid too large");
     const long long per_pixel = (long long)(p.cw + p.groups) * p.B;
     const long long units = (per_pixel + kThreads - 1) / kThreads;
-    const int pairs = (p.OH + kPoolRows - 1) / kPoolRows;
+    const bool in_turn = p.groups == 0 || units % 8 == 0 || total < kPoolFew;
+    const int rows = in_turn ? (int)std::min(8LL, std::max(1LL, total / (8192LL * 64))) : kPoolRows;
+    const int runs = (p.OH + rows - 1) / rows;
     // (32 bits hold a lane's bytes within a pixel and a workgroup's number, rounded up)
-    if (p.window == 3 && p.stride == 2 && pairs <= 65535 && per_pixel * 24 < (1LL << 32) - 24 * kThreads &&
-        (units * p.OW + 8) * pairs < (1LL << 31)) {
+    if (p.window == 3 && p.stride == 2 && runs <= 65535 && (!in_turn || p.OW <= 65535) && per_pixel * 24 < (1LL << 32) - 24 * kThreads &&
+        (units * p.OW + 8) * runs < (1LL << 31)) {
         const long long pixel = 4LL * p.cw * p.B + (p.fmt == TCBNN_RES_I12 ? 24LL : 16LL) * p.groups * p.B;
         const long long in_bytes = pixel * p.H * p.W, bytes = in_bytes + pixel * p.OH * p.OW;
-        const PoolOrder order = bytes < 165LL << 20 ? ROWS : (in_bytes <= 256LL << 20 ? COLUMNS : COLUMNS_BACK);
+        const PoolOrder order = in_turn ? TURN : (bytes < 165LL << 20 ? ROWS : (in_bytes <= 256LL << 20 ? COLUMNS : COLUMNS_BACK));
         const int per_xcd = (int)((units * p.OW + 7) / 8), across = std::min(per_xcd, 1 << 18);
-        const dim3 grid((unsigned)across * 8, (unsigned)((per_xcd + across - 1) / across), (unsigned)pairs);
-        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, p, (int)units, per_xcd, order); };
+        const dim3 grid = in_turn ? dim3((unsigned)units, (unsigned)p.OW, (unsigned)runs)
+                                  : dim3((unsigned)across * 8, (unsigned)((per_xcd + across - 1) / across), (unsigned)runs);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, p, (int)units, per_xcd, order, rows);
+        };
         if (p.fmt == TCBNN_RES_I12)
             launch(pool3x3s2_kernel<TCBNN_RES_I12>);
         else if (p.fmt == TCBNN_RES_I16)

@@ -1978,6 +1978,34 @@ def test_pool3x3_stride2(gpu, b, h, c, pad, fmt):
     test_pool128(gpu, b, h, c, 3, 2, pad, fmt)
 
 
+@pytest.mark.parametrize("b,h,c,pad,fmt", [
+    # in shares of rows to an XCD: odd frames, partly filled last workgroups
+    (150, 37, 64, 1, 0), (150, 37, 64, 1, 1), (150, 37, 64, 1, 2), (300, 29, 33, 2, 0), (300, 29, 33, 2, 1), (300, 29, 33, 2, 2),
+    # eight workgroups a pixel, in turn: two and three rows a thread, the last run short
+    (200, 57, 32, 0, 0), (64, 57, 200, 0, 1), (100, 57, 200, 0, 2)])
+def test_pool3x3_stride2_orders(gpu, b, h, c, pad, fmt):
+    test_pool128(gpu, b, h, c, 3, 2, pad, fmt)
+
+
+@pytest.mark.parametrize("b,h,c,pad", [(5, 9, 100, 1), (256, 61, 200, 1), (128, 61, 512, 2), (9, 224, 64, 0)])
+def test_pool3x3_stride2_of_bits(gpu, b, h, c, pad):
+    """No residual: up to eight rows a thread."""
+    from tcbnn_amd import layers
+    words = (c + 31) // 32
+    inp = rng(b + h + c).integers(0, 2 ** 32, size=(h, h, b, words), dtype=np.uint64).astype(np.uint32)
+    want, _ = orc.pool128(inp, c, 3, 2, pad)
+    layer = layers.Pool128LayerParam("p", h, h, c, b, 3, 2, pad)
+    src = gpuops.dev(np.ascontiguousarray(inp.transpose(0, 1, 3, 2)))
+    layer.initialize(src)
+    layer.output_gpu.fill(0xCD)
+    layer.forward()
+    gpuops.sync()
+    oh = layer.output_height
+    got = layer.output_gpu.to_numpy(np.uint32, (oh, oh, words, b)).transpose(0, 1, 3, 2)
+    np.testing.assert_array_equal(got, want)
+    layer.release()
+
+
 @pytest.mark.parametrize("b,h,c,fmt", [(70, 93, 64, 0), (130, 91, 64, 0)])
 def test_pool3x3_stride2_beyond_the_memory_side_cache(gpu, b, h, c, fmt):
     """Launches whose XCDs share the rows: from the first (152 MiB of input) and from the last (271)."""
