@@ -101,6 +101,10 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(res
     const float t = p.bn[n0 + lane];
     // s < t is s < ceil(t) for a whole number s
     mine[lane] = kMagic + (t == t ? fminf(fmaxf(ceilf(t), -kThrLimit), kThrLimit) : (p.nan_bit ? -kThrLimit : kThrLimit));
+    // (what other lanes wrote is read below: the order within the wave is said, not left to what the compiler cannot prove)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     v4i w[KS][kNT];
 #pragma unroll
     for (int nt = 0; nt < kNT; ++nt) {
