@@ -9,17 +9,18 @@
 // K loop of one tile (9 taps x Cin = 576..4608 bits: 36..288 MFMAs):
 //   - persistent workgroups: the FP4 weight fragments of a channel group (18..72 KiB, expanded from the
 //     filter's words in fragment order) and its thresholds are staged in LDS ONCE, then every wave walks a
-//     strided list of (pixel, 64-image) tiles; no barrier after the staging;
+//     strided list of (pixel, image tile) items; no barrier after the staging;
 //   - whole-chunk register prefetch: all activation words a wave needs for the next chunk of
 //     taps (the whole tile for Cin <= 128, one filter row above) are requested while the current
-//     chunk is multiplied, across tile boundaries; for Cin <= 128 the requests are issued two per
-//     k-step between the MFMAs of an interior tile (issued in one burst they hold the wave back);
+//     chunk is multiplied, across tile boundaries, two per k-step between the MFMAs of an interior tile
+//     where that gains (kBetween: for Cin <= 128 everywhere, for more in plain layers and with twelve
+//     waves; issued in one burst they hold the wave back);
 //   - wave-uniform border handling: a tap outside the frame is a cleared bit in a scalar mask
 //     (its loads and MFMAs are skipped), which is exactly the reference's "exclude" rule; pixel
 //     columns are skewed by the row so that every wave gets its share of the slower border tiles;
 //   - threshold folded into the accumulator: without a residual the accumulator starts from the
-//     negated integer threshold (operand C of the tile's first MFMA, always the centre tap), so the
-//     output bit is the sign of the finished accumulator;
+//     negated integer threshold (kStartInLds says how it gets there), so the output bit is the sign of
+//     the finished accumulator;
 //   - epilogue straight from the accumulator: one funnel shift per channel into a 16-channel half
 //     word, one lane swap, 128-byte stores of the batch-innermost layouts; residual add / save as
 //     contiguous 16-byte runs per lane.
@@ -206,15 +207,16 @@ conv3x3_mfma_f4_kernel(
 
     // start values of a lane's 16 channels per channel tile (zeros when a residual is added first); filled once
     // the thresholds are staged
-    v16f acc0[NT];  // (layers of one chunk per tile)
+    v16f acc0[NT];  // (not used with kStartInLds)
 
     // a wave's work items: output pixels, or 2x2 windows of them (row width `roww`)
     const int roww = kWin ? p.PW / 2 : p.PW;
     const int npix = kWin ? (p.PH / 2) * (p.PW / 2) : p.PH * p.PW;
     // First item of the wave (its later ones follow at stride dpi).  The items of the last, incomplete round go to
-    // the waves with the lowest first item.  An eight-wave workgroup has a CU to itself, two waves per SIMD: its
-    // waves 0-3 (one per SIMD) are numbered before the waves 4-7 of ANY workgroup, so that the left-over items fall
-    // one to a SIMD over all CUs instead of two to a SIMD in the first CUs and none in the others.
+    // the waves with the lowest first item.  A workgroup of eight or twelve waves has a CU to itself, two or three waves
+    // per SIMD: its waves 0-3 (one per SIMD) are numbered before the waves 4-7 of ANY workgroup, and these before the
+    // waves 8-11, so that the left-over items fall one to a SIMD over all CUs instead of two or three to a SIMD in the
+    // first CUs and none in the others.
     int pi = PSAVE ? stream  // (a window is taken by the whole workgroup)
                    : (kWaves >= 8 ? (wave >> 2) * (pix_streams * 4) + stream * 4 + (wave & 3) : stream * kWaves + wave);
     const int dpi = PSAVE ? pix_streams : pix_streams * kWaves;
@@ -253,10 +255,10 @@ conv3x3_mfma_f4_kernel(
         voff_bits[mt] = h == 0 && bimg[mt] < p.B ? (unsigned)bimg[mt] * 4u : kOutOfRange;
     }
 
-    // The tile's first MFMA must belong to a tap that is never outside the frame (it brings in the
-    // accumulator's start value): the centre tap.  Chunks of one filter row therefore come in the
-    // order middle, top, bottom, and the taps of a chunk start with its middle one; the sums are
-    // exact integers, so the order does not change them.
+    // Where the tile's first MFMA brings in the accumulator's start value (not with kStartInLds) it must belong
+    // to a tap that is never outside the frame: the centre tap.  Chunks of one filter row therefore come in
+    // the order middle, top, bottom, and the taps of a chunk start with its middle one; the sums are exact
+    // integers, so the order does not change them.
     auto chunk_row = [](int chunk) __attribute__((always_inline)) { return chunk == 0 ? 1 : (chunk == 1 ? 0 : 2); };
     // Requests the activation words of chunk `chunk` of the tile at pixel (yy, xx); returns the
     // wave-uniform mask of its in-frame taps.
@@ -358,9 +360,9 @@ conv3x3_mfma_f4_kernel(
     auto tap_of = [](int i) __attribute__((always_inline)) {
         return TPC == 9 ? (i == 0 ? 4 : (i <= 4 ? i - 1 : i)) : (i == 0 ? 1 : (i == 1 ? 0 : 2));
     };
-    // For Cin <= 128, interior pixels (every tap of the chunk in the frame: the bulk of a layer) run one
-    // straight-line block with the weight fragments of step i+1 read from LDS before step i is
-    // multiplied; border pixels test each tap and read ahead inside a tap only.
+    // Interior chunks (every tap in the frame: the bulk of a layer) run one straight-line block with the weight
+    // fragments of step i+1 read from LDS before step i is multiplied, for Cin <= 128 and wherever LOADS;
+    // others test each tap and read ahead inside a tap only.
     // LOADS: the words of the next chunk (interior as well) are requested two per step, in the shadow of
     // the MFMAs, instead of in one burst before the chunk.
     auto compute_chunk_as = [&](auto first_tag, auto loads_tag, int chunk, uint32_t (*buf)[MT], uint32_t mask,
@@ -1060,9 +1062,9 @@ conv3x3_mfma_f4_kernel(
     // the epilogue can take the bit from the sign of x - threshold.
     // Without a residual the sum s is an integer with |s| <= 9 Cin <= 4608, so s < threshold is
     // the same as s < ceil(threshold), and thresholds beyond +-8192 decide like +-8192.  The
-    // negated integer threshold is then what the accumulator STARTS from (operand C of the tile's
-    // first MFMA): the finished accumulator is s - ceil(threshold), exact in fp32, and its sign is
-    // the inverted output bit, with no per-value subtraction in the epilogue.
+    // negated integer threshold is then what the accumulator STARTS from (acc0, or start_tile): the
+    // finished accumulator is s - ceil(threshold), exact in fp32, and its sign is the inverted output
+    // bit, with no per-value subtraction in the epilogue.
     if (tid < NT * 32) {
         float t = thr_stage;
         t = t != t ? -__builtin_huge_valf() : t;
@@ -1086,8 +1088,8 @@ conv3x3_mfma_f4_kernel(
     auto step = [&](auto slot) __attribute__((always_inline)) {
         constexpr int I = decltype(slot)::value;
         constexpr int J = (I + LOOK) % NB;
-        // Both this chunk and the next one interior (Cin <= 128): the next one's loads ride along with
-        // this one's MFMAs.
+        // Both this chunk and the next one interior (with kBetween): the next one's loads ride along with this
+        // one's MFMAs.
         bool fused = false;
         unsigned nsoff = 0;
         const bool ahead = lc.pi < npix;  // (uniform) there is a chunk LOOK steps ahead
@@ -1210,7 +1212,7 @@ int launch_f(const BgemmParams& p, hipStream_t stream) {
     const int b_groups = (p.B + 32 * MT - 1) / (32 * MT);
     const int items = WIN != WIN_NONE ? (p.PH / 2) * (p.PW / 2) : p.PH * p.PW;  // pixels, or 2x2 windows of them
     // streams worth launching: one per item for workgroup-wide items; else one per kWaves items, or per 4 for
-    // eight-wave workgroups, whose waves 0-3 (one per SIMD) are served first (see the kernel's first item)
+    // workgroups of eight and twelve waves, whose waves 0-3 (one per SIMD) are served first (see the kernel's first item)
     constexpr int kServedFirst = kWaves >= 8 ? 4 : kWaves;
     const int quads = kWgItems ? items : (items + kServedFirst - 1) / kServedFirst;
     // Persistent workgroups, all resident at once: two per CU (three for residual layers), fewer
@@ -1265,10 +1267,10 @@ int launch_t(const BgemmParams& p, hipStream_t stream) {
 
 // Which instantiation serves a layer.  Measured on ResNet-18 and VGG-16 at batch 256 (10 launches back to back):
 // two channel tiles per wave (each expanded activation fragment feeds two MFMAs) everywhere except on layers of
-// Cin >= 384 that inject the 2 x 2 maximum of a larger tensor (the eight-wave workgroup below was 8 % slower
+// Cin >= 384 that inject the 2 x 2 maximum of a larger tensor (an eight-wave workgroup was 8 % slower
 // there: four times the residual operands per tile) and on the int32-output kernel for Cin = 192..384 (its LDS
 // staging area); from Cin = 384 on the weights of two channel tiles leave room for one workgroup per CU only, which
-// then has eight waves (waves_of).  Two image tiles per wave (each weight fragment read from LDS feeds two MFMAs)
+// then has eight or twelve waves (waves_of).  Two image tiles per wave (each weight fragment read from LDS feeds two MFMAs)
 // on the plain and int32-output layers up to Cin = 256; one on residual layers (their operands fill the registers)
 // and from Cin = 384 on (the activation ring of two image tiles no longer fits next to two channel tiles'
 // accumulators).
@@ -1365,7 +1367,7 @@ bool conv3x3_mfma_applicable(const BgemmParams& p) {
     const bool pool_ok = (p.pool_h == 1 && p.pool_w == 1) ||
                          (p.pool_h == 2 && p.pool_w == 2 && p.PH % 2 == 0 && p.PW % 2 == 0 && p.res_in == nullptr &&
                           p.res_out == nullptr);
-    // the centre tap of every output pixel lies inside the frame (the kernel starts each tile with it)
+    // the centre tap of every output pixel lies inside the frame (the kernel starts tiles with it)
     const bool centre_ok = p.pad_h <= 1 && p.pad_w <= 1 && (p.PH - 1) * p.stride_h - p.pad_h + 1 < p.H &&
                            (p.PW - 1) * p.stride_w - p.pad_w + 1 < p.W;
     // threshold epilogue, or the int32 dot products of an un-pooled convolution without residuals

@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
     __syncthreads();
 
     // Software pipeline, one k-step deep: while step q is multiplied, the weight fragments of step q + 1 are on
-    // their way from LDS and its row words are expanded (their ring slot is then asked for step q + 5).  Step q's
+    // their way from LDS and its row words are expanded (their ring slot is then asked for step q + 9).  Step q's
     // words sit in ring slot q % kAhead; kBlk is a multiple of kAhead, so the slot of step ql + d of a block is d.
     v4i anext[kNT], bnext[MT];
 #pragma unroll

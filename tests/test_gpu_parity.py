@@ -43,8 +43,8 @@ def test_bmm(gpu, variant, m, n, k):
 @pytest.mark.parametrize("m,n,k", [
     # few rows or columns and a long K: both sides of the line between the kernels for small and for large products
     (300, 4096, 4128), (257, 4128, 2624), (1220, 1056, 2624), (1184, 1024, 4096),
-    # two and four image tiles per wave: rows past the last one, a last column group of 32, rows of the weights that are
-    # no whole 128-bit units (1 to 3 words more), K that ends with a block, after one group of k-steps, within one
+    # two and (the fourth and the last) four image tiles per wave: rows past the last one, a last column group of 32, rows of the
+    # weights that are no whole 128-bit units (1 to 3 words more), K that ends with a block, after one group of k-steps, within one
     (3070, 2112, 1024), (3070, 2080, 1088), (2049, 3104, 544), (4095, 4064, 2080), (4097, 4096, 2528), (5000, 3104, 2112),
 ])
 def test_bmm_wide_requests(gpu, m, n, k):
@@ -52,6 +52,41 @@ def test_bmm_wide_requests(gpu, m, n, k):
     a = r.integers(0, 2 ** 32, size=(m, k // 32), dtype=np.uint64).astype(np.uint32)
     b = r.integers(0, 2 ** 32, size=(n, k // 32), dtype=np.uint64).astype(np.uint32)
     np.testing.assert_array_equal(gpuops.bmm(a, b, m, n, k, _variant(gpu, "mfma_f4")), orc.bmm(a, b, k))
+
+
+def _large_product_kernel(gpu, b, k, n, out=False):
+    """The FP4 engine's kernel for a fully connected layer of these sizes; a stand-alone product of the same sizes has as
+    many image tiles to a wave."""
+    import ctypes as C
+    name = C.create_string_buffer(128)
+    if out:
+        d = gpuops._lib.Out128Desc(1, 1, 1, 1, 1, b, k, n, _variant(gpu, "mfma_f4"))
+        gpuops.check(gpuops.lib.tcbnn_out128_kernel_name(C.byref(d), name, 128))
+    else:
+        d = gpuops._lib.Fc128Desc(1, 1, 1, 1, b, k, n, _variant(gpu, "mfma_f4"), None, 0)
+        gpuops.check(gpuops.lib.tcbnn_fc128_kernel_name(C.byref(d), name, 128))
+    return name.value.decode()
+
+
+@pytest.mark.parametrize("m,n,k", [
+    # rows past the last one, a last column group of 32 and none; K that ends with a whole block of sixteen k-steps, with half a one,
+    # within a group of eight, and with a row that is no whole 128-bit unit
+    (5000, 3104, 2048), (8192, 4096, 2048), (4999, 3104, 2304), (5000, 3104, 2176), (4999, 3104, 2592)])
+def test_bmm_four_image_tiles(gpu, m, n, k):
+    assert _large_product_kernel(gpu, m, k, n).startswith("gemm_mfma_f4_kernel<4,")
+    test_bmm_wide_requests(gpu, m, n, k)
+
+
+@pytest.mark.parametrize("b,k,n", [(5000, 2048, 3104), (4999, 2300, 3100)])
+def test_fc128_four_image_tiles(gpu, b, k, n):
+    assert _large_product_kernel(gpu, b, k, n) == "gemm_mfma_f4_kernel<4, 0, false>"
+    test_fc128(gpu, "mfma_f4", b, k, n)
+
+
+@pytest.mark.parametrize("b,k,n", [(5000, 2048, 3104), (4999, 2300, 3100)])
+def test_out128_four_image_tiles(gpu, b, k, n):
+    assert _large_product_kernel(gpu, b, k, n, out=True) == "gemm_mfma_f4_kernel<4, 1, false>"
+    test_out128(gpu, "mfma_f4", b, k, n)
 
 
 @pytest.mark.parametrize("k", [5161984, 5162016, 12000000])
