@@ -314,7 +314,8 @@ bool fc_mfma_applicable(const BgemmParams& p) {
 }
 
 namespace {
-constexpr int kCus = 256, kCuWaves = 16;  // compute units, and waves of these kernels that one holds (120 registers)
+constexpr int kCus = 256;       // compute units
+constexpr int kSimdWaves = 4;   // waves of these kernels that one of a compute unit's four SIMDs holds (120 registers)
 // Split of K over the waves of a workgroup: waves per tile, 8-word groups per wave, and how many groups the
 // kernel requests ahead of its first multiply (0: a streaming loop).
 struct FcPlan {
@@ -347,10 +348,12 @@ FcPlan fc_plan(const BgemmParams& p) {
     // busy, which is what binds (14 of its instructions to a product).  Four waves are taken all the same: they end at different times
     // and follow one another.  9216 inputs, 4096 outputs, batch 200: 9 waves in four rounds 13.6 us, 4 in one 9.3 (batch 128: 7.9 ->
     // 5.9, 384: 16.1 -> 12.2 with four waves in two rounds, 14.8 with two in one); 25088 -> 4096, batch 224: 27.0 -> 19.3;
-    // 32768 -> 512, batch 544: 16.0 -> 13.7; 16384 -> 2048, batch 256: 10.4 -> 8.9.
+    // 32768 -> 512, batch 544: 16.0 -> 13.7; 16384 -> 2048, batch 256: 10.4 -> 8.9.  A workgroup's waves are counted in fours,
+    // one to a SIMD: a fifth is a second wave of one SIMD, which then has as much again to do (513 .. 768 tiles with five waves,
+    // three workgroups a compute unit -> four waves, 35 layers: 0.75 .. 0.91 of the time; 8825 -> 3484, batch 212: 10.2 -> 8.3).
     const long long tiles = (long long)f.n_tiles * f.b_tiles;
     int kwaves = std::max(1, std::min(kMaxWaves, groups / 4));
-    while (kwaves > 4 && tiles > kCus * (kCuWaves / kwaves)) --kwaves;
+    while (kwaves > 4 && tiles > kCus * (kSimdWaves / ((kwaves + 3) / 4))) --kwaves;
     while (kwaves > 1 && tiles * kwaves > 8192) --kwaves;
     f.gpw = (groups + kwaves - 1) / kwaves;
     f.kwaves = (groups + f.gpw - 1) / f.gpw;

@@ -125,6 +125,14 @@ def test_large_products_only_where_their_sums_are_exact(out):
     assert "gemm_mfma" not in _fc_kernel(batch, (1 << 24) - 1, n, out)
 
 
+@pytest.mark.parametrize("batch,k,n,out,kernel", [
+    (212, 8825, 3484, False, "<0, 0, true>"), (94, 8794, 8046, True, "<1, 0, true>"),  # 763 and 756 tiles: nine groups a wave
+    (512, 8825, 1024, False, "<0, 7, true>"), (512, 8825, 1025, False, "<0, 0, true>")])  # 512 tiles: seven waves; 528
+def test_fc_layers_of_many_tiles_take_four_waves(batch, k, n, out, kernel):
+    """513 tiles and more: one wave to a SIMD, four workgroups to a compute unit; five waves leave a SIMD twice the work."""
+    assert _fc_kernel(batch, k, n, out) == "fc_mfma_f4_kernel" + kernel
+
+
 @pytest.mark.parametrize("frame,stride,served", [(1, 1, True), (2, 2, True), (5, 8, False), (3, 7, False)])
 def test_large_products_read_the_first_pixel(frame, stride, served):
     """One output pixel of a 1x1 filter is the frame's first one only without padding: ((5 + 8 - 5)/8 - 1)*8 + 1 - 5 = -4,

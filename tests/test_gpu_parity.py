@@ -217,6 +217,11 @@ def test_fc128_workgroups_at_once(gpu, b, k, n, name):
     fin.release()
 
 
+def test_out128_workgroups_at_once(gpu):
+    """Four waves a tile, nine groups each, the last with a part of them."""
+    test_out128(gpu, "mfma_f4", 94, 8794, 8046)
+
+
 @pytest.mark.parametrize("b,k,n,name", [
     (1, 100, 2000, "small_kernel<4>"), (16, 1537, 4096, "small_kernel<4>"),   # one wave and a part of a group; as many tiles as compute units
     (17, 8193, 1000, "small_kernel<4>"), (77, 25001, 520, "small_kernel<8>"),  # half a tile without neurons, images past the batch
