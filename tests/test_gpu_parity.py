@@ -83,9 +83,10 @@ def test_fc128_four_image_tiles(gpu, b, k, n):
     test_fc128(gpu, "mfma_f4", b, k, n)
 
 
-@pytest.mark.parametrize("b,k,n", [(5000, 2048, 3104), (4999, 2300, 3100)])
-def test_out128_four_image_tiles(gpu, b, k, n):
-    assert _large_product_kernel(gpu, b, k, n, out=True) == "gemm_mfma_f4_kernel<4, 1, false>"
+@pytest.mark.parametrize("b,k,n,tiles", [(5000, 2048, 3104, 4), (4999, 2300, 3101, 4), (8201, 300, 1002, 2), (4100, 129, 1039, 2)])
+def test_out128_large_products(gpu, b, k, n, tiles):
+    """Four values a request, at rows that begin at any word; runs of fewer than sixteen columns at the end."""
+    assert _large_product_kernel(gpu, b, k, n, out=True) == "gemm_mfma_f4_kernel<%d, 1, false>" % tiles
     test_out128(gpu, "mfma_f4", b, k, n)
 
 
