@@ -367,12 +367,15 @@ bool gemm_mfma_applicable(const BgemmParams& p) {
     // 32-bit buffer offsets: all rows' words, 64 columns' words
     if ((long long)p.cw * p.B * 4 >= (1LL << 31) || (long long)p.cw * 32 * kNT * 4 >= (1LL << 31)) return false;
     // Large enough to give every CU a workgroup with two image tiles per wave; smaller problems are bound by launch and fill and
-    // stay with the kernels written for them, but for int32 products of many 32 x 32 tiles and a long K (8 192 x 448 x 8 192
-    // 30.3 us there, 19.5 here; 200 x 8 192 x 8 192 24.6 / 17.0; 1 500 x 1 504 x 1 504 8.4 / 7.7; below the line 512 x 3 072 x 2 048
-    // 7.8 / 7.9, 2 048 x 1 024 x 1 024 6.2 / 6.8, 33 x 8 192 x 4 096 6.7 / 10.0).
+    // stay with the kernels written for them, but for int32 products that take those kernels' waves, one 32 x 32 tile each, more than
+    // one round of 1 024: the second one is as long as the first for however few tiles.  Two rounds from K = 3 840 on (332 x 4 224 x
+    // 3 872 10.8 us there, 10.5 here; 200 x 8 192 x 8 192 24.6 / 17.0; shorter ones 264 x 6 976 x 1 728 7.0 / 8.0, 2 450 x 608 x 2 592
+    // 8.3 / 9.2), more rounds at 100 000 words of tiles (8 192 x 448 x 8 192 30.3 / 19.5, 1 500 x 1 504 x 1 504 8.4 / 7.7, 2 433 x 1 312 x
+    // 1 696 10.4 / 8.8; below the line 1 812 x 1 312 x 864 6.3 / 6.8).  Over 800 products to either side of the lines none takes more
+    // than 3 % longer than with the other kernel.
     const long long wgs = (long long)((p.B + 32 * 2 * kWaves - 1) / (32 * 2 * kWaves)) * ((p.N + 32 * kNT - 1) / (32 * kNT));
     const long long tiles = (long long)((p.B + 31) / 32) * ((p.N + 31) / 32);
-    return wgs >= 256 || (p.mode == EPI_RAW && tiles >= 1200 && tiles * p.cw >= 100000);
+    return wgs >= 256 || (p.mode == EPI_RAW && ((tiles > 1024 && p.cw >= 120) || (tiles > 2048 && tiles * p.cw >= 100000)));
 }
 
 void gemm_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len) {

@@ -43,6 +43,8 @@ def test_bmm(gpu, variant, m, n, k):
 @pytest.mark.parametrize("m,n,k", [
     # few rows or columns and a long K: both sides of the line between the kernels for small and for large products
     (300, 4096, 4128), (257, 4128, 2624), (1220, 1056, 2624), (1184, 1024, 4096),
+    # (one tile more than a round, K on either side; two rounds and a few tiles more, words of tiles on either side)
+    (1025, 1024, 3840), (1025, 1024, 3808), (1024, 1024, 3840), (1472, 1440, 1568), (1472, 1440, 1504), (2048, 1024, 3808),
     # two and (the fourth and the last) four image tiles per wave: rows past the last one, a last column group of 32, rows of the
     # weights that are no whole 128-bit units (1 to 3 words more), K that ends with a block, after one group of k-steps, within one
     (3070, 2112, 1024), (3070, 2080, 1088), (2049, 3104, 544), (4095, 4064, 2080), (4097, 4096, 2528), (5000, 3104, 2112),
