@@ -206,7 +206,18 @@ bool conv1x1_mfma_applicable(const BgemmParams& p) {
     if ((p.cw != 2 && p.cw != 4 && p.cw != 8) || p.k_tap != 32 * p.cw || p.N % (32 * kNT) != 0 || p.bits_row_words != p.N / 32) return false;
     // windows inside the frame, and 32-bit offsets
     if ((p.PH - 1) * (long long)p.stride_h >= p.H || (p.PW - 1) * (long long)p.stride_w >= p.W) return false;
-    return (long long)p.PH * p.PW * p.B < (1LL << 30) && 4LL * p.H * p.W * p.cw * p.B < (1LL << 31);
+    // Int32 residuals, whose stores are nearly all of a launch: a persistent grid's waves drift apart and scatter the lines that they
+    // write, where bgemm_flat.hip's workgroups, dealt in order, keep together.  us, there -> here (MB of input and outputs): 256
+    // channels, 256 outputs at 21x21, batch 166 18.3 -> 15.3 (80 MB); from 120 MB on level within 5 %, even batches a little
+    // shorter, odd ones longer (192 outputs at 49x49, batch 69 25.3 -> 26.4, 137 MB); shorter again where the other launch has just
+    // left the 256 MiB memory-side cache (384 at 37x37, batch 136 68.7 -> 51.6, 301 MB); longer beyond (512 at 54x54, batch 185
+    // 245 -> 389).  Narrow residuals take 0.5 .. 0.9 of the time at all sizes to 1.5 GB.
+    const long long pixels = (long long)p.PH * p.PW * p.B;
+    if (p.res_out_fmt == TCBNN_RES_I32) {
+        const long long bytes = 4LL * p.N * pixels + 4LL * p.bits_row_words * pixels + 4LL * p.H * p.W * p.cw * p.B;
+        if (bytes > 120000000LL && (bytes < 268000000LL || bytes > 320000000LL)) return false;
+    }
+    return pixels < (1LL << 30) && 4LL * p.H * p.W * p.cw * p.B < (1LL << 31);
 }
 
 void conv1x1_mfma_kernel_name(const BgemmParams& p, char* buf, size_t len) {

@@ -147,6 +147,20 @@ def test_large_products_read_the_first_pixel(frame, stride, served):
     assert name.value.decode().startswith("gemm_mfma") == served, name.value
 
 
+@pytest.mark.parametrize("batch,frame,cout,fmt,kernel", [
+    (166, 21, 256, 0, "conv1x1"), (69, 49, 192, 0, "bgemm_flat"),                                    # 80 and 137 MB of int32
+    (136, 37, 384, 0, "conv1x1"), (185, 54, 512, 0, "bgemm_flat"), (185, 54, 512, 1, "conv1x1")])    # 301 MB; 1.1 GB, and in 16 bits
+def test_1x1_layers_with_large_int32_residuals(batch, frame, cout, fmt, kernel):
+    """Launches whose int32 stores a persistent grid would scatter go to the kernel whose workgroups are dealt in order."""
+    import ctypes as C
+    from tcbnn_amd import _lib
+    d = _lib.Conv128Desc(1, 1, 1, 1, None, 16, frame, frame, 256, 1, 1, cout, batch, 1, 1, 1, 1, 1, 0, 1, 0, 0, 0, 0,
+                         _lib.VARIANT_MFMA_F4, 0, fmt, 0)
+    name = C.create_string_buffer(128)
+    _lib.check(_lib.lib.tcbnn_conv128_kernel_name(C.byref(d), name, 128))
+    assert name.value.decode().startswith(kernel), name.value
+
+
 def _device_kernels():
     """Name -> record of every kernel in the library, as its code objects describe them (their AMDGPU metadata notes)."""
     import struct
