@@ -610,7 +610,8 @@ bool bgemm_flat_applicable(const BgemmParams& p) {
 // Both kernels serve the 3x3 layers of conv3x3_mfma.hip: which is faster?  An estimate of both launches in microseconds,
 // fitted to 623 measured pairs (all layers of five networks at batch 1 .. 200, and int32 convolutions with 64 .. 512
 // input channels, 64 .. 512 output channels, 8 x 8 .. 56 x 56 pixels, batch 2 .. 200): choosing by it costs 0.5 % over
-// choosing by measurement, always taking the persistent kernel 20 %.
+// choosing by measurement, always taking the persistent kernel 20 %.  (Measured with eight waves to a large workgroup and the
+// image tiles of conv3x3_mfma_image_tiles: where the persistent kernel has got faster since, the estimate charges it too much.)
 bool bgemm_flat_preferred(const BgemmParams& p) {
     if (!conv3x3_mfma_applicable(p) || !bgemm_flat_applicable(p)) return false;
     const double steps = 9.0 * p.cw / 2, pix = (double)p.PH * p.PW, n_tiles = (p.N + 31) / 32;

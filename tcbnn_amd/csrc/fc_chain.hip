@@ -284,7 +284,8 @@ __global__ __launch_bounds__(64 * kWaves) void fc_chain_kernel(const ChainArgs a
 bool fits(int batch, int k, int n) { return batch > 0 && k > 0 && n > 0 && k <= kMaxWidth && n <= kMaxWidth; }
 
 // Whether one launch is faster than one per layer, by what it saves (us), fitted to both sides' times of 380 runs (1 to 5 layers,
-// 10 to 2048 wide, batch 1 to 16384, launched on end).  A launch of its own costs a layer 1.75 us more than its share of this one, the
+// 10 to 2048 wide, batch 1 to 16384, launched on end; the layers' own launches have got faster since, with tiles of 16 x 16 and
+// large outputs four values a request).  A launch of its own costs a layer 1.75 us more than its share of this one, the
 // input's signs 0.7 and more where there is more to read, and this launch has 3.6 of its own.  A workgroup does a layer's products
 // for its 32 images on one compute unit, 1.85 us longer for 1024 x 1024 of them than all units together where there are few images, and
 // less where there are many; a layer of 4096 tiles or more is 2.4 us slower by itself; an output layer stores a number at a

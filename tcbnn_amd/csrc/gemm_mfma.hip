@@ -14,7 +14,7 @@
 //               addressing (a per-lane constant offset, the k-step in the scalar offset), eight k-steps ahead of their use.
 // Bound by the matrix pipe and by power: with operands like these the MFMA alone reaches 8.1 P (constants: 9.8), this kernel 5.8
 // on 8 192^3, of whose time a tenth is the output's.  Before (a row of the weights per lane, a request per image tile, one block
-// size): 8 192^3 214 us, 5 000 x 3 104 x 7 200 69, 3 072 x 3 072 x 8 192 51, 1 500 x 8 192 x 4 096 31.8; now 190, 56.5, 38.2, 25.0.
+// size): 8 192^3 223 us, 5 000 x 3 104 x 7 200 59, 3 072 x 3 072 x 8 192 53, 1 500 x 8 192 x 4 096 31.4; now 189, 47.4, 37.4, 24.0.
 // Operand roles, fragment order and the accumulator layout are those of bgemm_mfma.hip.
 #include "common.h"
 #include "mfma_util.h"
@@ -339,9 +339,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
 }
 
 // Image tiles per wave: two, whose smaller workgroups leave less of a last round empty and of which a compute unit runs three
-// (3 072 x 3 072 x 8 192 39.5 us against 45.0 with four, 8 000 x 2 080 x 6 016 51.8 / 56.9, 1 500 x 8 192 x 4 096 26.2 / 28.7); four, which multiply
+// (3 072 x 3 072 x 8 192 37.4 us against 44.3 with four, 8 000 x 2 080 x 6 016 48.0 / 54.6, 1 500 x 8 192 x 4 096 24.0 / 27.5); four, which multiply
 // every weight fragment twice as often, where they come out even over the compute units, at two workgroups in each or more,
-// and K is long (5 000 x 3 104 x 7 200 62 us with two, 58.6 with four; 8 192^3 217 / 201; 8 192 x 8 192 x 512 45.0 / 48.2).
+// and K is long (5 000 x 3 104 x 7 200 49.0 us with two, 47.3 with four; 8 192^3 200 / 184; 8 192 x 8 192 x 512 45.2 / 48.2).  Over 66
+// products the pick is at most 2.4 % slower than the other number of tiles.
 int gemm_mt(const BgemmParams& p) {
     constexpr int kCus = 256, kLongK = 64;  // (words)
     const long long n_groups = (p.N + 32 * kNT - 1) / (32 * kNT);
